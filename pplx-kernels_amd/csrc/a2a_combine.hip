@@ -88,31 +88,93 @@ __device__ __forceinline__ void gather_group(f32x8 (&acc)[VPL], uint64_t row_of_
   }
 }
 
+// What one wave of combine_gather adds up and where the sum goes.  Lane `base + k` holds the row
+// and the weight of pick k; `base` differs between the members of a DP group only.
+template <typename T, typename U, int KB, int VPL>
+__device__ __forceinline__ void reduce_row(const WorldDev &w, uint64_t row, float weight, uint32_t base,
+                                           bool all_rows, uint32_t segment, uint64_t out_of_lane,
+                                           uint64_t out_lanes) {
+  const uint32_t lane = lane_id();
+  const uint32_t nvec = w.H / 8;
+  const uint32_t K = w.K;
+  uint32_t vec_ld[VPL];
+  f32x8 acc[VPL];
+#pragma unroll
+  for (int v = 0; v < VPL; ++v) {
+    const uint32_t vec = (segment * VPL + v) * kWave + lane;
+    vec_ld[v] = vec < nvec ? vec : nvec - 1;  // clamp: loads stay unconditional
+    acc[v] = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  }
+  if (!all_rows) {
+    // A pick without a row (bad expert id or slot) contributes nothing.
+    for (uint32_t k = 0; k < K; ++k) {
+      if (read_lane64(row, base + k) != 0) gather_group<T, 1, VPL>(acc, row, weight, base + k, vec_ld);
+    }
+  } else {
+    uint32_t k = 0;
+    for (; k + KB <= K; k += KB) gather_group<T, KB, VPL>(acc, row, weight, base + k, vec_ld);
+    if constexpr (KB > 4) {
+      if ((K - k) & 4) { gather_group<T, 4, VPL>(acc, row, weight, base + k, vec_ld); k += 4; }
+    }
+    if constexpr (KB > 2) {
+      if ((K - k) & 2) { gather_group<T, 2, VPL>(acc, row, weight, base + k, vec_ld); k += 2; }
+    }
+    if constexpr (KB > 1) {
+      if ((K - k) & 1) { gather_group<T, 1, VPL>(acc, row, weight, base + k, vec_ld); }
+    }
+  }
+  for (; out_lanes != 0; out_lanes &= out_lanes - 1) {
+    U *out = reinterpret_cast<U *>(read_lane64(out_of_lane, (uint32_t)__builtin_ctzll(out_lanes)));
+#pragma unroll
+    for (int v = 0; v < VPL; ++v) {
+      const uint32_t vec = (segment * VPL + v) * kWave + lane;
+      if (vec < nvec) Store8<U>::at(out, vec, acc[v]);
+    }
+  }
+}
+
 // One wave owns VPL * 64 consecutive 8-element vectors of one output row (VPL KiB of a bf16
 // row) and takes the picks KB at a time, so KB * VPL row loads per lane are in flight: few
 // picks read long pieces of their rows, many picks shorter ones.
-template <typename T, typename U, class CT, int KB, int VPL>
-__global__ __launch_bounds__(256) void combine_gather(WorldDev w, CT tab, uint32_t segments, FastDiv by_segments,
-                                                      uint32_t first_rank, uint32_t rank_count) {
+//
+// GROUPED (DP groups of several ranks, dp * K <= 64): the members of a group hold the same
+// tokens, so the rows they gather are the same ones.  A wave then serves the token for all
+// members: lane i * K + k resolves pick k of member i, and members whose rows and weights agree
+// with those of the first present member (compared bit for bit, token by token: the operator
+// takes every rank's own indices and weights) share one gather and only store apart.  What is
+// bound by the gathered bytes moves up to dp times fewer of them: 8 ranks in groups of four, 3001
+// tokens of fp32 rows, 2880 wide, top-5: 150 us with a gather per rank, 54 us with one per
+// group (242 MB at 4.5 TB/s); groups of two, 4 x 128 bf16 tokens, 7168 wide, top-8: 16.5 and 15.0
+// us (the second gather of a step this small hits the last-level cache).
+template <typename T, typename U, class CT, int KB, int VPL, bool GROUPED>
+__global__ __launch_bounds__(256) void combine_gather(WorldDev w, CT tab, uint32_t segments, FastDiv by_segments) {
   const uint32_t lane = lane_id();
   const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / kWave) +
                                                        threadIdx.x / kWave);
   const uint32_t token = fast_div(wave, by_segments);
   const uint32_t segment = wave - token * segments;
-  const uint32_t r_local = group_of(w, token);
-  const uint32_t t = token - r_local * w.M;
-  if (r_local >= rank_count) return;
-  const uint32_t r = first_rank + r_local;
-  const CombineRank &c = tab.at(r);
-  if (t >= combine_rank_tokens(w, c)) return;
+  const uint32_t owner_index = group_of(w, token);  // the rank, or the DP group when GROUPED
+  const uint32_t t = token - owner_index * w.M;
+  if (owner_index >= (GROUPED ? w.G : w.R)) return;
+  const uint32_t member = GROUPED ? fast_div(lane, w.by_K) : 0;
+  const uint32_t pick = lane - member * w.K;
+  const bool has_pick = GROUPED ? member < w.dp : lane < w.K;
+  const uint32_t g = GROUPED ? owner_index : fast_div(owner_index, w.by_dp);
+  const CombineRank &c = tab.at(GROUPED ? g * w.dp + (has_pick ? member : 0) : owner_index);
+  bool present = t < combine_rank_tokens(w, c);
+  if constexpr (!GROUPED) {
+    if (!present) return;
+  }
+  present = present && has_pick;
+  if (GROUPED && __builtin_amdgcn_ballot_w64(present) == 0) return;
 
-  // Lane k resolves pick k: no LDS, no barrier.
-  uint64_t row = 0;
+  // Lane k (of its member) resolves pick k: no LDS, no barrier.
+  uint64_t row = 0, out = 0;
   float weight = 0.f;
-  if (lane < w.K) {
-    const uint32_t e = as_global(c.indices)[(size_t)t * w.K + lane];
-    const uint32_t slot = as_global(w.slot_map)[((size_t)fast_div(r, w.by_dp) * w.M + t) * w.K + lane];
-    weight = as_global(c.weights)[(int64_t)t * c.w_stride_row + lane];
+  if (present) {
+    const uint32_t e = as_global(c.indices)[(size_t)t * w.K + pick];
+    const uint32_t slot = as_global(w.slot_map)[((size_t)g * w.M + t) * w.K + pick];
+    weight = as_global(c.weights)[(int64_t)t * c.w_stride_row + pick];
     if (e < w.E && slot != kInvalidSlot) {
       const CombineRank &owner = tab.at(owner_of(w, e));
       if (slot < owner.y_rows) {
@@ -124,65 +186,54 @@ __global__ __launch_bounds__(256) void combine_gather(WorldDev w, CT tab, uint32
       }
     }
   }
-  const bool all_rows = __builtin_amdgcn_ballot_w64(lane < w.K && row == 0) == 0;
-
-  U *out = reinterpret_cast<U *>(c.out_tokens) + (int64_t)t * c.out_stride_row;
-  const uint32_t nvec = w.H / 8;
-  const uint32_t K = w.K;
-  if (!all_rows) {
-    // A pick without a row (bad expert id or slot) contributes nothing.
-    for (int v = 0; v < VPL; ++v) {
-      const uint32_t vec = (segment * VPL + v) * kWave + lane;
-      const uint32_t one[1] = {vec < nvec ? vec : nvec - 1};
-      f32x8 acc[1] = {{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
-      for (uint32_t k = 0; k < K; ++k) {
-        if (read_lane64(row, k) != 0) gather_group<T, 1, 1>(acc, row, weight, k, one);
+  if (has_pick) out = reinterpret_cast<uint64_t>(reinterpret_cast<U *>(c.out_tokens) + (int64_t)t * c.out_stride_row);
+  const uint64_t no_row = __builtin_amdgcn_ballot_w64(present && row == 0);
+  if constexpr (!GROUPED) {
+    reduce_row<T, U, KB, VPL>(w, row, weight, 0, no_row == 0, segment, out, 1ull);
+  } else {
+    const uint64_t heads = __builtin_amdgcn_ballot_w64(present && pick == 0);  // one lane per present member
+    for (uint64_t todo = heads; todo != 0;) {
+      const uint32_t base = (uint32_t)__builtin_ctzll(todo);
+      // members that want the same sum: every pick's row and weight as this member's
+      const int src = (int)((base + pick) & (kWave - 1));
+      const bool same = __shfl((uint32_t)row, src, kWave) == (uint32_t)row &&
+                        __shfl((uint32_t)(row >> 32), src, kWave) == (uint32_t)(row >> 32) &&
+                        __shfl(__float_as_uint(weight), src, kWave) == __float_as_uint(weight);
+      const uint64_t differs = __builtin_amdgcn_ballot_w64(present && !same);
+      uint64_t outs = 0;
+      const uint64_t picks = w.K == kWave ? ~0ull : (1ull << w.K) - 1;
+      for (uint64_t rest = todo; rest != 0; rest &= rest - 1) {
+        const uint32_t head = (uint32_t)__builtin_ctzll(rest);
+        if (((differs >> head) & picks) == 0) outs |= 1ull << head;
       }
-      if (vec < nvec) Store8<U>::at(out, vec, acc[0]);
+      reduce_row<T, U, KB, VPL>(w, row, weight, base, ((no_row >> base) & picks) == 0, segment, out, outs);
+      todo &= ~outs;
     }
-    return;
-  }
-  uint32_t vec_ld[VPL];
-  f32x8 acc[VPL];
-#pragma unroll
-  for (int v = 0; v < VPL; ++v) {
-    const uint32_t vec = (segment * VPL + v) * kWave + lane;
-    vec_ld[v] = vec < nvec ? vec : nvec - 1;  // clamp: loads stay unconditional
-    acc[v] = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  }
-  uint32_t k = 0;
-  for (; k + KB <= K; k += KB) gather_group<T, KB, VPL>(acc, row, weight, k, vec_ld);
-  if constexpr (KB > 4) {
-    if ((K - k) & 4) { gather_group<T, 4, VPL>(acc, row, weight, k, vec_ld); k += 4; }
-  }
-  if constexpr (KB > 2) {
-    if ((K - k) & 2) { gather_group<T, 2, VPL>(acc, row, weight, k, vec_ld); k += 2; }
-  }
-  if constexpr (KB > 1) {
-    if ((K - k) & 1) { gather_group<T, 1, VPL>(acc, row, weight, k, vec_ld); }
-  }
-#pragma unroll
-  for (int v = 0; v < VPL; ++v) {
-    const uint32_t vec = (segment * VPL + v) * kWave + lane;
-    if (vec < nvec) Store8<U>::at(out, vec, acc[v]);
   }
 }
 
 template <typename T, typename U, class CT, int KB, int VPL>
-int launch_combine_v(const WorldDev &w, const CT &tab, uint32_t first_rank, uint32_t rank_count, hipStream_t s) {
+int launch_combine_v(const WorldDev &w, const CT &tab, bool grouped, hipStream_t s) {
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
   const uint32_t segments = (nvec_segments + VPL - 1) / VPL;
-  const uint64_t waves = (uint64_t)rank_count * w.M * segments;
+  const uint64_t waves = (uint64_t)(grouped ? w.G : w.R) * w.M * segments;
   const dim3 grid((uint32_t)((waves + 3) / 4)), block(256);
-  hipLaunchKernelGGL((combine_gather<T, U, CT, KB, VPL>), grid, block, 0, s, w, tab, segments,
-                     make_fast_div(segments), first_rank, rank_count);
+  if (grouped) {
+    hipLaunchKernelGGL((combine_gather<T, U, CT, KB, VPL, true>), grid, block, 0, s, w, tab, segments,
+                       make_fast_div(segments));
+  } else {
+    hipLaunchKernelGGL((combine_gather<T, U, CT, KB, VPL, false>), grid, block, 0, s, w, tab, segments,
+                       make_fast_div(segments));
+  }
   return (int)hipGetLastError();
 }
 
 template <typename T, typename U, class CT>
-int launch_combine_k(const WorldDev &w, const CT &tab, uint32_t first_rank, uint32_t rank_count, hipStream_t s) {
-#define PPLX_COMBINE(KB, VPL) \
-  return launch_combine_v<T, U, CT, KB, VPL>(w, tab, first_rank, rank_count, s)
+int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
+#define PPLX_COMBINE(KB, VPL) return launch_combine_v<T, U, CT, KB, VPL>(w, tab, grouped, s)
+  // DP groups of several ranks gather once per group as long as a wave has a lane for every
+  // member's pick; beyond that (no routing in use comes near) every rank gathers for itself.
+  const bool grouped = w.dp > 1 && w.dp * w.K <= kWave;
   // Few picks: long pieces of each row, all picks at once.  Many picks: all of them at once,
   // 1 KiB of each (eight loads per lane in flight either way) -- except for steps of a few
   // hundred to two thousand tokens, whose waves are all resident at the same moment: there the
@@ -190,7 +241,7 @@ int launch_combine_k(const WorldDev &w, const CT &tab, uint32_t first_rank, uint
   // (8 x 128 DSv3 tokens, top-8: 23.4 us against 25.3 us; 8 x 256: 45.8 against 46.8; from
   // 8 x 512 on the wide form wins, 88.7 against 91.5 us, and below 8 x 64 too).
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
-  const uint64_t tokens = (uint64_t)rank_count * w.M;
+  const uint64_t tokens = (uint64_t)(grouped ? w.G : w.R) * w.M;
   if (w.K > 4 && tokens > 384 && tokens <= 2048 && nvec_segments >= 7) {
     if (nvec_segments % 7 == 0) PPLX_COMBINE(1, 7);
     PPLX_COMBINE(1, 8);
@@ -205,16 +256,15 @@ int launch_combine_k(const WorldDev &w, const CT &tab, uint32_t first_rank, uint
 }
 
 template <class CT>
-int launch_combine_t(const WorldDev &w, const CT &tab, int in_dtype, int out_dtype, hipStream_t s,
-                     uint32_t first_rank, uint32_t rank_count) {
+int launch_combine_t(const WorldDev &w, const CT &tab, int in_dtype, int out_dtype, hipStream_t s) {
   // dtype codes follow pplx_a2a_dtype: 0 = f32, 1 = bf16, 2 = f16.
   switch (in_dtype * 4 + out_dtype) {
-    case 0 * 4 + 1: return launch_combine_k<float, __bf16>(w, tab, first_rank, rank_count, s);
-    case 0 * 4 + 2: return launch_combine_k<float, _Float16>(w, tab, first_rank, rank_count, s);
-    case 1 * 4 + 1: return launch_combine_k<__bf16, __bf16>(w, tab, first_rank, rank_count, s);
-    case 1 * 4 + 2: return launch_combine_k<__bf16, _Float16>(w, tab, first_rank, rank_count, s);
-    case 2 * 4 + 1: return launch_combine_k<_Float16, __bf16>(w, tab, first_rank, rank_count, s);
-    case 2 * 4 + 2: return launch_combine_k<_Float16, _Float16>(w, tab, first_rank, rank_count, s);
+    case 0 * 4 + 1: return launch_combine_k<float, __bf16>(w, tab, s);
+    case 0 * 4 + 2: return launch_combine_k<float, _Float16>(w, tab, s);
+    case 1 * 4 + 1: return launch_combine_k<__bf16, __bf16>(w, tab, s);
+    case 1 * 4 + 2: return launch_combine_k<__bf16, _Float16>(w, tab, s);
+    case 2 * 4 + 1: return launch_combine_k<_Float16, __bf16>(w, tab, s);
+    case 2 * 4 + 2: return launch_combine_k<_Float16, _Float16>(w, tab, s);
     default: return (int)hipErrorInvalidValue;
   }
 }
@@ -224,8 +274,8 @@ int launch_combine_t(const WorldDev &w, const CT &tab, int in_dtype, int out_dty
 int launch_combine(const WorldDev &w, const CombineRank *inline_rows, int in_dtype, int out_dtype,
                    void *stream) {
   if (inline_rows)
-    return launch_combine_t(w, make_inline(w, inline_rows), in_dtype, out_dtype, (hipStream_t)stream, 0, w.R);
-  return launch_combine_t(w, HbmCombine{w.crank}, in_dtype, out_dtype, (hipStream_t)stream, 0, w.R);
+    return launch_combine_t(w, make_inline(w, inline_rows), in_dtype, out_dtype, (hipStream_t)stream);
+  return launch_combine_t(w, HbmCombine{w.crank}, in_dtype, out_dtype, (hipStream_t)stream);
 }
 
 }  // namespace pplx_amd

@@ -212,16 +212,16 @@ void fill_geometry(const pplx_a2a_config_t &cfg, WorldDev &d) {
   d.by_dp = make_fast_div(d.dp);
   d.by_L = make_fast_div(d.L);
   d.by_K = make_fast_div(d.K);
-  // Routing tiles of a whole step: small enough that a step has a few hundred of them (a tile
-  // is one workgroup, and routing is a chain of short launches that only parallelism shortens),
-  // at most 16 chunks of 64 tokens, and such that the LDS tables fit 64 KiB.
+  // Routing tiles of a whole step: 64-token chunks while a step has at most kScanFreeTiles of
+  // them, then as many chunks per tile as keep it there (the tiles' counts of an expert stay one
+  // cache line and need no scan), at most 16, and such that the LDS tables fit 64 KiB.
   const uint64_t step_chunks = ((uint64_t)d.G * d.M + kWave - 1) / kWave;
-  // A step of up to 1024 tokens is a single tile (one launch instead of three).
+  // A step of up to 1024 tokens is a single tile (one launch instead of two).
   d.tile_chunks = 1;
   if (step_chunks <= 16) {
     while (d.tile_chunks < step_chunks) d.tile_chunks *= 2;
   } else {
-    while (d.tile_chunks < 16 && step_chunks / d.tile_chunks > 256) d.tile_chunks *= 2;
+    while (d.tile_chunks < 16 && step_chunks > (uint64_t)kScanFreeTiles * d.tile_chunks) d.tile_chunks *= 2;
   }
   while (d.tile_chunks > 1 && route_lds_bytes(d.E, d.tile_chunks) > 65536u) d.tile_chunks /= 2;
   const uint64_t tile_tokens = (uint64_t)d.tile_chunks * kWave;

@@ -102,24 +102,33 @@ struct WorldDev {
   FastDiv by_M, by_dp, by_L, by_K;  // fast_div(n, by_X) == n / X
   DispatchRank *drank;   // [R]
   CombineRank *crank;    // [R]
-  uint32_t *tile_cnt;    // [num_tiles][E] tokens routed to e inside a tile; after route_scan the
-                         // tokens routed to e in all earlier tiles.  Behind it (route_tables):
-                         // [num_tiles * tile_chunks][E] 64-bit masks, one bit per token of a chunk
+  uint32_t *tile_cnt;    // tokens routed to each expert inside each tile, and behind them
+                         // (route_tables) [num_tiles * tile_chunks][E] 64-bit masks, one bit per
+                         // token of a chunk
   uint32_t *slot_map;    // [G * M][K] row of (token, pick) inside its expert
   uint32_t *faults;      // [1] sticky fault bits
 };
 
-// The routing scratch of a world is one block: the tiles' counts, then the chunks' masks.
+// The routing scratch of a world is one block: the tiles' counts, the chunks' masks, and for each
+// chunk the rows of its tile's earlier chunks.  The counts have one of two forms.  Steps of up to
+// kScanFreeTiles tiles keep them expert-major, 16 bits each (a tile holds at most 1024 tokens):
+// the kScanFreeTiles counts of an expert are one 128-byte line, short enough for whoever wants a
+// prefix of it to add it up.  Longer steps keep [num_tiles][E] 32-bit counts, which route_scan
+// turns into prefixes.
+constexpr uint32_t kScanFreeTiles = 64;
 struct RouteTables {
-  uint64_t mask_offset, bytes;
+  uint64_t mask_offset, base_offset, bytes;
 };
 #ifdef __HIPCC__
 __host__ __device__
 #endif
 inline RouteTables route_tables(uint32_t num_tiles, uint32_t tile_chunks, uint32_t experts) {
   RouteTables t;
-  t.mask_offset = ((uint64_t)num_tiles * experts * 4u + 7u) & ~7ull;
-  t.bytes = t.mask_offset + (uint64_t)num_tiles * tile_chunks * experts * 8u;
+  const uint64_t chunks = (uint64_t)num_tiles * tile_chunks;
+  const uint64_t scanned = (uint64_t)num_tiles * experts * 4u, rows = (uint64_t)experts * kScanFreeTiles * 2u;
+  t.mask_offset = ((scanned > rows ? scanned : rows) + 127u) & ~127ull;
+  t.base_offset = t.mask_offset + chunks * experts * 8u;
+  t.bytes = t.base_offset + chunks * experts * 2u;
   return t;
 }
 
@@ -129,10 +138,12 @@ struct RouteSpan {
   uint32_t v_count;       // virtual tokens covered
   uint32_t tile_chunks;   // 64-token chunks per tile (one workgroup)
   uint32_t pick_vector;   // expert ids one load may fetch (4, 2 or 1)
-  uint32_t *tile_cnt;     // [tiles][E]
+  uint32_t *tile_cnt;     // [tiles][E], scanned form; NULL: the counts go to tile_row
+  uint16_t *tile_row;     // [E][kScanFreeTiles], the form that needs no scan
   unsigned long long *tile_mask;  // [tiles * tile_chunks][E] route_count keeps the chunks' masks
                                   // here (and reports the faults) when set: the scatter that
                                   // follows works the slots out by itself
+  uint16_t *chunk_base;   // [tiles * tile_chunks][E], beside tile_mask: rows of the tile's earlier chunks
   uint32_t *slot_out;     // [G * M][K], indexed by absolute virtual token
 };
 
@@ -184,12 +195,12 @@ inline StageLayout stage_layout(uint32_t row_bytes, uint32_t scales, uint64_t to
 // arguments each.
 constexpr uint32_t kInlineRanks = 64;
 constexpr uint32_t kBindBatch = 64;
-// Steps of at most this many virtual tokens (DP groups x max_num_tokens) dispatch in one fused
-// launch.
-constexpr uint32_t kFusedMaxTokens = 3072;
 // A fused launch whose rows (all picks of all tokens) stay within this many bytes stores them
 // write-through into the 256 MB last-level cache instead of streaming them past it.
 constexpr uint64_t kWriteThroughMaxBytes = 192ull << 20;
+// Up to this many bytes of rows the fused launch is the faster one also for steps of many tokens
+// (dispatch_is_fused).
+constexpr uint64_t kFusedMaxBytes = 112ull << 20;
 
 // Device memory that pplx_a2a_static_step works in instead of a world's allocations: a fixed
 // array inside the library's code object (a2a_static.hip), one copy per GPU.

@@ -9,10 +9,11 @@
 //
 //   route_count      per routing tile: 64-token bitmasks per expert in LDS -> rows per
 //                    expert of the tile, and the masks themselves          (only if > 1 tile)
-//   route_scan       per expert: prefix of the tiles' rows, totals         (only if > 1 tile)
+//   route_scan       per expert: prefix of the tiles' rows, totals         (only if > 64 tiles)
 //   dispatch_scatter_slots  one wave per token (or per share of its K picks): the row is
 //                    read once into registers, lane k works the slot of pick k out of the
-//                    scanned rows and the masks, the row is stored K times, 16 B / lane
+//                    tiles' rows and the masks, the row is stored K times, 16 B / lane
+//                    (dispatch_scatter_scanned behind route_scan)
 //   route_slots + dispatch_scatter  the same with the slots written by a launch of their
 //                    own (single tile, rows beyond the register variants)
 //   dispatch_fused   small steps: routing and scatter in one launch; every
@@ -75,14 +76,18 @@ __global__ __launch_bounds__(256) void bind_rows(Row *table, Batch b) {
   }
 }
 
-// One wave per token (or per share of its picks).  ROUTED: the slot map was written by
-// route_slots; otherwise the wave works its token's slots out of the routing tables
-// (slots_from_masks) and writes the slot map itself.
-template <int NV, bool EXACT, class DT, bool ROUTED>
-__device__ __forceinline__ void scatter_token(const WorldDev &w, const DT &tab, uint32_t ksplit, uint32_t kper) {
+// Where a scatter wave gets its token's slots from.
+enum class Slots {
+  kMap,      // the slot map, which route_slots wrote
+  kScanned,  // the routing tables behind route_scan (the wave writes the slot map)
+  kTables,   // the routing tables as route_count left them (the same)
+};
+
+// One wave per token (or per share of its picks).
+template <int NV, bool EXACT, class DT, Slots SLOTS>
+__device__ __forceinline__ void scatter_token(const WorldDev &w, const DT &tab, uint32_t wave, uint32_t ksplit,
+                                              uint32_t kper) {
   const uint32_t lane = lane_id();
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / kWave) +
-                                                       threadIdx.x / kWave);
   const uint32_t v = wave >> __builtin_ctz(ksplit);  // (ksplit is a power of two)
   const uint32_t part = wave - v * ksplit;
   const uint32_t g = group_of(w, v);
@@ -90,23 +95,20 @@ __device__ __forceinline__ void scatter_token(const WorldDev &w, const DT &tab, 
   if (g >= w.G) return;
   if (t >= dispatch_group_tokens(w, tab, g)) return;
   const DispatchRank &src = tab.at(sender_of(w, g, t));
+  // The picks go out first: loads return in order, so what depends on them (the experts' buffers
+  // and the routing tables) is fetched while the row is still on its way.
+  const uint32_t e = lane < w.K ? as_global(src.indices)[(size_t)t * w.K + lane] : w.E;
   RowRegs<NV> regs;
   load_row<NV, EXACT>(w, src, t, lane, regs);
-  Destination dst;
-  if constexpr (ROUTED) {
-    if (lane < w.K) {
-      dst = resolve_destination(w, tab, as_global(src.indices)[(size_t)t * w.K + lane],
-                                as_global(w.slot_map)[(size_t)v * w.K + lane],
-                                part == 0);
-    }
+  ExpertBuffer buffer = expert_buffer(w, tab, e);
+  uint32_t slot = kInvalidSlot;
+  if constexpr (SLOTS == Slots::kMap) {
+    if (lane < w.K && e < w.E) slot = as_global(w.slot_map)[(size_t)v * w.K + lane];
   } else {
-    const uint32_t e = lane < w.K ? as_global(src.indices)[(size_t)t * w.K + lane] : w.E;
-    const uint32_t slot = slots_from_masks(w, v, lane, e);
-    if (lane < w.K) {
-      dst = resolve_destination(w, tab, e, slot, part == 0);
-      if (part == 0) as_global(w.slot_map)[(size_t)v * w.K + lane] = slot;
-    }
+    slot = slots_from_tables<SLOTS == Slots::kScanned>(w, v, lane, e);
+    if (lane < w.K && part == 0) as_global(w.slot_map)[(size_t)v * w.K + lane] = slot;
   }
+  const Destination dst = destination_of(w, buffer, slot, part == 0);
   const uint32_t k0 = part * kper;
   const uint32_t k1 = (k0 + kper < w.K) ? k0 + kper : w.K;
   // Rows stream past the caches; the 4-byte-per-lane scale rows are written through into the
@@ -118,13 +120,24 @@ __device__ __forceinline__ void scatter_token(const WorldDev &w, const DT &tab, 
 // Launched as one-wave workgroups whose dynamic LDS size caps how many of them a CU holds at a
 // time (see launch_scatter_t); the kernels themselves do not touch LDS.
 template <int NV, bool EXACT, class DT>
-__global__ __launch_bounds__(256) void dispatch_scatter(WorldDev w, DT tab, uint32_t ksplit, uint32_t kper) {
-  scatter_token<NV, EXACT, DT, true>(w, tab, ksplit, kper);
+__global__ __launch_bounds__(kWave) void dispatch_scatter(WorldDev w, DT tab, uint32_t ksplit, uint32_t kper) {
+  scatter_token<NV, EXACT, DT, Slots::kMap>(w, tab, blockIdx.x, ksplit, kper);
 }
 
 template <int NV, bool EXACT, class DT>
-__global__ __launch_bounds__(256) void dispatch_scatter_slots(WorldDev w, DT tab, uint32_t ksplit, uint32_t kper) {
-  scatter_token<NV, EXACT, DT, false>(w, tab, ksplit, kper);
+__global__ __launch_bounds__(kWave) void dispatch_scatter_scanned(WorldDev w, DT tab, uint32_t ksplit, uint32_t kper) {
+  scatter_token<NV, EXACT, DT, Slots::kScanned>(w, tab, blockIdx.x, ksplit, kper);
+}
+
+// The first ceil(E / 8) workgroups write the experts' totals.
+template <int NV, bool EXACT, class DT>
+__global__ __launch_bounds__(kWave) void dispatch_scatter_slots(WorldDev w, DT tab, uint32_t ksplit, uint32_t kper) {
+  const uint32_t totals = (w.E + 7) / 8;
+  if (blockIdx.x < totals) {
+    write_totals(w, tab, blockIdx.x, lane_id());
+    return;
+  }
+  scatter_token<NV, EXACT, DT, Slots::kTables>(w, tab, blockIdx.x - totals, ksplit, kper);
 }
 
 // Threads of a dispatch_fused workgroup: 16 waves (fewer, larger workgroups repeat less
@@ -315,7 +328,7 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   Destination dst;
   if (my_in_range && lane < w.K) {
     const size_t pair = (size_t)my_v * w.K + lane;
-    if (my_live) dst = resolve_destination(w, rows(), my_e, my_slot, my_part == 0);
+    if (my_live) dst = destination_of(w, expert_buffer(w, rows(), my_e), my_slot, my_part == 0);
     if (my_live && my_part == 0) {
       as_global(w.slot_map)[pair] = my_slot;
       if (my_e >= w.E) {
@@ -422,35 +435,44 @@ uint32_t fused_lds_bytes(const WorldDev &w, bool inline_table) {
   return table + 2u * w.E * (uint32_t)sizeof(uint32_t);
 }
 
-// Number of waves a row's K copies are spread over: few tokens -> more waves,
-// so that the launch still covers the 256 CUs (the row re-reads hit L2).
+// Number of waves a row's K copies are spread over (the row's re-reads hit L2).  Steps of one
+// routing tile need them to cover the 256 CUs.  Larger ones split only what leaves each wave long
+// runs of stores (8 ranks, us at one / two / four waves per token: 14 KiB rows, top-8, 1280 tokens
+// 38.8 / 36.4 / 38.6; 7 KiB rows, top-8, 2048 tokens 29.9 / 29.8 / 35.2; 4 KiB rows, top-8, 3072 tokens
+// 25.1 / 28.3 / 30.6; 8 KiB rows, top-2, 3072 tokens 18.1 / 20.4 / 30.6).
 uint32_t pick_ksplit(const WorldDev &w, uint32_t max_split) {
   const uint64_t tokens = (uint64_t)w.G * w.M;
+  const uint64_t stored = w.K * (w.Hb + 4ull * w.S);
   uint32_t ksplit = 1;
-  while (ksplit < max_split && ksplit < w.K && tokens * ksplit < 4096) ksplit *= 2;
+  while (ksplit < max_split && ksplit < w.K && tokens * ksplit < 4096 &&
+         (w.num_tiles == 1 || stored / (2 * ksplit) >= 48 * 1024)) ksplit *= 2;
   return ksplit;
 }
 
 // Scatter waves a CU should hold at a time (0 = as many as fit).
-// Measured on 8 x 4096 tokens with the slots worked out by the scatter's waves
-// (us at 3 / 4 / 6 / 8 / 12 / 16 waves per CU / full occupancy):
-//   112 KiB stored per wave (14 KiB rows, top-8)      847 / 844 / 851 / 855 / 860 / 858 / 857
-//   59 KiB (DSv3 fp8 rows, top-8)                     404 / 421 / 437 / 437 / 427 / 432 / 433
-//   32 KiB (4 KiB rows, top-8)                        206 / 211 / 215 / 216 / 217 / 220 / 221
-//   16 KiB (8 KiB rows, top-2)                        164 / 152 / 155 / 160 / 163 / 165 / 167
-//   17 KiB (2 KiB fp8 rows with scales, top-8)        163 / 133 / 106 / 104 / 109 / 110 / 111
-//   14 KiB (DSv3 fp8 rows, top-2)                     181 / 155 / 140 / 141 / 146 / 149 / 148
-//    8 KiB (1 KiB rows, top-8)                        122 / 100 /  77 /  64 /  57 /  60 /  60
-//    4 KiB (2 KiB rows, top-2)                        103 /  84 /  66 /  57 /  50 /  46 /  44
-// and on the Mixtral prefill (8 x 4096 tokens of 8 KiB, top-2, skewed routing) 147.5 us at 4
-// against 145.8 at 6.  A wave's launch, its loads and its slot arithmetic are dead time for the
-// stores, so the less a wave stores the more of them it takes to keep the CU's stores going.
+// Measured on 8 x 4096 tokens (us of a step, dispatch and combine, at 3 / 4 / 6 / 8 / 12 / 16 waves
+// per CU / full occupancy; only the dispatch varies, and up to 1 % of it is noise):
+//   112 KiB stored per wave (14 KiB rows, top-8)      1546 / 1549 / 1552 / 1560 / 1565 / 1562 / 1563
+//   59 KiB (DSv3 fp8 rows, top-8)                     1134 / 1145 / 1144 / 1135 / 1129 / 1137 / 1134
+//   32 KiB (4 KiB fp8 rows with scales, top-8)         649 /  632 /  641 /  642 /  642 /  642 /  641
+//   16 KiB (8 KiB rows, top-2)                         283 /  285 /  291 /  292 /  294 /  295 /  294
+//   17 KiB (2 KiB fp8 rows with scales, top-8)         357 /  337 /  316 /  311 /  312 /  314 /  315
+//   14 KiB (DSv3 fp8 rows, top-2)                      382 /  373 /  377 /  378 /  378 /  379 /  379
+//    8 KiB (1 KiB fp8 rows with scales, top-8)         226 /  202 /  179 /  169 /  159 /  159 /  160
+//    4 KiB (2 KiB fp8 rows with scales, top-2)         162 /  143 /  125 /  118 /  112 /  110 /  109
+// and on the Mixtral prefill (8 x 4096 tokens of 8 KiB, top-2, skewed routing) 271 / 267 / 276 / 279 /
+// 281.  Ragged and full steps of more than 16384 tokens of DSv3 rows do better with more waves (the
+// 8192-token prefill, half of its tokens absent: 1115 at 3, 1123 at 4, 1113 / 1108 / 1086 / 1100 at 6 / 8 /
+// 10 / 12: absent tokens' waves pass through the same slots), 14 KiB rows do not (8 x 4096 tokens, half of
+// them absent: 763 at 4, 774 at 10).  A wave's launch, its loads and its slot arithmetic are dead time for the stores, so the less
+// a wave stores the more of them it takes to keep the CU's stores going; where it stores much, few
+// waves per CU keep the stores in longer runs.
 uint32_t scatter_waves_per_cu(const WorldDev &w, uint32_t picks_per_wave) {
   if (w.lds_per_cu == 0) return 0;
   const uint64_t row = w.Hb + 4ull * w.S;
   const uint64_t stored = (uint64_t)picks_per_wave * row;
-  if (stored >= 24 * 1024) return 3;
-  if (stored >= 12 * 1024) return row >= 4096 ? 6 : 8;
+  if (stored >= 24 * 1024) return (uint64_t)w.G * w.M > 16384 && stored < 96 * 1024 ? 10 : 4;
+  if (stored >= 12 * 1024) return row >= 4096 ? 4 : 10;
   if (stored >= 6 * 1024) return 12;
   return 0;
 }
@@ -459,7 +481,7 @@ uint32_t scatter_waves_per_cu(const WorldDev &w, uint32_t picks_per_wave) {
 bool scatter_has_register_rows(const WorldDev &w) { return (w.Hb / 16 + kWave - 1) / kWave <= 32; }
 
 template <class DT>
-int launch_scatter_t(const WorldDev &w, const DT &tab, bool routed, hipStream_t s) {
+int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t s) {
   const uint32_t tokens = w.G * w.M;
   if (!scatter_has_register_rows(w)) {
     hipLaunchKernelGGL(dispatch_scatter_long<DT>, dim3(tokens), dim3(256), 0, s, w, tab);
@@ -478,14 +500,14 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, bool routed, hipStream_t 
   // what the intended number of workgroups leaves room for)
   uint32_t lds = waves_per_cu ? (w.lds_per_cu / waves_per_cu) & ~4095u : 0u;
   if (lds > 65536u) lds = 65536u;
-  const dim3 grid((uint32_t)waves), block(kWave);
+  const dim3 grid((uint32_t)waves + (slots == Slots::kTables ? (w.E + 7) / 8 : 0u)), block(kWave);
 #define PPLX_ROW_KERNEL_ARGS ksplit, kper
 #define PPLX_LAUNCH_LARGE_ROW_VARIANT(KERNEL)                                                    \
   do {                                                                                           \
     if (per_lane <= 16) PPLX_LAUNCH_ROW_VARIANT(KERNEL, 16, false);                              \
     else PPLX_LAUNCH_ROW_VARIANT(KERNEL, 32, false);                                             \
   } while (0)
-  if (routed) {
+  if (slots == Slots::kMap) {
     PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter);
   }
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
@@ -496,7 +518,9 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, bool routed, hipStream_t 
     if (per_lane <= 16) PPLX_LAUNCH_ROW_VARIANT(KERNEL, 16, false);                              \
     else return (int)hipErrorInvalidValue;                                                       \
   } while (0)
-  if (!routed) {
+  if (slots == Slots::kScanned) {
+    PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter_scanned);
+  } else if (slots == Slots::kTables) {
     PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter_slots);
   }
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
@@ -542,16 +566,20 @@ int launch_dispatch_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hi
   span.pick_vector = pick_vector;
   span.tile_cnt = w.tile_cnt;
   span.slot_out = w.slot_map;
-  // Steps of several tiles leave the last routing launch out: the scatter's waves work their
-  // own slots out of the tiles' tables.
-  const bool slots_in_scatter = w.num_tiles > 1 && (w.Hb / 16 + kWave - 1) / kWave <= 16;
-  if (slots_in_scatter) {
-    span.tile_mask = reinterpret_cast<unsigned long long *>(
-        reinterpret_cast<uint8_t *>(w.tile_cnt) + route_tables(w.num_tiles, w.tile_chunks, w.E).mask_offset);
+  // Steps of several tiles leave the last routing launch out (the scatter's waves work their own
+  // slots out of the tiles' tables), and the scan too as long as an expert's counts are one line.
+  Slots slots = Slots::kMap;
+  if (w.num_tiles > 1 && (w.Hb / 16 + kWave - 1) / kWave <= 16) {
+    slots = w.num_tiles <= kScanFreeTiles ? Slots::kTables : Slots::kScanned;
+    const RouteTables tables = route_tables(w.num_tiles, w.tile_chunks, w.E);
+    uint8_t *base = reinterpret_cast<uint8_t *>(w.tile_cnt);
+    span.tile_mask = reinterpret_cast<unsigned long long *>(base + tables.mask_offset);
+    span.chunk_base = reinterpret_cast<uint16_t *>(base + tables.base_offset);
+    if (slots == Slots::kTables) span.tile_row = reinterpret_cast<uint16_t *>(base);
   }
   int err = launch_route_t(w, tab, span, s);
   if (err) return err;
-  return launch_scatter_t(w, tab, !slots_in_scatter, s);
+  return launch_scatter_t(w, tab, slots, s);
 }
 
 }  // namespace
@@ -564,15 +592,23 @@ uint32_t route_lds_bytes(uint32_t num_experts, uint32_t tile_chunks) {
 }
 
 bool dispatch_is_fused(const WorldDev &w) {
-  // Every workgroup recounts all earlier tokens (work that grows with the square of the token
-  // count) and all of a workgroup's row waves store at once, while the scatter behind the two
-  // routing launches keeps few storing waves per CU.  Measured on 8 ranks (us, one launch /
-  // routing + scatter) at 2048, 3072, 4096, 6144 tokens: 7 KiB fp8 rows, top-8 of 256:
-  // 24 / 37, 45 / 48, 61 / 56, 86 / 79; 8 KiB rows, top-2 of 8: 15 / 21, 20 / 25, 26 / 27,
-  // 40 / 35; 4 KiB rows, top-8 of 64: 19 / 25, 26 / 32, 34 / 36, 49 / 49.  The one-launch form pays
-  // while the routing launches (about 10 us of latency) weigh more than the scatter's better rate.
+  if (!row_has_register_variant(w) || fused_lds_bytes(w, true) > 60 * 1024) return false;
+  // One launch while a workgroup per CU can own all tokens, one wave each: 4096 tokens, or 2048 of
+  // rows that take 512-thread workgroups (beyond that a second round of workgroups recounts
+  // everything: 8 ranks, 2 KiB rows, top-6 of 64: 4096 tokens 15.0 us against 15.9 with the routing
+  // in a launch of its own, 5120 tokens 24.2 against 20.0).  All of a workgroup's row waves store at
+  // once, though, where the scatter keeps few storing waves per CU, and that costs more than the
+  // routing launch once the rows no longer land in the last-level cache.  Measured on 8 ranks (us,
+  // one launch / routing + scatter; MB of rows stored): 7 KiB fp8 rows, top-8 of 256: 1536 tokens
+  // 18.9 / 24.8 (91), 1792 24.2 / 27.5 (106), 1920 28.4 / 28.6 (114), 2048 31.0 / 29.8 (121), 3072 45.3 /
+  // 40.4; 4 KiB rows, top-8 of 64: 3072 22.0 / 25.1 (104), 4080 32.2 / 31.5 (138); 8 KiB rows, top-2 of 8:
+  // 3072 14.2 / 18.1, 4080 20.6 / 21.2 (67); 14 KiB rows, top-8: 1280 34.2 / 36.4 (147), 2048 53.0 / 54.6,
+  // 2560 65.8 / 61.3.
   const uint64_t tokens = (uint64_t)w.G * w.M;
-  return tokens <= kFusedMaxTokens && row_has_register_variant(w) && fused_lds_bytes(w, true) <= 60 * 1024;
+  const uint32_t per_lane = (w.Hb / 16 + kWave - 1) / kWave;
+  const uint32_t waves = fused_threads((int)per_lane) / kWave;
+  const uint64_t stored = tokens * w.K * (w.Hb + 4ull * w.S);
+  return tokens <= 256u * waves && (waves < 16 || tokens <= 1792 || stored <= kFusedMaxBytes);
 }
 
 int launch_bind_dispatch(const WorldDev &w, const BindDispatchBatch &b, void *stream) {

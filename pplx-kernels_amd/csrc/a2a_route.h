@@ -1,5 +1,7 @@
 // Routing kernels: per-expert counts and the slot of every (token, pick) pair.
 #pragma once
+#include <type_traits>
+
 #include "a2a_common.h"
 
 namespace pplx_amd {
@@ -13,15 +15,19 @@ namespace {
 // workgroup).  Per chunk and expert a 64-bit mask in LDS holds one bit per token
 // routed to the expert (ds_or_b64); a token's row inside the expert is
 //     rows of earlier tiles + rows of earlier chunks of the tile + popc(mask & lanes below).
-// Three launches when a span has more than one tile, one otherwise:
-//   route_count   per tile: rows per expert                      -> tile_cnt[tile][e]
+//   route_count   per tile: rows per expert, kept with the masks (and reports the faults)
 //   route_scan    per expert: exclusive prefix over the tiles    -> tile_cnt[tile][e], totals
 //   route_slots   per tile: the masks again, slots               -> slot map
+// A span of one tile is one launch, route_slots.  With more tiles the scatter that follows works
+// each token's slots out by itself (slots_from_tables) from what route_count kept; up to
+// kScanFreeTiles tiles that is the only routing launch (the tiles' counts of an expert are one
+// cache line, and adding up a line per pick in the scatter's waves, behind their picks and beside
+// their row, costs less than the scan's launch: 8 x 509 DSv3 tokens count + scan + scatter 5.0 + 4.8
+// + 49.8 us, count + scatter 5.3 + 48.3; 8 x 1024 tokens of 2 KiB rows, top-6: 4.9 + 4.8 + 23.1 and
+// 4.9 + 21.7); beyond that the counts are scanned first.  Rows longer than the scatter's register variants
+// take all three.
 // An expert id repeated inside one token sets its bit once: the repeat takes no row, is not
 // counted, and is reported (kFaultDuplicateExpert).
-// With span.tile_mask set, route_count also keeps the masks and reports the faults, and there
-// is no route_slots launch: the scatter that follows works each token's slots out of the
-// scanned counts and the masks by itself (slots_from_masks).
 // ---------------------------------------------------------------------------
 
 // The token of this thread: which group and sender, whether its row of picks exists, and the
@@ -72,11 +78,17 @@ __global__ __launch_bounds__(1024) void route_count(WorldDev w, DT tab, RouteSpa
     }).codes;
   }
   __syncthreads();
-  uint32_t *out = span.tile_cnt + (size_t)blockIdx.x * w.E;
   for (uint32_t e = threadIdx.x; e < w.E; e += blockDim.x) {
     uint32_t rows = 0;
-    for (uint32_t c = 0; c < chunks; ++c) rows += __popcll(lds_mask[(size_t)c * w.E + e]);
-    out[e] = rows;
+    for (uint32_t c = 0; c < chunks; ++c) {
+      if (span.tile_mask != nullptr) span.chunk_base[((size_t)blockIdx.x * chunks + c) * w.E + e] = (uint16_t)rows;
+      rows += __popcll(lds_mask[(size_t)c * w.E + e]);
+    }
+    if (span.tile_row != nullptr) {
+      span.tile_row[(size_t)e * kScanFreeTiles + blockIdx.x] = (uint16_t)rows;
+    } else {
+      span.tile_cnt[(size_t)blockIdx.x * w.E + e] = rows;
+    }
   }
   if (span.tile_mask != nullptr) {
     unsigned long long *keep = span.tile_mask + (size_t)blockIdx.x * chunks * w.E;
@@ -88,39 +100,82 @@ __global__ __launch_bounds__(1024) void route_count(WorldDev w, DT tab, RouteSpa
   }
 }
 
-// What route_slots would have written for pick `lane` of virtual token v (wave-uniform), from
-// the scanned counts and the masks that route_count kept: rows of earlier tiles + rows of
-// earlier chunks of the tile + earlier tokens of the chunk.  A pick that repeats an earlier
-// one of its token, or names no expert, has no row.
-__device__ __forceinline__ uint32_t slots_from_masks(const WorldDev &w, uint32_t v, uint32_t lane, uint32_t e) {
-  const uint32_t chunks = w.tile_chunks;
-  const uint32_t chunk_abs = v / kWave;
-  const uint32_t tile = chunk_abs >> __builtin_ctz(chunks);  // (a tile is a power of two of chunks)
-  const uint32_t c = chunk_abs - tile * chunks;
+// Sum over an aligned group of `lanes` lanes (a power of two), in every lane of it.
+__device__ __forceinline__ uint32_t group_sum(uint32_t x, uint32_t lanes) {
+  auto moved = [](uint32_t v, auto ctrl) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xf, 0xf, false);
+  };
+  if (lanes > 1) x += moved(x, std::integral_constant<int, 0xB1>{});   // lane ^ 1
+  if (lanes > 2) x += moved(x, std::integral_constant<int, 0x4E>{});   // lane ^ 2
+  if (lanes > 4) x += moved(x, std::integral_constant<int, 0x141>{});  // 8 lanes mirrored: the other four
+  if (lanes > 8) x += moved(x, std::integral_constant<int, 0x140>{});  // 16 lanes mirrored: the other eight
+  if (lanes > 16) x += __shfl_xor(x, 16, kWave);
+  if (lanes > 32) x += __shfl_xor(x, 32, kWave);
+  return x;
+}
+
+// Rows of expert e in the tiles before `tile`, added up by the `lanes` lanes (a power of two) of
+// an aligned group that all pass the same e; every lane gets the sum.
+__device__ __forceinline__ uint32_t rows_of_earlier_tiles(const WorldDev &w, uint32_t e, uint32_t tile, uint32_t sub,
+                                                          uint32_t lanes) {
+  constexpr uint32_t kVec = 8;  // tiles per 16-byte vector
+  const PPLX_GLOBAL u32x4 *row = as_global(reinterpret_cast<const u32x4 *>(
+      reinterpret_cast<const uint16_t *>(w.tile_cnt) + (size_t)e * kScanFreeTiles));
+  uint32_t sum = 0;
+  for (uint32_t v = sub; v * kVec < tile; v += lanes) {
+    const u32x4 x = row[v];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+      if (v * kVec + 2 * i < tile) sum += x[i] & 0xffffu;
+      if (v * kVec + 2 * i + 1 < tile) sum += x[i] >> 16;
+    }
+  }
+  return group_sum(sum, lanes);
+}
+
+// What route_slots would have written for pick `lane` of virtual token v (wave-uniform), from the
+// tables that route_count kept: rows of earlier tiles + rows of earlier chunks of the tile +
+// earlier tokens of the chunk.  A pick that repeats an earlier one of its token, or names no
+// expert, has no row.
+template <bool SCANNED>
+__device__ __forceinline__ uint32_t slots_from_tables(const WorldDev &w, uint32_t v, uint32_t lane, uint32_t e) {
+  const uint32_t chunk = v / kWave;
+  const uint32_t tile = chunk >> __builtin_ctz(w.tile_chunks);  // (a tile is a power of two of chunks)
   const unsigned long long below = (1ull << (v & (kWave - 1))) - 1ull;
+  const RouteTables tables = route_tables(w.num_tiles, w.tile_chunks, w.E);
+  const uint8_t *base = reinterpret_cast<const uint8_t *>(w.tile_cnt);
+  // (unconditional loads, of expert 0 where there is no pick: all of them are in flight at once)
+  const uint32_t known = e < w.E ? e : 0;
+  const size_t at = (size_t)chunk * w.E + known;
+  const unsigned long long mask =
+      as_global(reinterpret_cast<const unsigned long long *>(base + tables.mask_offset))[at];
+  uint32_t slot = as_global(reinterpret_cast<const uint16_t *>(base + tables.base_offset))[at];
+  if constexpr (SCANNED) {
+    slot += as_global(w.tile_cnt)[(size_t)tile * w.E + known];
+  } else {
+    // 64 / (K rounded up to a power of two) lanes add up a pick's line of counts
+    const uint32_t shift = w.K > 1 ? 6 - (32 - __builtin_clz(w.K - 1)) : 6;  // log2 of the lanes per pick
+    const uint32_t e_of_pick = __shfl(known, (int)(lane >> shift), kWave);
+    const uint32_t sum = rows_of_earlier_tiles(w, e_of_pick, tile, lane & ((1u << shift) - 1), 1u << shift);
+    slot += __shfl(sum, (int)((lane << shift) & (kWave - 1)), kWave);
+  }
   bool has_row = lane < w.K && e < w.E;
   for (uint32_t k = 0; k + 1 < w.K; ++k) {
     const uint32_t earlier = (uint32_t)__builtin_amdgcn_readlane((int)e, (int)k);
     if (lane > k && earlier == e) has_row = false;
   }
-  if (!has_row) return kInvalidSlot;
-  const PPLX_GLOBAL unsigned long long *mask =
-      as_global(reinterpret_cast<const unsigned long long *>(
-          reinterpret_cast<const uint8_t *>(w.tile_cnt) + route_tables(w.num_tiles, chunks, w.E).mask_offset)) +
-      (size_t)tile * chunks * w.E + e;
-  uint32_t slot = as_global(w.tile_cnt)[(size_t)tile * w.E + e];
-  // four masks per trip (tiles of four chunks: one trip)
-  for (uint32_t c0 = 0; c0 <= c; c0 += 4) {
-    unsigned long long m[4];
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) m[i] = mask[(size_t)(c0 + i <= c ? c0 + i : c) * w.E];
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-      if (c0 + i < c) slot += __popcll(m[i]);
-      if (c0 + i == c) slot += __popcll(m[i] & below);
-    }
+  return has_row ? slot + (uint32_t)__popcll(mask & below) : kInvalidSlot;
+}
+
+// out_expert_num_tokens of the eight experts from 8 * i on, by one wave (scan-free form).
+template <class DT>
+__device__ __forceinline__ void write_totals(const WorldDev &w, const DT &tab, uint32_t i, uint32_t lane) {
+  const uint32_t e = i * 8 + lane / 8;
+  const uint32_t sum = rows_of_earlier_tiles(w, e < w.E ? e : 0, w.num_tiles, lane & 7, 8);
+  if (e < w.E && (lane & 7) == 0) {
+    const DispatchRank &owner = tab.at(owner_of(w, e));
+    as_global(owner.out_num_tokens)[(int64_t)local_of(w, e) * owner.out_num_tokens_stride] = (int32_t)sum;
   }
-  return slot;
 }
 
 // One wavefront per expert: tile_cnt[.][e] becomes its own exclusive prefix over the tiles, and
@@ -233,7 +288,8 @@ int launch_route_pv(const WorldDev &w, const DT &tab, const RouteSpan &span, hip
   if (tiles > 1) {
     hipLaunchKernelGGL((route_count<DT, PV>), dim3(tiles), dim3(block),
                        span.tile_chunks * w.E * sizeof(unsigned long long), s, w, tab, span);
-    hipLaunchKernelGGL((route_scan<DT>), dim3((w.E + 3) / 4), dim3(256), 0, s, w, tab, span, tiles);
+    if (span.tile_row == nullptr)
+      hipLaunchKernelGGL((route_scan<DT>), dim3((w.E + 3) / 4), dim3(256), 0, s, w, tab, span, tiles);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return (int)err;
     if (span.tile_mask != nullptr) return 0;  // the scatter works the slots out

@@ -44,20 +44,38 @@ struct Destination {
   int64_t scale_step = 0;
 };
 
+// The buffers of one expert, out of its owner's row of the rank table.  Fetched whole and without
+// conditions, so that it costs one trip to memory which can overlap with whatever finds the slot.
+struct ExpertBuffer {
+  uint64_t row, scale;
+  int64_t row_step, scale_step, scale_elem_step;
+  uint32_t rows;
+};
+
 template <class DT>
-__device__ __forceinline__ Destination resolve_destination(const WorldDev &w, const DT &tab, uint32_t e,
-                                                           uint32_t slot, bool report) {
+__device__ __forceinline__ ExpertBuffer expert_buffer(const WorldDev &w, const DT &tab, uint32_t e) {
+  const uint32_t known = e < w.E ? e : 0;
+  const DispatchRank &owner = tab.at(owner_of(w, known));
+  const uint32_t el = local_of(w, known);
+  ExpertBuffer b;
+  b.row = reinterpret_cast<uint64_t>(owner.expert_x + (int64_t)el * owner.x_stride_expert);
+  b.row_step = owner.x_stride_row;
+  b.scale = reinterpret_cast<uint64_t>(owner.expert_xs + (int64_t)el * owner.xs_stride_expert);
+  b.scale_step = owner.xs_stride_row;
+  b.scale_elem_step = owner.xs_stride_elem;
+  b.rows = owner.x_rows;
+  return b;
+}
+
+__device__ __forceinline__ Destination destination_of(const WorldDev &w, const ExpertBuffer &b, uint32_t slot,
+                                                      bool report) {
   Destination d;
-  if (e < w.E && slot != kInvalidSlot) {
-    const DispatchRank &dst = tab.at(owner_of(w, e));
-    const uint32_t el = local_of(w, e);
-    if (slot < dst.x_rows) {
-      d.row = reinterpret_cast<uint64_t>(dst.expert_x + (int64_t)el * dst.x_stride_expert +
-                                         (int64_t)slot * dst.x_stride_row);
+  if (slot != kInvalidSlot) {
+    if (slot < b.rows) {
+      d.row = b.row + (uint64_t)((int64_t)slot * b.row_step);
       if (w.S) {
-        d.scale = reinterpret_cast<uint64_t>(dst.expert_xs + (int64_t)el * dst.xs_stride_expert +
-                                             (int64_t)slot * dst.xs_stride_row);
-        d.scale_step = dst.xs_stride_elem;
+        d.scale = b.scale + 4u * (uint64_t)((int64_t)slot * b.scale_step);
+        d.scale_step = b.scale_elem_step;
       }
     } else if (report) {
       atomicOr(w.faults, kFaultRowDropped);

@@ -77,3 +77,61 @@ def test_members_of_a_dp_group_share_or_keep_their_own_sums(dp, K, E, H, M, y_dt
                 rtol=COMBINE_RTOL, atol=COMBINE_ATOL, err_msg=f"group {g} member {member}",
             )  # fmt: skip
             assert torch.isnan(got[data.n :]).all()
+
+
+# ---------------------------------------------------------------------------
+# Slots from the routing tables: one to sixty-four tiles without a scan, more with one
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize(
+    "E,K,M,R,hidden_bytes",
+    [
+        # (rows of 8208 bytes have no variant in the one-launch form)
+        (16, 1, 401, 8, 8208),  # 51 tiles of one chunk, 64 lanes to a pick, the last tile nearly empty
+        (64, 33, 129, 8, 8208),  # 17 tiles, one lane to a pick
+        (40, 5, 512, 8, 8208),  # exactly 64 tiles; lanes left over (8 to a pick, 5 picks)
+        (8, 3, 513, 8, 48),  # 65 chunks: 33 tiles of two
+        (24, 10, 4099, 8, 16),  # 513 chunks: 33 tiles of sixteen
+        (1024, 2, 2050, 8, 16),  # LDS limits tiles to four chunks: 65 tiles, scanned
+        (144, 4, 60, 72, 512),  # rank tables in HBM
+    ],
+)
+def test_slots_from_the_routing_tables(E, K, M, R, hidden_bytes):
+    spec = WorkloadSpec("tables", 72, R, E, K, hidden_bytes // 2, M, torch.bfloat16, tokens="uniform")
+    assert M * R > 4096 or hidden_bytes == 8208
+    groups = generate(spec, seed=E + K)
+    groups[0].n, groups[1].n, groups[-1].n = 0, M, M  # an empty rank; a full last tile
+    load = np.bincount(
+        np.concatenate([g.indices[: g.n].reshape(-1).numpy() for g in groups]), minlength=E
+    ).max()  # fmt: skip
+    step = DeviceStep(spec, groups, cap=int(load), alloc_expert_y=False)
+    world = make_world(spec, group_name="tables")
+    for _ in range(2):  # the tables of the step before must not show through
+        step.dispatch_world(world)
+        check_dispatch_against_oracle(step)
+    assert world.faults() == 0
+    world.destroy()
+
+
+@pytest.mark.parametrize(
+    "M,topk,hidden,in_dtype",
+    [
+        (1792, 8, 1792, torch.bfloat16),  # the last 3584-byte step of one launch by its row count
+        (1793, 8, 8192, torch.bfloat16),  # 235 MB of rows: routing and scatter
+        (2048, 1, 4096, torch.bfloat16),  # up to 4096 tokens in one launch while the rows are few
+        (4096, 1, 64, torch.bfloat16),
+        (4097, 1, 64, torch.bfloat16),  # routing and scatter
+        (2048, 1, 5120, torch.bfloat16),  # rows of 512-thread workgroups: up to 2048 tokens
+        (2049, 1, 5120, torch.bfloat16),
+    ],
+)
+def test_both_sides_of_the_one_launch_limit(M, topk, hidden, in_dtype):
+    spec = WorkloadSpec("limit", 73, 1, 16, topk, hidden, M, in_dtype)
+    groups = generate(spec, seed=M)
+    groups[0].n = M - 1
+    cap = int(np.bincount(groups[0].indices[: M - 1].reshape(-1).numpy(), minlength=16).max())
+    step = DeviceStep(spec, groups, cap=cap, alloc_expert_y=False)
+    world = make_world(spec, group_name="limit")
+    step.dispatch_world(world)
+    check_dispatch_against_oracle(step)
+    assert world.faults() == 0
+    world.destroy()

@@ -88,48 +88,31 @@ __device__ __forceinline__ void gather_group(f32x8 (&acc)[VPL], uint64_t row_of_
   }
 }
 
-// What one wave of combine_gather adds up and where the sum goes.  Lane `base + k` holds the row
-// and the weight of pick k; `base` differs between the members of a DP group only.
-template <typename T, typename U, int KB, int VPL>
-__device__ __forceinline__ void reduce_row(const WorldDev &w, uint64_t row, float weight, uint32_t base,
-                                           bool all_rows, uint32_t segment, uint64_t out_of_lane,
-                                           uint64_t out_lanes) {
-  const uint32_t lane = lane_id();
-  const uint32_t nvec = w.H / 8;
-  const uint32_t K = w.K;
-  uint32_t vec_ld[VPL];
-  f32x8 acc[VPL];
+constexpr uint32_t kWavesPerBlock = 4;
+
+// The sum of one output row's piece: lane `base + k` holds the row and the weight of pick k.
+template <typename T, int KB, int VPL>
+__device__ __forceinline__ void reduce_picks(f32x8 (&acc)[VPL], uint32_t K, uint64_t row, float weight, uint32_t base,
+                                             bool all_rows, const uint32_t (&vec)[VPL]) {
 #pragma unroll
-  for (int v = 0; v < VPL; ++v) {
-    const uint32_t vec = (segment * VPL + v) * kWave + lane;
-    vec_ld[v] = vec < nvec ? vec : nvec - 1;  // clamp: loads stay unconditional
-    acc[v] = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  }
+  for (int v = 0; v < VPL; ++v) acc[v] = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (!all_rows) {
     // A pick without a row (bad expert id or slot) contributes nothing.
     for (uint32_t k = 0; k < K; ++k) {
-      if (read_lane64(row, base + k) != 0) gather_group<T, 1, VPL>(acc, row, weight, base + k, vec_ld);
+      if (read_lane64(row, base + k) != 0) gather_group<T, 1, VPL>(acc, row, weight, base + k, vec);
     }
-  } else {
-    uint32_t k = 0;
-    for (; k + KB <= K; k += KB) gather_group<T, KB, VPL>(acc, row, weight, base + k, vec_ld);
-    if constexpr (KB > 4) {
-      if ((K - k) & 4) { gather_group<T, 4, VPL>(acc, row, weight, base + k, vec_ld); k += 4; }
-    }
-    if constexpr (KB > 2) {
-      if ((K - k) & 2) { gather_group<T, 2, VPL>(acc, row, weight, base + k, vec_ld); k += 2; }
-    }
-    if constexpr (KB > 1) {
-      if ((K - k) & 1) { gather_group<T, 1, VPL>(acc, row, weight, base + k, vec_ld); }
-    }
+    return;
   }
-  for (; out_lanes != 0; out_lanes &= out_lanes - 1) {
-    U *out = reinterpret_cast<U *>(read_lane64(out_of_lane, (uint32_t)__builtin_ctzll(out_lanes)));
-#pragma unroll
-    for (int v = 0; v < VPL; ++v) {
-      const uint32_t vec = (segment * VPL + v) * kWave + lane;
-      if (vec < nvec) Store8<U>::at(out, vec, acc[v]);
-    }
+  uint32_t k = 0;
+  for (; k + KB <= K; k += KB) gather_group<T, KB, VPL>(acc, row, weight, base + k, vec);
+  if constexpr (KB > 4) {
+    if ((K - k) & 4) { gather_group<T, 4, VPL>(acc, row, weight, base + k, vec); k += 4; }
+  }
+  if constexpr (KB > 2) {
+    if ((K - k) & 2) { gather_group<T, 2, VPL>(acc, row, weight, base + k, vec); k += 2; }
+  }
+  if constexpr (KB > 1) {
+    if ((K - k) & 1) { gather_group<T, 1, VPL>(acc, row, weight, base + k, vec); }
   }
 }
 
@@ -147,10 +130,10 @@ __device__ __forceinline__ void reduce_row(const WorldDev &w, uint64_t row, floa
 // group (242 MB at 4.5 TB/s); groups of two, 4 x 128 bf16 tokens, 7168 wide, top-8: 16.5 and 15.0
 // us (the second gather of a step this small hits the last-level cache).
 template <typename T, typename U, class CT, int KB, int VPL, bool GROUPED>
-__global__ __launch_bounds__(256) void combine_gather(WorldDev w, CT tab, uint32_t segments, FastDiv by_segments) {
+__global__ __launch_bounds__(kWavesPerBlock * kWave) void combine_gather(WorldDev w, CT tab, uint32_t segments,
+                                                                         FastDiv by_segments) {
   const uint32_t lane = lane_id();
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / kWave) +
-                                                       threadIdx.x / kWave);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave);
   const uint32_t token = fast_div(wave, by_segments);
   const uint32_t segment = wave - token * segments;
   const uint32_t owner_index = group_of(w, token);  // the rank, or the DP group when GROUPED
@@ -169,30 +152,52 @@ __global__ __launch_bounds__(256) void combine_gather(WorldDev w, CT tab, uint32
   if (GROUPED && __builtin_amdgcn_ballot_w64(present) == 0) return;
 
   // Lane k (of its member) resolves pick k: no LDS, no barrier.
-  uint64_t row = 0, out = 0;
+  uint64_t row = 0;
   float weight = 0.f;
   if (present) {
     const uint32_t e = as_global(c.indices)[(size_t)t * w.K + pick];
     const uint32_t slot = as_global(w.slot_map)[((size_t)g * w.M + t) * w.K + pick];
     weight = as_global(c.weights)[(int64_t)t * c.w_stride_row + pick];
     if (e < w.E && slot != kInvalidSlot) {
+      // (the buffer and its length in one trip, not the one behind the other)
       const CombineRank &owner = tab.at(owner_of(w, e));
-      if (slot < owner.y_rows) {
-        row = reinterpret_cast<uint64_t>(reinterpret_cast<const T *>(owner.expert_y) +
-                                         (int64_t)local_of(w, e) * owner.y_stride_expert +
-                                         (int64_t)slot * owner.y_stride_row);
+      const uint32_t y_rows = owner.y_rows;
+      uint64_t address = reinterpret_cast<uint64_t>(reinterpret_cast<const T *>(owner.expert_y) +
+                                                    (int64_t)local_of(w, e) * owner.y_stride_expert +
+                                                    (int64_t)slot * owner.y_stride_row);
+      settle(address);
+      if (slot < y_rows) {
+        row = address;
       } else if (segment == 0) {
         atomicOr(w.faults, kFaultBadSlot);
       }
     }
   }
-  if (has_pick) out = reinterpret_cast<uint64_t>(reinterpret_cast<U *>(c.out_tokens) + (int64_t)t * c.out_stride_row);
   const uint64_t no_row = __builtin_amdgcn_ballot_w64(present && row == 0);
+
+  const uint64_t out = reinterpret_cast<uint64_t>(reinterpret_cast<U *>(c.out_tokens) + (int64_t)t * c.out_stride_row);
+  const uint32_t nvec = w.H / 8;
+  uint32_t vec[VPL];
+#pragma unroll
+  for (int v = 0; v < VPL; ++v) {
+    vec[v] = (segment * VPL + v) * kWave + lane;
+    vec[v] = vec[v] < nvec ? vec[v] : nvec - 1;  // clamp: loads stay unconditional
+  }
+  f32x8 acc[VPL];
+  auto store = [&](uint64_t out) {
+#pragma unroll
+    for (int v = 0; v < VPL; ++v) {
+      const uint32_t at = (segment * VPL + v) * kWave + lane;
+      if (at < nvec) Store8<U>::at(reinterpret_cast<U *>(out), at, acc[v]);
+    }
+  };
   if constexpr (!GROUPED) {
-    reduce_row<T, U, KB, VPL>(w, row, weight, 0, no_row == 0, segment, out, 1ull);
+    reduce_picks<T, KB, VPL>(acc, w.K, row, weight, 0, no_row == 0, vec);
+    store(out);
   } else {
-    const uint64_t heads = __builtin_amdgcn_ballot_w64(present && pick == 0);  // one lane per present member
-    for (uint64_t todo = heads; todo != 0;) {
+    const uint64_t picks = w.K == kWave ? ~0ull : (1ull << w.K) - 1;
+    // one lane per present member
+    for (uint64_t todo = __builtin_amdgcn_ballot_w64(present && pick == 0); todo != 0;) {
       const uint32_t base = (uint32_t)__builtin_ctzll(todo);
       // members that want the same sum: every pick's row and weight as this member's
       const int src = (int)((base + pick) & (kWave - 1));
@@ -200,14 +205,13 @@ __global__ __launch_bounds__(256) void combine_gather(WorldDev w, CT tab, uint32
                         __shfl((uint32_t)(row >> 32), src, kWave) == (uint32_t)(row >> 32) &&
                         __shfl(__float_as_uint(weight), src, kWave) == __float_as_uint(weight);
       const uint64_t differs = __builtin_amdgcn_ballot_w64(present && !same);
-      uint64_t outs = 0;
-      const uint64_t picks = w.K == kWave ? ~0ull : (1ull << w.K) - 1;
+      reduce_picks<T, KB, VPL>(acc, w.K, row, weight, base, ((no_row >> base) & picks) == 0, vec);
       for (uint64_t rest = todo; rest != 0; rest &= rest - 1) {
         const uint32_t head = (uint32_t)__builtin_ctzll(rest);
-        if (((differs >> head) & picks) == 0) outs |= 1ull << head;
+        if (((differs >> head) & picks) != 0) continue;
+        store(read_lane64(out, head));
+        todo &= ~(1ull << head);
       }
-      reduce_row<T, U, KB, VPL>(w, row, weight, base, ((no_row >> base) & picks) == 0, segment, out, outs);
-      todo &= ~outs;
     }
   }
 }
@@ -217,7 +221,7 @@ int launch_combine_v(const WorldDev &w, const CT &tab, bool grouped, hipStream_t
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
   const uint32_t segments = (nvec_segments + VPL - 1) / VPL;
   const uint64_t waves = (uint64_t)(grouped ? w.G : w.R) * w.M * segments;
-  const dim3 grid((uint32_t)((waves + 3) / 4)), block(256);
+  const dim3 grid((uint32_t)((waves + kWavesPerBlock - 1) / kWavesPerBlock)), block(kWavesPerBlock * kWave);
   if (grouped) {
     hipLaunchKernelGGL((combine_gather<T, U, CT, KB, VPL, true>), grid, block, 0, s, w, tab, segments,
                        make_fast_div(segments));

@@ -203,8 +203,10 @@ constexpr uint64_t kWriteThroughMaxBytes = 192ull << 20;
 constexpr uint64_t kFusedMaxBytes = 112ull << 20;
 
 // Device memory that pplx_a2a_static_step works in instead of a world's allocations: a fixed
-// array inside the library's code object (a2a_static.hip), one copy per GPU.
-constexpr size_t kStaticScratchBytes = 8u << 20;
+// array inside the library's code object (a2a_static.hip), one copy per GPU.  The chunks' bases
+// beside the masks take up to 1.25 times what masks and counts take by themselves: every step whose
+// slot map, masks and counts fit 8 MiB has its room.
+constexpr size_t kStaticScratchBytes = 10u << 20;
 // Address of the calling thread's current device's copy (looked up once per device).
 int static_scratch_address(int device, void **out);
 // True once static_scratch_address has succeeded for `device`.

@@ -282,3 +282,23 @@ def test_bench_refuses_more_than_one_gpu():
         assert done.returncode == 2, done
         assert "single-GPU loopback" in done.stderr and "--gpus 1" in done.stderr
         assert done.stdout == ""
+
+
+@pytest.mark.parametrize(
+    "M,E,K",
+    [
+        (15000, 256, 8),  # 7.9 MiB of slot map, masks and counts, 8.3 MiB with the chunks' bases
+        (8192, 680, 8),  # 1024 chunks of 680 experts
+        (2050, 2504, 1),  # LDS limits the tiles to two chunks
+        (32000, 16, 7),  # mostly slot map
+    ],
+)
+def test_static_step_has_room_for_eight_mebibytes_of_slots_masks_and_counts(M, E, K):
+    # (the device number is refused behind the check of the room, so nothing runs)
+    tokens, chunks = 8 * M, -(-8 * M // 64)
+    assert 7 << 20 < tokens * K * 4 + chunks * E * 8 + 256 * E * 4 <= 8 << 20
+    cfg = ops.Config(M, E, K, 8, 1, 512, 512, 16)
+    args = (ops.DispatchArgs * 8)()
+    lib = ops.load_library()
+    st = lib.pplx_a2a_static_step(ctypes.byref(cfg), -1, args, None, None, None)
+    assert st != 0 and b"static array" not in lib.pplx_a2a_last_error()

@@ -250,6 +250,24 @@ int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
     if (nvec_segments % 7 == 0) PPLX_COMBINE(1, 7);
     PPLX_COMBINE(1, 8);
   }
+  // fp32 rows are twice as long, and gathering eight of them at a time in 2 KiB pieces leaves each
+  // wave's accesses scattered over too many of them; steps that fill the chip more than once take two
+  // picks in 8 KiB pieces, or three in 4 KiB pieces where the last of the 8 KiB ones would be mostly
+  // padding.  Measured on 8 ranks (us: as before / three in 4 KiB / two in 8 KiB): 1024 tokens a rank,
+  // top-8, 2048 wide 110.3 / 106.8 / 101.8, 4096 wide 217.9 / 214.3 / 204.7; 5120 wide, top-3 111.2 / 107.5
+  // / 106.9; 4096 wide, top-4 112.9 / 110.4 / 108.8; 1024 wide, top-10, 2048 a rank 136.6 / 131.4 / 135.3;
+  // 7168 wide, top-8, 2048 a rank 779 / 773 / 774, 512 and a ragged batch 101.7 / 101.6 / 97.9; 2880 wide,
+  // top-5, dp 4: 2 x 3001 tokens 98.9 / 94.1 / 94.4, ragged 52.0 / 50.6 / 53.0; dp 1, 8 x 1024 98.6 / 96.6 /
+  // 98.0.  Steps of a few hundred tokens lack the waves for it (64 tokens, 7168 wide, top-8: 5.8 / 7.9 /
+  // 11.0; 320 tokens, 1024 wide, top-6: 4.5 / 6.2 / 6.7); 16-bit rows do not care (within 1 %) or lose
+  // (the large ragged prefill of 7168-wide rows: 734 / 761 / 762).
+  if constexpr (sizeof(T) == 4) {
+    if (w.K > 2 && tokens > 2048) {
+      const uint32_t padding = (4 - nvec_segments % 4) % 4;
+      if (6 * padding <= nvec_segments) PPLX_COMBINE(2, 4);
+      PPLX_COMBINE(3, 2);
+    }
+  }
   switch (w.K) {
     case 1: PPLX_COMBINE(1, 8);
     case 2: PPLX_COMBINE(2, 4);

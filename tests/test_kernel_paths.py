@@ -15,6 +15,7 @@ from tests.all_to_all_utils import (
     ORACLE_DTYPE,
     DeviceStep,
     WorkloadSpec,
+    check_combine_against_oracle,
     check_dispatch_against_oracle,
     generate,
     make_world,
@@ -133,5 +134,40 @@ def test_both_sides_of_the_one_launch_limit(M, topk, hidden, in_dtype):
     world = make_world(spec, group_name="limit")
     step.dispatch_world(world)
     check_dispatch_against_oracle(step)
+    assert world.faults() == 0
+    world.destroy()
+
+
+# ---------------------------------------------------------------------------
+# Expert outputs in fp32: pieces of 2 KiB (up to 2048 tokens), 4 and 8 KiB of a row
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize(
+    "M,K,H,dp,out_dtype",
+    [
+        (1024, 5, 2048, 1, torch.bfloat16),  # eight picks at a time still
+        (1025, 3, 2048, 1, torch.bfloat16),  # two picks of 8 KiB, the third by itself
+        (1025, 8, 3592, 1, torch.float16),  # 8 segments, one vector in the last
+        (1025, 5, 2056, 1, torch.bfloat16),  # 5 segments: three picks of 4 KiB, then two
+        (1025, 10, 8, 1, torch.bfloat16),  # one vector; three times three picks, then one
+        (1025, 7, 1536, 2, torch.float16),  # the same for DP groups
+        (1025, 3, 2880, 4, torch.float16),
+    ],
+)
+def test_pieces_of_fp32_rows(M, K, H, dp, out_dtype):
+    spec = WorkloadSpec(
+        "pieces", 74, 2 * dp, 8 * dp if dp > 1 else 16, K, H, M, torch.bfloat16, out_dtype=out_dtype,
+        expert_y_dtype=torch.float32, dp_size=dp,
+    )  # fmt: skip
+    groups = generate(spec, seed=H + K)
+    groups[0].n, groups[1].n = M, M - 3
+    experts = np.concatenate([g.indices[: g.n].reshape(-1).numpy() for g in groups])
+    step = DeviceStep(spec, groups, cap=int(np.bincount(experts, minlength=spec.num_experts).max()))
+    world = make_world(spec, group_name="pieces")
+    step.dispatch_world(world)
+    expected = check_dispatch_against_oracle(step)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    step.expert_y_all.normal_(generator=gen)
+    step.combine_world(world)
+    check_combine_against_oracle(step, expected.slot_map)
     assert world.faults() == 0
     world.destroy()

@@ -218,6 +218,100 @@ int dtype_code(at::ScalarType t) {
   }
 }
 
+void check_dispatch(const at::Tensor &outExpertNumTokens, const at::Tensor &outExpertX,
+                    const at::Tensor *outExpertXScale, const at::Tensor &dpX, const at::Tensor *dpXScale,
+                    const at::Tensor &indices, const at::Tensor *boundM) {
+  check_tensor(outExpertNumTokens, 1, "outExpertNumTokens");
+  TORCH_CHECK(outExpertNumTokens.scalar_type() == at::kInt, "outExpertNumTokens must be of type Int");
+  check_tensor(outExpertX, 3, "outExpertX");
+  if (outExpertXScale) {
+    TORCH_CHECK(outExpertXScale->is_cuda(), "Tensor outExpertXScale must be on GPU");
+    TORCH_CHECK(outExpertXScale->dim() == 3, "Tensor outExpertXScale must be 3 dimensional");
+    TORCH_CHECK(outExpertXScale->scalar_type() == at::kFloat, "outExpertXScale must be of type Float");
+  }
+  check_tensor(dpX, 2, "dpX");
+  if (dpXScale) {
+    TORCH_CHECK(dpXScale->is_cuda(), "Tensor dpXScale must be on GPU");
+    TORCH_CHECK(dpXScale->dim() == 2, "Tensor dpXScale must be 2 dimensional");
+    TORCH_CHECK(dpXScale->scalar_type() == at::kFloat, "dpXScale must be of type Float");
+  }
+  check_tensor(indices, 2, "indices");
+  TORCH_CHECK(indices.scalar_type() == at::kUInt32, "indices must be of type UInt32");
+  check_bound_m(boundM);
+  TORCH_CHECK(indices.size(0) == dpX.size(0), "indices.size(0) must be equal to dpX.size(0)");
+}
+
+void check_picks(const at::Tensor &indices, uint64_t experts_per_token) {
+  TORCH_CHECK(indices.size(1) == (int64_t)experts_per_token, "indices.size(1) must be equal to the experts per token");
+}
+
+// The views of csrc/bindings/all_to_all_ops.cpp:165-195
+pplx_a2a_dispatch_args_t pack_dispatch(const at::Tensor &outExpertNumTokens, const at::Tensor &outExpertX,
+                                       const at::Tensor *outExpertXScale, const at::Tensor &dpX,
+                                       const at::Tensor *dpXScale, const at::Tensor &indices,
+                                       const at::Tensor *boundM) {
+  pplx_a2a_dispatch_args_t a{};
+  a.out_expert_num_tokens = static_cast<int32_t *>(outExpertNumTokens.data_ptr());
+  a.out_expert_num_tokens_stride = outExpertNumTokens.stride(0);
+  const int64_t esz = (int64_t)outExpertX.element_size();
+  a.out_expert_x = outExpertX.data_ptr();
+  a.out_expert_x_stride_row = outExpertX.stride(1) * esz;
+  a.out_expert_x_stride_expert = outExpertX.stride(0) * esz;
+  a.out_expert_x_rows = outExpertX.size(1);
+  if (outExpertXScale) {
+    a.out_expert_x_scale = static_cast<float *>(outExpertXScale->data_ptr());
+    a.out_expert_x_scale_stride_elem = outExpertXScale->stride(2);
+    a.out_expert_x_scale_stride_row = outExpertXScale->stride(1);
+    a.out_expert_x_scale_stride_expert = outExpertXScale->stride(0);
+  }
+  a.dp_x = dpX.data_ptr();
+  a.dp_x_stride_row = dpX.stride(0) * (int64_t)dpX.element_size();
+  if (dpXScale) {
+    a.dp_x_scale = static_cast<const float *>(dpXScale->data_ptr());
+    a.dp_x_scale_stride_elem = dpXScale->stride(1);
+    a.dp_x_scale_stride_row = dpXScale->stride(0);
+  }
+  a.indices = static_cast<const uint32_t *>(indices.data_ptr());
+  a.m = (uint32_t)indices.size(0);
+  a.bound_m = boundM ? static_cast<const uint32_t *>(boundM->data_ptr()) : nullptr;
+  return a;
+}
+
+void check_combine(const at::Tensor &outTokens, const at::Tensor &indices, const at::Tensor &weights,
+                   const at::Tensor &expertY, const at::Tensor *boundM) {
+  check_tensor(outTokens, 2, "outTokens");
+  check_tensor(indices, 2, "indices");
+  TORCH_CHECK(indices.scalar_type() == at::kUInt32, "indices must be of type UInt32");
+  check_tensor(weights, 2, "weights");
+  TORCH_CHECK(weights.scalar_type() == at::kFloat, "weights must be of type Float");
+  check_tensor(expertY, 3, "expertY");
+  check_bound_m(boundM);
+  TORCH_CHECK(dtype_code(expertY.scalar_type()) >= 0, "Unsupported dtype for expertY");
+  const int out_dtype = dtype_code(outTokens.scalar_type());
+  TORCH_CHECK(out_dtype == PPLX_A2A_BF16 || out_dtype == PPLX_A2A_F16, "Unsupported dtype for outTokens");
+}
+
+// The dtype switch of csrc/bindings/all_to_all_ops.cpp:265-310 and the element-stride views of :222-235
+pplx_a2a_combine_args_t pack_combine(const at::Tensor &outTokens, const at::Tensor &indices,
+                                     const at::Tensor &weights, const at::Tensor &expertY,
+                                     const at::Tensor *boundM) {
+  pplx_a2a_combine_args_t a{};
+  a.out_tokens = outTokens.data_ptr();
+  a.out_tokens_stride_row = outTokens.stride(0);
+  a.out_dtype = dtype_code(outTokens.scalar_type());
+  a.indices = static_cast<const uint32_t *>(indices.data_ptr());
+  a.weights = static_cast<const float *>(weights.data_ptr());
+  a.weights_stride_row = weights.stride(0);
+  a.expert_y = expertY.data_ptr();
+  a.expert_y_stride_row = expertY.stride(1);
+  a.expert_y_stride_expert = expertY.stride(0);
+  a.expert_y_rows = expertY.size(1);
+  a.in_dtype = dtype_code(expertY.scalar_type());
+  a.m = (uint32_t)indices.size(0);
+  a.bound_m = boundM ? static_cast<const uint32_t *>(boundM->data_ptr()) : nullptr;
+  return a;
+}
+
 RankRef find_rank(fptr_t ptr) {
   auto it = g_ranks.find(ptr);
   TORCH_CHECK(it != g_ranks.end(), "pplx_kernels: invalid state: the handle has been destroyed");
@@ -291,53 +385,13 @@ void dispatch_core(fptr_t ptr, const at::Tensor &outExpertNumTokens, const at::T
     // (a handle that is unknown is reported after the tensor checks, which need no handle)
     auto found = g_ranks.find(ptr);
     if (found != g_ranks.end()) world = found->second.world;
-    check_tensor(outExpertNumTokens, 1, "outExpertNumTokens");
-    TORCH_CHECK(outExpertNumTokens.scalar_type() == at::kInt, "outExpertNumTokens must be of type Int");
-    check_tensor(outExpertX, 3, "outExpertX");
-    if (outExpertXScale) {
-      TORCH_CHECK(outExpertXScale->is_cuda(), "Tensor outExpertXScale must be on GPU");
-      TORCH_CHECK(outExpertXScale->dim() == 3, "Tensor outExpertXScale must be 3 dimensional");
-      TORCH_CHECK(outExpertXScale->scalar_type() == at::kFloat, "outExpertXScale must be of type Float");
-    }
-    check_tensor(dpX, 2, "dpX");
-    if (dpXScale) {
-      TORCH_CHECK(dpXScale->is_cuda(), "Tensor dpXScale must be on GPU");
-      TORCH_CHECK(dpXScale->dim() == 2, "Tensor dpXScale must be 2 dimensional");
-      TORCH_CHECK(dpXScale->scalar_type() == at::kFloat, "dpXScale must be of type Float");
-    }
-    check_tensor(indices, 2, "indices");
-    TORCH_CHECK(indices.scalar_type() == at::kUInt32, "indices must be of type UInt32");
-    check_bound_m(boundM);
-    TORCH_CHECK(indices.size(0) == dpX.size(0), "indices.size(0) must be equal to dpX.size(0)");
+    check_dispatch(outExpertNumTokens, outExpertX, outExpertXScale, dpX, dpXScale, indices, boundM);
     const RankRef ref = find_rank(ptr);
-    TORCH_CHECK(indices.size(1) == (int64_t)world->cfg.experts_per_token,
-                "indices.size(1) must be equal to the experts per token");
+    check_picks(indices, world->cfg.experts_per_token);
     const int mode = split_mode_of(doSend, doRecv);
 
-    pplx_a2a_dispatch_args_t a{};
-    a.out_expert_num_tokens = static_cast<int32_t *>(outExpertNumTokens.data_ptr());
-    a.out_expert_num_tokens_stride = outExpertNumTokens.stride(0);
-    const int64_t esz = (int64_t)outExpertX.element_size();
-    a.out_expert_x = outExpertX.data_ptr();
-    a.out_expert_x_stride_row = outExpertX.stride(1) * esz;
-    a.out_expert_x_stride_expert = outExpertX.stride(0) * esz;
-    a.out_expert_x_rows = outExpertX.size(1);
-    if (outExpertXScale) {
-      a.out_expert_x_scale = static_cast<float *>(outExpertXScale->data_ptr());
-      a.out_expert_x_scale_stride_elem = outExpertXScale->stride(2);
-      a.out_expert_x_scale_stride_row = outExpertXScale->stride(1);
-      a.out_expert_x_scale_stride_expert = outExpertXScale->stride(0);
-    }
-    a.dp_x = dpX.data_ptr();
-    a.dp_x_stride_row = dpX.stride(0) * (int64_t)dpX.element_size();
-    if (dpXScale) {
-      a.dp_x_scale = static_cast<const float *>(dpXScale->data_ptr());
-      a.dp_x_scale_stride_elem = dpXScale->stride(1);
-      a.dp_x_scale_stride_row = dpXScale->stride(0);
-    }
-    a.indices = static_cast<const uint32_t *>(indices.data_ptr());
-    a.m = (uint32_t)indices.size(0);
-    a.bound_m = boundM ? static_cast<const uint32_t *>(boundM->data_ptr()) : nullptr;
+    const pplx_a2a_dispatch_args_t a =
+        pack_dispatch(outExpertNumTokens, outExpertX, outExpertXScale, dpX, dpXScale, indices, boundM);
 
     // Split calls go through staging that dispatch / combine never allocate; the reference's
     // callers do not know of it, so it is reserved the first time a rank splits a call.
@@ -366,34 +420,11 @@ void combine_core(fptr_t ptr, const at::Tensor &outTokens, const at::Tensor &ind
   try {
     auto found = g_ranks.find(ptr);
     if (found != g_ranks.end()) world = found->second.world;
-    check_tensor(outTokens, 2, "outTokens");
-    check_tensor(indices, 2, "indices");
-    TORCH_CHECK(indices.scalar_type() == at::kUInt32, "indices must be of type UInt32");
-    check_tensor(weights, 2, "weights");
-    TORCH_CHECK(weights.scalar_type() == at::kFloat, "weights must be of type Float");
-    check_tensor(expertY, 3, "expertY");
-    check_bound_m(boundM);
-    const int in_dtype = dtype_code(expertY.scalar_type());
-    TORCH_CHECK(in_dtype >= 0, "Unsupported dtype for expertY");
-    const int out_dtype = dtype_code(outTokens.scalar_type());
-    TORCH_CHECK(out_dtype == PPLX_A2A_BF16 || out_dtype == PPLX_A2A_F16, "Unsupported dtype for outTokens");
+    check_combine(outTokens, indices, weights, expertY, boundM);
     const RankRef ref = find_rank(ptr);
     const int mode = split_mode_of(doSend, doRecv);
 
-    pplx_a2a_combine_args_t a{};
-    a.out_tokens = outTokens.data_ptr();
-    a.out_tokens_stride_row = outTokens.stride(0);
-    a.out_dtype = out_dtype;
-    a.indices = static_cast<const uint32_t *>(indices.data_ptr());
-    a.weights = static_cast<const float *>(weights.data_ptr());
-    a.weights_stride_row = weights.stride(0);
-    a.expert_y = expertY.data_ptr();
-    a.expert_y_stride_row = expertY.stride(1);
-    a.expert_y_stride_expert = expertY.stride(0);
-    a.expert_y_rows = expertY.size(1);
-    a.in_dtype = in_dtype;
-    a.m = (uint32_t)indices.size(0);
-    a.bound_m = boundM ? static_cast<const uint32_t *>(boundM->data_ptr()) : nullptr;
+    const pplx_a2a_combine_args_t a = pack_combine(outTokens, indices, weights, expertY, boundM);
 
     arguments_refused = false;
     if (mode != PPLX_A2A_SPLIT_NONE) reserve_split_locked(*world, (int)expertY.element_size());
@@ -511,6 +542,124 @@ PyObject *py_combine(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// Entry r of a sequence argument; `keep` holds it until the call is over.
+struct Owned {
+  std::vector<PyObject *> refs;
+  explicit Owned(size_t n) { refs.reserve(n); }
+  Owned(const Owned &) = delete;
+  Owned &operator=(const Owned &) = delete;
+  ~Owned() {
+    for (PyObject *o : refs) Py_DECREF(o);
+  }
+};
+
+PyObject *entry(PyObject *seq, Py_ssize_t r, Owned &keep) {
+  PyObject *item = nullptr;
+  if (PyList_CheckExact(seq) && r < PyList_GET_SIZE(seq)) {
+    item = PyList_GET_ITEM(seq, r);
+    Py_INCREF(item);
+  } else {
+    PyObject *index = PyLong_FromSsize_t(r);
+    item = index ? PyObject_GetItem(seq, index) : nullptr;
+    Py_XDECREF(index);
+  }
+  if (!item) throw python_error();  // (the pending exception: an IndexError where a sequence is too short)
+  keep.refs.push_back(item);
+  return item;
+}
+
+// The library call itself runs without the interpreter lock.
+template <class Fn>
+int without_gil(Fn &&fn) {
+  PyThreadState *state = PyEval_SaveThread();
+  const int st = fn();
+  PyEval_RestoreThread(state);
+  return st;
+}
+
+pplx_a2a_config_t config_of_world(const pplx_a2a_world_t *ptr) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  for (const auto &named : g_worlds) {
+    if (named.second->ptr == ptr) return named.second->cfg;
+  }
+  TORCH_CHECK(false, "pplx_kernels: invalid state: the world has been destroyed");
+}
+
+pplx_a2a_world_t *world_arg(PyObject *obj) {
+  return reinterpret_cast<pplx_a2a_world_t *>((uintptr_t)int_arg(obj, "world"));
+}
+
+// world_dispatch(world, out_expert_num_tokens, out_expert_x, out_expert_x_scale, dp_x, dp_x_scale, indices,
+//                bound_m): entry r of every sequence is rank r's argument
+PyObject *py_world_dispatch(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  arity("world_dispatch", nargs, 8);
+  pplx_a2a_world_t *world = world_arg(args[0]);
+  const pplx_a2a_config_t cfg = config_of_world(world);
+  std::vector<pplx_a2a_dispatch_args_t> packed(cfg.world_size);
+  Owned keep(7 * (size_t)cfg.world_size);
+  void *stream = nullptr;
+  for (uint32_t r = 0; r < cfg.world_size; ++r) {
+    const at::Tensor &num_tokens = tensor_arg(entry(args[1], r, keep), "out_expert_num_tokens");
+    const at::Tensor &x = tensor_arg(entry(args[2], r, keep), "out_expert_x");
+    const at::Tensor *x_scale = optional_tensor_arg(entry(args[3], r, keep), "out_expert_x_scale");
+    const at::Tensor &dp_x = tensor_arg(entry(args[4], r, keep), "dp_x");
+    const at::Tensor *dp_x_scale = optional_tensor_arg(entry(args[5], r, keep), "dp_x_scale");
+    const at::Tensor &indices = tensor_arg(entry(args[6], r, keep), "indices");
+    const at::Tensor *bound_m = optional_tensor_arg(entry(args[7], r, keep), "bound_m");
+    check_dispatch(num_tokens, x, x_scale, dp_x, dp_x_scale, indices, bound_m);
+    check_picks(indices, cfg.experts_per_token);
+    packed[r] = pack_dispatch(num_tokens, x, x_scale, dp_x, dp_x_scale, indices, bound_m);
+    if (r == 0) stream = current_stream_of(indices);
+  }
+  A2A_CHECK(without_gil([&] { return pplx_a2a_world_dispatch(world, packed.data(), stream); }));
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// world_combine(world, out_tokens, indices, weights, expert_y, bound_m): the same
+PyObject *py_world_combine(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  arity("world_combine", nargs, 6);
+  pplx_a2a_world_t *world = world_arg(args[0]);
+  const pplx_a2a_config_t cfg = config_of_world(world);
+  std::vector<pplx_a2a_combine_args_t> packed(cfg.world_size);
+  Owned keep(5 * (size_t)cfg.world_size);
+  void *stream = nullptr;
+  for (uint32_t r = 0; r < cfg.world_size; ++r) {
+    const at::Tensor &out_tokens = tensor_arg(entry(args[1], r, keep), "out_tokens");
+    const at::Tensor &indices = tensor_arg(entry(args[2], r, keep), "indices");
+    const at::Tensor &weights = tensor_arg(entry(args[3], r, keep), "weights");
+    const at::Tensor &expert_y = tensor_arg(entry(args[4], r, keep), "expert_y");
+    const at::Tensor *bound_m = optional_tensor_arg(entry(args[5], r, keep), "bound_m");
+    check_combine(out_tokens, indices, weights, expert_y, bound_m);
+    packed[r] = pack_combine(out_tokens, indices, weights, expert_y, bound_m);
+    if (r == 0) stream = current_stream_of(indices);
+  }
+  A2A_CHECK(without_gil([&] { return pplx_a2a_world_combine(world, packed.data(), stream); }));
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// launch_bound(op, world, arguments, device): dispatch (op 0) or combine (op 1) of arguments that were
+// packed before (the address of `world_size` argument records), on the device's current stream
+PyObject *py_launch_bound(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  arity("launch_bound", nargs, 4);
+  const int64_t op = int_arg(args[0], "op");
+  pplx_a2a_world_t *world = world_arg(args[1]);
+  const void *packed = reinterpret_cast<const void *>((uintptr_t)int_arg(args[2], "arguments"));
+  const c10::DeviceIndex device = (c10::DeviceIndex)int_arg(args[3], "device");
+  (void)config_of_world(world);
+  void *stream = (void *)c10::hip::getCurrentHIPStream(device).stream();
+  A2A_CHECK(without_gil([&] {
+    return op == 0 ? pplx_a2a_world_dispatch(world, static_cast<const pplx_a2a_dispatch_args_t *>(packed), stream)
+                   : pplx_a2a_world_combine(world, static_cast<const pplx_a2a_combine_args_t *>(packed), stream);
+  }));
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
 PyObject *py_destroy_all(PyObject *, PyObject *) {
   HANDLE_TH_ERRORS
   destroy_all();
@@ -590,6 +739,14 @@ PyMethodDef kMethods[] = {
     {"combine", (PyCFunction)(void (*)(void))py_combine, METH_FASTCALL,
      "combine(fptr, out_tokens, indices, weights, expert_y, bound_m, do_send, do_recv): all_to_all_*_combine "
      "without the op dispatcher"},
+    {"world_dispatch", (PyCFunction)(void (*)(void))py_world_dispatch, METH_FASTCALL,
+     "world_dispatch(world, out_expert_num_tokens, out_expert_x, out_expert_x_scale, dp_x, dp_x_scale, indices, "
+     "bound_m): one dispatch step of all ranks; entry r of every sequence is rank r's argument"},
+    {"world_combine", (PyCFunction)(void (*)(void))py_world_combine, METH_FASTCALL,
+     "world_combine(world, out_tokens, indices, weights, expert_y, bound_m): one combine step of all ranks"},
+    {"launch_bound", (PyCFunction)(void (*)(void))py_launch_bound, METH_FASTCALL,
+     "launch_bound(op, world, arguments, device): dispatch (0) or combine (1) of packed arguments on the "
+     "device's current stream"},
     {"destroy_all", py_destroy_all, METH_NOARGS, "releases every rank handle and world"},
     {"is_live", py_is_live, METH_O, "is_live(fptr) -> bool"},
     {"world_ptr", py_world_ptr, METH_O, "world_ptr(fptr) -> address of the handle's pplx_a2a_world_t"},

@@ -8,10 +8,11 @@ Two shared objects sit next to this file (built by ``make -C pplx-kernels_amd/cs
   ``all_to_all_destroy`` with the reference's schemas (``all_to_all_ops.cpp:329-391``), as the
   reference's loader does with ``torch.ops.load_library`` (``src/pplx_kernels/ops.py:8-16``);
   its module functions ``_C.dispatch`` / ``_C.combine`` are the same code without the op
-  dispatcher, which ``AllToAll`` uses for eager calls.
+  dispatcher, which ``AllToAll`` uses for eager calls, and ``_C.world_dispatch`` /
+  ``_C.world_combine`` / ``_C.launch_bound`` take a step of all ranks for ``LoopbackWorld``.
 * ``libpplx_kernels.so`` -- the C ABI of ``include/pplx_a2a.h`` (kernels + host layer, no
-  torch types), which ``_C.so`` links against and which ``LoopbackWorld`` and the tests also
-  reach through ``ctypes``.
+  torch types), which ``_C.so`` links against and which ``LoopbackWorld`` (graphs, faults, arguments packed
+  once) and the tests also reach through ``ctypes``.
 
 A missing or unloadable library is an ``ImportError``: there is no fallback implementation.
 """

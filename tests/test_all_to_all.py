@@ -910,6 +910,52 @@ def test_bound_step_relaunches_with_new_inputs():
     world.destroy()
 
 
+def test_world_arguments_as_any_sequence():
+    """LoopbackWorld takes lists, tuples, stacked tensors and anything else that can be indexed, on
+    whatever stream is current; short sequences, foreign objects and wrong tensors are refused before
+    anything is launched."""
+    spec = _small_spec(name="sequences", in_dtype=FP8, hidden_dim=1024, tokens="uniform")
+    step = DeviceStep(spec, generate(spec))
+    world = make_world(spec, group_name="sequences")
+    step.expert_y_all.normal_()
+    R = spec.world_size
+    d = [step.expert_num_tokens_all, tuple(step.expert_x_all), {r: step.expert_x_scale_all[r] for r in range(R)},
+         step.dp_x + step.dp_x, step.dp_x_scale, tuple(step.indices), step.bound_m]  # fmt: skip
+    c = [tuple(step.out_tokens), step.indices, step.weights, step.expert_y_all, step.bound_m]
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        world.dispatch(*d)
+        world.combine(*c)
+    torch.cuda.current_stream().wait_stream(stream)
+    expected = check_dispatch_against_oracle(step)
+    check_combine_against_oracle(step, expected.slot_map)
+
+    with pytest.raises(IndexError):
+        world.dispatch(*d[:6], step.bound_m[:-1])
+    with pytest.raises(TypeError, match="weights must be a Tensor, not list"):
+        world.combine(*c[:2], [w.tolist() for w in step.weights], *c[3:])
+    with pytest.raises(RuntimeError, match="Tensor indices must be on GPU"):
+        world.dispatch(*d[:5], [i.cpu() for i in step.indices], d[6])
+    with pytest.raises(RuntimeError, match="indices.size\\(1\\) must be equal to the experts per token"):
+        world.dispatch(*d[:5], [i[:, :-1].contiguous() for i in step.indices], d[6])
+    with pytest.raises(RuntimeError, match="weights must be of type Float"):
+        world.combine(*c[:2], [w.double() for w in step.weights], *c[3:])
+    for t in step.out_tokens:
+        t.fill_(float("nan"))
+    bound = step.bind_world(world)
+    bound.dispatch(stream=torch.cuda.current_stream())
+    bound.combine()
+    expected = check_dispatch_against_oracle(step)
+    check_combine_against_oracle(step, expected.slot_map)
+    assert world.faults() == 0
+    world.destroy()
+    with pytest.raises(RuntimeError, match="the world has been destroyed"):
+        world.dispatch(*d)
+    with pytest.raises(RuntimeError, match="the world has been destroyed"):
+        bound.combine()
+
+
 def test_torch_cuda_graph_with_per_rank_calls():
     """The reference's "CUDA graph support" as a torch user meets it: torch.cuda.graph around
     the per-rank AllToAll calls, replayed with new inputs and a new bound_m."""

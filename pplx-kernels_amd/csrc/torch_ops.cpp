@@ -59,6 +59,7 @@ constexpr int kOps = 2, kModes = 3;  // (dispatch, combine) x (NONE, SEND, RECV)
 
 struct World {
   std::string key;
+  uint64_t id = 0;  // never given out again, unlike the address `ptr`
   pplx_a2a_config_t cfg{};
   pplx_a2a_world_t *ptr = nullptr;
   int handles = 0;
@@ -67,6 +68,13 @@ struct World {
   // called earlier are kept alive until then: a temporary such as x.to(device) must not go
   // back to the caching allocator before it has been read.
   std::array<std::vector<std::vector<at::Tensor>>, kOps * kModes> held;
+
+  World() = default;
+  World(const World &) = delete;
+  World &operator=(const World &) = delete;
+  ~World() {
+    if (ptr) (void)pplx_a2a_world_destroy(ptr);
+  }
 };
 
 struct RankRef {
@@ -75,14 +83,36 @@ struct RankRef {
 };
 
 std::mutex g_mu;  // guards the two maps and every World; held across a call into the library
-std::unordered_map<std::string, std::unique_ptr<World>> g_worlds;
+std::unordered_map<std::string, std::shared_ptr<World>> g_worlds;
 std::unordered_map<fptr_t, RankRef> g_ranks;
+
+// What a step of all ranks names its world by.  Such a step shares the world while it runs, so that
+// a world whose last rank goes meanwhile is freed behind it; `g_live_mu` is held for the lookup alone.
+std::mutex g_live_mu;
+std::unordered_map<uint64_t, std::shared_ptr<World>> g_live;
+uint64_t g_last_id = 0;
+
+std::shared_ptr<World> live_world(uint64_t id) {
+  std::lock_guard<std::mutex> lock(g_live_mu);
+  auto it = g_live.find(id);
+  TORCH_CHECK(it != g_live.end(), "pplx_kernels: invalid state: the world has been destroyed");
+  return it->second;
+}
 
 bool same_config(const pplx_a2a_config_t &a, const pplx_a2a_config_t &b) {
   return a.max_num_tokens == b.max_num_tokens && a.num_experts == b.num_experts &&
          a.experts_per_token == b.experts_per_token && a.world_size == b.world_size &&
          a.dp_size == b.dp_size && a.hidden_dim == b.hidden_dim &&
          a.hidden_dim_bytes == b.hidden_dim_bytes && a.hidden_dim_scale_bytes == b.hidden_dim_scale_bytes;
+}
+
+// Takes a world out of the maps; it goes when the caller, or a step that still runs, lets it go.
+std::shared_ptr<World> forget_world(std::unordered_map<std::string, std::shared_ptr<World>>::iterator it) {
+  std::shared_ptr<World> world = std::move(it->second);
+  g_worlds.erase(it);
+  std::lock_guard<std::mutex> lock(g_live_mu);
+  g_live.erase(world->id);
+  return world;
 }
 
 fptr_t create_rank(const std::string &transport, const std::string &group_name, int64_t maxNumTokens,
@@ -112,7 +142,7 @@ fptr_t create_rank(const std::string &transport, const std::string &group_name, 
                 "' already holds a world with a different configuration; destroy its ranks first or use "
                 "another group_name");
   } else {
-    auto world = std::make_unique<World>();
+    auto world = std::make_shared<World>();
     world->key = key;
     world->cfg = cfg;
     // The world lives on the caller's current device (device 0 when no GPU is visible, so that
@@ -120,6 +150,11 @@ fptr_t create_rank(const std::string &transport, const std::string &group_name, 
     const int device = c10::hip::device_count() > 0 ? (int)c10::hip::current_device() : 0;
     A2A_CHECK(pplx_a2a_world_create(&cfg, device, &world->ptr));
     for (auto &per_rank : world->held) per_rank.resize(cfg.world_size);
+    {
+      std::lock_guard<std::mutex> live(g_live_mu);
+      world->id = ++g_last_id;
+      g_live.emplace(world->id, world);
+    }
     it = g_worlds.emplace(key, std::move(world)).first;
   }
   World *world = it->second.get();
@@ -127,10 +162,7 @@ fptr_t create_rank(const std::string &transport, const std::string &group_name, 
   const int st = pplx_a2a_create(world->ptr, (uint32_t)rank, &handle);
   if (st != PPLX_A2A_OK) {
     const std::string msg = pplx_a2a_last_error();
-    if (world->handles == 0) {
-      (void)pplx_a2a_world_destroy(world->ptr);
-      g_worlds.erase(it);
-    }
+    if (world->handles == 0) (void)forget_world(it);
     TORCH_CHECK(false, "pplx_kernels: ", status_name(st), ": ", msg);
   }
   ++world->handles;
@@ -144,6 +176,7 @@ void release_held(World &world, uint32_t rank) {
 
 // csrc/bindings/all_to_all_ops.cpp:108
 void destroy(fptr_t ptr) {
+  std::shared_ptr<World> last;  // (let go behind the lock)
   std::lock_guard<std::mutex> lock(g_mu);
   auto it = g_ranks.find(ptr);
   TORCH_CHECK(it != g_ranks.end(), "pplx_kernels: unknown all-to-all handle ", ptr);
@@ -153,11 +186,12 @@ void destroy(fptr_t ptr) {
   g_ranks.erase(it);
   A2A_CHECK(pplx_a2a_destroy((pplx_a2a_t *)ptr));
   if (--world->handles == 0) {
-    const int st = pplx_a2a_world_destroy(world->ptr);
-    const std::string msg = st ? pplx_a2a_last_error() : "";
-    const std::string key = world->key;
-    g_worlds.erase(key);
-    TORCH_CHECK(st == PPLX_A2A_OK, "pplx_kernels: ", status_name(st), ": ", msg);
+    last = forget_world(g_worlds.find(world->key));
+    if (last.use_count() == 1) {  // (no step runs in it, and none can find it any more)
+      const int st = pplx_a2a_world_destroy(last->ptr);
+      last->ptr = nullptr;
+      A2A_CHECK(st);
+    }
   }
 }
 
@@ -166,8 +200,7 @@ void destroy_all() {
   std::lock_guard<std::mutex> lock(g_mu);
   for (auto &entry : g_ranks) (void)pplx_a2a_destroy((pplx_a2a_t *)entry.first);
   g_ranks.clear();
-  for (auto &entry : g_worlds) (void)pplx_a2a_world_destroy(entry.second->ptr);
-  g_worlds.clear();
+  while (!g_worlds.empty()) (void)forget_world(g_worlds.begin());
 }
 
 fptr_t create_intranode(int64_t maxNumTokens, int64_t numExperts, int64_t expertsPerToken, int64_t rank,
@@ -569,33 +602,26 @@ PyObject *entry(PyObject *seq, Py_ssize_t r, Owned &keep) {
 }
 
 // The library call itself runs without the interpreter lock.
+struct WithoutGil {
+  PyThreadState *state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
 template <class Fn>
 int without_gil(Fn &&fn) {
-  PyThreadState *state = PyEval_SaveThread();
-  const int st = fn();
-  PyEval_RestoreThread(state);
-  return st;
+  WithoutGil released;
+  return fn();
 }
 
-pplx_a2a_config_t config_of_world(const pplx_a2a_world_t *ptr) {
-  std::lock_guard<std::mutex> lock(g_mu);
-  for (const auto &named : g_worlds) {
-    if (named.second->ptr == ptr) return named.second->cfg;
-  }
-  TORCH_CHECK(false, "pplx_kernels: invalid state: the world has been destroyed");
-}
-
-pplx_a2a_world_t *world_arg(PyObject *obj) {
-  return reinterpret_cast<pplx_a2a_world_t *>((uintptr_t)int_arg(obj, "world"));
-}
+std::shared_ptr<World> world_arg(PyObject *obj) { return live_world((uint64_t)int_arg(obj, "world")); }
 
 // world_dispatch(world, out_expert_num_tokens, out_expert_x, out_expert_x_scale, dp_x, dp_x_scale, indices,
 //                bound_m): entry r of every sequence is rank r's argument
 PyObject *py_world_dispatch(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   arity("world_dispatch", nargs, 8);
-  pplx_a2a_world_t *world = world_arg(args[0]);
-  const pplx_a2a_config_t cfg = config_of_world(world);
+  const std::shared_ptr<World> world = world_arg(args[0]);
+  const pplx_a2a_config_t &cfg = world->cfg;
   std::vector<pplx_a2a_dispatch_args_t> packed(cfg.world_size);
   Owned keep(7 * (size_t)cfg.world_size);
   void *stream = nullptr;
@@ -612,7 +638,7 @@ PyObject *py_world_dispatch(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     packed[r] = pack_dispatch(num_tokens, x, x_scale, dp_x, dp_x_scale, indices, bound_m);
     if (r == 0) stream = current_stream_of(indices);
   }
-  A2A_CHECK(without_gil([&] { return pplx_a2a_world_dispatch(world, packed.data(), stream); }));
+  A2A_CHECK(without_gil([&] { return pplx_a2a_world_dispatch(world->ptr, packed.data(), stream); }));
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }
@@ -621,8 +647,8 @@ PyObject *py_world_dispatch(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 PyObject *py_world_combine(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   arity("world_combine", nargs, 6);
-  pplx_a2a_world_t *world = world_arg(args[0]);
-  const pplx_a2a_config_t cfg = config_of_world(world);
+  const std::shared_ptr<World> world = world_arg(args[0]);
+  const pplx_a2a_config_t &cfg = world->cfg;
   std::vector<pplx_a2a_combine_args_t> packed(cfg.world_size);
   Owned keep(5 * (size_t)cfg.world_size);
   void *stream = nullptr;
@@ -636,27 +662,41 @@ PyObject *py_world_combine(PyObject *, PyObject *const *args, Py_ssize_t nargs) 
     packed[r] = pack_combine(out_tokens, indices, weights, expert_y, bound_m);
     if (r == 0) stream = current_stream_of(indices);
   }
-  A2A_CHECK(without_gil([&] { return pplx_a2a_world_combine(world, packed.data(), stream); }));
+  A2A_CHECK(without_gil([&] { return pplx_a2a_world_combine(world->ptr, packed.data(), stream); }));
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }
 
-// launch_bound(op, world, arguments, device): dispatch (op 0) or combine (op 1) of arguments that were
-// packed before (the address of `world_size` argument records), on the device's current stream
+// launch_bound(op, world, arguments, device, stream): dispatch (op 0) or combine (op 1) of arguments that
+// were packed for this world before (the address of `world_size` argument records), on the stream with
+// this handle (None: the device's current one)
 PyObject *py_launch_bound(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  arity("launch_bound", nargs, 4);
+  arity("launch_bound", nargs, 5);
   const int64_t op = int_arg(args[0], "op");
-  pplx_a2a_world_t *world = world_arg(args[1]);
+  const std::shared_ptr<World> world = world_arg(args[1]);
   const void *packed = reinterpret_cast<const void *>((uintptr_t)int_arg(args[2], "arguments"));
-  const c10::DeviceIndex device = (c10::DeviceIndex)int_arg(args[3], "device");
-  (void)config_of_world(world);
-  void *stream = (void *)c10::hip::getCurrentHIPStream(device).stream();
+  void *stream = args[4] == Py_None
+                     ? (void *)c10::hip::getCurrentHIPStream((c10::DeviceIndex)int_arg(args[3], "device")).stream()
+                     : reinterpret_cast<void *>((uintptr_t)int_arg(args[4], "stream"));
   A2A_CHECK(without_gil([&] {
-    return op == 0 ? pplx_a2a_world_dispatch(world, static_cast<const pplx_a2a_dispatch_args_t *>(packed), stream)
-                   : pplx_a2a_world_combine(world, static_cast<const pplx_a2a_combine_args_t *>(packed), stream);
+    return op == 0
+               ? pplx_a2a_world_dispatch(world->ptr, static_cast<const pplx_a2a_dispatch_args_t *>(packed), stream)
+               : pplx_a2a_world_combine(world->ptr, static_cast<const pplx_a2a_combine_args_t *>(packed), stream);
   }));
   Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// world_faults(world, stream) -> the sticky fault bits since the last call (synchronises the stream)
+PyObject *py_world_faults(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  arity("world_faults", nargs, 2);
+  const std::shared_ptr<World> world = world_arg(args[0]);
+  void *stream = reinterpret_cast<void *>((uintptr_t)int_arg(args[1], "stream"));
+  uint32_t bits = 0;
+  A2A_CHECK(without_gil([&] { return pplx_a2a_world_faults(world->ptr, stream, &bits); }));
+  return PyLong_FromUnsignedLong(bits);
   END_HANDLE_TH_ERRORS
 }
 
@@ -681,6 +721,15 @@ PyObject *py_world_ptr(PyObject *, PyObject *arg) {
   const fptr_t ptr = int_arg(arg, "fptr");
   std::lock_guard<std::mutex> lock(g_mu);
   return PyLong_FromVoidPtr(find_rank(ptr).world->ptr);
+  END_HANDLE_TH_ERRORS
+}
+
+// world_id(fptr) -> the number of the handle's world, which no other world of the process gets
+PyObject *py_world_id(PyObject *, PyObject *arg) {
+  HANDLE_TH_ERRORS
+  const fptr_t ptr = int_arg(arg, "fptr");
+  std::lock_guard<std::mutex> lock(g_mu);
+  return PyLong_FromUnsignedLongLong(find_rank(ptr).world->id);
   END_HANDLE_TH_ERRORS
 }
 
@@ -745,11 +794,14 @@ PyMethodDef kMethods[] = {
     {"world_combine", (PyCFunction)(void (*)(void))py_world_combine, METH_FASTCALL,
      "world_combine(world, out_tokens, indices, weights, expert_y, bound_m): one combine step of all ranks"},
     {"launch_bound", (PyCFunction)(void (*)(void))py_launch_bound, METH_FASTCALL,
-     "launch_bound(op, world, arguments, device): dispatch (0) or combine (1) of packed arguments on the "
-     "device's current stream"},
+     "launch_bound(op, world, arguments, device, stream): dispatch (0) or combine (1) of packed arguments on "
+     "the stream with this handle, or the device's current one"},
+    {"world_faults", (PyCFunction)(void (*)(void))py_world_faults, METH_FASTCALL,
+     "world_faults(world, stream) -> sticky fault bits since the last call"},
     {"destroy_all", py_destroy_all, METH_NOARGS, "releases every rank handle and world"},
     {"is_live", py_is_live, METH_O, "is_live(fptr) -> bool"},
     {"world_ptr", py_world_ptr, METH_O, "world_ptr(fptr) -> address of the handle's pplx_a2a_world_t"},
+    {"world_id", py_world_id, METH_O, "world_id(fptr) -> number of the handle's world, never given out again"},
     {"reserve_split", (PyCFunction)(void (*)(void))py_reserve_split, METH_FASTCALL,
      "reserve_split(fptr, expert_y_elem_bytes)"},
     {"abandon_step", (PyCFunction)(void (*)(void))py_abandon_step, METH_FASTCALL,

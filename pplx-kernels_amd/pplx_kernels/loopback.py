@@ -59,31 +59,16 @@ class BoundStep:
     addresses, shapes and strides may not."""
 
     def __init__(self, world: "LoopbackWorld", dispatch_args, combine_args, device, keep: tuple) -> None:
-        self._world = world
-        self._dispatch_args = dispatch_args
-        self._combine_args = combine_args
-        self._device = device
-        self._keep = keep
-        self._lib = ops.load_library()
-        # what a launch on the current stream needs, as the plain numbers that _C takes
-        self._launch_dispatch = (0, world._world_ptr, ctypes.addressof(dispatch_args), device.index)
-        self._launch_combine = (1, world._world_ptr, ctypes.addressof(combine_args), device.index)
+        # (what the launches read: packed for this world, which is named by a number of its own)
+        self._keep = (dispatch_args, combine_args, keep)
+        self._launch_dispatch = (0, world._world_id, ctypes.addressof(dispatch_args), device.index)
+        self._launch_combine = (1, world._world_id, ctypes.addressof(combine_args), device.index)
 
     def dispatch(self, stream: torch.cuda.Stream | None = None) -> None:
-        if stream is None:
-            _launch_bound(*self._launch_dispatch)
-            return
-        ops.check_status(
-            self._lib.pplx_a2a_world_dispatch(self._world._world_ptr, self._dispatch_args, stream.cuda_stream)
-        )
+        _launch_bound(*self._launch_dispatch, None if stream is None else stream.cuda_stream)
 
     def combine(self, stream: torch.cuda.Stream | None = None) -> None:
-        if stream is None:
-            _launch_bound(*self._launch_combine)
-            return
-        ops.check_status(
-            self._lib.pplx_a2a_world_combine(self._world._world_ptr, self._combine_args, stream.cuda_stream)
-        )
+        _launch_bound(*self._launch_combine, None if stream is None else stream.cuda_stream)
 
 
 class LoopbackWorld:
@@ -117,7 +102,7 @@ class LoopbackWorld:
             )
             for r in range(world_size)
         ]
-        self._world_ptr = ops.world_of(self.ranks[0]._ptr).ptr
+        self._world_id = ops._C.world_id(self.ranks[0]._ptr)
 
     def dispatch(
         self,
@@ -131,7 +116,7 @@ class LoopbackWorld:
     ) -> None:
         """Entry ``r`` of every sequence is rank ``r``'s argument of ``AllToAll.dispatch``."""
         ops._C.world_dispatch(
-            self._world_ptr, out_expert_num_tokens, out_expert_x, out_expert_x_scale, dp_x, dp_x_scale, indices, bound_m
+            self._world_id, out_expert_num_tokens, out_expert_x, out_expert_x_scale, dp_x, dp_x_scale, indices, bound_m
         )
 
     def combine(
@@ -143,7 +128,7 @@ class LoopbackWorld:
         bound_m: Sequence[torch.Tensor | None],
     ) -> None:
         """Entry ``r`` of every sequence is rank ``r``'s argument of ``AllToAll.combine``."""
-        ops._C.world_combine(self._world_ptr, out_tokens, indices, weights, expert_y, bound_m)
+        ops._C.world_combine(self._world_id, out_tokens, indices, weights, expert_y, bound_m)
 
     def bind(
         self,
@@ -180,12 +165,7 @@ class LoopbackWorld:
         1 = a routed row did not fit ``out_expert_x.size(1)``, 2 = an expert index was out of
         range, 4 = combine met a slot beyond ``expert_y.size(1)``, 8 = an expert id repeated
         inside one token was dropped, 16 = a ``bound_m`` beyond ``max_num_tokens`` was clamped."""
-        bits = ctypes.c_uint32()
-        stream = torch.cuda.current_stream().cuda_stream
-        ops.check_status(
-            ops.load_library().pplx_a2a_world_faults(self._world_ptr, stream, ctypes.byref(bits))
-        )
-        return bits.value
+        return ops._C.world_faults(self._world_id, torch.cuda.current_stream().cuda_stream)
 
     @contextlib.contextmanager
     def capture(self):

@@ -956,6 +956,48 @@ def test_world_arguments_as_any_sequence():
         bound.combine()
 
 
+def test_a_world_that_replaces_another_does_not_run_its_bound_steps():
+    """Steps bound in a world of two ranks hold two records; worlds of eight ranks that come after it
+    (at the same address, for all the program knows) refuse them on either way to a stream."""
+    small = _small_spec(name="replaced", world_size=2, num_experts=8, hidden_dim=512)
+    large = _small_spec(name="replaced", world_size=8, num_experts=8, hidden_dim=512)
+    step = DeviceStep(small, generate(small))
+    for _ in range(4):
+        world = make_world(small, group_name="replaced")
+        bound = step.bind_world(world)
+        bound.dispatch()
+        check_dispatch_against_oracle(step)
+        world.destroy()
+        successor = make_world(large, group_name="replaced")
+        for launch in (bound.dispatch, bound.combine):
+            for kw in ({}, {"stream": torch.cuda.current_stream()}):
+                with pytest.raises(RuntimeError, match="the world has been destroyed"):
+                    launch(**kw)
+        with pytest.raises(RuntimeError, match="the world has been destroyed"):
+            world.faults()
+        assert successor.faults() == 0
+        successor.destroy()
+
+
+def test_a_world_outlives_the_step_that_runs_in_it():
+    """The last rank goes while a step's arguments are being read: the step still has its world."""
+    spec = _small_spec(name="outlives")
+    step = DeviceStep(spec, generate(spec))
+    world = make_world(spec, group_name="outlives")
+
+    class Destroys(list):
+        def __getitem__(self, r):
+            world.destroy()
+            return super().__getitem__(r)
+
+    world.dispatch(list(step.expert_num_tokens_all), list(step.expert_x_all), [None] * spec.world_size, step.dp_x,
+                   [None] * spec.world_size, step.indices, Destroys(step.bound_m))  # fmt: skip
+    assert world.ranks == []
+    check_dispatch_against_oracle(step)
+    with pytest.raises(RuntimeError, match="the world has been destroyed"):
+        world.faults()
+
+
 def test_torch_cuda_graph_with_per_rank_calls():
     """The reference's "CUDA graph support" as a torch user meets it: torch.cuda.graph around
     the per-rank AllToAll calls, replayed with new inputs and a new bound_m."""

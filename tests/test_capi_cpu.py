@@ -176,6 +176,18 @@ def test_operator_layer_checks_fire_before_the_device():
     with pytest.raises(RuntimeError, match="the handle has been destroyed"):
         C.world_ptr(12345)
     assert C.is_live(12345) is False
+    # a step of all ranks names its world by a number; whatever it comes with is not touched
+    for stream in (None, 0):
+        with pytest.raises(RuntimeError, match="the world has been destroyed"):
+            C.launch_bound(0, 12345, 0, 0, stream)
+    with pytest.raises(RuntimeError, match="the world has been destroyed"):
+        C.world_dispatch(12345, [], [], [], [], [], [], [])
+    with pytest.raises(RuntimeError, match="the world has been destroyed"):
+        C.world_combine(12345, [], [], [], [], [])
+    with pytest.raises(RuntimeError, match="the world has been destroyed"):
+        C.world_faults(12345, 0)
+    with pytest.raises(RuntimeError, match="the handle has been destroyed"):
+        C.world_id(12345)
     with pytest.raises(RuntimeError, match="negative rank"):
         torch.ops.pplx_kernels.all_to_all_intranode_create(8, 8, 2, -1, 4, 1, 64, 128, 0, "g")
     with pytest.raises(RuntimeError, match="negative or zero size"):

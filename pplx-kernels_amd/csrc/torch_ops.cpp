@@ -24,6 +24,7 @@
 #include <torch/library.h>
 
 #include <array>
+#include <iterator>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -82,7 +83,9 @@ struct RankRef {
   uint32_t rank;
 };
 
-std::mutex g_mu;  // guards the two maps and every World; held across a call into the library
+// Guards the two maps and every World; held across a call into the library, never while a tensor's last
+// reference goes (`Released`): a thread that holds it needs no interpreter lock.
+std::mutex g_mu;
 std::unordered_map<std::string, std::shared_ptr<World>> g_worlds;
 std::unordered_map<fptr_t, RankRef> g_ranks;
 
@@ -170,19 +173,31 @@ fptr_t create_rank(const std::string &transport, const std::string &group_name, 
   return (fptr_t)handle;
 }
 
-void release_held(World &world, uint32_t rank) {
-  for (auto &per_rank : world.held) per_rank[rank].clear();
+// Tensors that were kept for a step and are no longer: whoever takes g_mu declares one of these in
+// front of the lock, so that they go behind it.  The last reference to a tensor may need the
+// interpreter lock, which a thread that waits for g_mu may hold, and may run Python code that calls in
+// here again.
+typedef std::vector<at::Tensor> Released;
+
+void release(std::vector<at::Tensor> &kept, Released &released) {
+  released.insert(released.end(), std::make_move_iterator(kept.begin()), std::make_move_iterator(kept.end()));
+  kept.clear();
+}
+
+void release_held(World &world, uint32_t rank, Released &released) {
+  for (auto &per_rank : world.held) release(per_rank[rank], released);
 }
 
 // csrc/bindings/all_to_all_ops.cpp:108
 void destroy(fptr_t ptr) {
-  std::shared_ptr<World> last;  // (let go behind the lock)
+  std::shared_ptr<World> last;  // (let go behind the lock, like the tensors)
+  Released released;
   std::lock_guard<std::mutex> lock(g_mu);
   auto it = g_ranks.find(ptr);
   TORCH_CHECK(it != g_ranks.end(), "pplx_kernels: unknown all-to-all handle ", ptr);
   World *world = it->second.world;
   // (a handle that leaves in the middle of a step takes its half-made calls along)
-  release_held(*world, it->second.rank);
+  release_held(*world, it->second.rank, released);
   g_ranks.erase(it);
   A2A_CHECK(pplx_a2a_destroy((pplx_a2a_t *)ptr));
   if (--world->handles == 0) {
@@ -197,10 +212,11 @@ void destroy(fptr_t ptr) {
 
 // Interpreter exit: everything is released while the HIP runtime is still up.
 void destroy_all() {
+  std::vector<std::shared_ptr<World>> worlds;  // (let go behind the lock, with their tensors)
   std::lock_guard<std::mutex> lock(g_mu);
   for (auto &entry : g_ranks) (void)pplx_a2a_destroy((pplx_a2a_t *)entry.first);
   g_ranks.clear();
-  while (!g_worlds.empty()) (void)forget_world(g_worlds.begin());
+  while (!g_worlds.empty()) worlds.push_back(forget_world(g_worlds.begin()));
 }
 
 fptr_t create_intranode(int64_t maxNumTokens, int64_t numExperts, int64_t expertsPerToken, int64_t rank,
@@ -357,9 +373,9 @@ void reserve_split_locked(World &world, int expert_y_elem_bytes) {
   world.split_reserved = expert_y_elem_bytes;
 }
 
-void clear_held(World &world, int op) {
+void clear_held(World &world, int op, Released &released) {
   for (int mode = 0; mode < kModes; ++mode) {
-    for (auto &tensors : world.held[op * kModes + mode]) tensors.clear();
+    for (auto &tensors : world.held[op * kModes + mode]) release(tensors, released);
   }
 }
 
@@ -367,17 +383,18 @@ void clear_held(World &world, int op) {
 // for the phase is let go once the library holds no recorded call of it any more (the phase
 // has been launched, or the library gave the step up).
 void settle_held(World &world, uint32_t rank, int op, int mode, bool recorded,
-                 std::initializer_list<const at::Tensor *> tensors) {
+                 std::initializer_list<const at::Tensor *> tensors, Released &released) {
   uint32_t pending = 0;
   (void)pplx_a2a_world_recorded_calls(world.ptr, op, mode, &pending);
   auto &per_rank = world.held[op * kModes + mode];
   if (pending == 0) {
-    for (auto &kept : per_rank) kept.clear();
+    released.reserve(per_rank.size() * tensors.size());
+    for (auto &kept : per_rank) release(kept, released);
     return;
   }
   if (!recorded) return;
   auto &kept = per_rank[rank];
-  kept.clear();
+  release(kept, released);
   for (const at::Tensor *t : tensors) {
     if (t) kept.push_back(*t);
   }
@@ -387,12 +404,12 @@ void settle_held(World &world, uint32_t rank, int op, int mode, bool recorded,
 // the world waiting for it for good (every retry of an earlier rank "called twice"): the step
 // being assembled is given up, so that the caller can start it again from its first rank.
 // Returns the number of recorded calls that were dropped.
-uint32_t abandon_assembly(World *world, int op) {
+uint32_t abandon_assembly(World *world, int op, Released &released) {
   uint32_t dropped = 0;
   if (!world) return 0;
   (void)pplx_a2a_world_abandon_step(world->ptr, op == 0 ? PPLX_A2A_ABANDON_DISPATCH : PPLX_A2A_ABANDON_COMBINE,
                                     &dropped);
-  clear_held(*world, op);
+  clear_held(*world, op, released);
   return dropped;
 }
 
@@ -409,6 +426,7 @@ void *current_stream_of(const at::Tensor &t) {
 void dispatch_core(fptr_t ptr, const at::Tensor &outExpertNumTokens, const at::Tensor &outExpertX,
                    const at::Tensor *outExpertXScale, const at::Tensor &dpX, const at::Tensor *dpXScale,
                    const at::Tensor &indices, const at::Tensor *boundM, bool doSend, bool doRecv) {
+  Released released;
   std::lock_guard<std::mutex> lock(g_mu);
   World *world = nullptr;
   // What a failure means: refused arguments give the step being assembled up (below); call-order
@@ -434,11 +452,11 @@ void dispatch_core(fptr_t ptr, const at::Tensor &outExpertNumTokens, const at::T
     // stream is the current one of the tensors' device (csrc/bindings/all_to_all_ops.cpp:163,194).
     const int st = pplx_a2a_dispatch((pplx_a2a_t *)ptr, &a, mode, current_stream_of(indices));
     settle_held(*world, ref.rank, 0, mode, st == PPLX_A2A_OK,
-                {&outExpertNumTokens, &outExpertX, outExpertXScale, &dpX, dpXScale, &indices, boundM});
+                {&outExpertNumTokens, &outExpertX, outExpertXScale, &dpX, dpXScale, &indices, boundM}, released);
     arguments_refused = st == PPLX_A2A_INVALID_ARGUMENT;
     A2A_CHECK(st);
   } catch (const c10::Error &err) {
-    const uint32_t dropped = arguments_refused ? abandon_assembly(world, 0) : 0;
+    const uint32_t dropped = arguments_refused ? abandon_assembly(world, 0, released) : 0;
     if (dropped == 0) throw;
     A2A_RETHROW_ABANDONED(err, "dispatch", dropped);
   }
@@ -447,6 +465,7 @@ void dispatch_core(fptr_t ptr, const at::Tensor &outExpertNumTokens, const at::T
 // csrc/bindings/all_to_all_ops.cpp:238-311
 void combine_core(fptr_t ptr, const at::Tensor &outTokens, const at::Tensor &indices, const at::Tensor &weights,
                   const at::Tensor &expertY, const at::Tensor *boundM, bool doSend, bool doRecv) {
+  Released released;
   std::lock_guard<std::mutex> lock(g_mu);
   World *world = nullptr;
   bool arguments_refused = true;
@@ -462,11 +481,12 @@ void combine_core(fptr_t ptr, const at::Tensor &outTokens, const at::Tensor &ind
     arguments_refused = false;
     if (mode != PPLX_A2A_SPLIT_NONE) reserve_split_locked(*world, (int)expertY.element_size());
     const int st = pplx_a2a_combine((pplx_a2a_t *)ptr, &a, mode, current_stream_of(indices));
-    settle_held(*world, ref.rank, 1, mode, st == PPLX_A2A_OK, {&outTokens, &indices, &weights, &expertY, boundM});
+    settle_held(*world, ref.rank, 1, mode, st == PPLX_A2A_OK, {&outTokens, &indices, &weights, &expertY, boundM},
+                released);
     arguments_refused = st == PPLX_A2A_INVALID_ARGUMENT;
     A2A_CHECK(st);
   } catch (const c10::Error &err) {
-    const uint32_t dropped = arguments_refused ? abandon_assembly(world, 1) : 0;
+    const uint32_t dropped = arguments_refused ? abandon_assembly(world, 1, released) : 0;
     if (dropped == 0) throw;
     A2A_RETHROW_ABANDONED(err, "combine", dropped);
   }
@@ -751,12 +771,13 @@ PyObject *py_abandon_step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   arity("abandon_step", nargs, 2);
   const fptr_t ptr = int_arg(args[0], "fptr");
   const int64_t which = int_arg(args[1], "which");
+  Released released;
   std::lock_guard<std::mutex> lock(g_mu);
   World *world = find_rank(ptr).world;
   uint32_t dropped = 0;
   A2A_CHECK(pplx_a2a_world_abandon_step(world->ptr, (uint32_t)which, &dropped));
-  if (which & PPLX_A2A_ABANDON_DISPATCH) clear_held(*world, 0);
-  if (which & PPLX_A2A_ABANDON_COMBINE) clear_held(*world, 1);
+  if (which & PPLX_A2A_ABANDON_DISPATCH) clear_held(*world, 0, released);
+  if (which & PPLX_A2A_ABANDON_COMBINE) clear_held(*world, 1, released);
   return PyLong_FromUnsignedLong(dropped);
   END_HANDLE_TH_ERRORS
 }

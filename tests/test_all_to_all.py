@@ -1107,6 +1107,41 @@ def test_a_rank_replaced_in_the_middle_of_a_step():
         a.destroy()
 
 
+def test_a_kept_tensor_may_call_back_when_it_goes():
+    """A temporary that only the recorded call keeps alive runs a callback into the operator layer
+    with its last reference: wherever that goes, no lock is held any more."""
+    import weakref
+
+    from pplx_kernels import ops
+
+    spec = _small_spec(name="callback")
+    step = DeviceStep(spec, generate(spec))
+    ranks = _make_ranks(spec, "callback")
+    seen: list[str] = []
+
+    def dispatch_temporary(what: str) -> None:
+        kw = _dispatch_kw(step, 0)
+        kw["dp_x"] = kw["dp_x"].clone()
+        weakref.finalize(kw["dp_x"], lambda: seen.append(f"{what}: {ops._C.held_tensors(ranks[1]._ptr)} kept"))
+        ranks[0].dispatch(**kw)
+
+    dispatch_temporary("launched")
+    assert seen == []
+    for r in range(1, spec.world_size):
+        ranks[r].dispatch(**_dispatch_kw(step, r))
+    check_dispatch_against_oracle(step)
+    dispatch_temporary("refused")
+    with pytest.raises(RuntimeError, match="indices must be of type UInt32"):
+        ranks[1].dispatch(**{**_dispatch_kw(step, 1), "indices": step.indices[1].to(torch.int32)})
+    dispatch_temporary("abandoned")
+    assert ops.abandon_step(ranks[2]._ptr) == 1
+    dispatch_temporary("destroyed")
+    ranks[0].destroy()
+    assert seen == [f"{what}: 0 kept" for what in ("launched", "refused", "abandoned", "destroyed")]
+    for a in ranks[1:]:
+        a.destroy()
+
+
 def test_a_step_is_abandoned_when_a_rank_is_refused():
     """Rank 2's arguments fail their checks after ranks 0 and 1 have called: the half-assembled
     step is given up (nothing of it has reached the GPU), the tensors kept for it are let go,

@@ -220,6 +220,22 @@ int pplx_a2a_static_step(const pplx_a2a_config_t *cfg, int device,
                          const pplx_a2a_combine_args_t *combine_per_rank, uint32_t *fault_bits,
                          void *stream);
 
+/* Which kernels a step of a geometry runs as; for tests and tools.  Needs no GPU (it answers for one
+ * with 160 KiB of LDS per compute unit). */
+typedef enum pplx_a2a_dispatch_form {
+  PPLX_A2A_DISPATCH_ONE_LAUNCH = 0,     /* routing and scatter in one */
+  PPLX_A2A_DISPATCH_SLOT_MAP = 1,       /* the routing launches write the slots */
+  PPLX_A2A_DISPATCH_TABLES = 2,         /* the scatter works the slots out of the routing tables */
+  PPLX_A2A_DISPATCH_SCANNED_TABLES = 3  /* the same behind a scan of the tiles' counts */
+} pplx_a2a_dispatch_form;
+typedef struct pplx_a2a_plan {
+  int32_t dispatch_form;          /* pplx_a2a_dispatch_form */
+  uint32_t routing_tiles;
+  uint32_t scatter_waves_per_cu;  /* 0 = as many as fit, or no scatter launch */
+  int32_t scatter_in_turn;   /* 1: its waves fetch row, slots and buffers one behind the other */
+} pplx_a2a_plan_t;
+int pplx_a2a_plan(const pplx_a2a_config_t *cfg, pplx_a2a_plan_t *out);
+
 /* Parts of a step for pplx_a2a_world_abandon_step. */
 #define PPLX_A2A_ABANDON_DISPATCH 1u
 #define PPLX_A2A_ABANDON_COMBINE 2u

@@ -1099,6 +1099,22 @@ int pplx_a2a_static_step(const pplx_a2a_config_t *cfg, int device,
   return PPLX_A2A_OK;
 }
 
+int pplx_a2a_plan(const pplx_a2a_config_t *cfg, pplx_a2a_plan_t *out) {
+  if (!cfg || !out) return fail(PPLX_A2A_INVALID_ARGUMENT, "cfg / out is NULL");
+  if (int st = check_config(*cfg)) return st;
+  WorldDev d{};
+  fill_geometry(*cfg, d);
+  d.lds_per_cu = 160u << 10;
+  const DispatchPlan dispatch = dispatch_plan(d);
+  pplx_a2a_plan_t plan{};
+  plan.dispatch_form = (int32_t)dispatch.form;
+  plan.routing_tiles = d.num_tiles;
+  plan.scatter_waves_per_cu = dispatch.scatter_waves_per_cu;
+  plan.scatter_in_turn = dispatch.scatter_in_turn;
+  *out = plan;
+  return PPLX_A2A_OK;
+}
+
 int pplx_a2a_world_faults(pplx_a2a_world_t *w, void *stream, uint32_t *out_bits) {
   if (!w || !out_bits) return fail(PPLX_A2A_INVALID_ARGUMENT, "world / out_bits is NULL");
   DeviceScope scope(w->device);

@@ -244,6 +244,14 @@ int launch_split_stage_tokens(const WorldDev &w, const SplitDev &sp, const Dispa
 int launch_split_deliver(const WorldDev &w, const SplitDev &sp, const CombineRank *inline_rows, void *stream);
 // True when dispatch runs as the single fused launch for this geometry.
 bool dispatch_is_fused(const WorldDev &w);
+// What launch_dispatch does with this geometry (the values of pplx_a2a_plan_t).
+enum class DispatchForm : uint32_t { kOneLaunch = 0, kSlotMap = 1, kTables = 2, kScannedTables = 3 };
+struct DispatchPlan {
+  DispatchForm form;
+  uint32_t scatter_waves_per_cu;
+  bool scatter_in_turn;
+};
+DispatchPlan dispatch_plan(const WorldDev &w);
 // LDS bytes the routing kernels need for a given geometry.
 uint32_t route_lds_bytes(uint32_t num_experts, uint32_t tile_chunks);
 

@@ -83,8 +83,11 @@ enum class Slots {
   kTables,   // the routing tables as route_count left them (the same)
 };
 
-// One wave per token (or per share of its picks).
-template <int NV, bool EXACT, class DT, Slots SLOTS>
+// One wave per token (or per share of its picks).  It needs the row, the picks' slots and their experts'
+// buffers.  IN_TURN fetches them one behind the other; otherwise the picks go out first (loads return
+// in order) and what depends on them, the buffers and the routing tables, is fetched while the row is
+// still on its way.  Which steps want which: scatter_plan.
+template <int NV, bool EXACT, class DT, Slots SLOTS, bool IN_TURN>
 __device__ __forceinline__ void scatter_token(const WorldDev &w, const DT &tab, uint32_t wave, uint32_t ksplit,
                                               uint32_t kper) {
   const uint32_t lane = lane_id();
@@ -95,18 +98,22 @@ __device__ __forceinline__ void scatter_token(const WorldDev &w, const DT &tab, 
   if (g >= w.G) return;
   if (t >= dispatch_group_tokens(w, tab, g)) return;
   const DispatchRank &src = tab.at(sender_of(w, g, t));
-  // The picks go out first: loads return in order, so what depends on them (the experts' buffers
-  // and the routing tables) is fetched while the row is still on its way.
-  const uint32_t e = lane < w.K ? as_global(src.indices)[(size_t)t * w.K + lane] : w.E;
   RowRegs<NV> regs;
-  load_row<NV, EXACT>(w, src, t, lane, regs);
-  ExpertBuffer buffer = expert_buffer(w, tab, e);
+  if constexpr (IN_TURN) load_row<NV, EXACT>(w, src, t, lane, regs);
+  const uint32_t e = lane < w.K ? as_global(src.indices)[(size_t)t * w.K + lane] : w.E;
+  if constexpr (!IN_TURN) load_row<NV, EXACT>(w, src, t, lane, regs);
+  ExpertBuffer buffer;
+  if constexpr (!IN_TURN) buffer = expert_buffer(w, tab, e);
   uint32_t slot = kInvalidSlot;
   if constexpr (SLOTS == Slots::kMap) {
     if (lane < w.K && e < w.E) slot = as_global(w.slot_map)[(size_t)v * w.K + lane];
   } else {
     slot = slots_from_tables<SLOTS == Slots::kScanned>(w, v, lane, e);
     if (lane < w.K && part == 0) as_global(w.slot_map)[(size_t)v * w.K + lane] = slot;
+  }
+  if constexpr (IN_TURN) {
+    settle(slot);
+    buffer = expert_buffer(w, tab, e);
   }
   const Destination dst = destination_of(w, buffer, slot, part == 0);
   const uint32_t k0 = part * kper;
@@ -121,23 +128,23 @@ __device__ __forceinline__ void scatter_token(const WorldDev &w, const DT &tab, 
 // time (see launch_scatter_t); the kernels themselves do not touch LDS.
 template <int NV, bool EXACT, class DT>
 __global__ __launch_bounds__(kWave) void dispatch_scatter(WorldDev w, DT tab, uint32_t ksplit, uint32_t kper) {
-  scatter_token<NV, EXACT, DT, Slots::kMap>(w, tab, blockIdx.x, ksplit, kper);
+  scatter_token<NV, EXACT, DT, Slots::kMap, false>(w, tab, blockIdx.x, ksplit, kper);
 }
 
-template <int NV, bool EXACT, class DT>
+template <int NV, bool EXACT, class DT, bool IN_TURN>
 __global__ __launch_bounds__(kWave) void dispatch_scatter_scanned(WorldDev w, DT tab, uint32_t ksplit, uint32_t kper) {
-  scatter_token<NV, EXACT, DT, Slots::kScanned>(w, tab, blockIdx.x, ksplit, kper);
+  scatter_token<NV, EXACT, DT, Slots::kScanned, IN_TURN>(w, tab, blockIdx.x, ksplit, kper);
 }
 
 // The first ceil(E / 8) workgroups write the experts' totals.
-template <int NV, bool EXACT, class DT>
+template <int NV, bool EXACT, class DT, bool IN_TURN>
 __global__ __launch_bounds__(kWave) void dispatch_scatter_slots(WorldDev w, DT tab, uint32_t ksplit, uint32_t kper) {
   const uint32_t totals = (w.E + 7) / 8;
   if (blockIdx.x < totals) {
     write_totals(w, tab, blockIdx.x, lane_id());
     return;
   }
-  scatter_token<NV, EXACT, DT, Slots::kTables>(w, tab, blockIdx.x - totals, ksplit, kper);
+  scatter_token<NV, EXACT, DT, Slots::kTables, IN_TURN>(w, tab, blockIdx.x - totals, ksplit, kper);
 }
 
 // Threads of a dispatch_fused workgroup: 16 waves (fewer, larger workgroups repeat less
@@ -449,32 +456,52 @@ uint32_t pick_ksplit(const WorldDev &w, uint32_t max_split) {
   return ksplit;
 }
 
-// Scatter waves a CU should hold at a time (0 = as many as fit).
-// Measured on 8 x 4096 tokens (us of a step, dispatch and combine, at 3 / 4 / 6 / 8 / 12 / 16 waves
-// per CU / full occupancy; only the dispatch varies, and up to 1 % of it is noise):
-//   112 KiB stored per wave (14 KiB rows, top-8)      1546 / 1549 / 1552 / 1560 / 1565 / 1562 / 1563
-//   59 KiB (DSv3 fp8 rows, top-8)                     1134 / 1145 / 1144 / 1135 / 1129 / 1137 / 1134
-//   32 KiB (4 KiB fp8 rows with scales, top-8)         649 /  632 /  641 /  642 /  642 /  642 /  641
+// How the scatter's waves go about their stores: how many of them a CU holds at a time (0 = as many
+// as fit), and whether they take the row, the slots and the experts' buffers one behind the other
+// (scatter_token).  A wave's launch, its loads and its slot arithmetic are dead time for the stores, so
+// the less a wave stores the more of them it takes to keep the CU's stores going; where it stores much,
+// few waves keep the stores in longer runs, and large steps do best with three whose stores start
+// later.  Dispatch on 8 ranks, us, all forms alternating in one process on the same buffers (whose
+// place in memory moves all of them by up to 15 % from one process to the next); side by side at 4 and
+// 10 waves / one behind the other at 3:
+//   59 KiB stored per wave (DSv3 fp8 rows, top-8 of 256)
+//     8 x 509    52.7 /  -  / 53.0     8 x 1024  97.8 /  -  / 98.4    8 x 2048  184 / 189 / 185
+//     8 x 4096    432 / 431 / 430      8 x 6000   645 / 626 / 610     8 x 8192  859 / 843 / 826
+//     8 x 10000  1070 / 1038 / 1010    8 x 8192, half of the tokens absent  430 / 430 / 424
+//   48 KiB (6 KiB fp8 rows, top-8)     8 x 4096   338 / 337 / 325     8 x 8192  744 / 730 / 710
+//   64 KiB (8 KiB rows, top-8 of 64)   8 x 4096   428 / 442 / 431     8 x 8192   -  / 974 / 941
+//  112 KiB (14 KiB rows, top-8)        8 x 4096   852 /  -  / 845     8 x 8192 1682 /  -  / 1679
+//   40 KiB (10 KiB rows, top-4 of 32)  8 x 4096   328 / 332 / 311     8 x 8192   -  / 672 / 620
+//   32 KiB (8 KiB rows, top-4 of 32)   8 x 4096    -  / 225 / 208     8 x 8192   -  / 531 / 472
+//   32 KiB (4 KiB fp8 rows, top-8)     8 x 509   33.6 /  -  / 37.1    8 x 2048  108 / 109 / 107
+//     8 x 4096    209 / 212 / 206      8 x 6000   320 / 330 / 367     8 x 8192  458 / 478 / 584
+//   25 KiB (4 KiB rows, top-6 of 64)   8 x 4096   155 / 159 /  -      8 x 1024 43.7 / 45.8 / -
+//   24 KiB (3 KiB fp8 rows, top-8)     8 x 4096   157 / 162 / 172     8 x 8192  351 / 340 / 450
+// and whole steps of 8 x 4096 tokens at 3 / 4 / 6 / 8 / 12 / 16 waves / full occupancy, side by side:
 //   16 KiB (8 KiB rows, top-2)                         283 /  285 /  291 /  292 /  294 /  295 /  294
 //   17 KiB (2 KiB fp8 rows with scales, top-8)         357 /  337 /  316 /  311 /  312 /  314 /  315
 //   14 KiB (DSv3 fp8 rows, top-2)                      382 /  373 /  377 /  378 /  378 /  379 /  379
 //    8 KiB (1 KiB fp8 rows with scales, top-8)         226 /  202 /  179 /  169 /  159 /  159 /  160
 //    4 KiB (2 KiB fp8 rows with scales, top-2)         162 /  143 /  125 /  118 /  112 /  110 /  109
-// and on the Mixtral prefill (8 x 4096 tokens of 8 KiB, top-2, skewed routing) 271 / 267 / 276 / 279 /
-// 281.  Ragged and full steps of more than 16384 tokens of DSv3 rows do better with more waves (the
-// 8192-token prefill, half of its tokens absent: 1115 at 3, 1123 at 4, 1113 / 1108 / 1086 / 1100 at 6 / 8 /
-// 10 / 12: absent tokens' waves pass through the same slots), 14 KiB rows do not (8 x 4096 tokens, half of
-// them absent: 763 at 4, 774 at 10).  A wave's launch, its loads and its slot arithmetic are dead time for the stores, so the less
-// a wave stores the more of them it takes to keep the CU's stores going; where it stores much, few
-// waves per CU keep the stores in longer runs.
-uint32_t scatter_waves_per_cu(const WorldDev &w, uint32_t picks_per_wave) {
-  if (w.lds_per_cu == 0) return 0;
+// (one behind the other they lose: 8 x 4096 tokens of 8 KiB, top-2, skewed: 123 and 130; 2 KiB rows,
+// top-6, 8 x 1024: 26.2 and 27.5).
+struct ScatterPlan {
+  uint32_t waves_per_cu;
+  bool in_turn;
+};
+
+ScatterPlan scatter_plan(const WorldDev &w, uint32_t picks_per_wave) {
+  if (w.lds_per_cu == 0) return {0, false};
+  const uint64_t tokens = (uint64_t)w.G * w.M;
   const uint64_t row = w.Hb + 4ull * w.S;
   const uint64_t stored = (uint64_t)picks_per_wave * row;
-  if (stored >= 24 * 1024) return (uint64_t)w.G * w.M > 16384 && stored < 96 * 1024 ? 10 : 4;
-  if (stored >= 12 * 1024) return row >= 4096 ? 4 : 10;
-  if (stored >= 6 * 1024) return 12;
-  return 0;
+  if (stored >= 24 * 1024) {
+    if (tokens <= 16384) return {4, false};
+    if (stored >= 48 * 1024 || (stored >= 32 * 1024 && (row >= 8192 || tokens <= 32768))) return {3, true};
+    return {stored >= 32 * 1024 || tokens <= 32768 ? 4u : 10u, false};
+  }
+  if (stored >= 12 * 1024) return {row >= 4096 ? 4u : 10u, false};
+  return {stored >= 6 * 1024 ? 12u : 0u, false};
 }
 
 // Rows that dispatch_scatter holds in registers (longer ones stream through dispatch_scatter_long).
@@ -493,12 +520,12 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t 
   // One wave per workgroup, and few of them per CU at a time.  A wave reads one row and then
   // has up to K rows of stores to issue; HBM takes those stores best when a CU sends the rows of
   // three or four waves at a time rather than those of thirty-two interleaved (figures at
-  // scatter_waves_per_cu).  The hardware has no such knob, so each workgroup asks for a share of
+  // scatter_plan).  The hardware has no such knob, so each workgroup asks for a share of
   // the CU's LDS that only that many fit into.
-  const uint32_t waves_per_cu = scatter_waves_per_cu(w, kper);
+  const ScatterPlan plan = scatter_plan(w, kper);
   // (LDS is handed out in blocks: a share that is not a multiple of 4 KiB can round up past
   // what the intended number of workgroups leaves room for)
-  uint32_t lds = waves_per_cu ? (w.lds_per_cu / waves_per_cu) & ~4095u : 0u;
+  uint32_t lds = plan.waves_per_cu ? (w.lds_per_cu / plan.waves_per_cu) & ~4095u : 0u;
   if (lds > 65536u) lds = 65536u;
   const dim3 grid((uint32_t)waves + (slots == Slots::kTables ? (w.E + 7) / 8 : 0u)), block(kWave);
 #define PPLX_ROW_KERNEL_ARGS ksplit, kper
@@ -511,18 +538,29 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t 
     PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter);
   }
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
-  // (rows beyond 16 KiB leave no registers for the slot arithmetic: slots_in_scatter() sends
-  // them through route_slots and the kernel above)
+  // (rows beyond 16 KiB leave no registers for the slot arithmetic: slots_of() sends them through
+  // route_slots and the kernel above)
 #define PPLX_LAUNCH_LARGE_ROW_VARIANT(KERNEL)                                                    \
   do {                                                                                           \
     if (per_lane <= 16) PPLX_LAUNCH_ROW_VARIANT(KERNEL, 16, false);                              \
     else return (int)hipErrorInvalidValue;                                                       \
+  } while (0)
+#undef PPLX_LAUNCH_ROW_VARIANT
+#define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                               \
+  do {                                                                                           \
+    if (plan.in_turn)                                                                       \
+      hipLaunchKernelGGL((KERNEL<NV, EXACT, DT, true>), grid, block, lds, s, w, tab, ksplit, kper);  \
+    else                                                                                         \
+      hipLaunchKernelGGL((KERNEL<NV, EXACT, DT, false>), grid, block, lds, s, w, tab, ksplit, kper); \
   } while (0)
   if (slots == Slots::kScanned) {
     PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter_scanned);
   } else if (slots == Slots::kTables) {
     PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter_slots);
   }
+#undef PPLX_LAUNCH_ROW_VARIANT
+#define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                               \
+  hipLaunchKernelGGL((KERNEL<NV, EXACT, DT>), grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS)
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
 #undef PPLX_ROW_KERNEL_ARGS
   return (int)hipGetLastError();
@@ -556,6 +594,13 @@ int launch_fused_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hipSt
   return (int)hipGetLastError();
 }
 
+// Steps of several tiles leave the last routing launch out (the scatter's waves work their own
+// slots out of the tiles' tables), and the scan too as long as an expert's counts are one line.
+Slots slots_of(const WorldDev &w) {
+  if (w.num_tiles == 1 || (w.Hb / 16 + kWave - 1) / kWave > 16) return Slots::kMap;
+  return w.num_tiles <= kScanFreeTiles ? Slots::kTables : Slots::kScanned;
+}
+
 template <class DT>
 int launch_dispatch_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hipStream_t s) {
   if (dispatch_is_fused(w)) return launch_fused_t(w, tab, pick_vector, s);
@@ -566,11 +611,8 @@ int launch_dispatch_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hi
   span.pick_vector = pick_vector;
   span.tile_cnt = w.tile_cnt;
   span.slot_out = w.slot_map;
-  // Steps of several tiles leave the last routing launch out (the scatter's waves work their own
-  // slots out of the tiles' tables), and the scan too as long as an expert's counts are one line.
-  Slots slots = Slots::kMap;
-  if (w.num_tiles > 1 && (w.Hb / 16 + kWave - 1) / kWave <= 16) {
-    slots = w.num_tiles <= kScanFreeTiles ? Slots::kTables : Slots::kScanned;
+  const Slots slots = slots_of(w);
+  if (slots != Slots::kMap) {
     const RouteTables tables = route_tables(w.num_tiles, w.tile_chunks, w.E);
     uint8_t *base = reinterpret_cast<uint8_t *>(w.tile_cnt);
     span.tile_mask = reinterpret_cast<unsigned long long *>(base + tables.mask_offset);
@@ -609,6 +651,18 @@ bool dispatch_is_fused(const WorldDev &w) {
   const uint32_t waves = fused_threads((int)per_lane) / kWave;
   const uint64_t stored = tokens * w.K * (w.Hb + 4ull * w.S);
   return tokens <= 256u * waves && (waves < 16 || tokens <= 1792 || stored <= kFusedMaxBytes);
+}
+
+DispatchPlan dispatch_plan(const WorldDev &w) {
+  if (dispatch_is_fused(w)) return {DispatchForm::kOneLaunch, 0, false};
+  const Slots slots = slots_of(w);
+  const DispatchForm form = slots == Slots::kMap      ? DispatchForm::kSlotMap
+                            : slots == Slots::kTables ? DispatchForm::kTables
+                                                      : DispatchForm::kScannedTables;
+  if (!scatter_has_register_rows(w)) return {form, 0, false};
+  const uint32_t ksplit = pick_ksplit(w, kWave);
+  const ScatterPlan plan = scatter_plan(w, (w.K + ksplit - 1) / ksplit);
+  return {form, plan.waves_per_cu, plan.in_turn && slots != Slots::kMap};
 }
 
 int launch_bind_dispatch(const WorldDev &w, const BindDispatchBatch &b, void *stream) {

@@ -54,6 +54,7 @@ EXPORTED_SYMBOLS = (
     "pplx_a2a_world_dispatch",
     "pplx_a2a_world_combine",
     "pplx_a2a_static_step",
+    "pplx_a2a_plan",
     "pplx_a2a_world_recorded_calls",
     "pplx_a2a_world_abandon_step",
     "pplx_a2a_world_reserve_split",
@@ -80,6 +81,17 @@ class Config(ctypes.Structure):
         ("hidden_dim", ctypes.c_uint64),
         ("hidden_dim_bytes", ctypes.c_uint64),
         ("hidden_dim_scale_bytes", ctypes.c_uint64),
+    ]
+
+
+class Plan(ctypes.Structure):
+    """pplx_a2a_plan_t"""
+
+    _fields_ = [
+        ("dispatch_form", ctypes.c_int32),
+        ("routing_tiles", ctypes.c_uint32),
+        ("scatter_waves_per_cu", ctypes.c_uint32),
+        ("scatter_in_turn", ctypes.c_int32),
     ]
 
 
@@ -165,6 +177,7 @@ def load_library() -> ctypes.CDLL:
         lib.pplx_a2a_static_step.argtypes = [
             ctypes.POINTER(Config), i32, ctypes.POINTER(DispatchArgs), ctypes.POINTER(CombineArgs), vp, vp,
         ]  # fmt: skip
+        lib.pplx_a2a_plan.argtypes = [ctypes.POINTER(Config), ctypes.POINTER(Plan)]
         lib.pplx_a2a_world_of.argtypes = [vp]
         lib.pplx_a2a_world_of.restype = vp
         lib.pplx_a2a_world_recorded_calls.argtypes = [vp, i32, i32, ctypes.POINTER(u32)]
@@ -182,6 +195,13 @@ def load_library() -> ctypes.CDLL:
             getattr(lib, name)  # AttributeError here means a stale or foreign library
         _lib = lib
     return _lib
+
+
+def plan_of(config: Config) -> Plan:
+    """Which kernels a step of this geometry runs as (no GPU needed)."""
+    plan = Plan()
+    check_status(load_library().pplx_a2a_plan(ctypes.byref(config), ctypes.byref(plan)))
+    return plan
 
 
 def check_status(status: int) -> None:

@@ -9,9 +9,11 @@ import numpy as np
 import pytest
 import torch
 
+from pplx_kernels import ops
 from tests.all_to_all_utils import (
     COMBINE_ATOL,
     COMBINE_RTOL,
+    FP8,
     ORACLE_DTYPE,
     DeviceStep,
     WorkloadSpec,
@@ -22,8 +24,12 @@ from tests.all_to_all_utils import (
     to_oracle_groups,
     torch_bits,
 )
+from tests.test_contract import FAULT_BAD_EXPERT, FAULT_DUPLICATE, FAULT_ROW_DROPPED, _check_with_repeats_dropped
 
 pytestmark = pytest.mark.gpu
+
+# pplx_a2a_dispatch_form
+ONE_LAUNCH, SLOT_MAP, TABLES, SCANNED_TABLES = range(4)
 
 
 # ---------------------------------------------------------------------------
@@ -110,6 +116,47 @@ def test_slots_from_the_routing_tables(E, K, M, R, hidden_bytes):
         step.dispatch_world(world)
         check_dispatch_against_oracle(step)
     assert world.faults() == 0
+    world.destroy()
+
+
+@pytest.mark.parametrize(
+    "E,K,M,R,hidden_bytes,form",
+    [
+        (64, 8, 2100, 8, 7168, TABLES),
+        (40, 5, 2100, 8, 8208, TABLES),  # no whole registers
+        (24, 3, 2100, 8, 16384, TABLES),  # the longest rows that do
+        (256, 8, 8200, 8, 7168, SCANNED_TABLES),
+        (144, 7, 240, 72, 7168, TABLES),  # rank tables in HBM
+    ],
+)
+@pytest.mark.parametrize("faults", [False, True], ids=["", "faults"])
+def test_scatter_that_fetches_row_slots_and_buffers_in_turn(E, K, M, R, hidden_bytes, form, faults):
+    fp8 = hidden_bytes == 7168
+    spec = WorkloadSpec(
+        "in-turn", 75, R, E, K, hidden_bytes if fp8 else hidden_bytes // 2, M, FP8 if fp8 else torch.bfloat16
+    )
+    groups = generate(spec, seed=E)
+    for i, g in enumerate(groups):  # (the batch need not be full for the form to be the one of full ones)
+        g.n = (i * 37 + 5) % 90
+    if faults:
+        groups[1].indices[3, 1] = E + 7
+        groups[2].indices[4, K - 1] = groups[2].indices[4, 0]
+    ids = np.concatenate([g.indices[: g.n].reshape(-1).numpy() for g in groups])
+    load = int(np.bincount(ids[ids < E], minlength=E).max())
+    step = DeviceStep(spec, groups, cap=load - 2 if faults else load, alloc_expert_y=False)
+    plan = ops.plan_of(
+        ops.Config(M, E, K, R, 1, spec.hidden_dim, spec.hidden_dim_bytes, spec.hidden_dim_scale_bytes)
+    )
+    assert plan.dispatch_form == form and plan.scatter_in_turn
+    world = make_world(spec, group_name="in-turn")
+    for _ in range(2):
+        step.dispatch_world(world)
+        if faults:
+            _check_with_repeats_dropped(step, after_combine=False)
+            assert world.faults() == FAULT_ROW_DROPPED | FAULT_BAD_EXPERT | FAULT_DUPLICATE
+        else:
+            check_dispatch_against_oracle(step)
+            assert world.faults() == 0
     world.destroy()
 
 

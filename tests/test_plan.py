@@ -1,0 +1,62 @@
+"""Which kernels a step runs as, on both sides of every line of the rules (no GPU needed)."""
+
+from __future__ import annotations
+
+import pytest
+
+from pplx_kernels import ops
+
+ONE_LAUNCH, SLOT_MAP, TABLES, SCANNED_TABLES = range(4)
+
+
+def plan(tokens, row, topk, experts=64, scales=0, ranks=8, dp=1):
+    """`tokens` of all groups, rows of `row` bytes with `scales` floats."""
+    assert tokens * dp % ranks == 0
+    return ops.plan_of(
+        ops.Config(tokens * dp // ranks, experts, topk, ranks, dp, row // 2, row, 4 * scales)
+    )
+
+
+@pytest.mark.parametrize(
+    "tokens,row,scales,topk,waves,in_turn",
+    [
+        # 48 KiB and more per wave: three waves, one fetch behind the other, beyond 16384 tokens
+        (16384, 7168, 56, 8, 4, False),
+        (16392, 7168, 56, 8, 3, True),
+        (65536, 7168, 56, 8, 3, True),
+        (80000, 7168, 56, 8, 3, True),
+        (32768, 14336, 0, 8, 3, True),
+        (65536, 16384, 0, 3, 3, True),
+        # from 32 KiB on: the same up to 32768 tokens, or for rows of 8 KiB and more
+        (16384, 4096, 0, 8, 4, False),
+        (16392, 4096, 0, 8, 3, True),
+        (32768, 4096, 0, 8, 3, True),
+        (32776, 4096, 0, 8, 4, False),
+        (32776, 8192, 0, 4, 3, True),
+        (32776, 8176, 0, 6, 4, False),
+        (65536, 10240, 0, 4, 3, True),
+        # from 24 KiB on
+        (16392, 4096, 0, 6, 4, False),
+        (32768, 8192, 0, 3, 4, False),
+        (32776, 8192, 0, 3, 10, False),
+        # less
+        (32768, 8192, 0, 2, 4, False),
+        (32768, 2048, 16, 8, 10, False),
+        (32768, 1024, 8, 8, 12, False),
+        (32768, 2048, 16, 2, 0, False),
+    ],
+)
+def test_scatter(tokens, row, scales, topk, waves, in_turn):
+    p = plan(tokens, row, topk, scales=scales)
+    assert p.dispatch_form == (TABLES if tokens <= 65536 else SCANNED_TABLES)
+    assert (p.scatter_waves_per_cu, bool(p.scatter_in_turn)) == (waves, in_turn)
+
+
+def test_forms_of_the_routing():
+    assert plan(4104, 1024, 2).dispatch_form == TABLES  # 65 chunks
+    assert plan(65536, 1024, 2).routing_tiles == 64
+    assert plan(65544, 1024, 2).dispatch_form == SCANNED_TABLES
+    assert plan(4104, 16384 + 16, 2).dispatch_form == SLOT_MAP  # beyond the register variants
+    assert plan(8, 1024, 2).dispatch_form == ONE_LAUNCH
+    with pytest.raises(RuntimeError, match="experts_per_token"):
+        plan(8, 1024, 0)

@@ -198,9 +198,6 @@ constexpr uint32_t kBindBatch = 64;
 // A fused launch whose rows (all picks of all tokens) stay within this many bytes stores them
 // write-through into the 256 MB last-level cache instead of streaming them past it.
 constexpr uint64_t kWriteThroughMaxBytes = 192ull << 20;
-// Up to this many bytes of rows the fused launch is the faster one also for steps of many tokens
-// (dispatch_is_fused).
-constexpr uint64_t kFusedMaxBytes = 112ull << 20;
 
 // Device memory that pplx_a2a_static_step works in instead of a world's allocations: a fixed
 // array inside the library's code object (a2a_static.hip), one copy per GPU.  The chunks' bases

@@ -638,19 +638,34 @@ bool dispatch_is_fused(const WorldDev &w) {
   // One launch while a workgroup per CU can own all tokens, one wave each: 4096 tokens, or 2048 of
   // rows that take 512-thread workgroups (beyond that a second round of workgroups recounts
   // everything: 8 ranks, 2 KiB rows, top-6 of 64: 4096 tokens 15.0 us against 15.9 with the routing
-  // in a launch of its own, 5120 tokens 24.2 against 20.0).  All of a workgroup's row waves store at
-  // once, though, where the scatter keeps few storing waves per CU, and that costs more than the
-  // routing launch once the rows no longer land in the last-level cache.  Measured on 8 ranks (us,
-  // one launch / routing + scatter; MB of rows stored): 7 KiB fp8 rows, top-8 of 256: 1536 tokens
-  // 18.9 / 24.8 (91), 1792 24.2 / 27.5 (106), 1920 28.4 / 28.6 (114), 2048 31.0 / 29.8 (121), 3072 45.3 /
-  // 40.4; 4 KiB rows, top-8 of 64: 3072 22.0 / 25.1 (104), 4080 32.2 / 31.5 (138); 8 KiB rows, top-2 of 8:
-  // 3072 14.2 / 18.1, 4080 20.6 / 21.2 (67); 14 KiB rows, top-8: 1280 34.2 / 36.4 (147), 2048 53.0 / 54.6,
-  // 2560 65.8 / 61.3.
+  // in a launch of its own, 5120 tokens 24.2 against 20.0; 14 KiB rows, top-8: 2048 tokens 53.0 / 54.6,
+  // 2560 65.8 / 61.3).  All of a workgroup's row waves store at once, though, where the scatter keeps few
+  // storing waves per CU, and that costs more than the routing launch once the rows fill the last-level
+  // cache.  Where that is depends on the rows; on 8 ranks, top-8 (us, one launch / routing + scatter; MiB of
+  // rows stored):
+  //   fp8 rows with scales, 7 KiB: 108 29.5 / 30.4, 116 31.1 / 31.8, 130 34.1 / 33.8, 144 37.3 / 36.5,
+  //     159 42.1 / 40.9; 6 KiB: 111 29.0 / 31.2, 148 36.4 / 36.7; 5 KiB: 124 33.2 / 31.1, 144 37.2 / 36.0;
+  //     4 KiB: 107 26.9 / 29.1, 116 28.8 / 33.8, 132 32.0 / 32.7
+  //   whole lines only (no scales), 8 KiB: 116 28.6 / 30.5, 144 34.5 / 36.9, 160 37.8 / 42.2, 176 40.7 /
+  //     42.8, 192 45.2 / 45.8; 7 KiB: 126 30.8 / 33.4, 140 33.9 / 35.8, 154 36.5 / 38.7; the same with half of
+  //     the tokens absent (8 KiB, 144: 21.3 / 23.2), and for 8 KiB rows with scales (148 35.5 / 37.9,
+  //     182 42.8 / 44.2): these run up to 176
+  // The recount weighs more where it cannot take four picks at a time, or has more than eight: 8 KiB rows,
+  // top-5 120 33.1 / 31.2; top-6 120 32.7 / 32.0; top-9 117 33.3 / 31.7; top-10 120 33.8 / 32.7, 140 38.3 / 36.4;
+  // top-12 120 34.4 / 31.5; top-16 160 58.4 / 41.2 (but 113 39.4 / 42.4, 120 42.1 / 44.5: up to 1024 tokens
+  // the slots take a launch of a single workgroup).
   const uint64_t tokens = (uint64_t)w.G * w.M;
   const uint32_t per_lane = (w.Hb / 16 + kWave - 1) / kWave;
   const uint32_t waves = fused_threads((int)per_lane) / kWave;
   const uint64_t stored = tokens * w.K * (w.Hb + 4ull * w.S);
-  return tokens <= 256u * waves && (waves < 16 || tokens <= 1792 || stored <= kFusedMaxBytes);
+  if (tokens > 256u * waves) return false;
+  if (waves < 16) return true;
+  const bool quick_count = w.K % 4 == 0 && w.K <= 8;
+  const bool whole_lines = w.S == 0 || w.Hb >= 8192;
+  uint64_t limit = 112ull << 20;
+  if (quick_count || (tokens <= 1024 && w.K <= 16)) limit = 120ull << 20;
+  if (quick_count && whole_lines && tokens <= 3072) limit = 176ull << 20;
+  return stored <= limit;
 }
 
 DispatchPlan dispatch_plan(const WorldDev &w) {

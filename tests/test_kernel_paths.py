@@ -161,19 +161,30 @@ def test_scatter_that_fetches_row_slots_and_buffers_in_turn(E, K, M, R, hidden_b
 
 
 @pytest.mark.parametrize(
-    "M,topk,hidden,in_dtype",
+    "M,topk,hidden,in_dtype,form",
     [
-        (1792, 8, 1792, torch.bfloat16),  # the last 3584-byte step of one launch by its row count
-        (1793, 8, 8192, torch.bfloat16),  # 235 MB of rows: routing and scatter
-        (2048, 1, 4096, torch.bfloat16),  # up to 4096 tokens in one launch while the rows are few
-        (4096, 1, 64, torch.bfloat16),
-        (4097, 1, 64, torch.bfloat16),  # routing and scatter
-        (2048, 1, 5120, torch.bfloat16),  # rows of 512-thread workgroups: up to 2048 tokens
-        (2049, 1, 5120, torch.bfloat16),
+        (1792, 8, 1792, torch.bfloat16, ONE_LAUNCH),
+        (1793, 8, 8192, torch.bfloat16, ONE_LAUNCH),  # 512-thread workgroups: no limit of bytes
+        (2048, 1, 4096, torch.bfloat16, ONE_LAUNCH),
+        (4096, 1, 64, torch.bfloat16, ONE_LAUNCH),  # the last step that a workgroup per CU can own
+        (4097, 1, 64, torch.bfloat16, TABLES),
+        (2048, 1, 5120, torch.bfloat16, ONE_LAUNCH),  # the last one of 512-thread workgroups
+        (2049, 1, 5120, torch.bfloat16, TABLES),
+        (2816, 8, 4096, torch.bfloat16, ONE_LAUNCH),  # 176 MiB of whole lines
+        (2817, 8, 4096, torch.bfloat16, TABLES),
+        (2127, 8, 7168, FP8, ONE_LAUNCH),  # 120 MiB with scales
+        (2128, 8, 7168, FP8, TABLES),
+        (1792, 8, 4096, torch.bfloat16, ONE_LAUNCH),  # 112 MiB
+        (1592, 9, 4096, torch.bfloat16, ONE_LAUNCH),  # 112 MiB of picks that are counted one at a time
+        (1593, 9, 4096, torch.bfloat16, TABLES),
     ],
 )
-def test_both_sides_of_the_one_launch_limit(M, topk, hidden, in_dtype):
+def test_both_sides_of_the_one_launch_limit(M, topk, hidden, in_dtype, form):
     spec = WorkloadSpec("limit", 73, 1, 16, topk, hidden, M, in_dtype)
+    plan = ops.plan_of(
+        ops.Config(M, 16, topk, 1, 1, hidden, spec.hidden_dim_bytes, spec.hidden_dim_scale_bytes)
+    )
+    assert plan.dispatch_form == form
     groups = generate(spec, seed=M)
     groups[0].n = M - 1
     cap = int(np.bincount(groups[0].indices[: M - 1].reshape(-1).numpy(), minlength=16).max())

@@ -52,6 +52,42 @@ def test_scatter(tokens, row, scales, topk, waves, in_turn):
     assert (p.scatter_waves_per_cu, bool(p.scatter_in_turn)) == (waves, in_turn)
 
 
+@pytest.mark.parametrize(
+    "tokens,row,scales,topk,one_launch",
+    [
+        # a wave per token in a workgroup per CU
+        (4096, 1024, 0, 2, True),
+        (4104, 1024, 0, 2, False),
+        (2048, 10240, 0, 8, True),
+        (2056, 10240, 0, 1, False),
+        # bytes of rows: 112 MiB for any number of picks
+        (1792, 8192, 0, 8, True),
+        (1400, 8192, 0, 10, True),  # 109 MiB
+        (1440, 8192, 0, 10, False),  # 112.5
+        (2864, 8192, 0, 5, True),  # 111.9
+        (2872, 8192, 0, 5, False),  # 112.2
+        (1792, 8192, 0, 9, False),  # 126
+        # 120 MiB for picks that are counted four at a time, and up to 1024 tokens
+        (2120, 7168, 56, 8, True),  # 119.6
+        (2128, 7168, 56, 8, False),  # 120.0, 8 KiB beyond
+        (3840, 4096, 0, 8, True),  # 120 MiB
+        (3848, 4096, 0, 8, False),
+        (960, 8192, 0, 16, True),  # 120 MiB
+        (968, 8192, 0, 16, False),
+        (960, 8192, 0, 17, False),
+        # 176 MiB for rows of whole lines, or of 8 KiB, up to 3072 tokens
+        (2816, 8192, 0, 8, True),  # 176 MiB
+        (2824, 8192, 0, 8, False),
+        (2728, 8192, 64, 8, True),  # 175.8
+        (2736, 8192, 64, 8, False),  # 176.3
+        (3072, 7168, 0, 8, True),  # 168
+        (3080, 7168, 0, 8, False),
+    ],
+)
+def test_one_launch(tokens, row, scales, topk, one_launch):
+    assert (plan(tokens, row, topk, scales=scales).dispatch_form == ONE_LAUNCH) == one_launch
+
+
 def test_forms_of_the_routing():
     assert plan(4104, 1024, 2).dispatch_form == TABLES  # 65 chunks
     assert plan(65536, 1024, 2).routing_tiles == 64

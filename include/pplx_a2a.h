@@ -233,8 +233,10 @@ typedef struct pplx_a2a_plan {
   uint32_t routing_tiles;
   uint32_t scatter_waves_per_cu;  /* 0 = as many as fit, or no scatter launch */
   int32_t scatter_in_turn;   /* 1: its waves fetch row, slots and buffers one behind the other */
+  int32_t combine_per_group;      /* 1: combine gathers once for the ranks of a DP group */
 } pplx_a2a_plan_t;
-int pplx_a2a_plan(const pplx_a2a_config_t *cfg, pplx_a2a_plan_t *out);
+/* in_dtype: pplx_a2a_dtype of expert_y */
+int pplx_a2a_plan(const pplx_a2a_config_t *cfg, int in_dtype, pplx_a2a_plan_t *out);
 
 /* Parts of a step for pplx_a2a_world_abandon_step. */
 #define PPLX_A2A_ABANDON_DISPATCH 1u

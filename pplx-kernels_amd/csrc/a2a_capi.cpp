@@ -1099,7 +1099,7 @@ int pplx_a2a_static_step(const pplx_a2a_config_t *cfg, int device,
   return PPLX_A2A_OK;
 }
 
-int pplx_a2a_plan(const pplx_a2a_config_t *cfg, pplx_a2a_plan_t *out) {
+int pplx_a2a_plan(const pplx_a2a_config_t *cfg, int in_dtype, pplx_a2a_plan_t *out) {
   if (!cfg || !out) return fail(PPLX_A2A_INVALID_ARGUMENT, "cfg / out is NULL");
   if (int st = check_config(*cfg)) return st;
   WorldDev d{};
@@ -1111,6 +1111,7 @@ int pplx_a2a_plan(const pplx_a2a_config_t *cfg, pplx_a2a_plan_t *out) {
   plan.routing_tiles = d.num_tiles;
   plan.scatter_waves_per_cu = dispatch.scatter_waves_per_cu;
   plan.scatter_in_turn = dispatch.scatter_in_turn;
+  plan.combine_per_group = combine_gathers_per_group(d, in_dtype);
   *out = plan;
   return PPLX_A2A_OK;
 }

@@ -128,7 +128,10 @@ __device__ __forceinline__ void reduce_picks(f32x8 (&acc)[VPL], uint32_t K, uint
 // bound by the gathered bytes moves up to dp times fewer of them: 8 ranks in groups of four, 3001
 // tokens of fp32 rows, 2880 wide, top-5: 150 us with a gather per rank, 54 us with one per
 // group (242 MB at 4.5 TB/s); groups of two, 4 x 128 bf16 tokens, 7168 wide, top-8: 16.5 and 15.0
-// us (the second gather of a step this small hits the last-level cache).
+// us (the second gather of a step this small hits the last-level cache).  Members that do not agree are
+// gathered for one after the other by the same wave: if every token's weights differ, a step of 4 x 128
+// tokens takes 41 us where a gather per rank takes 33 (groups of four, 2 x 128: 36 and 25), one of 4 x
+// 1024 tokens 267 and 275.  Copies of a token carry the same weights, so nothing is made of that case.
 template <typename T, typename U, class CT, int KB, int VPL, bool GROUPED>
 __global__ __launch_bounds__(kWavesPerBlock * kWave) void combine_gather(WorldDev w, CT tab, uint32_t segments,
                                                                          FastDiv by_segments) {
@@ -216,6 +219,20 @@ __global__ __launch_bounds__(kWavesPerBlock * kWave) void combine_gather(WorldDe
   }
 }
 
+// DP groups of several ranks gather once per group as long as a wave has a lane for every member's
+// pick; beyond that (no routing in use comes near) every rank gathers for itself.  So it does in steps
+// whose ranks gather up to 10 MiB together: there the bytes cost less than the longer chain in front of
+// them (dispatch + combine, us, per rank / per group, at the MiB that all ranks gather): 8 ranks in groups
+// of two, 7168-wide bf16, top-8: 14 12.5 / 12.8, 19 14.4 / 13.8, 64 28.2 / 22.9; 2048 wide, top-6: 3 10.8 / 11.3,
+// 14 14.0 / 13.7; 4096 wide, top-2: 8 10.7 / 11.4, 14 12.9 / 13.3, 32 20.6 / 19.3; groups of four, 7168 wide:
+// 3.5 10.3 / 10.7, 19 14.3 / 12.8; 1024-wide f16, top-4: 8 10.2 / 11.1, 14 11.5 / 11.8, 32 14.6 / 13.9; 2880-wide
+// fp32, top-5: 7 11.0 / 11.8, 14 13.9 / 12.6; 64 ranks in groups of four, 10 13.8 / 12.6.
+constexpr uint64_t kGroupGatherMinBytes = 10ull << 20;
+bool combine_per_group(const WorldDev &w, size_t elem_bytes) {
+  return w.dp > 1 && w.dp * w.K <= kWave &&
+         (uint64_t)w.R * w.M * w.K * w.H * elem_bytes > kGroupGatherMinBytes;
+}
+
 template <typename T, typename U, class CT, int KB, int VPL>
 int launch_combine_v(const WorldDev &w, const CT &tab, bool grouped, hipStream_t s) {
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
@@ -235,9 +252,7 @@ int launch_combine_v(const WorldDev &w, const CT &tab, bool grouped, hipStream_t
 template <typename T, typename U, class CT>
 int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
 #define PPLX_COMBINE(KB, VPL) return launch_combine_v<T, U, CT, KB, VPL>(w, tab, grouped, s)
-  // DP groups of several ranks gather once per group as long as a wave has a lane for every
-  // member's pick; beyond that (no routing in use comes near) every rank gathers for itself.
-  const bool grouped = w.dp > 1 && w.dp * w.K <= kWave;
+  const bool grouped = combine_per_group(w, sizeof(T));
   // Few picks: long pieces of each row, all picks at once.  Many picks: all of them at once,
   // 1 KiB of each (eight loads per lane in flight either way) -- except for steps of a few
   // hundred to two thousand tokens, whose waves are all resident at the same moment: there the
@@ -292,6 +307,10 @@ int launch_combine_t(const WorldDev &w, const CT &tab, int in_dtype, int out_dty
 }
 
 }  // namespace
+
+bool combine_gathers_per_group(const WorldDev &w, int in_dtype) {
+  return combine_per_group(w, in_dtype == 0 ? 4 : 2);
+}
 
 int launch_combine(const WorldDev &w, const CombineRank *inline_rows, int in_dtype, int out_dtype,
                    void *stream) {

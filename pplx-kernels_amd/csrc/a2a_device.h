@@ -249,6 +249,8 @@ struct DispatchPlan {
   bool scatter_in_turn;
 };
 DispatchPlan dispatch_plan(const WorldDev &w);
+// True when combine gathers the rows of a DP group once for its ranks (in_dtype: pplx_a2a_dtype).
+bool combine_gathers_per_group(const WorldDev &w, int in_dtype);
 // LDS bytes the routing kernels need for a given geometry.
 uint32_t route_lds_bytes(uint32_t num_experts, uint32_t tile_chunks);
 

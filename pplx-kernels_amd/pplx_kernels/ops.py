@@ -92,6 +92,7 @@ class Plan(ctypes.Structure):
         ("routing_tiles", ctypes.c_uint32),
         ("scatter_waves_per_cu", ctypes.c_uint32),
         ("scatter_in_turn", ctypes.c_int32),
+        ("combine_per_group", ctypes.c_int32),
     ]
 
 
@@ -177,7 +178,7 @@ def load_library() -> ctypes.CDLL:
         lib.pplx_a2a_static_step.argtypes = [
             ctypes.POINTER(Config), i32, ctypes.POINTER(DispatchArgs), ctypes.POINTER(CombineArgs), vp, vp,
         ]  # fmt: skip
-        lib.pplx_a2a_plan.argtypes = [ctypes.POINTER(Config), ctypes.POINTER(Plan)]
+        lib.pplx_a2a_plan.argtypes = [ctypes.POINTER(Config), i32, ctypes.POINTER(Plan)]
         lib.pplx_a2a_world_of.argtypes = [vp]
         lib.pplx_a2a_world_of.restype = vp
         lib.pplx_a2a_world_recorded_calls.argtypes = [vp, i32, i32, ctypes.POINTER(u32)]
@@ -197,10 +198,10 @@ def load_library() -> ctypes.CDLL:
     return _lib
 
 
-def plan_of(config: Config) -> Plan:
+def plan_of(config: Config, in_dtype: torch.dtype = torch.bfloat16) -> Plan:
     """Which kernels a step of this geometry runs as (no GPU needed)."""
     plan = Plan()
-    check_status(load_library().pplx_a2a_plan(ctypes.byref(config), ctypes.byref(plan)))
+    check_status(load_library().pplx_a2a_plan(ctypes.byref(config), DTYPE_CODE[in_dtype], ctypes.byref(plan)))
     return plan
 
 

@@ -69,7 +69,7 @@ def test_ctypes_structs_match_the_header_layout():
     assert ctypes.sizeof(ops.Config) == 56
     assert ctypes.sizeof(ops.DispatchArgs) == 18 * 8
     assert ctypes.sizeof(ops.CombineArgs) == 12 * 8
-    assert ctypes.sizeof(ops.Plan) == 4 * 4
+    assert ctypes.sizeof(ops.Plan) == 5 * 4
     assert ops.DispatchArgs.bound_m.offset == 17 * 8
     assert ops.CombineArgs.in_dtype.offset == 10 * 8 and ops.CombineArgs.m.offset == 10 * 8 + 4
 

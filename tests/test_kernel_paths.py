@@ -36,17 +36,21 @@ ONE_LAUNCH, SLOT_MAP, TABLES, SCANNED_TABLES = range(4)
 # Combine of DP groups: one gather for the members that agree
 # ---------------------------------------------------------------------------
 @pytest.mark.parametrize(
-    "dp,K,E,H,M,y_dtype,out_dtype",
+    "dp,K,E,H,M,y_dtype,out_dtype,shared",
     [
-        (2, 8, 32, 7168, 120, torch.bfloat16, torch.bfloat16),  # long pieces of each row
-        (4, 5, 32, 1000, 7, torch.float32, torch.float16),  # tail of picks, row no multiple of 512
-        (2, 1, 8, 8, 1, torch.float16, torch.float16),  # the smallest row and step
-        (4, 16, 64, 520, 9, torch.bfloat16, torch.bfloat16),  # every lane holds a pick
-        (4, 17, 64, 520, 9, torch.bfloat16, torch.bfloat16),  # one pick too many for a shared wave
-        (8, 8, 64, 264, 5, torch.bfloat16, torch.float16),  # a single group of eight
+        (2, 8, 32, 7168, 120, torch.bfloat16, torch.bfloat16, True),  # long pieces of each row
+        (4, 5, 32, 1000, 7, torch.float32, torch.float16, False),
+        (4, 5, 32, 1000, 110, torch.float32, torch.float16, True),  # tail of picks, row no multiple of 512
+        (2, 1, 8, 8, 1, torch.float16, torch.float16, False),  # the smallest row and step
+        (2, 1, 8, 8, 132000, torch.float16, torch.float16, True),  # the smallest row
+        (4, 16, 64, 520, 9, torch.bfloat16, torch.bfloat16, False),
+        (4, 16, 64, 520, 140, torch.bfloat16, torch.bfloat16, True),  # every lane holds a pick
+        (4, 17, 64, 520, 140, torch.bfloat16, torch.bfloat16, False),  # one pick too many for a shared wave
+        (8, 8, 64, 264, 5, torch.bfloat16, torch.float16, False),
+        (8, 8, 64, 264, 520, torch.bfloat16, torch.float16, True),  # a single group of eight
     ],
 )
-def test_members_of_a_dp_group_share_or_keep_their_own_sums(dp, K, E, H, M, y_dtype, out_dtype):
+def test_members_of_a_dp_group_share_or_keep_their_own_sums(dp, K, E, H, M, y_dtype, out_dtype, shared):
     """Member 0 and the last member agree on every token; member 1's weights differ on every
     third token, and it has fewer tokens (so for the rest of them it is absent)."""
     from oracle import a2a_oracle as orc
@@ -55,7 +59,10 @@ def test_members_of_a_dp_group_share_or_keep_their_own_sums(dp, K, E, H, M, y_dt
         "dpshare", 71, 8, E, K, H, M, torch.bfloat16, out_dtype=out_dtype, expert_y_dtype=y_dtype, dp_size=dp,
         tokens="uniform",
     )  # fmt: skip
+    assert ops.plan_of(ops.Config(M, E, K, 8, dp, H, 2 * H, 0), y_dtype).combine_per_group == shared
     groups = generate(spec, seed=dp * 100 + K)
+    for g in groups:
+        g.n = min(g.n, 150)
     step = DeviceStep(spec, groups)
     own = [dataclasses.replace(groups[r // dp]) for r in range(8)]
     for r in range(1, 8, dp):

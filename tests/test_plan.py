@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 import pytest
+import torch
 
 from pplx_kernels import ops
 
@@ -86,6 +87,27 @@ def test_scatter(tokens, row, scales, topk, waves, in_turn):
 )
 def test_one_launch(tokens, row, scales, topk, one_launch):
     assert (plan(tokens, row, topk, scales=scales).dispatch_form == ONE_LAUNCH) == one_launch
+
+
+@pytest.mark.parametrize(
+    "ranks,dp,max_tokens,topk,hidden,dtype,per_group",
+    [
+        # 10 MiB gathered by all ranks
+        (8, 2, 80, 8, 1024, torch.bfloat16, False),
+        (8, 2, 81, 8, 1024, torch.bfloat16, True),
+        (8, 2, 40, 8, 1024, torch.float32, False),
+        (8, 4, 41, 8, 1024, torch.float32, True),
+        (64, 4, 1, 8, 7168, torch.bfloat16, False),
+        (64, 4, 4, 8, 7168, torch.bfloat16, True),
+        # a lane for every member's pick
+        (8, 8, 1024, 8, 1024, torch.bfloat16, True),
+        (8, 8, 1024, 9, 1024, torch.bfloat16, False),
+        (8, 1, 1024, 8, 1024, torch.bfloat16, False),
+    ],
+)
+def test_combine_per_group(ranks, dp, max_tokens, topk, hidden, dtype, per_group):
+    p = ops.plan_of(ops.Config(max_tokens, 64, topk, ranks, dp, hidden, 2 * hidden, 0), dtype)
+    assert bool(p.combine_per_group) == per_group
 
 
 def test_forms_of_the_routing():

@@ -275,9 +275,13 @@ int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
   // top-5, dp 4: 2 x 3001 tokens 98.9 / 94.1 / 94.4, ragged 52.0 / 50.6 / 53.0; dp 1, 8 x 1024 98.6 / 96.6 /
   // 98.0.  Steps of a few hundred tokens lack the waves for it (64 tokens, 7168 wide, top-8: 5.8 / 7.9 /
   // 11.0; 320 tokens, 1024 wide, top-6: 4.5 / 6.2 / 6.7); 16-bit rows do not care (within 1 %) or lose
-  // (the large ragged prefill of 7168-wide rows: 734 / 761 / 762).
+  // (the large ragged prefill of 7168-wide rows: 734 / 761 / 762).  Rows of up to 512 columns are one
+  // 2 KiB piece, and a longer one is only padding: more than four picks of them stay eight at a time
+  // (8 x 2048 tokens, dispatch and combine, eight picks of 2 KiB / three of 4 KiB: 512 wide, top-8 92.7 / 93.8, top-6
+  // 71.8 / 74.0; 256 wide, top-10 62.3 / 66.2; 8 wide, top-8 35.2 / 41.6; 8 x 8192, 512 wide, top-8, combine
+  // alone 221.4 / 226.6).
   if constexpr (sizeof(T) == 4) {
-    if (w.K > 2 && tokens > 2048) {
+    if (w.K > 2 && tokens > 2048 && (w.K <= 4 || nvec_segments > 1)) {
       const uint32_t padding = (4 - nvec_segments % 4) % 4;
       if (6 * padding <= nvec_segments) PPLX_COMBINE(2, 4);
       PPLX_COMBINE(3, 2);

@@ -213,7 +213,10 @@ def test_both_sides_of_the_one_launch_limit(M, topk, hidden, in_dtype, form):
         (1025, 3, 2048, 1, torch.bfloat16),  # two picks of 8 KiB, the third by itself
         (1025, 8, 3592, 1, torch.float16),  # 8 segments, one vector in the last
         (1025, 5, 2056, 1, torch.bfloat16),  # 5 segments: three picks of 4 KiB, then two
-        (1025, 10, 8, 1, torch.bfloat16),  # one vector; three times three picks, then one
+        (1025, 10, 520, 1, torch.bfloat16),  # one vector beyond a segment; three times three picks, then one
+        (1025, 10, 8, 1, torch.bfloat16),  # one segment, of one vector: eight picks, then two
+        (1025, 5, 512, 1, torch.float16),  # a full segment: four picks, then one
+        (1025, 4, 512, 1, torch.bfloat16),  # three picks, then one
         (1025, 7, 1536, 2, torch.float16),  # the same for DP groups
         (1025, 3, 2880, 4, torch.float16),
     ],

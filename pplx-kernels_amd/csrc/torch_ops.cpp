@@ -177,15 +177,43 @@ fptr_t create_rank(const std::string &transport, const std::string &group_name, 
 // front of the lock, so that they go behind it.  The last reference to a tensor may need the
 // interpreter lock, which a thread that waits for g_mu may hold, and may run Python code that calls in
 // here again.
-typedef std::vector<at::Tensor> Released;
+//
+// A launched step's tensors change places with the cleared vectors of the thread's step before, so that
+// neither side allocates again from step to step.
+struct Released {
+  typedef std::vector<std::vector<at::Tensor>> PerRank;
+  PerRank step;
+  std::vector<at::Tensor> others;
+  bool has_step = false;
 
-void release(std::vector<at::Tensor> &kept, Released &released) {
-  released.insert(released.end(), std::make_move_iterator(kept.begin()), std::make_move_iterator(kept.end()));
-  kept.clear();
-}
+  Released() = default;
+  Released(const Released &) = delete;
+  Released &operator=(const Released &) = delete;
+  ~Released() {
+    if (!has_step) return;
+    for (auto &tensors : step) tensors.clear();
+    if (spare().empty()) spare().swap(step);  // (a callback of a tensor may have left its own)
+  }
+  void take_step(PerRank &held) {
+    step.swap(spare());
+    step.resize(held.size());
+    held.swap(step);
+    has_step = true;
+  }
+  void take(std::vector<at::Tensor> &kept) {
+    others.insert(others.end(), std::make_move_iterator(kept.begin()), std::make_move_iterator(kept.end()));
+    kept.clear();
+  }
+
+ private:
+  static PerRank &spare() {
+    static thread_local PerRank vectors;
+    return vectors;
+  }
+};
 
 void release_held(World &world, uint32_t rank, Released &released) {
-  for (auto &per_rank : world.held) release(per_rank[rank], released);
+  for (auto &per_rank : world.held) released.take(per_rank[rank]);
 }
 
 // csrc/bindings/all_to_all_ops.cpp:108
@@ -375,7 +403,7 @@ void reserve_split_locked(World &world, int expert_y_elem_bytes) {
 
 void clear_held(World &world, int op, Released &released) {
   for (int mode = 0; mode < kModes; ++mode) {
-    for (auto &tensors : world.held[op * kModes + mode]) release(tensors, released);
+    for (auto &tensors : world.held[op * kModes + mode]) released.take(tensors);
   }
 }
 
@@ -388,13 +416,12 @@ void settle_held(World &world, uint32_t rank, int op, int mode, bool recorded,
   (void)pplx_a2a_world_recorded_calls(world.ptr, op, mode, &pending);
   auto &per_rank = world.held[op * kModes + mode];
   if (pending == 0) {
-    released.reserve(per_rank.size() * tensors.size());
-    for (auto &kept : per_rank) release(kept, released);
+    released.take_step(per_rank);
     return;
   }
   if (!recorded) return;
   auto &kept = per_rank[rank];
-  release(kept, released);
+  if (!kept.empty()) released.take(kept);
   for (const at::Tensor *t : tensors) {
     if (t) kept.push_back(*t);
   }

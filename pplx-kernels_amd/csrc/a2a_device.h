@@ -138,8 +138,8 @@ struct RouteSpan {
   uint32_t v_count;       // virtual tokens covered
   uint32_t tile_chunks;   // 64-token chunks per tile (one workgroup)
   uint32_t pick_vector;   // expert ids one load may fetch (4, 2 or 1)
-  uint32_t *tile_cnt;     // [tiles][E], scanned form; NULL: the counts go to tile_row
-  uint16_t *tile_row;     // [E][kScanFreeTiles], the form that needs no scan
+  uint32_t *tile_cnt;     // [tiles][E], scanned form
+  uint16_t *tile_row;     // [E][kScanFreeTiles], the form that needs no scan; NULL: the counts go to tile_cnt
   unsigned long long *tile_mask;  // [tiles * tile_chunks][E] route_count keeps the chunks' masks
                                   // here (and reports the faults) when set: the scatter that
                                   // follows works the slots out by itself

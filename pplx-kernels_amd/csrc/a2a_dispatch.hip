@@ -444,7 +444,7 @@ uint32_t fused_lds_bytes(const WorldDev &w, bool inline_table) {
 
 // Number of waves a row's K copies are spread over (the row's re-reads hit L2).  Steps of one
 // routing tile need them to cover the 256 CUs.  Larger ones split only what leaves each wave long
-// runs of stores (8 ranks, us at one / two / four waves per token: 14 KiB rows, top-8, 1280 tokens
+// runs of stores (8 ranks, us in this form at one / two / four waves per token: 14 KiB rows, top-8, 1280 tokens
 // 38.8 / 36.4 / 38.6; 7 KiB rows, top-8, 2048 tokens 29.9 / 29.8 / 35.2; 4 KiB rows, top-8, 3072 tokens
 // 25.1 / 28.3 / 30.6; 8 KiB rows, top-2, 3072 tokens 18.1 / 20.4 / 30.6).
 uint32_t pick_ksplit(const WorldDev &w, uint32_t max_split) {
@@ -519,8 +519,8 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t 
   const uint64_t waves = (uint64_t)tokens * ksplit;
   // One wave per workgroup, and few of them per CU at a time.  A wave reads one row and then
   // has up to K rows of stores to issue; HBM takes those stores best when a CU sends the rows of
-  // three or four waves at a time rather than those of thirty-two interleaved (figures at
-  // scatter_plan).  The hardware has no such knob, so each workgroup asks for a share of
+  // a few waves at a time (three or four where each stores much) rather than those of thirty-two
+  // interleaved (figures at scatter_plan).  The hardware has no such knob, so each workgroup asks for a share of
   // the CU's LDS that only that many fit into.
   const ScatterPlan plan = scatter_plan(w, kper);
   // (LDS is handed out in blocks: a share that is not a multiple of 4 KiB can round up past

@@ -98,10 +98,20 @@ __device__ __forceinline__ void scatter_token(const WorldDev &w, const DT &tab, 
   if (g >= w.G) return;
   if (t >= dispatch_group_tokens(w, tab, g)) return;
   const DispatchRank &src = tab.at(sender_of(w, g, t));
-  RowRegs<NV> regs;
-  if constexpr (IN_TURN) load_row<NV, EXACT>(w, src, t, lane, regs);
+  constexpr bool kStaged = NV == 0;  // the row goes through LDS
+  extern __shared__ u32x4 lds_row[];
+  RowRegs<kStaged ? 1 : NV> regs;
+  auto fetch_row = [&]() {
+    if constexpr (kStaged) {
+      regs.sc = load_scale(w, src, t, lane);
+      stage_row(w, src, t, lane, 0, 1, lds_row);
+    } else {
+      load_row<NV, EXACT>(w, src, t, lane, regs);
+    }
+  };
+  if constexpr (IN_TURN) fetch_row();
   const uint32_t e = lane < w.K ? as_global(src.indices)[(size_t)t * w.K + lane] : w.E;
-  if constexpr (!IN_TURN) load_row<NV, EXACT>(w, src, t, lane, regs);
+  if constexpr (!IN_TURN) fetch_row();
   ExpertBuffer buffer;
   if constexpr (!IN_TURN) buffer = expert_buffer(w, tab, e);
   uint32_t slot = kInvalidSlot;
@@ -121,11 +131,16 @@ __device__ __forceinline__ void scatter_token(const WorldDev &w, const DT &tab, 
   // Rows stream past the caches; the 4-byte-per-lane scale rows are written through into the
   // last-level cache instead, where the partial lines of neighbouring rows meet before they go
   // to HBM (3-4 % of the kernel's time at 224-byte scale rows).
-  store_row<NV, EXACT, RowStore::kStreamThrough, RowStore::kKeep>(w, src, t, lane, dst, k0, k1, regs);
+  if constexpr (kStaged) {
+    row_staged();
+    store_staged_row<RowStore::kStream, RowStore::kKeep, RowStore::kKeep>(w, src, t, lane, dst, k0, k1, regs.sc, lds_row);
+  } else {
+    store_row<NV, EXACT, RowStore::kStreamThrough, RowStore::kKeep>(w, src, t, lane, dst, k0, k1, regs);
+  }
 }
 
 // Launched as one-wave workgroups whose dynamic LDS size caps how many of them a CU holds at a
-// time (see launch_scatter_t); the kernels themselves do not touch LDS.
+// time (see launch_scatter_t); only the variants for rows that share lines (NV = 0) use it, for the row.
 template <int NV, bool EXACT, class DT>
 __global__ __launch_bounds__(kWave) void dispatch_scatter(WorldDev w, DT tab, uint32_t ksplit, uint32_t kper) {
   scatter_token<NV, EXACT, DT, Slots::kMap, false>(w, tab, blockIdx.x, ksplit, kper);
@@ -272,6 +287,8 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   }
   uint32_t *hist = reinterpret_cast<uint32_t *>(lds_u64 + table_words);  // [E] tokens before the workgroup's own
   uint32_t *own_mask = hist + w.E;                                       // [E] bit j: own token j goes to e
+  // NV = 0: the workgroup's rows (those that share lines), one behind the other
+  u32x4 *own_rows = reinterpret_cast<u32x4 *>(lds_u64 + ((table_words + w.E + 1) & ~1u));
   for (uint32_t e = threadIdx.x; e < 2 * w.E; e += kFusedThreads) hist[e] = 0;
   // Orders the zeroing (and the staged table) before the first counter update of any wave.
   __syncthreads();
@@ -324,8 +341,19 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   const bool my_pick_has_row = my_live && my_e < w.E && !my_repeats;
   if (my_pick_has_row && my_part == 0) atomicOr(&own_mask[my_e], 1u << my_j);
   timeline.mark(3);
-  RowRegs<NV> regs;
-  if (my_live) load_row<NV, EXACT>(w, my_src, my_t, lane, regs);
+  constexpr bool kRowInLds = NV == 0;
+  RowRegs<kRowInLds ? 1 : NV> regs;
+  u32x4 *my_row = own_rows + (size_t)my_j * (w.Hb / 16);
+  if constexpr (kRowInLds) {
+    regs.sc = 0.f;
+    if (my_live) {
+      regs.sc = load_scale(w, my_src, my_t, lane);
+      stage_row(w, my_src, my_t, lane, my_part, ksplit, my_row);
+    }
+    row_staged();
+  } else {
+    if (my_live) load_row<NV, EXACT>(w, my_src, my_t, lane, regs);
+  }
   __syncthreads();
   timeline.mark(4);
 
@@ -360,7 +388,13 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
     timeline.mark(6);
     const uint32_t k0 = my_part * kper;
     const uint32_t k1 = (k0 + kper < w.K) ? k0 + kper : w.K;
-    if (write_through) {
+    if constexpr (kRowInLds) {
+      if (write_through) {
+        store_staged_row<RowStore::kKeep, RowStore::kKeep, RowStore::kKeep>(w, my_src, my_t, lane, dst, k0, k1, regs.sc, my_row);
+      } else {
+        store_staged_row<RowStore::kStream, RowStore::kKeep, RowStore::kKeep>(w, my_src, my_t, lane, dst, k0, k1, regs.sc, my_row);
+      }
+    } else if (write_through) {
       store_row<NV, EXACT, RowStore::kKeep>(w, my_src, my_t, lane, dst, k0, k1, regs);
     } else {
       store_row<NV, EXACT, RowStore::kStream>(w, my_src, my_t, lane, dst, k0, k1, regs);
@@ -439,7 +473,35 @@ __global__ __launch_bounds__(256) void dispatch_scatter_long(WorldDev w, DT tab)
 // the mask of the workgroup's own tokens.
 uint32_t fused_lds_bytes(const WorldDev &w, bool inline_table) {
   const uint32_t table = inline_table ? w.R * (uint32_t)sizeof(DispatchRank) : 0u;
-  return table + 2u * w.E * (uint32_t)sizeof(uint32_t);
+  return (table + 2u * w.E * (uint32_t)sizeof(uint32_t) + 15u) & ~15u;
+}
+// Tokens of a dispatch_fused workgroup: as few as still give every CU a workgroup (all of a workgroup's
+// waves help with the counting; only the waves that own a token, or a share of one, load and store
+// rows, and few storing waves per CU suit the memory system better than sixteen: 8 x 128 DSv3
+// tokens take 14.7 us with 4 row waves per workgroup against 15.1 us with 16).
+uint32_t fused_tokens_per_block(uint32_t tokens, uint32_t waves) {
+  const uint32_t n = (tokens + 255) / 256;
+  return n > waves ? waves : n < 1 ? 1 : n;
+}
+// Whether dispatch_fused keeps its rows in LDS: those that no register variant fits, and those that share
+// lines once a step and each of its tokens store enough for that to matter (the way through LDS costs 0.3-0.8 us
+// in front of the first store, and the reads from it are repeated for every copy).  Dispatch + combine, us, on
+// three buffer sets in turn, which the last-level cache holds while a set is small / on sixteen, in registers and
+// in LDS at the MiB of rows stored: 3088-byte rows, top-8 7 10.5 10.5 / 11.4 11.6, 23 15.8 16.1 / 21.9 20.2, 47 26.0 26.6 / 37.0
+// 32.6, 95 56.1 47.5 / 64.9 47.7; 5264 bytes, top-8 15 13.3 13.3 / 16.5 16.1, 47 25.9 26.0 / 37.8 31.8, 95 56.6 47.5 / 64.9 47.4, 127
+// 80.0 63.1 / 79.6 62.4; 8176 bytes, top-6 31 21.0 20.6 / 28.4 24.2, 63 36.8 33.7 / 48.4 38.6, 169 99.7 82.0 / 99.9 81.3.  Shorter rows
+// lose what they gain: 1552 bytes, top-8 31 20.6 21.8 (three sets); 2064 bytes, top-8 31 20.2 20.9, 63 36.2 36.4.
+// Rows without a register variant took two launches; dispatch, two launches / one: 12016 bytes, top-8 0.7 8.8 / 6.4, 46
+// 27.6 / 13.5, 93 41.5 / 23.6; 13312 bytes, top-5 32 23.8 / 10.8; 9216 bytes, top-4 18 12.8 / 7.7.
+bool fused_rows_in_lds(const WorldDev &w) {
+  if (!row_has_register_variant(w)) return true;
+  if (!row_shares_lines(w)) return false;
+  const uint64_t stored = (uint64_t)w.G * w.M * w.K * (w.Hb + 4ull * w.S);
+  return w.Hb >= 3072 ? stored > 16ull << 20 : w.Hb >= 2048 && stored > 64ull << 20;
+}
+uint32_t fused_waves(const WorldDev &w) {
+  const uint32_t per_lane = (w.Hb / 16 + kWave - 1) / kWave;
+  return fused_threads(fused_rows_in_lds(w) ? 0 : (int)per_lane) / kWave;
 }
 
 // Number of waves a row's K copies are spread over (the row's re-reads hit L2).  Steps of one
@@ -485,6 +547,19 @@ uint32_t pick_ksplit(const WorldDev &w, uint32_t max_split) {
 //    4 KiB (2 KiB fp8 rows with scales, top-2)         162 /  143 /  125 /  118 /  112 /  110 /  109
 // (one behind the other they lose: 8 x 4096 tokens of 8 KiB, top-2, skewed: 123 and 130; 2 KiB rows,
 // top-6, 8 x 1024: 26.2 and 27.5).
+// Rows that share lines (a2a_rows.h) spend more time in front of and between their stores, and want twice
+// as many waves; so scatter_plan gives half of what a CU holds, and launch_scatter_t halves the share of LDS.  Us
+// at 6 / 8 / 12 / 16 / 24 waves, side by side unless it says otherwise:
+//   66 KiB (8656-byte rows, top-10 of 128)  2 x 1252  54.1 / 56.6 / 55.4 / 55.8 /  -
+//   41 KiB (5264-byte rows, top-8 of 256)   8 x 513   42.0 / 44.1 / 43.3 /  -        8 x 2048  139 / 140 / 143 / 143
+//     8 x 5000   339 / 339 / 342 (in turn 348 / 343 / 343; four waves 404, three 455)
+//   48 KiB (8176-byte rows, top-6 of 64)    8 x 4097   347 / 348 / 359
+//   40 KiB (8208-byte rows, top-5 of 40)    8 x 2100   137 / 138 / 139 (in turn 140)  8 x 6100  449 / 466 / 461 (in turn 443)
+//   23 KiB (2976-byte rows, top-8 of 16)    4 x 4903   95.1 / 92.1 / 94.4 / 96.6
+//   17 KiB (4240-byte rows, top-4 of 4)     4 x 6712   59.7 / 54.2 / 52.6 / 53.0
+//    8 KiB (1040-byte rows, top-8 of 64)    8 x 8000    -  / 186 / 137 / 109 / 104
+//    7 KiB (2576-byte rows, top-3 of 16)    4 x 3587   42.4 / 38.5 / 35.0 / 32.9
+//    5 KiB (2528-byte rows, top-2 of 64)    8 x 8000    -  / 143 / 109 / 101 / 97.5, as many as fit 97.6
 struct ScatterPlan {
   uint32_t waves_per_cu;
   bool in_turn;
@@ -495,6 +570,15 @@ ScatterPlan scatter_plan(const WorldDev &w, uint32_t picks_per_wave) {
   const uint64_t tokens = (uint64_t)w.G * w.M;
   const uint64_t row = w.Hb + 4ull * w.S;
   const uint64_t stored = (uint64_t)picks_per_wave * row;
+  if (row_shares_lines(w)) {
+    if (stored >= 32 * 1024) {
+      if (tokens > 16384 && row >= 8192) return {3, true};
+      return {tokens > 32768 ? 4u : 3u, false};
+    }
+    if (stored >= 20 * 1024) return {4, false};
+    if (stored >= 12 * 1024) return {6, false};
+    return {stored >= 6 * 1024 ? 12u : 0u, false};
+  }
   if (stored >= 24 * 1024) {
     if (tokens <= 16384) return {4, false};
     if (stored >= 48 * 1024 || (stored >= 32 * 1024 && (row >= 8192 || tokens <= 32768))) return {3, true};
@@ -523,10 +607,16 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t 
   // interleaved (figures at scatter_plan).  The hardware has no such knob, so each workgroup asks for a share of
   // the CU's LDS that only that many fit into.
   const ScatterPlan plan = scatter_plan(w, kper);
+  const bool staged = row_shares_lines(w);
   // (LDS is handed out in blocks: a share that is not a multiple of 4 KiB can round up past
   // what the intended number of workgroups leaves room for)
   uint32_t lds = plan.waves_per_cu ? (w.lds_per_cu / plan.waves_per_cu) & ~4095u : 0u;
   if (lds > 65536u) lds = 65536u;
+  if (staged) {
+    lds = (lds / 2) & ~4095u;
+    const uint32_t row = (w.Hb + 1023u) & ~1023u;
+    if (lds < row) lds = row;
+  }
   const dim3 grid((uint32_t)waves + (slots == Slots::kTables ? (w.E + 7) / 8 : 0u)), block(kWave);
 #define PPLX_ROW_KERNEL_ARGS ksplit, kper
 #define PPLX_LAUNCH_LARGE_ROW_VARIANT(KERNEL)                                                    \
@@ -535,7 +625,8 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t 
     else PPLX_LAUNCH_ROW_VARIANT(KERNEL, 32, false);                                             \
   } while (0)
   if (slots == Slots::kMap) {
-    PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter);
+    if (staged) PPLX_LAUNCH_ROW_VARIANT(dispatch_scatter, 0, false);
+    else PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter);
   }
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
   // (rows beyond 16 KiB leave no registers for the slot arithmetic: slots_of() sends them through
@@ -554,9 +645,11 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t 
       hipLaunchKernelGGL((KERNEL<NV, EXACT, DT, false>), grid, block, lds, s, w, tab, ksplit, kper); \
   } while (0)
   if (slots == Slots::kScanned) {
-    PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter_scanned);
+    if (staged) PPLX_LAUNCH_ROW_VARIANT(dispatch_scatter_scanned, 0, false);
+    else PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter_scanned);
   } else if (slots == Slots::kTables) {
-    PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter_slots);
+    if (staged) PPLX_LAUNCH_ROW_VARIANT(dispatch_scatter_slots, 0, false);
+    else PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter_slots);
   }
 #undef PPLX_LAUNCH_ROW_VARIANT
 #define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                               \
@@ -569,26 +662,28 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t 
 template <class DT>
 int launch_fused_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hipStream_t s) {
   const uint32_t tokens = w.G * w.M;
-  const uint32_t kWaves = fused_threads((int)((w.Hb / 16 + kWave - 1) / kWave)) / kWave;
-  // Tokens per workgroup: as few as still give every CU a workgroup (all of a workgroup's waves
-  // help with the counting; only the waves that own a token, or a share of one, load and store
-  // rows, and few storing waves per CU suit the memory system better than sixteen: 8 x 128 DSv3
-  // tokens take 14.7 us with 4 row waves per workgroup against 15.1 us with 16).  Steps of fewer
-  // than 1024 tokens spread each token's picks over several waves instead.
-  uint32_t tokens_per_block = (tokens + 255) / 256;
-  if (tokens_per_block > kWaves) tokens_per_block = kWaves;
-  if (tokens_per_block < 1) tokens_per_block = 1;
+  const uint32_t kWaves = fused_waves(w);
+  const uint32_t tokens_per_block = fused_tokens_per_block(tokens, kWaves);
+  // Steps of fewer than 1024 tokens spread each token's picks over several waves; rows in LDS, which the waves
+  // share, up to 4096 (4240-byte rows, top-4, 1024 tokens 8.0 us at one wave per token, 7.7 at all of a
+  // workgroup's; 15984-byte rows, top-4 17.8 and 17.2; 5264-byte rows, top-8, 2048 tokens 21.3 and 21.2).
+  const bool staged = fused_rows_in_lds(w);
+  const uint64_t spread_below = staged ? 4096 : 1024;
   uint32_t ksplit = 1;
-  while (ksplit * 2 <= w.K && tokens_per_block * ksplit * 2 <= kWaves && (uint64_t)tokens * ksplit < 1024) ksplit *= 2;
+  while (ksplit * 2 <= w.K && tokens_per_block * ksplit * 2 <= kWaves && (uint64_t)tokens * ksplit < spread_below) ksplit *= 2;
   const uint32_t kper = (w.K + ksplit - 1) / ksplit;
   const dim3 grid((tokens + tokens_per_block - 1) / tokens_per_block), block(kWaves * kWave);
-  const uint32_t lds = fused_lds_bytes(w, DT::kInline && w.R <= kInlineRanks);
-  // Rows that fit the last-level cache with room to spare are written through into it.
+  const uint32_t lds = fused_lds_bytes(w, DT::kInline && w.R <= kInlineRanks) + (staged ? tokens_per_block * w.Hb : 0u);
+  // Rows that fit the last-level cache with room to spare are written through into it.  Rows in LDS less far:
+  // dispatch + combine, us, on three buffer sets in turn / on sixteen, written through and streamed at the MiB of rows
+  // stored: 5264-byte rows, top-8 31 19.5 20.1 / 24.4 20.9, 63 32.2 34.2 / 38.9 34.1, 95 49.7 47.5 / 52.7 47.4; 8176 bytes, top-6
+  // 47 25.5 26.8 / 30.3 27.0, 95 48.9 46.8 / 51.3 46.5; 12016 bytes, top-8 (three sets) 63 31.4 33.3, 95 50.1 50.1, 127 63.7 59.8.
   const uint64_t row_bytes = (uint64_t)tokens * w.K * (w.Hb + 4ull * w.S);
-  const uint32_t write_through = row_bytes <= kWriteThroughMaxBytes ? 1u : 0u;
+  const uint32_t write_through = row_bytes <= (staged ? 64ull << 20 : kWriteThroughMaxBytes) ? 1u : 0u;
 #define PPLX_ROW_KERNEL_ARGS ksplit, kper, tokens_per_block, pick_vector, write_through
 #define PPLX_LAUNCH_LARGE_ROW_VARIANT(KERNEL) return (int)hipErrorInvalidValue
-  PPLX_DISPATCH_ROW_VARIANTS(dispatch_fused);
+  if (staged) PPLX_LAUNCH_ROW_VARIANT(dispatch_fused, 0, false);
+  else PPLX_DISPATCH_ROW_VARIANTS(dispatch_fused);
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
 #undef PPLX_ROW_KERNEL_ARGS
   return (int)hipGetLastError();
@@ -634,7 +729,9 @@ uint32_t route_lds_bytes(uint32_t num_experts, uint32_t tile_chunks) {
 }
 
 bool dispatch_is_fused(const WorldDev &w) {
-  if (!row_has_register_variant(w) || fused_lds_bytes(w, true) > 60 * 1024) return false;
+  if (fused_lds_bytes(w, true) > 60 * 1024) return false;
+  const bool in_lds = fused_rows_in_lds(w);
+  if (in_lds && w.Hb > 16 * 1024) return false;
   // One launch while a workgroup per CU can own all tokens, one wave each: 4096 tokens, or 2048 of
   // rows that take 512-thread workgroups (beyond that a second round of workgroups recounts
   // everything: 8 ranks, 2 KiB rows, top-6 of 64: 4096 tokens 15.0 us against 15.9 with the routing
@@ -655,10 +752,17 @@ bool dispatch_is_fused(const WorldDev &w) {
   // top-12 120 34.4 / 31.5; top-16 160 58.4 / 41.2 (but 113 39.4 / 42.4, 120 42.1 / 44.5: up to 1024 tokens
   // the slots take a launch of a single workgroup).
   const uint64_t tokens = (uint64_t)w.G * w.M;
-  const uint32_t per_lane = (w.Hb / 16 + kWave - 1) / kWave;
-  const uint32_t waves = fused_threads((int)per_lane) / kWave;
+  const uint32_t waves = fused_waves(w);
   const uint64_t stored = tokens * w.K * (w.Hb + 4ull * w.S);
   if (tokens > 256u * waves) return false;
+  // Rows in LDS (dispatch + combine, us, one launch / two): 8176 bytes, top-6 127 62.4 / 66.0, 169 82.0 / 83.8; 12016 bytes,
+  // top-8 127 59.8 / 65.2, 169 76.9 / 83.4; 15984 bytes, top-4 127 66.1 / 69.3; whole lines without a register variant
+  // 9216 bytes, top-4 95 50.6 / 52.0 and 127 63.5 / 63.3, 13312 bytes, top-5 127 61.7 / 61.9 and 169 82.0 / 81.0.
+  if (in_lds) {
+    const uint64_t rows = (uint64_t)fused_tokens_per_block((uint32_t)tokens, waves) * w.Hb;
+    const uint64_t limit = row_shares_lines(w) ? 180ull << 20 : 128ull << 20;
+    return fused_lds_bytes(w, true) + rows <= 160 * 1024 && stored <= limit && (row_shares_lines(w) || tokens <= 2048);
+  }
   if (waves < 16) return true;
   const bool quick_count = w.K % 4 == 0 && w.K <= 8;
   const bool whole_lines = w.S == 0 || w.Hb >= 8192;

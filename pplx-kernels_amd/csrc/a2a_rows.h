@@ -17,6 +17,13 @@ struct RowRegs {
   float sc;      // scale `lane` of the row (lanes >= S hold a copy of the last one)
 };
 
+// Scale `lane` of row t (0 when there are none).
+__device__ __forceinline__ float load_scale(const WorldDev &w, const DispatchRank &src, uint32_t t, uint32_t lane) {
+  if (w.S == 0) return 0.f;
+  const uint32_t j = lane < w.S ? lane : w.S - 1;
+  return as_global(src.dp_xs)[(int64_t)t * src.dp_xs_stride_row + (int64_t)j * src.dp_xs_stride_elem];
+}
+
 // First half: issues the loads of row t of `src`; needs t < src.m only.
 template <int NV, bool EXACT>
 __device__ __forceinline__ void load_row(const WorldDev &w, const DispatchRank &src, uint32_t t,
@@ -30,11 +37,7 @@ __device__ __forceinline__ void load_row(const WorldDev &w, const DispatchRank &
     if (!EXACT) j = j < nvec ? j : nvec - 1;  // clamp: loads stay unconditional
     regs.x[i] = row[j];
   }
-  regs.sc = 0.f;
-  if (w.S) {
-    const uint32_t j = lane < w.S ? lane : w.S - 1;
-    regs.sc = as_global(src.dp_xs)[(int64_t)t * src.dp_xs_stride_row + (int64_t)j * src.dp_xs_stride_elem];
-  }
+  regs.sc = load_scale(w, src, t, lane);
 }
 
 // Where pick (expert e, row `slot`) of a token lands: row address, scale-row address and the
@@ -84,13 +87,29 @@ __device__ __forceinline__ Destination destination_of(const WorldDev &w, const E
   return d;
 }
 
+// The scale row of pick k; `scale` is scale `lane` of the token.
+template <RowStore POLICY>
+__device__ __forceinline__ void store_scales(const WorldDev &w, const DispatchRank &src, uint32_t t, uint32_t lane,
+                                             const Destination &dst, uint32_t k, float scale) {
+  const uint32_t S = w.S;
+  if (S == 0) return;
+  PPLX_GLOBAL float *sout = global_ptr<float>(read_lane64(dst.scale, k));
+  const int64_t step = (int64_t)read_lane64((uint64_t)dst.scale_step, k);
+  if (lane < S) row_store<POLICY>(scale, sout + (int64_t)lane * step);
+  if (S > kWave) {
+    const PPLX_GLOBAL float *srow = as_global(src.dp_xs) + (int64_t)t * src.dp_xs_stride_row;
+    for (uint32_t j = lane + kWave; j < S; j += kWave) {
+      sout[(int64_t)j * step] = srow[(int64_t)j * src.dp_xs_stride_elem];
+    }
+  }
+}
+
 // Second half: lane k holds the destination of pick k; the row is stored for picks [k0, k1).
 template <int NV, bool EXACT, RowStore POLICY = RowStore::kStream, RowStore SCALE_POLICY = POLICY>
 __device__ __forceinline__ void store_row(const WorldDev &w, const DispatchRank &src, uint32_t t,
                                           uint32_t lane, Destination dst, uint32_t k0, uint32_t k1,
                                           RowRegs<NV> &regs) {
   const uint32_t nvec = w.Hb / 16;
-  const uint32_t S = w.S;
 #pragma unroll
   for (int i = 0; i < NV; ++i) settle(regs.x[i]);
   settle(regs.sc);
@@ -107,17 +126,83 @@ __device__ __forceinline__ void store_row(const WorldDev &w, const DispatchRank 
       const uint32_t j = lane + i * kWave;
       if (EXACT || j < nvec) row_store<POLICY>(regs.x[i], out + j);
     }
-    if (S) {
-      PPLX_GLOBAL float *sout = global_ptr<float>(read_lane64(dst.scale, k));
-      const int64_t step = (int64_t)read_lane64((uint64_t)dst.scale_step, k);
-      if (lane < S) row_store<SCALE_POLICY>(regs.sc, sout + (int64_t)lane * step);
-      if (S > kWave) {
-        const PPLX_GLOBAL float *srow = as_global(src.dp_xs) + (int64_t)t * src.dp_xs_stride_row;
-        for (uint32_t j = lane + kWave; j < S; j += kWave) {
-          sout[(int64_t)j * step] = srow[(int64_t)j * src.dp_xs_stride_elem];
-        }
+    store_scales<SCALE_POLICY>(w, src, t, lane, dst, k, regs.sc);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Rows whose length is no multiple of a 128-byte line.  Every copy of such a row begins somewhere else
+// inside a line, so a wave that stores 64 vectors from the row's start at a time cuts a line in two at each
+// of its stores, and the halves reach the memory as two partial writes.  The row is therefore kept in
+// LDS instead of registers (fetched with loads that write LDS directly), and for every pick the lanes
+// take it from there shifted by the copy's offset in its line: all stores but the ends of the row
+// cover whole lines.  The lines that two rows share are written through into the last-level cache
+// ("sc1"), where their parts meet; the others stream.  Dispatch, us, registers streamed through ("sc1
+// nt") / registers non-temporal / LDS non-temporal / LDS with shared lines written through:
+//   5264-byte rows, top-8 of 256, 8 x 2048 tokens  210 / 175 / 160 / 139
+//   2976-byte rows, top-8 of 16, 4 x 4903          125 / 116 / 105 / 92
+//   8656-byte rows, top-10 of 128, 2 x 1252        74 / 61 / 58 / 54
+//   3296-byte rows, top-3 of 16, 25979             79 / 65 / 62 / 59
+//   2528-byte rows, top-1 of 64, 2 x 16358         43 / 38 / 39 / 39
+// (whole lines, half a KiB left over: 4608-byte rows with scales, 8 x 2048 tokens 120 in registers, 124
+// through LDS; 5760-byte rows, top-5, 8 x 3001 71 / 73; 512-byte rows 61 / 89: these stay in registers.)
+// ---------------------------------------------------------------------------
+constexpr uint32_t kLineBytes = 128;
+inline bool row_shares_lines(const WorldDev &w) { return w.Hb % kLineBytes != 0; }
+
+// Vectors first, first + step, ... (64 each) of row t go to the same place in `lds`, which the calling wave
+// may read once its loads have returned (row_staged).
+__device__ __forceinline__ void stage_row(const WorldDev &w, const DispatchRank &src, uint32_t t, uint32_t lane,
+                                          uint32_t first, uint32_t step, u32x4 *lds) {
+  const uint32_t nvec = w.Hb / 16;
+  const PPLX_GLOBAL u32x4 *row =
+      as_global(reinterpret_cast<const u32x4 *>(src.dp_x + (int64_t)t * src.dp_x_stride_row));
+  for (uint32_t j = first * kWave; j < nvec; j += step * kWave) {
+    if (j + lane < nvec) {
+      __builtin_amdgcn_global_load_lds((const PPLX_GLOBAL void *)(row + j + lane),
+                                       (__attribute__((address_space(3))) void *)(lds + j), 16, 0, 0);
+    }
+  }
+}
+
+// All loads of the wave have returned.  (The builtin, which the compiler counts, and not inline asm:
+// it would otherwise wait for the stores of one pick before it reads LDS for the next.)
+__device__ __forceinline__ void row_staged() {
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  asm volatile("" ::: "memory");
+}
+
+// store_row for a row in LDS.
+template <RowStore POLICY, RowStore EDGE_POLICY, RowStore SCALE_POLICY>
+__device__ __forceinline__ void store_staged_row(const WorldDev &w, const DispatchRank &src, uint32_t t, uint32_t lane,
+                                                 Destination dst, uint32_t k0, uint32_t k1, float scale,
+                                                 const u32x4 *lds) {
+  constexpr uint32_t kLineVecs = kLineBytes / 16;
+  const uint32_t nvec = w.Hb / 16;
+  settle(scale);
+  settle(dst.row);
+  settle(dst.scale);
+  settle(dst.scale_step);
+  for (uint32_t k = k0; k < k1; ++k) {
+    const uint64_t p = read_lane64(dst.row, k);
+    if (p == 0) continue;
+    PPLX_GLOBAL u32x4 *out = global_ptr<u32x4>(p);
+    // vector j of the row is vector j + shift of the lines it covers
+    const uint32_t shift = (uint32_t)(p / 16) % kLineVecs;
+    const uint32_t end = nvec + shift;
+    // (64 vectors a trip: two, four and eight times as many with their LDS reads in front measured the same
+    // for long rows and up to 25 % more for rows of a few hundred vectors)
+    for (uint32_t first = 0; first < end; first += kWave) {
+      const uint32_t at = first + lane, j = at - shift;  // (j wraps beyond nvec in front of the row)
+      if (j >= nvec) continue;
+      const u32x4 x = lds[j];
+      if ((shift != 0 && at < kLineVecs) || at / kLineVecs == end / kLineVecs) {
+        row_store<EDGE_POLICY>(x, out + j);
+      } else {
+        row_store<POLICY>(x, out + j);
       }
     }
+    store_scales<SCALE_POLICY>(w, src, t, lane, dst, k, scale);
   }
 }
 

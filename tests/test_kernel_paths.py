@@ -3,6 +3,7 @@ can go wrong, against the CPU oracle."""
 
 from __future__ import annotations
 
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -239,3 +240,83 @@ def test_pieces_of_fp32_rows(M, K, H, dp, out_dtype):
     check_combine_against_oracle(step, expected.slot_map)
     assert world.faults() == 0
     world.destroy()
+
+
+# ---------------------------------------------------------------------------
+# Rows that share 128-byte lines, and rows without a register variant: through LDS
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize(
+    "E,K,M,R,row_bytes,form",
+    [
+        (16, 3, 2, 8, 8208, ONE_LAUNCH),  # no register variant, one vector more than a line
+        (16, 2, 3, 8, 16368, ONE_LAUNCH),  # the longest that shares lines
+        (8, 1, 1, 8, 8304, ONE_LAUNCH),  # one vector less than a line
+        (16, 4, 33, 8, 9344, ONE_LAUNCH),  # whole lines without a register variant
+        (64, 16, 261, 8, 2064, ONE_LAUNCH),  # 65.8 MiB of short rows
+        (64, 8, 129, 8, 3088, ONE_LAUNCH),  # two waves to a token
+        (64, 6, 512, 8, 5136, ONE_LAUNCH),  # sixteen rows to a workgroup
+        (40, 5, 520, 8, 1040, TABLES),
+        (24, 4, 521, 8, 4208, TABLES),
+        (16, 1, 523, 8, 8080, TABLES),
+        (8, 8, 530, 8, 16, TABLES),  # eight rows to a line
+        (24, 3, 8200, 8, 112, SCANNED_TABLES),
+        (16, 2, 5, 8, 16400, SLOT_MAP),
+        (16, 2, 5, 8, 32752, SLOT_MAP),  # the longest that goes through LDS
+        (144, 3, 3, 72, 8208, ONE_LAUNCH),  # rank tables in HBM
+        (144, 3, 60, 72, 1040, TABLES),
+        (16, 3, 2, 8, -8592, ONE_LAUNCH),  # (fp8 with 68 scales)
+        (32, 6, 520, 8, -2000, TABLES),
+    ],
+)
+@pytest.mark.parametrize("strided", [False, True], ids=["", "strided"])
+def test_rows_through_lds(E, K, M, R, row_bytes, form, strided):
+    fp8, row_bytes = row_bytes < 0, abs(row_bytes)
+    spec = WorkloadSpec(
+        "lds-rows", 76, R, E, K, row_bytes if fp8 else row_bytes // 2, M, FP8 if fp8 else torch.bfloat16
+    )
+    if K * M * R > 20000:
+        spec = dataclasses.replace(spec, tokens="uniform")
+    assert form == ops.plan_of(
+        ops.Config(M, E, K, R, 1, spec.hidden_dim, spec.hidden_dim_bytes, spec.hidden_dim_scale_bytes)
+    ).dispatch_form  # fmt: skip
+    groups = generate(spec, seed=E + K + row_bytes)
+    groups[R // 2].n = min(1, groups[R // 2].n)
+    ids = np.concatenate([g.indices[: g.n].reshape(-1).numpy() for g in groups])
+    step = DeviceStep(spec, groups, cap=int(np.bincount(ids, minlength=E).max()), alloc_expert_y=False)
+    if not strided:
+        world = make_world(spec, group_name="lds-rows")
+        for _ in range(2):
+            step.dispatch_world(world)
+            check_dispatch_against_oracle(step)
+        assert world.faults() == 0
+        world.destroy()
+        return
+    # Through the C ABI, which takes rows at any multiple of 16 bytes: copies 48 bytes apart from 16 bytes behind
+    # a line on, sources 16 bytes apart.
+    lib = ops.load_library()
+    args = (ops.DispatchArgs * R)()
+    pitch, rows = row_bytes + 48, E * step.cap
+    guard = torch.full((16 + rows * pitch,), 0xA5, dtype=torch.uint8, device="cuda")
+    sources = []
+    for r in range(R):
+        ops.pack_dispatch_args(
+            K, step.expert_num_tokens[r], step.expert_x[r], step.expert_x_scale[r], step.dp_x[r], step.dp_x_scale[r],
+            step.indices[r], step.bound_m[r], out=args[r],
+        )  # fmt: skip
+        wide = torch.zeros(step.dp_x[r].shape[0], row_bytes + 16, dtype=torch.uint8, device="cuda")
+        wide[:, :row_bytes] = step.dp_x[r].view(torch.uint8)
+        sources.append(wide)
+        args[r].dp_x, args[r].dp_x_stride_row = wide.data_ptr(), row_bytes + 16
+        args[r].out_expert_x = guard.data_ptr() + 16 + r * (E // R) * step.cap * pitch
+        args[r].out_expert_x_stride_row, args[r].out_expert_x_stride_expert = pitch, step.cap * pitch
+    config = ops.Config(M, E, K, R, 1, spec.hidden_dim, spec.hidden_dim_bytes, spec.hidden_dim_scale_bytes)
+    handle = ctypes.c_void_p()
+    ops.check_status(lib.pplx_a2a_world_create(ctypes.byref(config), 0, ctypes.byref(handle)))
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ops.check_status(lib.pplx_a2a_world_dispatch(handle, args, stream))
+    torch.cuda.synchronize()
+    ops.check_status(lib.pplx_a2a_world_destroy(handle))
+    copies = guard[16:].view(rows, pitch)
+    step.expert_x_all.view(torch.uint8).view(rows, row_bytes).copy_(copies[:, :row_bytes])
+    check_dispatch_against_oracle(step)
+    assert (copies[:, row_bytes:] == 0xA5).all() and (guard[:16] == 0xA5).all()

@@ -174,24 +174,42 @@ struct LdsDispatch {
   __device__ __forceinline__ const DispatchRank &at(uint32_t i) const { return rows[i]; }
 };
 
+// Picks first, ..., first + NP - 1 of a token in registers, fetched PV at a time by loads that are issued
+// together.  Positions beyond the token's K picks hold copies of others; FULL: K == NP.
+template <int PV, int NP, bool FULL> struct PickBlock {
+  typedef PickVector<PV> Vec;
+  typename Vec::type v[NP / PV];
+  __device__ __forceinline__ void load(const PPLX_GLOBAL typename Vec::type *idx, uint32_t first, uint32_t K) {
+    const uint32_t from = first / PV;
+    if constexpr (FULL) {
+#pragma unroll
+      for (uint32_t i = 0; i < NP / PV; ++i) v[i] = idx[i];
+      return;
+    }
+    uint32_t last = K / PV - 1;
+    settle(last);  // (a vector register: sixteen clamped offsets do not fit beside the scalars)
+#pragma unroll
+    for (uint32_t i = 0; i < NP / PV; ++i) v[i] = idx[from + i < last ? from + i : last];
+  }
+  __device__ __forceinline__ uint32_t at(int u) const { return Vec::at(v[u / PV], u % PV); }
+};
+
 // Counts, per expert, the tokens before virtual token v_end that are routed to it, into the LDS
 // histogram `hist`: one thread per token and pass, PV picks per load (K % PV == 0 and every
-// indices pointer aligned to the vector: the host checks both).  Every expert a token names
-// counts once (a repeat inside the token takes no row).
+// indices pointer aligned to the vector: the host checks both), NP picks of a token in registers at a time.
+// Every expert a token names counts once (a repeat inside the token takes no row).
 //
-// The loads of a token (its group's token count and its first two vectors of picks) are
+// The loads of a token (its group's token count and its first NP picks) are
 // unconditional, from a harmless address when the thread has no token, and sit in
 // straight-line code: they are issued together and cost one trip to memory, and the count is
 // applied afterwards.  The loads of the next pass are issued before the picks of this one are
 // counted, so a step of several passes pays one trip, not one per pass.
-template <int PV, uint32_t THREADS, class Table>
+template <int PV, int NP, bool FULL, uint32_t THREADS, class Table>
 __device__ __forceinline__ void count_earlier_picks(const WorldDev &w, const Table &rows, uint32_t v_end,
                                                     uint32_t *hist) {
-  typedef PickVector<PV> Vec;
-  typedef typename Vec::type vec_t;
-  const uint32_t vectors = w.K / PV;
+  typedef typename PickVector<PV>::type vec_t;
   struct Fetch {
-    vec_t a, b;           // vectors 0 and 1 of the token's picks (b repeats a when there is one)
+    PickBlock<PV, NP, FULL> picks;
     uint32_t n;           // tokens present in the group
     uint32_t t;           // token inside its group
     const PPLX_GLOBAL vec_t *idx;
@@ -208,37 +226,55 @@ __device__ __forceinline__ void count_earlier_picks(const WorldDev &w, const Tab
     const bool bounded = f.valid && head.bound_m != nullptr;
     const uint32_t loaded_n = *as_global(bounded ? head.bound_m : w.faults);
     f.idx = as_global(reinterpret_cast<const vec_t *>(f.valid ? src.indices + (size_t)f.t * w.K : w.slot_map));
-    f.a = f.idx[0];
-    f.b = f.idx[vectors > 1 ? 1 : 0];
+    f.picks.load(f.idx, 0, w.K);
     f.n = bounded ? loaded_n : head.m;
     return f;
   };
-  auto place = [&](uint32_t j, vec_t a, vec_t b, const Fetch &f) {
-    const bool second = j + 1 < vectors;
-    // The picks of this call are compared in registers; those of earlier calls for the same
-    // token (top-k beyond two vectors) are read again.
-    uint32_t e[2 * PV];
+  // Picks first, ... of the token, of which the earlier ones have been counted.
+  auto count = [&](const PickBlock<PV, NP, FULL> &picks, uint32_t first, const PPLX_GLOBAL vec_t *idx) {
+    if constexpr (FULL) {
 #pragma unroll
-    for (int u = 0; u < PV; ++u) {
-      e[u] = Vec::at(a, u);
-      e[PV + u] = second ? Vec::at(b, u) : w.E;
+      for (int u = 0; u < NP; ++u) {
+        bool counts = picks.at(u) < w.E;
+#pragma unroll
+        for (int p = 0; p < u; ++p) counts = counts && picks.at(p) != picks.at(u);
+        if (counts) atomicAdd(&hist[picks.at(u)], 1u);
+      }
+      return;
+    }
+    // bit u: pick first + u does not exist, or repeats an earlier one
+    unsigned skip = w.K - first < NP ? ~0u << (w.K - first) : 0u;
+    settle(skip);
+    if (NP > 8 && first != 0) {
+      const PPLX_GLOBAL uint32_t *before = reinterpret_cast<const PPLX_GLOBAL uint32_t *>(idx);
+      for (uint32_t p = 0; p < first; ++p) {
+        const uint32_t earlier = before[p];
+#pragma unroll
+        for (int u = 0; u < NP; ++u) skip |= (unsigned)(earlier == picks.at(u)) << u;
+      }
     }
 #pragma unroll
-    for (int u = 0; u < 2 * PV; ++u) {
-      bool counts = e[u] < w.E;
+    for (int u = 1; u < NP; ++u) {
+      bool repeats = false;
 #pragma unroll
-      for (int p = 0; p < u; ++p) counts = counts && e[p] != e[u];
-      if (counts && j != 0) {
-        const PPLX_GLOBAL uint32_t *before = reinterpret_cast<const PPLX_GLOBAL uint32_t *>(f.idx);
-        for (uint32_t p = 0; p < j * PV; ++p) counts = counts && before[p] != e[u];
-      }
-      if (counts) atomicAdd(&hist[e[u]], 1u);
+      for (int p = 0; p < u; ++p) repeats = repeats || picks.at(p) == picks.at(u);
+      skip |= (unsigned)repeats << u;
+      settle(skip);  // (bits in a register, not a condition mask per comparison)
+    }
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      if (picks.at(u) < w.E && !((skip >> u) & 1u)) atomicAdd(&hist[picks.at(u)], 1u);
     }
   };
   auto consume = [&](const Fetch &f) {
     if (!f.valid || f.t >= f.n) return;
-    place(0, f.a, f.b, f);
-    for (uint32_t j = 2; j < vectors; j += 2) place(j, f.idx[j], f.idx[j + 1 < vectors ? j + 1 : j], f);
+    PickBlock<PV, NP, FULL> picks = f.picks;
+    for (uint32_t first = 0;;) {
+      count(picks, first, f.idx);
+      first += NP;
+      if (NP <= 8 || first >= w.K) break;
+      picks.load(f.idx, first, w.K);
+    }
   };
 
   Fetch current = issue(threadIdx.x);
@@ -319,12 +355,19 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   const uint32_t my_loaded_e = *as_global(has_pick ? my_src.indices + (size_t)my_t * w.K + lane : w.faults);
 
   // 2. picks of all earlier tokens
-  if (pick_vector == 4) {
-    count_earlier_picks<4, kFusedThreads>(w, rows(), v0, hist);
-  } else if (pick_vector == 2) {
-    count_earlier_picks<2, kFusedThreads>(w, rows(), v0, hist);
+  if (w.K > 8) {
+    if (pick_vector > 1) count_earlier_picks<2, 16, false, kFusedThreads>(w, rows(), v0, hist);
+    else count_earlier_picks<1, 16, false, kFusedThreads>(w, rows(), v0, hist);
+  } else if (w.K > 4) {
+    if (pick_vector == 4) count_earlier_picks<4, 8, true, kFusedThreads>(w, rows(), v0, hist);
+    else if (pick_vector == 2) count_earlier_picks<2, 8, false, kFusedThreads>(w, rows(), v0, hist);
+    else count_earlier_picks<1, 8, false, kFusedThreads>(w, rows(), v0, hist);
+  } else if (w.K > 2) {
+    if (pick_vector == 4) count_earlier_picks<4, 4, true, kFusedThreads>(w, rows(), v0, hist);
+    else count_earlier_picks<1, 4, false, kFusedThreads>(w, rows(), v0, hist);
   } else {
-    count_earlier_picks<1, kFusedThreads>(w, rows(), v0, hist);
+    if (pick_vector == 2) count_earlier_picks<2, 2, true, kFusedThreads>(w, rows(), v0, hist);
+    else count_earlier_picks<1, 2, false, kFusedThreads>(w, rows(), v0, hist);
   }
   timeline.mark(2);
   // ... and the workgroup's own: a pick that names no expert, or repeats an earlier pick of its
@@ -755,6 +798,13 @@ bool dispatch_is_fused(const WorldDev &w) {
   const uint32_t waves = fused_waves(w);
   const uint64_t stored = tokens * w.K * (w.Hb + 4ull * w.S);
   if (tokens > 256u * waves) return false;
+  // Picks beyond eight weigh more, the most where they can only be fetched one by one or do not fit the registers
+  // (us, one launch / routing + scatter): 2 KiB rows, top-9 1024 tokens 9.8 / 16.6, 2048 16.9 / 14.9, 4096 31.0 / 21.9;
+  // 8 KiB rows, top-9 2048 35.5 / 36.2; 4720-byte rows, top-9 2048 29.9 / 30.2, 4096 54.3 / 45.2; 2 KiB rows, top-24 1024
+  // 21.4 / 32.2, 2048 40.0 / 28.4; top-32 1024 28.5 / 45.2.  (2 KiB rows, top-10 2048 14.3 / 15.9, 4096 23.8 / 24.6; top-16
+  // 2048 19.3 / 21.5.)
+  if (tokens > 1024 && w.K > 16) return false;
+  if (tokens > 1024 && w.K > 8 && w.K % 2 != 0 && (w.Hb < 4096 || tokens > 2048)) return false;
   // Rows in LDS (dispatch + combine, us, one launch / two): 8176 bytes, top-6 127 62.4 / 66.0, 169 82.0 / 83.8; 12016 bytes,
   // top-8 127 59.8 / 65.2, 169 76.9 / 83.4; 15984 bytes, top-4 127 66.1 / 69.3; whole lines without a register variant
   // 9216 bytes, top-4 95 50.6 / 52.0 and 127 63.5 / 63.3, 13312 bytes, top-5 127 61.7 / 61.9 and 169 82.0 / 81.0.

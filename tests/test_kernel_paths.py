@@ -255,6 +255,7 @@ def test_pieces_of_fp32_rows(M, K, H, dp, out_dtype):
         (64, 16, 261, 8, 2064, ONE_LAUNCH),  # 65.8 MiB of short rows
         (64, 8, 129, 8, 3088, ONE_LAUNCH),  # two waves to a token
         (64, 6, 512, 8, 5136, ONE_LAUNCH),  # sixteen rows to a workgroup
+        (64, 9, 258, 8, 1392, TABLES),  # picks that are counted one by one
         (40, 5, 520, 8, 1040, TABLES),
         (24, 4, 521, 8, 4208, TABLES),
         (16, 1, 523, 8, 8080, TABLES),
@@ -320,3 +321,28 @@ def test_rows_through_lds(E, K, M, R, row_bytes, form, strided):
     step.expert_x_all.view(torch.uint8).view(rows, row_bytes).copy_(copies[:, :row_bytes])
     check_dispatch_against_oracle(step)
     assert (copies[:, row_bytes:] == 0xA5).all() and (guard[:16] == 0xA5).all()
+
+
+@pytest.mark.parametrize("K", [8, 9, 10, 12, 16, 17, 24, 33, 64])
+@pytest.mark.parametrize("aligned", [True, False], ids=["", "misaligned-picks"])
+def test_one_launch_with_many_picks(K, aligned):
+    """Picks beyond eight are held sixteen at a time; repeats are found across those pieces."""
+    spec = WorkloadSpec("many-picks", 77, 8, 64, K, 512, 90, torch.bfloat16, tokens="uniform")
+    assert ops.plan_of(ops.Config(90, 64, K, 8, 1, 512, 1024, 0)).dispatch_form == ONE_LAUNCH
+    groups = generate(spec, seed=K)
+    groups[1].n = groups[3].n = 90
+    groups[1].indices[3, K - 1] = groups[1].indices[3, 0]
+    groups[1].indices[4, K // 2] = groups[1].indices[4, 1]
+    groups[3].indices[0, 0] = 64
+    groups[3].indices[7] = groups[3].indices[7, 0].item()
+    step = DeviceStep(spec, groups, alloc_expert_y=False)
+    if not aligned:
+        for r, idx in enumerate(step.indices):
+            flat = torch.zeros(idx.numel() + 1, dtype=torch.int32, device="cuda").view(torch.uint32)
+            flat[1:] = idx.reshape(-1)
+            step.indices[r] = flat[1:].view(idx.shape)
+    world = make_world(spec, group_name="many-picks")
+    step.dispatch_world(world)
+    _check_with_repeats_dropped(step, after_combine=False)
+    assert world.faults() == FAULT_BAD_EXPERT | FAULT_DUPLICATE
+    world.destroy()

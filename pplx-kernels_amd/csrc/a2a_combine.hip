@@ -253,12 +253,20 @@ template <typename T, typename U, class CT>
 int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
 #define PPLX_COMBINE(KB, VPL) return launch_combine_v<T, U, CT, KB, VPL>(w, tab, grouped, s)
   const bool grouped = combine_per_group(w, sizeof(T));
-  // Few picks: long pieces of each row, all picks at once.  Many picks: all of them at once,
-  // 1 KiB of each (eight loads per lane in flight either way) -- except for steps of a few
-  // hundred to two thousand tokens, whose waves are all resident at the same moment: there the
+  // All picks of 1 KiB of a row at once where they are three to eight, longer pieces of fewer (two to eight
+  // loads per lane in flight either way, and no piece longer than the row) -- except for steps of a few
+  // hundred to two thousand tokens, whose waves are all resident at the same moment: there more than four
   // picks are better taken one after the other in 7 or 8 KiB pieces by a quarter as many waves
   // (8 x 128 DSv3 tokens, top-8: 23.4 us against 25.3 us; 8 x 256: 45.8 against 46.8; from
   // 8 x 512 on the wide form wins, 88.7 against 91.5 us, and below 8 x 64 too).
+  // Dispatch + combine, 8 ranks, bf16, us, formerly / now: top-1 (one pick of 8 KiB / of up to 3), 16384 tokens 512 wide
+  // 30.8 / 24.1, 1024 wide 37.0 / 32.3, 8192 wide 203.5 / 195.7 (1 KiB pieces 217); top-2 (two of 4 / of up to 2 KiB), 8192 tokens
+  // 512 wide 21.7 / 19.8, 1024 wide 27.0 / 26.0, 6656 wide 125.4 / 124.4; top-3 (eight places, so two picks and then one /
+  // three of 1 KiB), 8192 tokens 2048 wide 57.0 / 52.4, 4096 wide 99.5 / 90.4, 4096 tokens 7168 wide 89.9 / 81.7; top-5 (four, then
+  // one / five of 1 KiB), 16000 tokens 512 wide 43.4 / 41.6, 4096 tokens 7168 wide 124.6 / 122.5, 320 tokens 4096 wide 13.3 /
+  // 12.8.  A wave that serves a DP group compares its members first, so pieces stay as long as formerly there unless that
+  // is mostly padding (groups of two, 4 x 512 tokens, short / long pieces: 2048 wide, top-1 13.8 / 12.8, top-2 16.5 / 15.4; 4096
+  // wide, top-1 20.8 / 18.7, top-2 26.1 / 25.5; but 4600 wide, nine KiB, top-1 23.5 / 30.4, top-2 29.9 / 39.9).  Top-6 and top-7 in one go measure the same as four picks and the rest (145.0 / 145.9, 165.3 / 165.0).
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
   const uint64_t tokens = (uint64_t)(grouped ? w.G : w.R) * w.M;
   if (w.K > 4 && tokens > 384 && tokens <= 2048 && nvec_segments >= 7) {
@@ -288,9 +296,21 @@ int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
     }
   }
   switch (w.K) {
-    case 1: PPLX_COMBINE(1, 8);
-    case 2: PPLX_COMBINE(2, 4);
-    case 4: PPLX_COMBINE(4, 2);
+    case 1:
+      if (nvec_segments == 1) PPLX_COMBINE(1, 1);
+      if (nvec_segments == 2) PPLX_COMBINE(1, 2);
+      if (nvec_segments == 4) PPLX_COMBINE(1, 4);
+      if (grouped && nvec_segments > 4 && 8 * ((8 - nvec_segments % 8) % 8) <= 5 * nvec_segments) PPLX_COMBINE(1, 8);
+      PPLX_COMBINE(1, 3);
+    case 2:
+      if (nvec_segments == 1) PPLX_COMBINE(2, 1);
+      if (grouped && nvec_segments > 2 && (nvec_segments + 1) % 4 <= 1) PPLX_COMBINE(2, 4);
+      PPLX_COMBINE(2, 2);
+    case 3: PPLX_COMBINE(3, 1);
+    case 4:
+      if (nvec_segments == 1) PPLX_COMBINE(4, 1);
+      PPLX_COMBINE(4, 2);
+    case 5: PPLX_COMBINE(5, 1);
     default: PPLX_COMBINE(8, 1);
   }
 #undef PPLX_COMBINE

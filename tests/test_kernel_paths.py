@@ -346,3 +346,40 @@ def test_one_launch_with_many_picks(K, aligned):
     _check_with_repeats_dropped(step, after_combine=False)
     assert world.faults() == FAULT_BAD_EXPERT | FAULT_DUPLICATE
     world.destroy()
+
+
+# ---------------------------------------------------------------------------
+# Combine of few picks: pieces that are no longer than the row
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize(
+    "H,dp,y_dtype,out_dtype",
+    [
+        (8, 1, torch.bfloat16, torch.bfloat16),  # one vector
+        (512, 1, torch.float16, torch.float16),  # a full segment
+        (520, 1, torch.bfloat16, torch.bfloat16),  # one vector in the second
+        (1032, 1, torch.bfloat16, torch.float16),  # one vector in the third
+        (1536, 2, torch.float16, torch.bfloat16),  # three segments
+        (1544, 1, torch.bfloat16, torch.bfloat16),  # a second piece of one vector
+        (4096, 2, torch.bfloat16, torch.bfloat16),
+        (1032, 1, torch.float32, torch.bfloat16),
+        (504, 4, torch.float32, torch.float16),
+    ],
+)
+def test_pieces_of_few_picks(K, H, dp, y_dtype, out_dtype):
+    M = 90
+    spec = WorkloadSpec(
+        "few-picks", 78, 8, 16, K, H, M, torch.bfloat16, out_dtype=out_dtype, expert_y_dtype=y_dtype, dp_size=dp,
+        tokens="uniform",
+    )  # fmt: skip
+    groups = generate(spec, seed=H + K)
+    groups[0].n, groups[-1].n = M, 1
+    step = DeviceStep(spec, groups)
+    world = make_world(spec, group_name="few-picks")
+    step.dispatch_world(world)
+    expected = check_dispatch_against_oracle(step)
+    step.expert_y_all.normal_(generator=torch.Generator(device="cuda").manual_seed(7))
+    step.combine_world(world)
+    check_combine_against_oracle(step, expected.slot_map)
+    assert world.faults() == 0
+    world.destroy()

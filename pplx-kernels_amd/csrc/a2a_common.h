@@ -67,8 +67,8 @@ __device__ __forceinline__ PPLX_GLOBAL V *as_global(V *p) {
 //   kKeep          written through at agent scope ("sc1"): the data stays in the last-level
 //                  cache, where the experts' GEMMs will look for it next, and a step whose rows
 //                  fit there no longer waits for HBM to take them (dispatch of 8 x 128 DSv3
-//                  tokens: 18.9 instead of 22.6 us); beyond kWriteThroughMaxBytes it is the
-//                  slowest of the three.
+//                  tokens: 18.9 instead of 22.6 us; from about 240 MB per step on it is the
+//                  slowest of the three).
 // The compiler offers no builtin for the scoped forms, hence the asm; they are plain vector stores.
 enum class RowStore { kStream, kStreamThrough, kKeep, kPlain };
 

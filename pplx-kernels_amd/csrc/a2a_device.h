@@ -195,18 +195,9 @@ inline StageLayout stage_layout(uint32_t row_bytes, uint32_t scales, uint64_t to
 // arguments each.
 constexpr uint32_t kInlineRanks = 64;
 constexpr uint32_t kBindBatch = 64;
-// A one-launch dispatch whose rows (all picks of all tokens) stay within this many bytes stores them
-// write-through into the 256 MB last-level cache, larger ones stream them (non-temporal).  The line lies where
-// three buffer sets used in turn no longer find their lines in the cache; dispatch + combine, us, on three sets,
-// written through / streamed at the MiB of rows stored: 7 KiB fp8 rows, top-8 56 37.3 / 40.2, 95 66.7 / 67.3, 112 78.5 / 77.0;
-// 8 KiB rows, top-8 64 29.4 / 31.4, 96 44.6 / 46.0, 112 51.1 / 51.2, 140 65.0 / 63.8, 170 77.1 / 75.9; 14 KiB rows, top-8 95 44.1 / 45.7,
-// 112 53.7 / 52.9, 140 65.9 / 64.6; 5760-byte rows, top-5 79 41.3 / 42.5, 95 50.9 / 48.9, 111 59.8 / 55.7.  On sixteen sets, none of
-// which is still in the cache when its turn comes, streaming is ahead from 8 MiB on (4 KiB rows, top-4 16 15.9 / 14.1, 64 36.9
-// / 35.0; 7 KiB fp8 rows 32 30.3 / 28.6, 64 51.5 / 49.7): a layer's buffers are usually the last layer's, so the line is the one
-// of buffers that come back.
-constexpr uint64_t kWriteThroughMaxBytes = 108ull << 20;
-// A split SEND's staged rows are read by the RECV that follows, and stay in the cache while they fit.
-constexpr uint64_t kStageWriteThroughMaxBytes = 192ull << 20;
+// A fused launch whose rows (all picks of all tokens) stay within this many bytes stores them
+// write-through into the 256 MB last-level cache instead of streaming them past it.
+constexpr uint64_t kWriteThroughMaxBytes = 192ull << 20;
 
 // Device memory that pplx_a2a_static_step works in instead of a world's allocations: a fixed
 // array inside the library's code object (a2a_static.hip), one copy per GPU.  The chunks' bases

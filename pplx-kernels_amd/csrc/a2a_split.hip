@@ -151,7 +151,7 @@ int launch_split_stage_tokens_t(const WorldDev &w, const SplitDev &sp, const DT 
     return (int)hipGetLastError();
   }
   const uint64_t row_bytes = (uint64_t)tokens * sp.token_stride;
-  const uint32_t write_through = row_bytes <= kStageWriteThroughMaxBytes ? 1u : 0u;
+  const uint32_t write_through = row_bytes <= kWriteThroughMaxBytes ? 1u : 0u;
   const dim3 grid((tokens + 3) / 4), block(256);
 #define PPLX_ROW_KERNEL_ARGS sp, write_through
 #define PPLX_LAUNCH_LARGE_ROW_VARIANT(KERNEL) return (int)hipErrorInvalidValue

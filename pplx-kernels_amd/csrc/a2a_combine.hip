@@ -117,8 +117,8 @@ __device__ __forceinline__ void reduce_picks(f32x8 (&acc)[VPL], uint32_t K, uint
 }
 
 // One wave owns VPL * 64 consecutive 8-element vectors of one output row (VPL KiB of a bf16
-// row) and takes the picks KB at a time, so KB * VPL row loads per lane are in flight: few
-// picks read long pieces of their rows, many picks shorter ones.
+// row) and takes the picks KB at a time, so KB * VPL row loads per lane are in flight
+// (which of the two: launch_combine_k).
 //
 // GROUPED (DP groups of several ranks, dp * K <= 64): the members of a group hold the same
 // tokens, so the rows they gather are the same ones.  A wave then serves the token for all

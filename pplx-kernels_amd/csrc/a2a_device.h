@@ -196,7 +196,11 @@ inline StageLayout stage_layout(uint32_t row_bytes, uint32_t scales, uint64_t to
 constexpr uint32_t kInlineRanks = 64;
 constexpr uint32_t kBindBatch = 64;
 // A fused launch whose rows (all picks of all tokens) stay within this many bytes stores them
-// write-through into the 256 MB last-level cache instead of streaming them past it.
+// write-through into the 256 MB last-level cache instead of streaming them past it.  That pays where a step's
+// buffers come back soon: 14 KiB rows, top-8, 1024 tokens (112 MiB), one buffer set, dispatch alone 25.9 us written
+// through / 30.4 streamed.  With three sets in turn the two are level from about 108 MiB on (step, 112 MiB 55.1 / 53.2; 8 KiB
+// rows 112 MiB 51.1 / 51.2, 140 65.0 / 63.8; 7 KiB fp8 rows 56 MiB 37.3 / 40.2, 95 66.7 / 67.3, 112 78.5 / 77.0), and with sixteen
+// streaming is ahead from 8 MiB on (7 KiB fp8 rows, 32 MiB 30.3 / 28.6, 64 51.5 / 49.7).
 constexpr uint64_t kWriteThroughMaxBytes = 192ull << 20;
 
 // Device memory that pplx_a2a_static_step works in instead of a world's allocations: a fixed

@@ -306,6 +306,7 @@ __device__ __forceinline__ void count_earlier_picks(const WorldDev &w, const Tab
 //      lane resolves its destination row and keeps it in registers;
 //   4. the waves fan their rows out.  The last workgroup has counted everything and writes
 //      out_expert_num_tokens.
+// NV = 0: the rows go through LDS; the waves that share a token fetch its row together (fused_rows_in_lds).
 template <int NV, bool EXACT, class DT>
 __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, DT tab, uint32_t ksplit,
                                                                   uint32_t kper, uint32_t tokens_per_block,
@@ -790,10 +791,10 @@ bool dispatch_is_fused(const WorldDev &w) {
   //     42.8, 192 45.2 / 45.8; 7 KiB: 126 30.8 / 33.4, 140 33.9 / 35.8, 154 36.5 / 38.7; the same with half of
   //     the tokens absent (8 KiB, 144: 21.3 / 23.2), and for 8 KiB rows with scales (148 35.5 / 37.9,
   //     182 42.8 / 44.2): these run up to 176
-  // The recount weighs more where it cannot take four picks at a time, or has more than eight: 8 KiB rows,
-  // top-5 120 33.1 / 31.2; top-6 120 32.7 / 32.0; top-9 117 33.3 / 31.7; top-10 120 33.8 / 32.7, 140 38.3 / 36.4;
-  // top-12 120 34.4 / 31.5; top-16 160 58.4 / 41.2 (but 113 39.4 / 42.4, 120 42.1 / 44.5: up to 1024 tokens
-  // the slots take a launch of a single workgroup).
+  // Picks that are not counted four at a time, or more than eight, run up to 112 (120 in steps of up to 1024 tokens),
+  // where the forms come level: 8 KiB rows, top-5 80 21.3 / 23.4, 160 39.8 / 38.3; top-9 144 35.5 / 36.2; top-10 160 38.4 / 38.7;
+  // top-12 192 45.1 / 44.9.  (Up to 1024 tokens the slots take a launch of a single workgroup, and one launch is ahead
+  // beyond that as well: top-16 128 31.1 / 43.6; not taken up.)
   const uint64_t tokens = (uint64_t)w.G * w.M;
   const uint32_t waves = fused_waves(w);
   const uint64_t stored = tokens * w.K * (w.Hb + 4ull * w.S);

@@ -212,8 +212,8 @@ __device__ __forceinline__ void store_staged_row(const WorldDev &w, const Dispat
 namespace pplx_amd {
 namespace {
 // Rows of up to 8 KiB and rows of exactly 10, 12, 14 or 16 KiB (5120-, 6144-, 7168- and 8192-wide
-// bf16) have a register variant in every row kernel; other sizes beyond 8 KiB take
-// dispatch_scatter's padded variants or the streaming kernels.
+// bf16) have a register variant in every row kernel; other sizes beyond 8 KiB go through LDS (the one-launch
+// dispatch; the scatter too where they share lines), take the scatter's padded variants or the streaming kernels.
 inline bool row_has_register_variant(const WorldDev &w) {
   const uint32_t nvec = w.Hb / 16;
   const uint32_t per_lane = (nvec + kWave - 1) / kWave;

@@ -256,6 +256,10 @@ def test_pieces_of_fp32_rows(M, K, H, dp, out_dtype):
         (64, 8, 129, 8, 3088, ONE_LAUNCH),  # two waves to a token
         (64, 6, 512, 8, 5136, ONE_LAUNCH),  # sixteen rows to a workgroup
         (64, 9, 258, 8, 1392, TABLES),  # picks that are counted one by one
+        (64, 1, 512, 8, 10128, ONE_LAUNCH),  # sixteen rows and the tables fill a CU's LDS
+        (64, 1, 512, 8, 10144, TABLES),  # ... and no longer fit it; 64 tiles of one chunk, 64 lanes to a pick
+        (40, 5, 512, 8, 10240, TABLES),  # whole lines; 64 tiles of one chunk, lanes left over
+        (16, 1, 401, 8, 10240, TABLES),  # 51 tiles of one chunk, the last nearly empty
         (40, 5, 520, 8, 1040, TABLES),
         (24, 4, 521, 8, 4208, TABLES),
         (16, 1, 523, 8, 8080, TABLES),

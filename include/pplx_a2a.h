@@ -238,6 +238,10 @@ typedef struct pplx_a2a_plan {
 } pplx_a2a_plan_t;
 /* in_dtype: pplx_a2a_dtype of expert_y */
 int pplx_a2a_plan(const pplx_a2a_config_t *cfg, int in_dtype, pplx_a2a_plan_t *out);
+/* The same for a GPU with `lds_per_cu` bytes of LDS per compute unit (0: it does not say).
+ * `rows_in_lds` (optional) receives 1 when dispatch takes its rows through LDS, not registers. */
+int pplx_a2a_plan_on(const pplx_a2a_config_t *cfg, int in_dtype, uint32_t lds_per_cu, pplx_a2a_plan_t *out,
+                     int32_t *rows_in_lds);
 
 /* Parts of a step for pplx_a2a_world_abandon_step. */
 #define PPLX_A2A_ABANDON_DISPATCH 1u

@@ -1100,11 +1100,16 @@ int pplx_a2a_static_step(const pplx_a2a_config_t *cfg, int device,
 }
 
 int pplx_a2a_plan(const pplx_a2a_config_t *cfg, int in_dtype, pplx_a2a_plan_t *out) {
+  return pplx_a2a_plan_on(cfg, in_dtype, 160u << 10, out, nullptr);
+}
+
+int pplx_a2a_plan_on(const pplx_a2a_config_t *cfg, int in_dtype, uint32_t lds_per_cu, pplx_a2a_plan_t *out,
+                     int32_t *rows_in_lds) {
   if (!cfg || !out) return fail(PPLX_A2A_INVALID_ARGUMENT, "cfg / out is NULL");
   if (int st = check_config(*cfg)) return st;
   WorldDev d{};
   fill_geometry(*cfg, d);
-  d.lds_per_cu = 160u << 10;
+  d.lds_per_cu = lds_per_cu;
   const DispatchPlan dispatch = dispatch_plan(d);
   pplx_a2a_plan_t plan{};
   plan.dispatch_form = (int32_t)dispatch.form;
@@ -1113,6 +1118,7 @@ int pplx_a2a_plan(const pplx_a2a_config_t *cfg, int in_dtype, pplx_a2a_plan_t *o
   plan.scatter_in_turn = dispatch.scatter_in_turn;
   plan.combine_per_group = combine_gathers_per_group(d, in_dtype);
   *out = plan;
+  if (rows_in_lds) *rows_in_lds = dispatch.rows_in_lds;
   return PPLX_A2A_OK;
 }
 

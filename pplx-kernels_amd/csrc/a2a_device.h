@@ -251,6 +251,7 @@ struct DispatchPlan {
   DispatchForm form;
   uint32_t scatter_waves_per_cu;
   bool scatter_in_turn;
+  bool rows_in_lds;
 };
 DispatchPlan dispatch_plan(const WorldDev &w);
 // True when combine gathers the rows of a DP group once for its ranks (in_dtype: pplx_a2a_dtype).

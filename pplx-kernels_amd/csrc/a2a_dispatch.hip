@@ -812,7 +812,9 @@ bool dispatch_is_fused(const WorldDev &w) {
   if (in_lds) {
     const uint64_t rows = (uint64_t)fused_tokens_per_block((uint32_t)tokens, waves) * w.Hb;
     const uint64_t limit = row_shares_lines(w) ? 180ull << 20 : 128ull << 20;
-    return fused_lds_bytes(w, true) + rows <= 160 * 1024 && stored <= limit && (row_shares_lines(w) || tokens <= 2048);
+    // (a device that does not say how much LDS it has is taken to have the 64 KiB of any)
+    const uint32_t lds = w.lds_per_cu ? w.lds_per_cu : 64u << 10;
+    return fused_lds_bytes(w, true) + rows <= lds && stored <= limit && (row_shares_lines(w) || tokens <= 2048);
   }
   if (waves < 16) return true;
   const bool quick_count = w.K % 4 == 0 && w.K <= 8;
@@ -824,15 +826,15 @@ bool dispatch_is_fused(const WorldDev &w) {
 }
 
 DispatchPlan dispatch_plan(const WorldDev &w) {
-  if (dispatch_is_fused(w)) return {DispatchForm::kOneLaunch, 0, false};
+  if (dispatch_is_fused(w)) return {DispatchForm::kOneLaunch, 0, false, fused_rows_in_lds(w)};
   const Slots slots = slots_of(w);
   const DispatchForm form = slots == Slots::kMap      ? DispatchForm::kSlotMap
                             : slots == Slots::kTables ? DispatchForm::kTables
                                                       : DispatchForm::kScannedTables;
-  if (!scatter_has_register_rows(w)) return {form, 0, false};
+  if (!scatter_has_register_rows(w)) return {form, 0, false, false};
   const uint32_t ksplit = pick_ksplit(w, kWave);
   const ScatterPlan plan = scatter_plan(w, (w.K + ksplit - 1) / ksplit);
-  return {form, plan.waves_per_cu, plan.in_turn && slots != Slots::kMap};
+  return {form, plan.waves_per_cu, plan.in_turn && slots != Slots::kMap, row_shares_lines(w)};
 }
 
 int launch_bind_dispatch(const WorldDev &w, const BindDispatchBatch &b, void *stream) {

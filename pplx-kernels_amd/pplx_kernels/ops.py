@@ -55,6 +55,7 @@ EXPORTED_SYMBOLS = (
     "pplx_a2a_world_combine",
     "pplx_a2a_static_step",
     "pplx_a2a_plan",
+    "pplx_a2a_plan_on",
     "pplx_a2a_world_recorded_calls",
     "pplx_a2a_world_abandon_step",
     "pplx_a2a_world_reserve_split",
@@ -179,6 +180,9 @@ def load_library() -> ctypes.CDLL:
             ctypes.POINTER(Config), i32, ctypes.POINTER(DispatchArgs), ctypes.POINTER(CombineArgs), vp, vp,
         ]  # fmt: skip
         lib.pplx_a2a_plan.argtypes = [ctypes.POINTER(Config), i32, ctypes.POINTER(Plan)]
+        lib.pplx_a2a_plan_on.argtypes = [
+            ctypes.POINTER(Config), i32, u32, ctypes.POINTER(Plan), ctypes.POINTER(i32),
+        ]  # fmt: skip
         lib.pplx_a2a_world_of.argtypes = [vp]
         lib.pplx_a2a_world_of.restype = vp
         lib.pplx_a2a_world_recorded_calls.argtypes = [vp, i32, i32, ctypes.POINTER(u32)]
@@ -203,6 +207,18 @@ def plan_of(config: Config, in_dtype: torch.dtype = torch.bfloat16) -> Plan:
     plan = Plan()
     check_status(load_library().pplx_a2a_plan(ctypes.byref(config), DTYPE_CODE[in_dtype], ctypes.byref(plan)))
     return plan
+
+
+def plan_on(config: Config, lds_per_cu: int = 160 << 10, in_dtype: torch.dtype = torch.bfloat16) -> tuple[Plan, bool]:
+    """The same for a GPU with ``lds_per_cu`` bytes of LDS per compute unit (0: unknown), and whether dispatch takes
+    its rows through LDS."""
+    plan, rows_in_lds = Plan(), ctypes.c_int32()
+    check_status(
+        load_library().pplx_a2a_plan_on(
+            ctypes.byref(config), DTYPE_CODE[in_dtype], lds_per_cu, ctypes.byref(plan), ctypes.byref(rows_in_lds)
+        )
+    )
+    return plan, bool(rows_in_lds.value)
 
 
 def check_status(status: int) -> None:

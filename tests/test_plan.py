@@ -110,6 +110,26 @@ def test_combine_per_group(ranks, dp, max_tokens, topk, hidden, dtype, per_group
     assert bool(p.combine_per_group) == per_group
 
 
+@pytest.mark.parametrize(
+    "lds,tokens,row,topk,one_launch",
+    [
+        # 8 x 2 rows of 12 KiB and the tables beside them fit any device's LDS, sixteen rows of 10128 bytes only
+        # one of 160 KiB (163712 of its 163840 bytes)
+        (160 << 10, 16, 12016, 2, True),
+        (64 << 10, 16, 12016, 2, True),
+        (0, 16, 12016, 2, True),
+        (160 << 10, 4096, 10128, 1, True),
+        (163711, 4096, 10128, 1, False),
+        (64 << 10, 4096, 10128, 1, False),
+        (0, 4096, 10128, 1, False),
+        (64 << 10, 4096, 8192, 1, True),  # rows in registers need none
+    ],
+)
+def test_rows_in_lds_need_a_device_that_holds_them(lds, tokens, row, topk, one_launch):
+    p, _ = ops.plan_on(ops.Config(tokens // 8, 64, topk, 8, 1, row // 2, row, 0), lds)
+    assert (p.dispatch_form == ONE_LAUNCH) == one_launch
+
+
 def test_forms_of_the_routing():
     assert plan(4104, 1024, 2).dispatch_form == TABLES  # 65 chunks
     assert plan(65536, 1024, 2).routing_tiles == 64

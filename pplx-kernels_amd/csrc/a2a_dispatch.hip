@@ -307,7 +307,11 @@ __device__ __forceinline__ void count_earlier_picks(const WorldDev &w, const Tab
 //   4. the waves fan their rows out.  The last workgroup has counted everything and writes
 //      out_expert_num_tokens.
 // NV = 0: the rows go through LDS; the waves that share a token fetch its row together (fused_rows_in_lds).
-template <int NV, bool EXACT, class DT>
+// MANY: more than eight picks.  Counting them takes 70 registers, in a kernel of its own so that the others do not pay
+// for them: rows of 1, 2 and 3 KiB get by with 42, 45 and 55, and two workgroups fit a CU (kernel alone, us, all
+// numbers of picks in one kernel / apart, medians of two runs of 360 launches: 512-byte rows, 8 x 128 tokens, top-8 6.28 6.36 /
+// 6.12 6.24, 8 x 512, top-4 7.64 7.72 / 7.44 7.64; 1 KiB rows, 8 x 128, top-8 level at 6.20 - 6.32).
+template <int NV, bool EXACT, class DT, bool MANY>
 __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, DT tab, uint32_t ksplit,
                                                                   uint32_t kper, uint32_t tokens_per_block,
                                                                   uint32_t pick_vector, uint32_t write_through) {
@@ -356,7 +360,7 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   const uint32_t my_loaded_e = *as_global(has_pick ? my_src.indices + (size_t)my_t * w.K + lane : w.faults);
 
   // 2. picks of all earlier tokens
-  if (w.K > 8) {
+  if constexpr (MANY) {
     if (pick_vector > 1) count_earlier_picks<2, 16, false, kFusedThreads>(w, rows(), v0, hist);
     else count_earlier_picks<1, 16, false, kFusedThreads>(w, rows(), v0, hist);
   } else if (w.K > 4) {
@@ -696,8 +700,6 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t 
     else PPLX_DISPATCH_ROW_VARIANTS(dispatch_scatter_slots);
   }
 #undef PPLX_LAUNCH_ROW_VARIANT
-#define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                               \
-  hipLaunchKernelGGL((KERNEL<NV, EXACT, DT>), grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS)
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
 #undef PPLX_ROW_KERNEL_ARGS
   return (int)hipGetLastError();
@@ -725,10 +727,18 @@ int launch_fused_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hipSt
   const uint64_t row_bytes = (uint64_t)tokens * w.K * (w.Hb + 4ull * w.S);
   const uint32_t write_through = row_bytes <= (staged ? 64ull << 20 : kWriteThroughMaxBytes) ? 1u : 0u;
 #define PPLX_ROW_KERNEL_ARGS ksplit, kper, tokens_per_block, pick_vector, write_through
+#define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                                                       \
+  do {                                                                                                                   \
+    if (w.K > 8)                                                                                                         \
+      hipLaunchKernelGGL((KERNEL<NV, EXACT, DT, true>), grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS);              \
+    else                                                                                                                 \
+      hipLaunchKernelGGL((KERNEL<NV, EXACT, DT, false>), grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS);             \
+  } while (0)
 #define PPLX_LAUNCH_LARGE_ROW_VARIANT(KERNEL) return (int)hipErrorInvalidValue
   if (staged) PPLX_LAUNCH_ROW_VARIANT(dispatch_fused, 0, false);
   else PPLX_DISPATCH_ROW_VARIANTS(dispatch_fused);
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
+#undef PPLX_LAUNCH_ROW_VARIANT
 #undef PPLX_ROW_KERNEL_ARGS
   return (int)hipGetLastError();
 }

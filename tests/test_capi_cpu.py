@@ -278,6 +278,16 @@ def test_no_kernel_spills_or_uses_scratch():
     assert not offenders, offenders
 
 
+def test_one_launch_dispatch_of_short_rows_leaves_room_for_two_workgroups():
+    """The one-launch dispatch of rows of up to 3 KiB and up to eight picks keeps to 64 vector registers, so that two of
+    its workgroups (1024 threads) fit the 512 registers that a lane of each of a CU's four SIMDs has."""
+    name = re.compile(r"14dispatch_fusedILi([123])ELb1E.*Lb0EEE")
+    kernels = [(name.search(k[".name"]), k) for k in _gpu_kernels_of(ops._LIB_PATH)]
+    short = {k[".name"]: k[".vgpr_count"] for found, k in kernels if found}
+    assert len(short) == 6  # three lengths, two places of the rank tables
+    assert all(v <= 64 for v in short.values()), short
+
+
 def test_bench_refuses_more_than_one_gpu():
     """Every simulated rank shares one GPU's HBM: `bench.py --gpus N` with N above 1 (or under a
     launcher that sets WORLD_SIZE) exits with a message that says so, before it touches a GPU."""

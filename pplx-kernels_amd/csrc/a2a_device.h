@@ -195,13 +195,23 @@ inline StageLayout stage_layout(uint32_t row_bytes, uint32_t scales, uint64_t to
 // arguments each.
 constexpr uint32_t kInlineRanks = 64;
 constexpr uint32_t kBindBatch = 64;
-// A fused launch whose rows (all picks of all tokens) stay within this many bytes stores them
-// write-through into the 256 MB last-level cache instead of streaming them past it.  That pays where a step's
-// buffers come back soon: 14 KiB rows, top-8, 1024 tokens (112 MiB), one buffer set, dispatch alone 25.9 us written
-// through / 30.4 streamed.  With three sets in turn the two are level from about 108 MiB on (step, 112 MiB 55.1 / 53.2; 8 KiB
-// rows 112 MiB 51.1 / 51.2, 140 65.0 / 63.8; 7 KiB fp8 rows 56 MiB 37.3 / 40.2, 95 66.7 / 67.3, 112 78.5 / 77.0), and with sixteen
-// streaming is ahead from 8 MiB on (7 KiB fp8 rows, 32 MiB 30.3 / 28.6, 64 51.5 / 49.7).
+// A one-launch dispatch whose rows (all picks of all tokens) stay within this many bytes and go through registers
+// stores them write-through into the 256 MB last-level cache instead of streaming them past it.  That pays where
+// a step's buffers come back soon: 14 KiB rows, top-8, 1024 tokens (112 MiB), one buffer set, dispatch alone 25.9
+// us written through / 30.4 streamed.  With three sets in turn the two are level from about 108 MiB on (step,
+// 112 MiB 55.1 / 53.2; 8 KiB rows 112 MiB 51.1 / 51.2, 140 65.0 / 63.8; 7 KiB fp8 rows 56 MiB 37.3 / 40.2,
+// 95 66.7 / 67.3, 112 78.5 / 77.0), and with sixteen streaming is ahead from 8 MiB on (7 KiB fp8 rows,
+// 32 MiB 30.3 / 28.6, 64 51.5 / 49.7).
 constexpr uint64_t kWriteThroughMaxBytes = 192ull << 20;
+// The same for rows that go through LDS, whose whole lines stream well: up to where the two are level on three sets.
+// Us, written through / streamed, 8 ranks, top-8, at the MiB of rows stored; one set: dispatch alone, others: step:
+//                one set                              three sets                           sixteen sets
+//                66          80          95           66          80          95           66          80
+//   2576 bytes   16.5 18.0   18.1 20.6                35.2 35.4   41.5 40.9                42.5 36.1   48.8 42.7
+//   4240 bytes   15.3 17.4   18.2 21.8   20.2 23.2    33.8 35.0   41.8 42.5   48.2 46.7    40.5 35.4   48.1 43.1
+//   5264 bytes   15.3 17.6   17.3 21.4   20.3 23.6    33.1 34.8   42.0 43.7   49.7 46.8    39.5 34.9   48.4 44.0
+//   8176 bytes   15.3 17.8   17.1 20.0   19.1 24.5    35.8 37.0   40.4 40.6   47.1 46.4    41.0 37.4   44.9 40.9
+constexpr uint64_t kLdsWriteThroughMaxBytes = 80ull << 20;
 
 // Device memory that pplx_a2a_static_step works in instead of a world's allocations: a fixed
 // array inside the library's code object (a2a_static.hip), one copy per GPU.  The chunks' bases

@@ -720,12 +720,9 @@ int launch_fused_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hipSt
   const uint32_t kper = (w.K + ksplit - 1) / ksplit;
   const dim3 grid((tokens + tokens_per_block - 1) / tokens_per_block), block(kWaves * kWave);
   const uint32_t lds = fused_lds_bytes(w, DT::kInline && w.R <= kInlineRanks) + (staged ? tokens_per_block * w.Hb : 0u);
-  // Rows that fit the last-level cache with room to spare are written through into it.  Rows in LDS less far:
-  // dispatch + combine, us, on three buffer sets in turn / on sixteen, written through and streamed at the MiB of rows
-  // stored: 5264-byte rows, top-8 31 19.5 20.1 / 24.4 20.9, 63 32.2 34.2 / 38.9 34.1, 95 49.7 47.5 / 52.7 47.4; 8176 bytes, top-6
-  // 47 25.5 26.8 / 30.3 27.0, 95 48.9 46.8 / 51.3 46.5; 12016 bytes, top-8 (three sets) 63 31.4 33.3, 95 50.1 50.1, 127 63.7 59.8.
+  // Rows that fit the last-level cache with room to spare are written through into it.
   const uint64_t row_bytes = (uint64_t)tokens * w.K * (w.Hb + 4ull * w.S);
-  const uint32_t write_through = row_bytes <= (staged ? 64ull << 20 : kWriteThroughMaxBytes) ? 1u : 0u;
+  const uint32_t write_through = row_bytes <= (staged ? kLdsWriteThroughMaxBytes : kWriteThroughMaxBytes) ? 1u : 0u;
 #define PPLX_ROW_KERNEL_ARGS ksplit, kper, tokens_per_block, pick_vector, write_through
 #define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                                                       \
   do {                                                                                                                   \

@@ -566,6 +566,25 @@ uint32_t pick_ksplit(const WorldDev &w, uint32_t max_split) {
   return ksplit;
 }
 
+// Whether the scatter takes rows that share lines through LDS.  A row costs a trip to LDS in front of its
+// first store and another read of it per copy there, which short rows of small steps, bound by the chain of a wave and
+// not by the memory, do not get back.  Dispatch on three buffer sets, experts 64, LDS : registers at 4200, 8000 and
+// 20000 tokens
+//               top-4              top-8              top-10             top-16             top-64
+//   112 bytes   1.02 1.02 1.01     1.07 1.04 1.00     1.10 1.03 0.98     1.12 1.03 0.93     0.91 0.76 0.83
+//   144 bytes   1.04 1.01 1.01     1.09 1.02 0.97     1.12 1.00 0.99     1.09 0.97 0.87     0.92 0.77 0.80
+//   272 bytes   1.02 0.99 0.95     1.08 0.96 0.89     1.07 0.94 0.81     1.06 0.88 0.76     1.00 0.90 0.96
+//   400 bytes   1.01 0.96 0.90     1.04 0.91 0.81     1.01 0.86 0.77     0.91 0.71 0.68     0.90 0.83 0.90
+//   528 bytes   1.00 0.97 0.83     0.99 0.83 0.71     0.97 0.79 0.66     0.81 0.63 0.63     0.87 0.95 0.88
+// The two are level where the step's rows, read once, come to 2 MiB, or what it stores to 24.  Rows of 96 bytes and
+// less lose (16 bytes 1.03 - 1.44, 48 bytes 1.0 - 1.26, 64 bytes, which cut no line, 1.20 - 1.44, 96 bytes 1.0 - 1.12)
+// except for some steps of 64 picks (80 and 96 bytes 0.85 - 0.91).
+bool scatter_rows_in_lds(const WorldDev &w) {
+  if (!row_shares_lines(w) || w.Hb < 112) return false;
+  const uint64_t read = (uint64_t)w.G * w.M * w.Hb;
+  return w.Hb >= 1024 || read >= 2u << 20 || read * w.K >= 24u << 20;
+}
+
 // How the scatter's waves go about their stores: how many of them a CU holds at a time (0 = as many
 // as fit), and whether they take the row, the slots and the experts' buffers one behind the other
 // (scatter_token).  A wave's launch, its loads and its slot arithmetic are dead time for the stores, so
@@ -618,7 +637,7 @@ ScatterPlan scatter_plan(const WorldDev &w, uint32_t picks_per_wave) {
   const uint64_t tokens = (uint64_t)w.G * w.M;
   const uint64_t row = w.Hb + 4ull * w.S;
   const uint64_t stored = (uint64_t)picks_per_wave * row;
-  if (row_shares_lines(w)) {
+  if (scatter_rows_in_lds(w)) {
     if (stored >= 32 * 1024) {
       if (tokens > 16384 && row >= 8192) return {3, true};
       return {tokens > 32768 ? 4u : 3u, false};
@@ -655,7 +674,7 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t 
   // interleaved (figures at scatter_plan).  The hardware has no such knob, so each workgroup asks for a share of
   // the CU's LDS that only that many fit into.
   const ScatterPlan plan = scatter_plan(w, kper);
-  const bool staged = row_shares_lines(w);
+  const bool staged = scatter_rows_in_lds(w);
   // (LDS is handed out in blocks: a share that is not a multiple of 4 KiB can round up past
   // what the intended number of workgroups leaves room for)
   uint32_t lds = plan.waves_per_cu ? (w.lds_per_cu / plan.waves_per_cu) & ~4095u : 0u;
@@ -841,7 +860,7 @@ DispatchPlan dispatch_plan(const WorldDev &w) {
   if (!scatter_has_register_rows(w)) return {form, 0, false, false};
   const uint32_t ksplit = pick_ksplit(w, kWave);
   const ScatterPlan plan = scatter_plan(w, (w.K + ksplit - 1) / ksplit);
-  return {form, plan.waves_per_cu, plan.in_turn && slots != Slots::kMap, row_shares_lines(w)};
+  return {form, plan.waves_per_cu, plan.in_turn && slots != Slots::kMap, scatter_rows_in_lds(w)};
 }
 
 int launch_bind_dispatch(const WorldDev &w, const BindDispatchBatch &b, void *stream) {

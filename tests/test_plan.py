@@ -130,6 +130,31 @@ def test_rows_in_lds_need_a_device_that_holds_them(lds, tokens, row, topk, one_l
     assert (p.dispatch_form == ONE_LAUNCH) == one_launch
 
 
+@pytest.mark.parametrize(
+    "tokens,row,topk,in_lds",
+    [
+        (40000, 96, 10, False),
+        (18728, 112, 3, True),  # rows of 2 MiB together
+        (18720, 112, 3, False),
+        (5248, 400, 2, True),
+        (5240, 400, 2, False),
+        (4104, 112, 55, True),  # copies of 24 MiB together
+        (4104, 112, 54, False),
+        (4104, 512, 8, False),  # whole lines
+        (4104, 1008, 1, True),
+        (4104, 1040, 8, True),
+        (1024, 8192 + 16, 32, True),  # rows from 1 KiB on
+        (4104, 10240, 8, False),
+        (4104, 32752, 2, True),
+        (4104, 32784, 2, False),  # beyond the kernels of one wave per token
+    ],
+)
+def test_rows_of_the_scatter_in_lds(tokens, row, topk, in_lds):
+    p, rows_in_lds = ops.plan_on(ops.Config(tokens // 8, 64, topk, 8, 1, row // 2, row, 0))
+    assert p.dispatch_form != ONE_LAUNCH
+    assert rows_in_lds == in_lds
+
+
 def test_forms_of_the_routing():
     assert plan(4104, 1024, 2).dispatch_form == TABLES  # 65 chunks
     assert plan(65536, 1024, 2).routing_tiles == 64

@@ -231,8 +231,7 @@ typedef enum pplx_a2a_dispatch_form {
 typedef struct pplx_a2a_plan {
   int32_t dispatch_form;          /* pplx_a2a_dispatch_form */
   uint32_t routing_tiles;
-  uint32_t scatter_waves_per_cu;  /* 0 = as many as fit, or no scatter launch; rows of no whole number of
-                                     128-byte lines: half of the waves */
+  uint32_t scatter_waves_per_cu;  /* 0 = as many as fit, or no scatter launch */
   int32_t scatter_in_turn;   /* 1: its waves fetch row, slots and buffers one behind the other */
   int32_t combine_per_group;      /* 1: combine gathers once for the ranks of a DP group */
 } pplx_a2a_plan_t;

@@ -592,7 +592,7 @@ bool scatter_rows_in_lds(const WorldDev &w) {
 // few waves keep the stores in longer runs, and large steps do best with three whose stores start
 // later.  Dispatch on 8 ranks, us, all forms alternating in one process on the same buffers (whose
 // place in memory moves all of them by up to 15 % from one process to the next); side by side at 4 and
-// 10 waves / one behind the other at 3:
+// 10 waves (nine, in fact: see kLdsBlock; the two are within 0.8 %) / one behind the other at 3:
 //   59 KiB stored per wave (DSv3 fp8 rows, top-8 of 256)
 //     8 x 509    52.7 /  -  / 53.0     8 x 1024  97.8 /  -  / 98.4    8 x 2048  184 / 189 / 185
 //     8 x 4096    432 / 431 / 430      8 x 6000   645 / 626 / 610     8 x 8192  859 / 843 / 826
@@ -614,9 +614,8 @@ bool scatter_rows_in_lds(const WorldDev &w) {
 //    4 KiB (2 KiB fp8 rows with scales, top-2)         162 /  143 /  125 /  118 /  112 /  110 /  109
 // (one behind the other they lose: 8 x 4096 tokens of 8 KiB, top-2, skewed: 123 and 130; 2 KiB rows,
 // top-6, 8 x 1024: 26.2 and 27.5).
-// Rows that share lines (a2a_rows.h) spend more time in front of and between their stores, and want twice
-// as many waves; so scatter_plan gives half of what a CU holds, and launch_scatter_t halves the share of LDS.  Us
-// at 6 / 8 / 12 / 16 / 24 waves, side by side unless it says otherwise:
+// Rows in LDS (a2a_rows.h) spend more time in front of and between their stores and want more waves.  Us at 6 / 8 / 12 /
+// 16 waves / as many as fit, side by side unless it says otherwise:
 //   66 KiB (8656-byte rows, top-10 of 128)  2 x 1252  54.1 / 56.6 / 55.4 / 55.8 /  -
 //   41 KiB (5264-byte rows, top-8 of 256)   8 x 513   42.0 / 44.1 / 43.3 /  -        8 x 2048  139 / 140 / 143 / 143
 //     8 x 5000   339 / 339 / 342 (in turn 348 / 343 / 343; four waves 404, three 455)
@@ -624,9 +623,13 @@ bool scatter_rows_in_lds(const WorldDev &w) {
 //   40 KiB (8208-byte rows, top-5 of 40)    8 x 2100   137 / 138 / 139 (in turn 140)  8 x 6100  449 / 466 / 461 (in turn 443)
 //   23 KiB (2976-byte rows, top-8 of 16)    4 x 4903   95.1 / 92.1 / 94.4 / 96.6
 //   17 KiB (4240-byte rows, top-4 of 4)     4 x 6712   59.7 / 54.2 / 52.6 / 53.0
-//    8 KiB (1040-byte rows, top-8 of 64)    8 x 8000    -  / 186 / 137 / 109 / 104
-//    7 KiB (2576-byte rows, top-3 of 16)    4 x 3587   42.4 / 38.5 / 35.0 / 32.9
-//    5 KiB (2528-byte rows, top-2 of 64)    8 x 8000    -  / 143 / 109 / 101 / 97.5, as many as fit 97.6
+//    5 KiB (2528-byte rows, top-2 of 64)    8 x 8000    -  / 143 / 109 / 101 / 97.6
+// and on two buffer sets in turn, at 12 / 16 / 25 waves / as many as fit:
+//    9 KiB (3088-byte rows, top-3 of 64)    8 x 5000  110 / 106 / 105 / 106
+//    8 KiB (1040-byte rows, top-8 of 64)    8 x 8000  175 / 161 / 158 / 153
+//    8 KiB (2064-byte rows, top-4 of 64)    8 x 8000  152 / 139 / 136 / 138    8 x 1000  22.8 / 22.1 / 21.3 / 21.9
+//    7 KiB (784-byte rows, top-10 of 64)    8 x 6000  108 / 95.1 / 83.9 / 80.9
+//    6 KiB (3088-byte rows, top-2 of 64)    8 x 2000  34.4 / 31.6 / 30.0 / 29.8
 struct ScatterPlan {
   uint32_t waves_per_cu;
   bool in_turn;
@@ -639,12 +642,11 @@ ScatterPlan scatter_plan(const WorldDev &w, uint32_t picks_per_wave) {
   const uint64_t stored = (uint64_t)picks_per_wave * row;
   if (scatter_rows_in_lds(w)) {
     if (stored >= 32 * 1024) {
-      if (tokens > 16384 && row >= 8192) return {3, true};
-      return {tokens > 32768 ? 4u : 3u, false};
+      if (tokens > 16384 && row >= 8192) return {6, true};
+      return {tokens > 32768 ? 8u : 6u, false};
     }
-    if (stored >= 20 * 1024) return {4, false};
-    if (stored >= 12 * 1024) return {6, false};
-    return {stored >= 6 * 1024 ? 12u : 0u, false};
+    if (stored >= 20 * 1024) return {8, false};
+    return {stored >= 12 * 1024 ? 12u : 0u, false};
   }
   if (stored >= 24 * 1024) {
     if (tokens <= 16384) return {4, false};
@@ -653,6 +655,15 @@ ScatterPlan scatter_plan(const WorldDev &w, uint32_t picks_per_wave) {
   }
   if (stored >= 12 * 1024) return {row >= 4096 ? 4u : 10u, false};
   return {stored >= 6 * 1024 ? 12u : 0u, false};
+}
+
+// Dynamic LDS of a scatter workgroup (one wave): the row if it goes through LDS, and the share of a CU's LDS of which as
+// many fit as the plan wants.  LDS is handed out in blocks of 1280 bytes, 128 to a CU (one-wave workgroups that hold 16384
+// bytes run nine to a CU, with 15360 ten; 12288 and 12800 twelve).
+constexpr uint32_t kLdsBlock = 1280;
+uint32_t scatter_lds(const WorldDev &w, const ScatterPlan &plan) {
+  const uint32_t share = plan.waves_per_cu ? w.lds_per_cu / kLdsBlock / plan.waves_per_cu * kLdsBlock : 0;
+  return scatter_rows_in_lds(w) && share < w.Hb ? w.Hb : share;
 }
 
 // Rows that dispatch_scatter holds in registers (longer ones stream through dispatch_scatter_long).
@@ -675,15 +686,7 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t 
   // the CU's LDS that only that many fit into.
   const ScatterPlan plan = scatter_plan(w, kper);
   const bool staged = scatter_rows_in_lds(w);
-  // (LDS is handed out in blocks: a share that is not a multiple of 4 KiB can round up past
-  // what the intended number of workgroups leaves room for)
-  uint32_t lds = plan.waves_per_cu ? (w.lds_per_cu / plan.waves_per_cu) & ~4095u : 0u;
-  if (lds > 65536u) lds = 65536u;
-  if (staged) {
-    lds = (lds / 2) & ~4095u;
-    const uint32_t row = (w.Hb + 1023u) & ~1023u;
-    if (lds < row) lds = row;
-  }
+  const uint32_t lds = scatter_lds(w, plan);
   const dim3 grid((uint32_t)waves + (slots == Slots::kTables ? (w.E + 7) / 8 : 0u)), block(kWave);
 #define PPLX_ROW_KERNEL_ARGS ksplit, kper
 #define PPLX_LAUNCH_LARGE_ROW_VARIANT(KERNEL)                                                    \
@@ -860,7 +863,13 @@ DispatchPlan dispatch_plan(const WorldDev &w) {
   if (!scatter_has_register_rows(w)) return {form, 0, false, false};
   const uint32_t ksplit = pick_ksplit(w, kWave);
   const ScatterPlan plan = scatter_plan(w, (w.K + ksplit - 1) / ksplit);
-  return {form, plan.waves_per_cu, plan.in_turn && slots != Slots::kMap, scatter_rows_in_lds(w)};
+  uint32_t waves = plan.waves_per_cu;
+  if (waves) {  // (fewer where the rows take more than their share)
+    const uint32_t blocks = (scatter_lds(w, plan) + kLdsBlock - 1) / kLdsBlock;
+    const uint32_t fit = w.lds_per_cu / kLdsBlock / (blocks ? blocks : 1);
+    if (waves > fit) waves = fit;
+  }
+  return {form, waves, plan.in_turn && slots != Slots::kMap, scatter_rows_in_lds(w)};
 }
 
 int launch_bind_dispatch(const WorldDev &w, const BindDispatchBatch &b, void *stream) {

@@ -34,7 +34,6 @@ def plan(tokens, row, topk, experts=64, scales=0, ranks=8, dp=1):
         (32768, 4096, 0, 8, 3, True),
         (32776, 4096, 0, 8, 4, False),
         (32776, 8192, 0, 4, 3, True),
-        (32776, 8176, 0, 6, 4, False),
         (65536, 10240, 0, 4, 3, True),
         # from 24 KiB on
         (16392, 4096, 0, 6, 4, False),
@@ -45,6 +44,17 @@ def plan(tokens, row, topk, experts=64, scales=0, ranks=8, dp=1):
         (32768, 2048, 16, 8, 10, False),
         (32768, 1024, 8, 8, 12, False),
         (32768, 2048, 16, 2, 0, False),
+        # rows that share lines, through LDS: from 32 KiB on six waves, or eight beyond 32768 tokens; ...
+        (16384, 8208, 0, 4, 6, False),
+        (16392, 8208, 0, 4, 6, True),  # ... in turn from 8 KiB rows and 16384 tokens on
+        (32776, 8208, 0, 4, 6, True),
+        (32768, 8176, 0, 6, 6, False),
+        (32776, 8176, 0, 6, 8, False),
+        (32776, 8176, 0, 3, 8, False),  # from 20 KiB on
+        (32776, 8176, 0, 2, 12, False),  # from 12 KiB on
+        (32776, 8176, 0, 1, 0, False),
+        (32776, 2064, 0, 5, 0, False),
+        (32776, 2064, 0, 6, 12, False),
     ],
 )
 def test_scatter(tokens, row, scales, topk, waves, in_turn):
@@ -128,6 +138,13 @@ def test_combine_per_group(ranks, dp, max_tokens, topk, hidden, dtype, per_group
 def test_rows_in_lds_need_a_device_that_holds_them(lds, tokens, row, topk, one_launch):
     p, _ = ops.plan_on(ops.Config(tokens // 8, 64, topk, 8, 1, row // 2, row, 0), lds)
     assert (p.dispatch_form == ONE_LAUNCH) == one_launch
+
+
+@pytest.mark.parametrize("row,waves", [(26864, 6), (26896, 5), (32752, 4)])
+def test_long_rows_in_lds_leave_room_for_fewer_waves(row, waves):
+    """LDS is handed out in 128 blocks of 1280 bytes: six rows of 21 blocks, five of 22, four of 26."""
+    p = plan(16384, row, 2)
+    assert p.dispatch_form == SLOT_MAP and p.scatter_waves_per_cu == waves
 
 
 @pytest.mark.parametrize(

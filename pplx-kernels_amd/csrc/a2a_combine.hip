@@ -249,24 +249,25 @@ int launch_combine_v(const WorldDev &w, const CT &tab, bool grouped, hipStream_t
   return (int)hipGetLastError();
 }
 
+// Whether pieces of `length` KiB of a 16-bit row make workgroups that come out even, `least` to four of them to each of the
+// 256 CUs, with at most 1 KiB of padding to a piece.
+bool even_pieces(uint64_t tokens, uint32_t segments, uint32_t length, uint32_t least) {
+  const uint32_t pieces = (segments + length - 1) / length;
+  if (pieces * length - segments > pieces) return false;
+  const uint64_t workgroups = (tokens * pieces + kWavesPerBlock - 1) / kWavesPerBlock;
+  const uint64_t per_cu = (workgroups + 255) / 256;
+  return per_cu >= least && per_cu <= 4 && 256 * per_cu - workgroups <= 16;
+}
+
 template <typename T, typename U, class CT>
 int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
 #define PPLX_COMBINE(KB, VPL) return launch_combine_v<T, U, CT, KB, VPL>(w, tab, grouped, s)
   const bool grouped = combine_per_group(w, sizeof(T));
-  // All picks of 1 KiB of a row at once where they are three to eight, longer pieces of fewer (two to eight
-  // loads per lane in flight either way, and no piece longer than the row) -- except for steps of a few
+  // Five picks and more are taken up to eight at a time, 1 KiB of a row each -- except for steps of a few
   // hundred to two thousand tokens, whose waves are all resident at the same moment: there more than four
   // picks are better taken one after the other in 7 or 8 KiB pieces by a quarter as many waves
   // (8 x 128 DSv3 tokens, top-8: 23.4 us against 25.3 us; 8 x 256: 45.8 against 46.8; from
-  // 8 x 512 on the wide form wins, 88.7 against 91.5 us, and below 8 x 64 too).
-  // Dispatch + combine, 8 ranks, bf16, us, formerly / now: top-1 (one pick of 8 KiB / of up to 3), 16384 tokens 512 wide
-  // 30.8 / 24.1, 1024 wide 37.0 / 32.3, 8192 wide 203.5 / 195.7 (1 KiB pieces 217); top-2 (two of 4 / of up to 2 KiB), 8192 tokens
-  // 512 wide 21.7 / 19.8, 1024 wide 27.0 / 26.0, 6656 wide 125.4 / 124.4; top-3 (eight places, so two picks and then one /
-  // three of 1 KiB), 8192 tokens 2048 wide 57.0 / 52.4, 4096 wide 99.5 / 90.4, 4096 tokens 7168 wide 89.9 / 81.7; top-5 (four, then
-  // one / five of 1 KiB), 16000 tokens 512 wide 43.4 / 41.6, 4096 tokens 7168 wide 124.6 / 122.5, 320 tokens 4096 wide 13.3 /
-  // 12.8.  A wave that serves a DP group compares its members first, so pieces stay as long as formerly there unless that
-  // is mostly padding (groups of two, 4 x 512 tokens, short / long pieces: 2048 wide, top-1 13.8 / 12.8, top-2 16.5 / 15.4; 4096
-  // wide, top-1 20.8 / 18.7, top-2 26.1 / 25.5; but 4600 wide, nine KiB, top-1 23.5 / 30.4, top-2 29.9 / 39.9).  Top-6 and top-7 in one go measure the same as four picks and the rest (145.0 / 145.9, 165.3 / 165.0).
+  // 8 x 512 on the wide form wins, 88.7 against 91.5 us, and below 8 x 64 too).  Fewer picks: at the switch below.
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
   const uint64_t tokens = (uint64_t)(grouped ? w.G : w.R) * w.M;
   if (w.K > 4 && tokens > 384 && tokens <= 2048 && nvec_segments >= 7) {
@@ -295,16 +296,36 @@ int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
       PPLX_COMBINE(3, 2);
     }
   }
+  // Of what is left, up to five picks are taken all at once.  One or two leave a wave of 1 KiB with little in flight, so they read longer
+  // pieces: up to 3 KiB of one pick and 2 KiB of two, which is ahead of 8 and of 4 KiB nearly everywhere (dispatch +
+  // combine, 8 ranks, us, long / short pieces: one pick of 16-bit rows, 512 tokens, 2048 wide 8.3 / 7.8, 4096 wide 9.2 /
+  // 8.8, 8192 wide 12.0 / 11.4; 8192 tokens, 52.3 / 51.0 and 105.9 / 103.6; two picks, 512 tokens, 8.7 / 8.3, 10.0 /
+  // 10.0 and 14.1 / 13.9; 8192 tokens, 71.6 / 70.5 and 151.8 / 150.2; not one pick, 1024 tokens, 2560 wide 9.2 / 9.6, 3072
+  // 9.6 / 10.1), except
+  //  - where the workgroups of the long pieces come out even over the CUs (even_pieces): one pick, 2048 tokens, 3584 wide
+  //    15.1 / 15.7, 4096 wide 16.0 / 16.7, 8192 wide 28.9 / 29.5; 4096 tokens of 4096 29.5 / 30.2; 1536 of 7168 19.6 / 20.5 (but
+  //    uneven, 4096 wide, 1536 tokens 15.1 / 14.3, 2560 19.8 / 19.8, 3584 25.1 / 24.6); two picks of fp32 rows only where
+  //    there are four workgroups to a CU: 4096 tokens, 2048 wide 27.9 / 28.8; 2048 tokens, 4096 wide 27.6 / 28.4
+  //    (three, 3072 tokens, 2048 wide 22.8 / 22.9; 3584 tokens 26.2 / 25.4; two, 1024 tokens, 4096 wide 17.2 / 17.1);
+  //  - for DP groups, whose waves compare the members first.  They keep the long pieces for rows that are longer than half
+  //    of one (groups of two, 4 x 512 tokens, one pick, 4096 wide 18.8 / 20.6, 7168 wide 32.1 / 31.4; groups of four, 2 x 512,
+  //    15.0 / 15.1 and 22.1 / 24.0; two picks, 25.2 / 25.9 and 44.3 / 44.4, 17.3 / 19.2 and 28.3 / 28.9), one pick also unless
+  //    the last piece would be all but empty (4608 wide, nine KiB, 23.3 / 22.4).
+  // Picks of one go, against eight places of 1 KiB: top-3 (two picks and then one), 8192 tokens, 2048 wide 57.0 / 52.4, 4096
+  // wide 99.5 / 90.4; top-5 (four and one), 16000 tokens, 512 wide 43.4 / 41.6, 4096 tokens, 7168 wide 124.6 / 122.5.
+  // Top-6 and top-7 in one go measure the same as four picks and the rest (145.0 / 145.9, 165.3 / 165.0).
   switch (w.K) {
     case 1:
       if (nvec_segments == 1) PPLX_COMBINE(1, 1);
       if (nvec_segments == 2) PPLX_COMBINE(1, 2);
       if (nvec_segments == 4) PPLX_COMBINE(1, 4);
       if (grouped && nvec_segments > 4 && 8 * ((8 - nvec_segments % 8) % 8) <= 5 * nvec_segments) PPLX_COMBINE(1, 8);
+      if (!grouped && sizeof(T) == 2 && even_pieces(tokens, nvec_segments, 8, 2)) PPLX_COMBINE(1, 8);
       PPLX_COMBINE(1, 3);
     case 2:
       if (nvec_segments == 1) PPLX_COMBINE(2, 1);
-      if (grouped && nvec_segments > 2 && (nvec_segments + 1) % 4 <= 1) PPLX_COMBINE(2, 4);
+      if (grouped && nvec_segments > 2) PPLX_COMBINE(2, 4);
+      if (!grouped && sizeof(T) == 4 && even_pieces(tokens, nvec_segments, 4, 4)) PPLX_COMBINE(2, 4);
       PPLX_COMBINE(2, 2);
     case 3: PPLX_COMBINE(3, 1);
     case 4:

@@ -387,3 +387,31 @@ def test_pieces_of_few_picks(K, H, dp, y_dtype, out_dtype):
     check_combine_against_oracle(step, expected.slot_map)
     assert world.faults() == 0
     world.destroy()
+
+
+@pytest.mark.parametrize(
+    "K,H,M,y_dtype,dp",
+    [
+        (1, 3584, 256, torch.bfloat16, 1),  # 8 KiB pieces, two workgroups to a CU
+        (1, 3208, 250, torch.float16, 1),  # ... a few less, the last of seven KiB a single vector
+        (1, 7680, 256, torch.bfloat16, 1),  # ... four workgroups, two pieces to a row
+        (2, 1544, 512, torch.float32, 1),  # 4 KiB pieces, four workgroups
+        (2, 2560, 300, torch.bfloat16, 2),  # five KiB of a DP group's rows
+        (2, 1032, 300, torch.float16, 4),  # a single vector in the third
+    ],
+)
+def test_long_pieces_of_few_picks(K, H, M, y_dtype, dp):
+    spec = WorkloadSpec(
+        "long-pieces", 79, 8, 16, K, H, M, torch.bfloat16, expert_y_dtype=y_dtype, dp_size=dp, tokens="uniform"
+    )  # fmt: skip
+    groups = generate(spec, seed=H + K)
+    groups[0].n, groups[-1].n = M, 1
+    step = DeviceStep(spec, groups)
+    world = make_world(spec, group_name="long-pieces")
+    step.dispatch_world(world)
+    expected = check_dispatch_against_oracle(step)
+    step.expert_y_all.normal_(generator=torch.Generator(device="cuda").manual_seed(8))
+    step.combine_world(world)
+    check_combine_against_oracle(step, expected.slot_map)
+    assert world.faults() == 0
+    world.destroy()

@@ -100,10 +100,10 @@ def test_members_of_a_dp_group_share_or_keep_their_own_sums(dp, K, E, H, M, y_dt
 @pytest.mark.parametrize(
     "E,K,M,R,hidden_bytes",
     [
-        # (rows of 8208 bytes have no variant in the one-launch form)
-        (16, 1, 401, 8, 8208),  # 51 tiles of one chunk, 64 lanes to a pick, the last tile nearly empty
+        # (the rows of a workgroup of the one-launch form would not fit LDS)
+        (16, 1, 401, 8, 16368),  # 51 tiles of one chunk, 64 lanes to a pick, the last tile nearly empty
         (64, 33, 129, 8, 8208),  # 17 tiles, one lane to a pick
-        (40, 5, 512, 8, 8208),  # exactly 64 tiles; lanes left over (8 to a pick, 5 picks)
+        (40, 5, 512, 8, 16368),  # exactly 64 tiles; lanes left over (8 to a pick, 5 picks)
         (8, 3, 513, 8, 48),  # 65 chunks: 33 tiles of two
         (24, 10, 4099, 8, 16),  # 513 chunks: 33 tiles of sixteen
         (1024, 2, 2050, 8, 16),  # LDS limits tiles to four chunks: 65 tiles, scanned
@@ -112,7 +112,8 @@ def test_members_of_a_dp_group_share_or_keep_their_own_sums(dp, K, E, H, M, y_dt
 )
 def test_slots_from_the_routing_tables(E, K, M, R, hidden_bytes):
     spec = WorkloadSpec("tables", 72, R, E, K, hidden_bytes // 2, M, torch.bfloat16, tokens="uniform")
-    assert M * R > 4096 or hidden_bytes == 8208
+    form = ops.plan_of(ops.Config(M, E, K, R, 1, spec.hidden_dim, hidden_bytes, 0)).dispatch_form
+    assert form == (SCANNED_TABLES if E == 1024 else TABLES)
     groups = generate(spec, seed=E + K)
     groups[0].n, groups[1].n, groups[-1].n = 0, M, M  # an empty rank; a full last tile
     load = np.bincount(
@@ -281,9 +282,11 @@ def test_rows_through_lds(E, K, M, R, row_bytes, form, strided):
     )
     if K * M * R > 20000:
         spec = dataclasses.replace(spec, tokens="uniform")
-    assert form == ops.plan_of(
+    plan, in_lds = ops.plan_on(
         ops.Config(M, E, K, R, 1, spec.hidden_dim, spec.hidden_dim_bytes, spec.hidden_dim_scale_bytes)
-    ).dispatch_form  # fmt: skip
+    )
+    assert plan.dispatch_form == form
+    assert in_lds == (row_bytes not in (16, 10240))  # (those stay in registers)
     groups = generate(spec, seed=E + K + row_bytes)
     groups[R // 2].n = min(1, groups[R // 2].n)
     ids = np.concatenate([g.indices[: g.n].reshape(-1).numpy() for g in groups])
@@ -325,6 +328,57 @@ def test_rows_through_lds(E, K, M, R, row_bytes, form, strided):
     step.expert_x_all.view(torch.uint8).view(rows, row_bytes).copy_(copies[:, :row_bytes])
     check_dispatch_against_oracle(step)
     assert (copies[:, row_bytes:] == 0xA5).all() and (guard[:16] == 0xA5).all()
+
+
+@pytest.mark.parametrize(
+    "E,K,M,dp,row_bytes,faults",
+    [
+        (16, 4, 21, 2, 8208, False),
+        (16, 4, 21, 4, 9344, True),  # whole lines without a register variant; a group's rows from four ranks
+        (64, 8, 128, 2, 5136, True),  # 20 MiB of rows that a register variant would fit; two waves to a token
+        (64, 7, 200, 1, 12304, True),  # seven tokens to a workgroup, picks that the shares of a token do not divide
+    ],
+)
+def test_one_launch_rows_in_lds_of_groups_and_of_faults(E, K, M, dp, row_bytes, faults):
+    """Rows in LDS of the one-launch form: eager, dropped rows and bad and repeated picks among them, and replayed from a
+    graph."""
+    spec = WorkloadSpec("lds-one", 80, 8, E, K, row_bytes // 2, M, torch.bfloat16, dp_size=dp, tokens="uniform")
+    plan, in_lds = ops.plan_on(ops.Config(M, E, K, 8, dp, spec.hidden_dim, row_bytes, 0))
+    assert plan.dispatch_form == ONE_LAUNCH and in_lds
+    groups = generate(spec, seed=row_bytes)
+    groups[0].n = M
+    if faults:
+        groups[0].indices[3, 1] = E + 9
+        groups[0].indices[M - 1, K - 1] = groups[0].indices[M - 1, 0]
+    ids = np.concatenate([g.indices[: g.n].reshape(-1).numpy() for g in groups])
+    load = int(np.bincount(ids[ids < E], minlength=E).max())
+    step = DeviceStep(spec, groups, cap=load - 2 if faults else load, alloc_expert_y=False)
+    world = make_world(spec, group_name="lds-one")
+
+    def check():
+        if faults:
+            _check_with_repeats_dropped(step, after_combine=False)
+            assert world.faults() == FAULT_ROW_DROPPED | FAULT_BAD_EXPERT | FAULT_DUPLICATE
+        else:
+            check_dispatch_against_oracle(step)
+            assert world.faults() == 0
+
+    step.dispatch_world(world)
+    check()
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        with world.capture() as cap:
+            step.dispatch_world(world)
+        for _ in range(3):
+            step.expert_x_all.zero_()
+            step.expert_num_tokens_all.zero_()
+            stream.synchronize()
+            cap.graph.replay(stream)
+            stream.synchronize()
+            check()
+        cap.graph.destroy()
+    world.destroy()
 
 
 @pytest.mark.parametrize("K", [8, 9, 10, 12, 16, 17, 24, 33, 64])

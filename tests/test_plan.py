@@ -93,6 +93,25 @@ def test_scatter(tokens, row, scales, topk, waves, in_turn):
         (2736, 8192, 64, 8, False),  # 176.3
         (3072, 7168, 0, 8, True),  # 168
         (3080, 7168, 0, 8, False),
+        # more than sixteen picks, and more than eight that can only be fetched one by one
+        (1024, 2048, 0, 17, True),
+        (1032, 2048, 0, 17, False),
+        (4096, 1024, 0, 16, True),
+        (1024, 2048, 0, 9, True),
+        (1032, 2048, 0, 9, False),
+        (1032, 4096, 0, 9, True),
+        (2048, 4096, 0, 9, True),
+        (2056, 4096, 0, 9, False),
+        (4096, 1024, 0, 10, True),
+        # rows in LDS: 180 MiB where they share lines, 128 MiB and 2048 tokens where they do not
+        (2880, 8176, 0, 8, True),  # 179.6
+        (2888, 8176, 0, 8, False),  # 180.1
+        (1816, 9216, 0, 8, True),  # 127.7
+        (1824, 9216, 0, 8, False),  # 128.3
+        (2048, 9216, 0, 1, True),
+        (2056, 9216, 0, 1, False),
+        (16, 16368, 0, 2, True),  # the longest that share lines
+        (16, 16400, 0, 2, False),
     ],
 )
 def test_one_launch(tokens, row, scales, topk, one_launch):
@@ -138,6 +157,26 @@ def test_combine_per_group(ranks, dp, max_tokens, topk, hidden, dtype, per_group
 def test_rows_in_lds_need_a_device_that_holds_them(lds, tokens, row, topk, one_launch):
     p, _ = ops.plan_on(ops.Config(tokens // 8, 64, topk, 8, 1, row // 2, row, 0), lds)
     assert (p.dispatch_form == ONE_LAUNCH) == one_launch
+
+
+@pytest.mark.parametrize(
+    "tokens,row,topk,in_lds",
+    [
+        (8, 8208, 1, True),  # no register variant
+        (8, 9216, 1, True),
+        (8, 10240, 1, False),
+        (672, 3088, 8, False),  # 15.8 MiB of rows that share lines
+        (680, 3088, 8, True),  # 16.02
+        (2744, 3056, 8, False),  # 63.98 MiB of shorter ones
+        (2752, 3056, 8, True),  # 64.2
+        (4096, 2032, 14, False),  # shorter still
+        (2752, 3072, 8, False),  # whole lines
+    ],
+)
+def test_rows_of_one_launch_in_lds(tokens, row, topk, in_lds):
+    p, rows_in_lds = ops.plan_on(ops.Config(tokens // 8, 64, topk, 8, 1, row // 2, row, 0))
+    assert p.dispatch_form == ONE_LAUNCH
+    assert rows_in_lds == in_lds
 
 
 @pytest.mark.parametrize("row,waves", [(26864, 6), (26896, 5), (32752, 4)])

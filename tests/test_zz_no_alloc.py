@@ -143,6 +143,9 @@ def test_static_step_matches_the_world_path_on_calls_in_a_row():
     _compare(tiled, groups, fault_word, cap=max(int(expert_counts(groups, tiled.num_experts).max()), 1))
     # 5. and a small one once more
     _compare(small, generate(small, seed=9), fault_word)
+    # 6. one launch with its rows in LDS
+    lds = _spec(name="d", hidden_dim=4104, max_num_tokens=24, in_dtype=torch.bfloat16)
+    _compare(lds, generate(lds), fault_word)
 
 
 def test_static_step_reports_faults_and_refuses_what_does_not_fit():

@@ -296,8 +296,8 @@ int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
       PPLX_COMBINE(3, 2);
     }
   }
-  // Of what is left, up to five picks are taken all at once.  One or two leave a wave of 1 KiB with little in flight, so they read longer
-  // pieces: up to 3 KiB of one pick and 2 KiB of two, which is ahead of 8 and of 4 KiB nearly everywhere (dispatch +
+  // Of what is left, up to five picks are taken all at once.  One or two leave a wave of 1 KiB with little in flight, so
+  // they read longer pieces: up to 3 KiB of one pick and 2 KiB of two, which is ahead of 8 and of 4 KiB nearly everywhere (dispatch +
   // combine, 8 ranks, us, long / short pieces: one pick of 16-bit rows, 512 tokens, 2048 wide 8.3 / 7.8, 4096 wide 9.2 /
   // 8.8, 8192 wide 12.0 / 11.4; 8192 tokens, 52.3 / 51.0 and 105.9 / 103.6; two picks, 512 tokens, 8.7 / 8.3, 10.0 /
   // 10.0 and 14.1 / 13.9; 8192 tokens, 71.6 / 70.5 and 151.8 / 150.2; not one pick, 1024 tokens, 2560 wide 9.2 / 9.6, 3072

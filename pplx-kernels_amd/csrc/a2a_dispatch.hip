@@ -18,6 +18,8 @@
 //                    own (single tile, rows beyond the register variants)
 //   dispatch_fused   small steps: routing and scatter in one launch; every
 //                    workgroup recounts the picks of the tokens before its own
+//                    (rows that share 128-byte lines go through LDS instead of registers in
+//                    both, and so do those that no register variant of dispatch_fused fits)
 //   combine_gather   one wave per 1 KiB of an output row: K rows gathered through
 //                    the slot map, fp32 accumulate in pick order, 16 B stores
 //
@@ -140,7 +142,7 @@ __device__ __forceinline__ void scatter_token(const WorldDev &w, const DT &tab, 
 }
 
 // Launched as one-wave workgroups whose dynamic LDS size caps how many of them a CU holds at a
-// time (see launch_scatter_t); only the variants for rows that share lines (NV = 0) use it, for the row.
+// time (scatter_lds); only the variants for rows that go through LDS (NV = 0) use it, for the row.
 template <int NV, bool EXACT, class DT>
 __global__ __launch_bounds__(kWave) void dispatch_scatter(WorldDev w, DT tab, uint32_t ksplit, uint32_t kper) {
   scatter_token<NV, EXACT, DT, Slots::kMap, false>(w, tab, blockIdx.x, ksplit, kper);
@@ -328,7 +330,7 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   }
   uint32_t *hist = reinterpret_cast<uint32_t *>(lds_u64 + table_words);  // [E] tokens before the workgroup's own
   uint32_t *own_mask = hist + w.E;                                       // [E] bit j: own token j goes to e
-  // NV = 0: the workgroup's rows (those that share lines), one behind the other
+  // NV = 0: the workgroup's rows, one behind the other
   u32x4 *own_rows = reinterpret_cast<u32x4 *>(lds_u64 + ((table_words + w.E + 1) & ~1u));
   for (uint32_t e = threadIdx.x; e < 2 * w.E; e += kFusedThreads) hist[e] = 0;
   // Orders the zeroing (and the staged table) before the first counter update of any wave.
@@ -531,16 +533,24 @@ uint32_t fused_tokens_per_block(uint32_t tokens, uint32_t waves) {
   const uint32_t n = (tokens + 255) / 256;
   return n > waves ? waves : n < 1 ? 1 : n;
 }
-// Whether dispatch_fused keeps its rows in LDS: those that no register variant fits, and those that share
-// lines once a step and each of its tokens store enough for that to matter (the way through LDS costs 0.3-0.8 us
-// in front of the first store, and the reads from it are repeated for every copy).  Dispatch + combine, us, on
-// three buffer sets in turn, which the last-level cache holds while a set is small / on sixteen, in registers and
-// in LDS at the MiB of rows stored: 3088-byte rows, top-8 7 10.5 10.5 / 11.4 11.6, 23 15.8 16.1 / 21.9 20.2, 47 26.0 26.6 / 37.0
-// 32.6, 95 56.1 47.5 / 64.9 47.7; 5264 bytes, top-8 15 13.3 13.3 / 16.5 16.1, 47 25.9 26.0 / 37.8 31.8, 95 56.6 47.5 / 64.9 47.4, 127
-// 80.0 63.1 / 79.6 62.4; 8176 bytes, top-6 31 21.0 20.6 / 28.4 24.2, 63 36.8 33.7 / 48.4 38.6, 169 99.7 82.0 / 99.9 81.3.  Shorter rows
-// lose what they gain: 1552 bytes, top-8 31 20.6 21.8 (three sets); 2064 bytes, top-8 31 20.2 20.9, 63 36.2 36.4.
-// Rows without a register variant took two launches; dispatch, two launches / one: 12016 bytes, top-8 0.7 8.8 / 6.4, 46
-// 27.6 / 13.5, 93 41.5 / 23.6; 13312 bytes, top-5 32 23.8 / 10.8; 9216 bytes, top-4 18 12.8 / 7.7.
+// Whether dispatch_fused keeps its rows in LDS: those that no register variant fits, and those that share lines once a
+// step stores enough for whole lines to matter (the way through LDS costs 0.3-0.8 us in front of the first store, and
+// every copy reads the row from there again).  How much that is depends on where a step's buffers are: the lines lie
+// where little is lost while the last-level cache still holds them, although cold buffers gain from far smaller steps
+// on.  Dispatch + combine, top-8, us, registers / LDS as stored here, at the MiB of rows stored, on three buffer sets in
+// turn and on sixteen, nothing of which is cached:
+//                  three sets                                          sixteen sets
+//                  24          40          56          66          80          24          40          56          66
+//   2064 bytes *   16.9 17.2   24.2 25.2   31.2 31.8                           23.3 21.8   34.0 31.6   43.8 39.9
+//   2576 bytes *   16.4 16.7   23.0 23.6   30.0 30.7   34.8 35.1   42.3 40.5   23.1 21.0   32.5 29.7   42.9 37.8   48.8 42.7
+//   3088 bytes     15.9 16.2   22.4 23.1   29.6 30.6   35.0 35.1   42.4 40.4   21.9 20.3   32.4 29.1   42.5 37.1   48.1 41.5
+//   3600 bytes     16.0 16.2   22.5 22.9   29.7 29.5   34.1 34.0   42.8 40.5   22.5 20.7   32.4 28.5   41.5 35.9
+//   4240 bytes     16.0 16.2   22.8 22.9   29.4 29.8   34.4 33.8   45.3 41.8   22.5 20.2   32.4 28.0   42.6 36.1   48.2 40.5
+//   5264 bytes     16.1 16.3   22.2 22.5   29.6 29.3   33.5 33.2   44.3 41.4   22.7 20.5   31.6 27.0   42.9 35.6   48.5 39.8
+//   8176 bytes     15.6 15.7   23.3 23.5   27.0 27.2   37.0 35.8   48.1 40.4   22.4 20.3   32.8 27.9   40.0 32.8   49.8 41.0
+// (* below 64 MiB these two stay in registers.)  Rows without a register variant took two launches; dispatch, two
+// launches / one: 12016 bytes, top-8 0.7 MiB 8.8 / 6.4, 46 27.6 / 13.5, 93 41.5 / 23.6; 13312 bytes, top-5 32 23.8 / 10.8;
+// 9216 bytes, top-4 18 12.8 / 7.7.
 bool fused_rows_in_lds(const WorldDev &w) {
   if (!row_has_register_variant(w)) return true;
   if (!row_shares_lines(w)) return false;
@@ -592,7 +602,7 @@ bool scatter_rows_in_lds(const WorldDev &w) {
 // few waves keep the stores in longer runs, and large steps do best with three whose stores start
 // later.  Dispatch on 8 ranks, us, all forms alternating in one process on the same buffers (whose
 // place in memory moves all of them by up to 15 % from one process to the next); side by side at 4 and
-// 10 waves (nine, in fact: see kLdsBlock; the two are within 0.8 %) / one behind the other at 3:
+// 9 waves / one behind the other at 3:
 //   59 KiB stored per wave (DSv3 fp8 rows, top-8 of 256)
 //     8 x 509    52.7 /  -  / 53.0     8 x 1024  97.8 /  -  / 98.4    8 x 2048  184 / 189 / 185
 //     8 x 4096    432 / 431 / 430      8 x 6000   645 / 626 / 610     8 x 8192  859 / 843 / 826
@@ -612,6 +622,8 @@ bool scatter_rows_in_lds(const WorldDev &w) {
 //   14 KiB (DSv3 fp8 rows, top-2)                      382 /  373 /  377 /  378 /  378 /  379 /  379
 //    8 KiB (1 KiB fp8 rows with scales, top-8)         226 /  202 /  179 /  169 /  159 /  159 /  160
 //    4 KiB (2 KiB fp8 rows with scales, top-2)         162 /  143 /  125 /  118 /  112 /  110 /  109
+// (8 / 9 / 10 / 12: 8 x 4096 tokens, 16 KiB 106.7 / 107.2 / 107.6 / 108.6, 24 KiB 212.5 / 213.5 / 213.5 / 215.2; 8 x 1024,
+// 13 KiB, step 67.9 at nine, 68.3 at ten)
 // (one behind the other they lose: 8 x 4096 tokens of 8 KiB, top-2, skewed: 123 and 130; 2 KiB rows,
 // top-6, 8 x 1024: 26.2 and 27.5).
 // Rows in LDS (a2a_rows.h) spend more time in front of and between their stores and want more waves.  Us at 6 / 8 / 12 /
@@ -651,9 +663,9 @@ ScatterPlan scatter_plan(const WorldDev &w, uint32_t picks_per_wave) {
   if (stored >= 24 * 1024) {
     if (tokens <= 16384) return {4, false};
     if (stored >= 48 * 1024 || (stored >= 32 * 1024 && (row >= 8192 || tokens <= 32768))) return {3, true};
-    return {stored >= 32 * 1024 || tokens <= 32768 ? 4u : 10u, false};
+    return {stored >= 32 * 1024 || tokens <= 32768 ? 4u : 9u, false};
   }
-  if (stored >= 12 * 1024) return {row >= 4096 ? 4u : 10u, false};
+  if (stored >= 12 * 1024) return {row >= 4096 ? 4u : 9u, false};
   return {stored >= 6 * 1024 ? 12u : 0u, false};
 }
 
@@ -820,10 +832,10 @@ bool dispatch_is_fused(const WorldDev &w) {
   //     42.8, 192 45.2 / 45.8; 7 KiB: 126 30.8 / 33.4, 140 33.9 / 35.8, 154 36.5 / 38.7; the same with half of
   //     the tokens absent (8 KiB, 144: 21.3 / 23.2), and for 8 KiB rows with scales (148 35.5 / 37.9,
   //     182 42.8 / 44.2): these run up to 176
-  // Picks that are not counted four at a time, or more than eight, run up to 112 (120 in steps of up to 1024 tokens),
-  // where the forms come level: 8 KiB rows, top-5 80 21.3 / 23.4, 160 39.8 / 38.3; top-9 144 35.5 / 36.2; top-10 160 38.4 / 38.7;
-  // top-12 192 45.1 / 44.9.  (Up to 1024 tokens the slots take a launch of a single workgroup, and one launch is ahead
-  // beyond that as well: top-16 128 31.1 / 43.6; not taken up.)
+  // Picks that are not counted four at a time, or more than eight, run up to 112 (120 in steps of up to 1024 tokens).
+  // That is safe for all of them, and short of where the forms come level for most: 8 KiB rows, top-5 80 21.3 / 23.4,
+  // 160 39.8 / 38.3; top-9 144 35.5 / 36.2; top-10 160 38.4 / 38.7; top-12 192 45.1 / 44.9; up to 1024 tokens the slots
+  // take a launch of a single workgroup, and one launch is ahead beyond 120 too (top-16 128 31.1 / 43.6).
   const uint64_t tokens = (uint64_t)w.G * w.M;
   const uint32_t waves = fused_waves(w);
   const uint64_t stored = tokens * w.K * (w.Hb + 4ull * w.S);
@@ -835,9 +847,17 @@ bool dispatch_is_fused(const WorldDev &w) {
   // 2048 19.3 / 21.5.)
   if (tokens > 1024 && w.K > 16) return false;
   if (tokens > 1024 && w.K > 8 && w.K % 2 != 0 && (w.Hb < 4096 || tokens > 2048)) return false;
-  // Rows in LDS (dispatch + combine, us, one launch / two): 8176 bytes, top-6 127 62.4 / 66.0, 169 82.0 / 83.8; 12016 bytes,
-  // top-8 127 59.8 / 65.2, 169 76.9 / 83.4; 15984 bytes, top-4 127 66.1 / 69.3; whole lines without a register variant
-  // 9216 bytes, top-4 95 50.6 / 52.0 and 127 63.5 / 63.3, 13312 bytes, top-5 127 61.7 / 61.9 and 169 82.0 / 81.0.
+  // Rows in LDS, dispatch + combine on three buffer sets, us, one launch / two:
+  //   sharing lines, MiB of rows   150           169           180           192           205
+  //     5264 bytes, top-10         71.5 / 72.6   81.6 / 83.7                 88.4 / 88.7   94.7 / 94.5
+  //     6160 bytes, top-8          71.1 / 75.6   80.2 / 82.8   83.3 / 84.8   88.6 / 89.8
+  //     8176 bytes, top-6          74.2 / 78.0   80.3 / 83.0   85.0 / 86.2   90.3 / 90.7
+  //     12016 bytes, top-8         70.6 / 79.4   75.5 / 82.1   81.4 / 85.9   89.1 / 92.6
+  //     4240 bytes, top-12         69.0 / 70.8   78.1 / 81.6   83.2 / 84.8   88.3 / 87.9
+  //   whole lines: 13312 bytes, top-5 102 52.6 / 53.6, 130 62.6 / 63.0, 169 82.0 / 81.0; 9216 bytes, top-4 72 38.0 / 40.4, 99
+  //     51.0 / 51.6, 117 59.2 / 59.1; 11264 bytes, top-8 129 59.5 / 62.3, 146 68.6 / 70.0.  Their limit of 2048 tokens is
+  //     that of 512-thread workgroups and on the safe side: 9216 bytes, 2304 tokens, top-1 20.3 / 23.4, 4096 32.8 / 34.2;
+  //     13312 bytes, top-3 2816 57.1 / 57.6, 3072 61.0 / 60.6.
   if (in_lds) {
     const uint64_t rows = (uint64_t)fused_tokens_per_block((uint32_t)tokens, waves) * w.Hb;
     const uint64_t limit = row_shares_lines(w) ? 180ull << 20 : 128ull << 20;

@@ -1,4 +1,5 @@
-// Row fan-out in registers, shared by the dispatch kernels, and the macro that picks the register variant for a row size.
+// Row fan-out in registers and through LDS, shared by the dispatch kernels, and the macro that picks the register variant
+// for a row size.
 #pragma once
 #include "a2a_common.h"
 
@@ -131,9 +132,9 @@ __device__ __forceinline__ void store_row(const WorldDev &w, const DispatchRank 
 }
 
 // ---------------------------------------------------------------------------
-// Rows whose length is no multiple of a 128-byte line.  Every copy of such a row begins somewhere else
+// Rows through LDS.  They are for rows whose length is no multiple of a 128-byte line.  Every copy of such a row begins somewhere else
 // inside a line, so a wave that stores 64 vectors from the row's start at a time cuts a line in two at each
-// of its stores, and the halves reach the memory as two partial writes.  The row is therefore kept in
+// of its stores, and the halves reach the memory as two partial writes.  Such a row is kept in
 // LDS instead of registers (fetched with loads that write LDS directly), and for every pick the lanes
 // take it from there shifted by the copy's offset in its line: all stores but the ends of the row
 // cover whole lines.  The lines that two rows share are written through into the last-level cache
@@ -145,7 +146,9 @@ __device__ __forceinline__ void store_row(const WorldDev &w, const DispatchRank 
 //   3296-byte rows, top-3 of 16, 25979             79 / 65 / 62 / 59
 //   2528-byte rows, top-1 of 64, 2 x 16358         43 / 38 / 39 / 39
 // (whole lines, half a KiB left over: 4608-byte rows with scales, 8 x 2048 tokens 120 in registers, 124
-// through LDS; 5760-byte rows, top-5, 8 x 3001 71 / 73; 512-byte rows 61 / 89: these stay in registers.)
+// through LDS; 5760-byte rows, top-5, 8 x 3001 71 / 73; 512-byte rows 61 / 89: these stay in registers.)  Which rows
+// and steps take it: scatter_rows_in_lds, and fused_rows_in_lds for the one-launch dispatch, which also holds rows of
+// whole lines there that no register variant fits.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kLineBytes = 128;
 inline bool row_shares_lines(const WorldDev &w) { return w.Hb % kLineBytes != 0; }

@@ -38,10 +38,10 @@ def plan(tokens, row, topk, experts=64, scales=0, ranks=8, dp=1):
         # from 24 KiB on
         (16392, 4096, 0, 6, 4, False),
         (32768, 8192, 0, 3, 4, False),
-        (32776, 8192, 0, 3, 10, False),
+        (32776, 8192, 0, 3, 9, False),
         # less
         (32768, 8192, 0, 2, 4, False),
-        (32768, 2048, 16, 8, 10, False),
+        (32768, 2048, 16, 8, 9, False),
         (32768, 1024, 8, 8, 12, False),
         (32768, 2048, 16, 2, 0, False),
         # rows that share lines, through LDS: from 32 KiB on six waves, or eight beyond 32768 tokens; ...

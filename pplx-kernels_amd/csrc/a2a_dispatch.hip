@@ -18,7 +18,7 @@
 //                    own (single tile, rows beyond the register variants)
 //   dispatch_fused   small steps: routing and scatter in one launch; every
 //                    workgroup recounts the picks of the tokens before its own
-//                    (rows that share 128-byte lines go through LDS instead of registers in
+//                    (rows that cut 64-byte half lines go through LDS instead of registers in
 //                    both, and so do those that no register variant of dispatch_fused fits)
 //   combine_gather   one wave per 1 KiB of an output row: K rows gathered through
 //                    the slot map, fp32 accumulate in pick order, 16 B stores
@@ -533,7 +533,7 @@ uint32_t fused_tokens_per_block(uint32_t tokens, uint32_t waves) {
   const uint32_t n = (tokens + 255) / 256;
   return n > waves ? waves : n < 1 ? 1 : n;
 }
-// Whether dispatch_fused keeps its rows in LDS: those that no register variant fits, and those that share lines once a
+// Whether dispatch_fused keeps its rows in LDS: those that no register variant fits, and those that cut half lines once a
 // step stores enough for whole lines to matter (the way through LDS costs 0.3-0.8 us in front of the first store, and
 // every copy reads the row from there again).  How much that is depends on where a step's buffers are: the lines lie
 // where little is lost while the last-level cache still holds them, although cold buffers gain from far smaller steps
@@ -553,7 +553,7 @@ uint32_t fused_tokens_per_block(uint32_t tokens, uint32_t waves) {
 // 9216 bytes, top-4 18 12.8 / 7.7.
 bool fused_rows_in_lds(const WorldDev &w) {
   if (!row_has_register_variant(w)) return true;
-  if (!row_shares_lines(w)) return false;
+  if (!row_cuts_half_lines(w)) return false;
   const uint64_t stored = (uint64_t)w.G * w.M * w.K * (w.Hb + 4ull * w.S);
   return w.Hb >= 3072 ? stored > 16ull << 20 : w.Hb >= 2048 && stored > 64ull << 20;
 }
@@ -576,7 +576,7 @@ uint32_t pick_ksplit(const WorldDev &w, uint32_t max_split) {
   return ksplit;
 }
 
-// Whether the scatter takes rows that share lines through LDS.  A row costs a trip to LDS in front of its
+// Whether the scatter takes rows that cut half lines through LDS.  A row costs a trip to LDS in front of its
 // first store and another read of it per copy there, which short rows of small steps, bound by the chain of a wave and
 // not by the memory, do not get back.  Dispatch on three buffer sets, experts 64, LDS : registers at 4200, 8000 and
 // 20000 tokens
@@ -590,7 +590,7 @@ uint32_t pick_ksplit(const WorldDev &w, uint32_t max_split) {
 // less lose (16 bytes 1.03 - 1.44, 48 bytes 1.0 - 1.26, 64 bytes, which cut no line, 1.20 - 1.44, 96 bytes 1.0 - 1.12)
 // except for some steps of 64 picks (80 and 96 bytes 0.85 - 0.91).
 bool scatter_rows_in_lds(const WorldDev &w) {
-  if (!row_shares_lines(w) || w.Hb < 112) return false;
+  if (!row_cuts_half_lines(w) || w.Hb < 112) return false;
   const uint64_t read = (uint64_t)w.G * w.M * w.Hb;
   return w.Hb >= 1024 || read >= 2u << 20 || read * w.K >= 24u << 20;
 }
@@ -848,22 +848,21 @@ bool dispatch_is_fused(const WorldDev &w) {
   if (tokens > 1024 && w.K > 16) return false;
   if (tokens > 1024 && w.K > 8 && w.K % 2 != 0 && (w.Hb < 4096 || tokens > 2048)) return false;
   // Rows in LDS, dispatch + combine on three buffer sets, us, one launch / two:
-  //   sharing lines, MiB of rows   150           169           180           192           205
+  //   cutting half lines, MiB     150           169           180           192           205
   //     5264 bytes, top-10         71.5 / 72.6   81.6 / 83.7                 88.4 / 88.7   94.7 / 94.5
   //     6160 bytes, top-8          71.1 / 75.6   80.2 / 82.8   83.3 / 84.8   88.6 / 89.8
   //     8176 bytes, top-6          74.2 / 78.0   80.3 / 83.0   85.0 / 86.2   90.3 / 90.7
   //     12016 bytes, top-8         70.6 / 79.4   75.5 / 82.1   81.4 / 85.9   89.1 / 92.6
   //     4240 bytes, top-12         69.0 / 70.8   78.1 / 81.6   83.2 / 84.8   88.3 / 87.9
-  //   whole lines: 13312 bytes, top-5 102 52.6 / 53.6, 130 62.6 / 63.0, 169 82.0 / 81.0; 9216 bytes, top-4 72 38.0 / 40.4, 99
-  //     51.0 / 51.6, 117 59.2 / 59.1; 11264 bytes, top-8 129 59.5 / 62.3, 146 68.6 / 70.0.  Their limit of 2048 tokens is
-  //     that of 512-thread workgroups and on the safe side: 9216 bytes, 2304 tokens, top-1 20.3 / 23.4, 4096 32.8 / 34.2;
-  //     13312 bytes, top-3 2816 57.1 / 57.6, 3072 61.0 / 60.6.
+  //   whole half lines: 13312 bytes, top-5 102 52.6 / 53.6, 130 62.6 / 63.0, 169 82.0 / 81.0, top-3 107 57.1 / 57.6, 117 61.0 /
+  //     60.6; 9216 bytes, top-4 72 38.0 / 40.4, 99 51.0 / 51.6, 117 59.2 / 59.1, top-1, 4096 tokens 32.8 / 34.2; 9280 bytes, top-4
+  //     85 44.6 / 45.8; 11264 bytes, top-8 129 59.5 / 62.3, 146 68.6 / 70.0; 10304 bytes, top-4 156 77.0 / 74.1
   if (in_lds) {
     const uint64_t rows = (uint64_t)fused_tokens_per_block((uint32_t)tokens, waves) * w.Hb;
-    const uint64_t limit = row_shares_lines(w) ? 180ull << 20 : 128ull << 20;
+    const uint64_t limit = row_cuts_half_lines(w) ? 180ull << 20 : 128ull << 20;
     // (a device that does not say how much LDS it has is taken to have the 64 KiB of any)
     const uint32_t lds = w.lds_per_cu ? w.lds_per_cu : 64u << 10;
-    return fused_lds_bytes(w, true) + rows <= lds && stored <= limit && (row_shares_lines(w) || tokens <= 2048);
+    return fused_lds_bytes(w, true) + rows <= lds && stored <= limit;
   }
   if (waves < 16) return true;
   const bool quick_count = w.K % 4 == 0 && w.K <= 8;

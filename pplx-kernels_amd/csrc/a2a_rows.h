@@ -132,26 +132,28 @@ __device__ __forceinline__ void store_row(const WorldDev &w, const DispatchRank 
 }
 
 // ---------------------------------------------------------------------------
-// Rows through LDS.  They are for rows whose length is no multiple of a 128-byte line.  Every copy of such a row begins somewhere else
-// inside a line, so a wave that stores 64 vectors from the row's start at a time cuts a line in two at each
-// of its stores, and the halves reach the memory as two partial writes.  Such a row is kept in
-// LDS instead of registers (fetched with loads that write LDS directly), and for every pick the lanes
-// take it from there shifted by the copy's offset in its line: all stores but the ends of the row
-// cover whole lines.  The lines that two rows share are written through into the last-level cache
-// ("sc1"), where their parts meet; the others stream.  Dispatch, us, registers streamed through ("sc1
-// nt") / registers non-temporal / LDS non-temporal / LDS with shared lines written through:
+// Rows through LDS.  They are for rows whose length is no multiple of half a 128-byte line, the unit in which memory
+// takes writes.  Every copy of such a row begins somewhere else inside a line, so a wave that stores 64 vectors from the
+// row's start at a time cuts a half line in two at each of its stores, and the parts reach the memory as partial
+// writes.  Such a row is kept in LDS instead of registers (fetched with loads that write LDS directly), and for every
+// pick the lanes take it from there shifted by the copy's offset in its line: all stores but the ends of the row cover
+// whole lines.  The lines that two rows share are written through into the last-level cache ("sc1"), where their parts
+// meet; the others stream.  Dispatch, us, registers streamed through ("sc1 nt") / registers non-temporal / LDS
+// non-temporal / LDS with shared lines written through:
 //   5264-byte rows, top-8 of 256, 8 x 2048 tokens  210 / 175 / 160 / 139
 //   2976-byte rows, top-8 of 16, 4 x 4903          125 / 116 / 105 / 92
 //   8656-byte rows, top-10 of 128, 2 x 1252        74 / 61 / 58 / 54
 //   3296-byte rows, top-3 of 16, 25979             79 / 65 / 62 / 59
 //   2528-byte rows, top-1 of 64, 2 x 16358         43 / 38 / 39 / 39
-// (whole lines, half a KiB left over: 4608-byte rows with scales, 8 x 2048 tokens 120 in registers, 124
-// through LDS; 5760-byte rows, top-5, 8 x 3001 71 / 73; 512-byte rows 61 / 89: these stay in registers.)  Which rows
-// and steps take it: scatter_rows_in_lds, and fused_rows_in_lds for the one-launch dispatch, which also holds rows of
-// whole lines there that no register variant fits.
+// Rows of whole half lines stay in registers.  Dispatch on three buffer sets, top-8, registers / LDS: 192 bytes, 8000 tokens
+// 11.4 / 14.4; 320 bytes, top-10, 20000 20.5 / 27.4; 1856 bytes, top-6, 42394 97 / 117; 3264 bytes, 4712 29.9 / 32.0; 8256
+// bytes, top-6, 9408 94 / 101; 14400 bytes, 3124 73.6 / 79.5; with half a KiB left over 4608 bytes with scales, 8 x 2048
+// 120 / 124; 5760 bytes, top-5, 8 x 3001 71 / 73; 512 bytes 61 / 89.  Which of the
+// others take it: scatter_rows_in_lds, and fused_rows_in_lds for the one-launch dispatch, which also holds rows of whole
+// half lines there that no register variant fits.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kLineBytes = 128;
-inline bool row_shares_lines(const WorldDev &w) { return w.Hb % kLineBytes != 0; }
+inline bool row_cuts_half_lines(const WorldDev &w) { return w.Hb % (kLineBytes / 2) != 0; }
 
 // Vectors first, first + step, ... (64 each) of row t go to the same place in `lds`, which the calling wave
 // may read once its loads have returned (row_staged).
@@ -216,7 +218,7 @@ namespace pplx_amd {
 namespace {
 // Rows of up to 8 KiB and rows of exactly 10, 12, 14 or 16 KiB (5120-, 6144-, 7168- and 8192-wide
 // bf16) have a register variant in every row kernel; other sizes beyond 8 KiB go through LDS (the one-launch
-// dispatch; the scatter too where they share lines), take the scatter's padded variants or the streaming kernels.
+// dispatch; the scatter too where they cut half lines), take the scatter's padded variants or the streaming kernels.
 inline bool row_has_register_variant(const WorldDev &w) {
   const uint32_t nvec = w.Hb / 16;
   const uint32_t per_lane = (nvec + kWave - 1) / kWave;

@@ -244,13 +244,13 @@ def test_pieces_of_fp32_rows(M, K, H, dp, out_dtype):
 
 
 # ---------------------------------------------------------------------------
-# Rows that share 128-byte lines, and rows without a register variant: through LDS
+# Rows that cut 64-byte half lines, and rows without a register variant: through LDS
 # ---------------------------------------------------------------------------
 @pytest.mark.parametrize(
     "E,K,M,R,row_bytes,form",
     [
         (16, 3, 2, 8, 8208, ONE_LAUNCH),  # no register variant, one vector more than a line
-        (16, 2, 3, 8, 16368, ONE_LAUNCH),  # the longest that shares lines
+        (16, 2, 3, 8, 16368, ONE_LAUNCH),  # the longest that cuts half lines
         (8, 1, 1, 8, 8304, ONE_LAUNCH),  # one vector less than a line
         (16, 4, 33, 8, 9344, ONE_LAUNCH),  # whole lines without a register variant
         (64, 16, 261, 8, 2064, ONE_LAUNCH),  # 65.8 MiB of short rows

@@ -44,7 +44,7 @@ def plan(tokens, row, topk, experts=64, scales=0, ranks=8, dp=1):
         (32768, 2048, 16, 8, 9, False),
         (32768, 1024, 8, 8, 12, False),
         (32768, 2048, 16, 2, 0, False),
-        # rows that share lines, through LDS: from 32 KiB on six waves, or eight beyond 32768 tokens; ...
+        # rows that cut half lines, through LDS: from 32 KiB on six waves, or eight beyond 32768 tokens; ...
         (16384, 8208, 0, 4, 6, False),
         (16392, 8208, 0, 4, 6, True),  # ... in turn from 8 KiB rows and 16384 tokens on
         (32776, 8208, 0, 4, 6, True),
@@ -103,14 +103,14 @@ def test_scatter(tokens, row, scales, topk, waves, in_turn):
         (2048, 4096, 0, 9, True),
         (2056, 4096, 0, 9, False),
         (4096, 1024, 0, 10, True),
-        # rows in LDS: 180 MiB where they share lines, 128 MiB and 2048 tokens where they do not
+        # rows in LDS: 180 MiB where they cut half lines, 128 MiB where they do not
         (2880, 8176, 0, 8, True),  # 179.6
         (2888, 8176, 0, 8, False),  # 180.1
         (1816, 9216, 0, 8, True),  # 127.7
         (1824, 9216, 0, 8, False),  # 128.3
-        (2048, 9216, 0, 1, True),
-        (2056, 9216, 0, 1, False),
-        (16, 16368, 0, 2, True),  # the longest that share lines
+        (1824, 9280, 0, 8, False),  # half a line over
+        (4096, 9216, 0, 1, True),
+        (16, 16368, 0, 2, True),  # the longest that cut half lines
         (16, 16400, 0, 2, False),
     ],
 )
@@ -165,12 +165,14 @@ def test_rows_in_lds_need_a_device_that_holds_them(lds, tokens, row, topk, one_l
         (8, 8208, 1, True),  # no register variant
         (8, 9216, 1, True),
         (8, 10240, 1, False),
-        (672, 3088, 8, False),  # 15.8 MiB of rows that share lines
+        (672, 3088, 8, False),  # 15.8 MiB of rows that cut half lines
         (680, 3088, 8, True),  # 16.02
         (2744, 3056, 8, False),  # 63.98 MiB of shorter ones
         (2752, 3056, 8, True),  # 64.2
         (4096, 2032, 14, False),  # shorter still
         (2752, 3072, 8, False),  # whole lines
+        (2752, 3136, 8, False),  # half a line over
+        (8, 8256, 1, True),  # ... and no register variant
     ],
 )
 def test_rows_of_one_launch_in_lds(tokens, row, topk, in_lds):
@@ -197,6 +199,8 @@ def test_long_rows_in_lds_leave_room_for_fewer_waves(row, waves):
         (4104, 112, 55, True),  # copies of 24 MiB together
         (4104, 112, 54, False),
         (4104, 512, 8, False),  # whole lines
+        (4104, 1088, 8, False),  # half a line over
+        (16384, 8256, 4, False),
         (4104, 1008, 1, True),
         (4104, 1040, 8, True),
         (1024, 8192 + 16, 32, True),  # rows from 1 KiB on

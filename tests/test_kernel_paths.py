@@ -406,6 +406,18 @@ def test_one_launch_with_many_picks(K, aligned):
     world.destroy()
 
 
+@pytest.mark.parametrize("row_bytes", [1024, 1040, 8208])
+def test_one_launch_with_many_picks_and_rank_tables_in_hbm(row_bytes):
+    spec = WorkloadSpec("many-ranks", 81, 72, 144, 10, row_bytes // 2, 8, torch.bfloat16, tokens="uniform")
+    assert ops.plan_of(ops.Config(8, 144, 10, 72, 1, row_bytes // 2, row_bytes, 0)).dispatch_form == ONE_LAUNCH
+    step = DeviceStep(spec, generate(spec, seed=row_bytes), alloc_expert_y=False)
+    world = make_world(spec, group_name="many-ranks")
+    step.dispatch_world(world)
+    check_dispatch_against_oracle(step)
+    assert world.faults() == 0
+    world.destroy()
+
+
 # ---------------------------------------------------------------------------
 # Combine of few picks: pieces that are no longer than the row
 # ---------------------------------------------------------------------------

@@ -10,14 +10,42 @@ namespace {
 // with k ascending and fp32 accumulation
 // (csrc/all_to_all/intranode_combine.cu:141-168).
 // ---------------------------------------------------------------------------
+// What a lane has of a piece of a row (64 x 8 elements): where it lies, how it is fetched and stored.  In 16-bit rows that
+// is one vector of 8 elements.  In fp32 rows it is two vectors of 4 elements that lie 1 KiB apart, so that every load of
+// the wave covers whole lines: with the 32 bytes of 8 elements in one lane each of the two loads touches all lines of 2 KiB
+// and takes half of each.  Combine alone on three buffer sets, us, 8 elements in one lane / two vectors apart: 7168 wide, top-8,
+// 8 x 128 tokens 46.0 / 41.5, 8 x 1024 381.8 / 347.4; 512 wide, top-8, 8 x 2048 56.7 / 47.8; 4096 wide, top-2, 8 x 2048
+// 118.1 / 110.0, top-1 72.5 / 66.1; 520 wide, top-6, 8 x 1024 25.7 / 21.4; 2880 wide, top-5, groups of four, 3001 tokens
+// 50.6 / 46.1 (242 MB: 4.8 -> 5.25 TB/s; the stores, 8 bytes a lane, still cover whole lines).
+template <typename U> struct OutVectors;
+template <> struct OutVectors<__bf16> {
+  typedef __bf16 by4 __attribute__((ext_vector_type(4)));
+  typedef bf16x8 by8;
+};
+template <> struct OutVectors<_Float16> {
+  typedef _Float16 by4 __attribute__((ext_vector_type(4)));
+  typedef f16x8 by8;
+};
+
 template <typename T> struct Row8;
 template <> struct Row8<float> {
   struct Raw {
     f32x4 a, b;
   };
-  static __device__ __forceinline__ Raw load(uint64_t row, uint32_t vec) {
-    const PPLX_GLOBAL f32x4 *p = global_cptr<f32x4>(row) + 2 * (size_t)vec;
-    return Raw{__builtin_nontemporal_load(p), __builtin_nontemporal_load(p + 1)};
+  struct Place {
+    uint32_t a, b;  // in vectors of 4 elements
+  };
+  static __device__ __forceinline__ Place place(uint32_t piece, uint32_t lane) {
+    return Place{2 * piece * kWave + lane, (2 * piece + 1) * kWave + lane};
+  }
+  // (beyond the row its last vector is fetched: loads stay unconditional)
+  static __device__ __forceinline__ Place clamped(Place p, uint32_t H) {
+    const uint32_t last = H / 4 - 1;
+    return Place{p.a < last ? p.a : last, p.b < last ? p.b : last};
+  }
+  static __device__ __forceinline__ Raw load(uint64_t row, Place p) {
+    const PPLX_GLOBAL f32x4 *x = global_cptr<f32x4>(row);
+    return Raw{__builtin_nontemporal_load(x + p.a), __builtin_nontemporal_load(x + p.b)};
   }
   static __device__ __forceinline__ f32x8 widen(const Raw &r) {
     return __builtin_shufflevector(r.a, r.b, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -26,12 +54,35 @@ template <> struct Row8<float> {
   template <int N> static __device__ __forceinline__ void settle(Raw *raw) {
     SettleAll<2 * N>::of(reinterpret_cast<f32x4 *>(raw));
   }
-};
-template <> struct Row8<__bf16> {
-  typedef u32x4 Raw;
-  static __device__ __forceinline__ Raw load(uint64_t row, uint32_t vec) {
-    return __builtin_nontemporal_load(global_cptr<u32x4>(row) + vec);
+  template <typename U>
+  static __device__ __forceinline__ void store(uint64_t row, Place p, uint32_t H, const f32x8 &acc) {
+    typedef typename OutVectors<U>::by4 vec_t;
+    PPLX_GLOBAL vec_t *out = global_ptr<vec_t>(row);
+    const f32x4 a = __builtin_shufflevector(acc, acc, 0, 1, 2, 3), b = __builtin_shufflevector(acc, acc, 4, 5, 6, 7);
+    if (p.a < H / 4) __builtin_nontemporal_store(__builtin_convertvector(a, vec_t), out + p.a);
+    if (p.b < H / 4) __builtin_nontemporal_store(__builtin_convertvector(b, vec_t), out + p.b);
   }
+};
+// The 16-bit types.
+template <typename V> struct Row8By16 {
+  typedef V Raw;
+  typedef uint32_t Place;  // in vectors of 8 elements
+  static __device__ __forceinline__ Place place(uint32_t piece, uint32_t lane) { return piece * kWave + lane; }
+  static __device__ __forceinline__ Place clamped(Place p, uint32_t H) {
+    const uint32_t last = H / 8 - 1;
+    return p < last ? p : last;
+  }
+  static __device__ __forceinline__ Raw load(uint64_t row, Place p) {
+    return __builtin_nontemporal_load(global_cptr<V>(row) + p);
+  }
+  template <int N> static __device__ __forceinline__ void settle(Raw *raw) { SettleAll<N>::of(raw); }
+  template <typename U>
+  static __device__ __forceinline__ void store(uint64_t row, Place p, uint32_t H, const f32x8 &acc) {
+    typedef typename OutVectors<U>::by8 vec_t;
+    if (p < H / 8) __builtin_nontemporal_store(__builtin_convertvector(acc, vec_t), global_ptr<vec_t>(row) + p);
+  }
+};
+template <> struct Row8<__bf16> : Row8By16<u32x4> {
   static __device__ __forceinline__ f32x8 widen(const Raw &raw) {
     f32x8 out;
 #pragma unroll
@@ -41,42 +92,20 @@ template <> struct Row8<__bf16> {
     }
     return out;
   }
-  template <int N> static __device__ __forceinline__ void settle(Raw *raw) { SettleAll<N>::of(raw); }
 };
-template <> struct Row8<_Float16> {
-  typedef f16x8 Raw;
-  static __device__ __forceinline__ Raw load(uint64_t row, uint32_t vec) {
-    return __builtin_nontemporal_load(global_cptr<f16x8>(row) + vec);
-  }
-  static __device__ __forceinline__ f32x8 widen(const Raw &raw) {
-    return __builtin_convertvector(raw, f32x8);
-  }
-  template <int N> static __device__ __forceinline__ void settle(Raw *raw) { SettleAll<N>::of(raw); }
-};
-
-template <typename U> struct Store8;
-template <> struct Store8<__bf16> {
-  static __device__ __forceinline__ void at(void *row, uint32_t vec, const f32x8 &acc) {
-    __builtin_nontemporal_store(__builtin_convertvector(acc, bf16x8),
-                                as_global(reinterpret_cast<bf16x8 *>(row)) + vec);
-  }
-};
-template <> struct Store8<_Float16> {
-  static __device__ __forceinline__ void at(void *row, uint32_t vec, const f32x8 &acc) {
-    __builtin_nontemporal_store(__builtin_convertvector(acc, f16x8),
-                                as_global(reinterpret_cast<f16x8 *>(row)) + vec);
-  }
+template <> struct Row8<_Float16> : Row8By16<f16x8> {
+  static __device__ __forceinline__ f32x8 widen(const Raw &raw) { return __builtin_convertvector(raw, f32x8); }
 };
 
 // N picks starting at k, VPL vectors of each: all N * VPL loads are issued before the first is used.
 template <typename T, int N, int VPL>
 __device__ __forceinline__ void gather_group(f32x8 (&acc)[VPL], uint64_t row_of_lane, float weight_of_lane,
-                                             uint32_t k, const uint32_t (&vec)[VPL]) {
+                                             uint32_t k, const typename Row8<T>::Place (&at)[VPL]) {
   typename Row8<T>::Raw raw[VPL][N];
 #pragma unroll
   for (int v = 0; v < VPL; ++v) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) raw[v][i] = Row8<T>::load(read_lane64(row_of_lane, k + i), vec[v]);
+    for (int i = 0; i < N; ++i) raw[v][i] = Row8<T>::load(read_lane64(row_of_lane, k + i), at[v]);
   }
   Row8<T>::template settle<VPL * N>(&raw[0][0]);
 #pragma unroll
@@ -93,26 +122,26 @@ constexpr uint32_t kWavesPerBlock = 4;
 // The sum of one output row's piece: lane `base + k` holds the row and the weight of pick k.
 template <typename T, int KB, int VPL>
 __device__ __forceinline__ void reduce_picks(f32x8 (&acc)[VPL], uint32_t K, uint64_t row, float weight, uint32_t base,
-                                             bool all_rows, const uint32_t (&vec)[VPL]) {
+                                             bool all_rows, const typename Row8<T>::Place (&at)[VPL]) {
 #pragma unroll
   for (int v = 0; v < VPL; ++v) acc[v] = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (!all_rows) {
     // A pick without a row (bad expert id or slot) contributes nothing.
     for (uint32_t k = 0; k < K; ++k) {
-      if (read_lane64(row, base + k) != 0) gather_group<T, 1, VPL>(acc, row, weight, base + k, vec);
+      if (read_lane64(row, base + k) != 0) gather_group<T, 1, VPL>(acc, row, weight, base + k, at);
     }
     return;
   }
   uint32_t k = 0;
-  for (; k + KB <= K; k += KB) gather_group<T, KB, VPL>(acc, row, weight, base + k, vec);
+  for (; k + KB <= K; k += KB) gather_group<T, KB, VPL>(acc, row, weight, base + k, at);
   if constexpr (KB > 4) {
-    if ((K - k) & 4) { gather_group<T, 4, VPL>(acc, row, weight, base + k, vec); k += 4; }
+    if ((K - k) & 4) { gather_group<T, 4, VPL>(acc, row, weight, base + k, at); k += 4; }
   }
   if constexpr (KB > 2) {
-    if ((K - k) & 2) { gather_group<T, 2, VPL>(acc, row, weight, base + k, vec); k += 2; }
+    if ((K - k) & 2) { gather_group<T, 2, VPL>(acc, row, weight, base + k, at); k += 2; }
   }
   if constexpr (KB > 1) {
-    if ((K - k) & 1) { gather_group<T, 1, VPL>(acc, row, weight, base + k, vec); }
+    if ((K - k) & 1) { gather_group<T, 1, VPL>(acc, row, weight, base + k, at); }
   }
 }
 
@@ -179,23 +208,17 @@ __global__ __launch_bounds__(kWavesPerBlock * kWave) void combine_gather(WorldDe
   const uint64_t no_row = __builtin_amdgcn_ballot_w64(present && row == 0);
 
   const uint64_t out = reinterpret_cast<uint64_t>(reinterpret_cast<U *>(c.out_tokens) + (int64_t)t * c.out_stride_row);
-  const uint32_t nvec = w.H / 8;
-  uint32_t vec[VPL];
+  typedef Row8<T> Row;
+  typename Row::Place at[VPL];
 #pragma unroll
-  for (int v = 0; v < VPL; ++v) {
-    vec[v] = (segment * VPL + v) * kWave + lane;
-    vec[v] = vec[v] < nvec ? vec[v] : nvec - 1;  // clamp: loads stay unconditional
-  }
+  for (int v = 0; v < VPL; ++v) at[v] = Row::clamped(Row::place(segment * VPL + v, lane), w.H);
   f32x8 acc[VPL];
   auto store = [&](uint64_t out) {
 #pragma unroll
-    for (int v = 0; v < VPL; ++v) {
-      const uint32_t at = (segment * VPL + v) * kWave + lane;
-      if (at < nvec) Store8<U>::at(reinterpret_cast<U *>(out), at, acc[v]);
-    }
+    for (int v = 0; v < VPL; ++v) Row::template store<U>(out, Row::place(segment * VPL + v, lane), w.H, acc[v]);
   };
   if constexpr (!GROUPED) {
-    reduce_picks<T, KB, VPL>(acc, w.K, row, weight, 0, no_row == 0, vec);
+    reduce_picks<T, KB, VPL>(acc, w.K, row, weight, 0, no_row == 0, at);
     store(out);
   } else {
     const uint64_t picks = w.K == kWave ? ~0ull : (1ull << w.K) - 1;
@@ -208,7 +231,7 @@ __global__ __launch_bounds__(kWavesPerBlock * kWave) void combine_gather(WorldDe
                         __shfl((uint32_t)(row >> 32), src, kWave) == (uint32_t)(row >> 32) &&
                         __shfl(__float_as_uint(weight), src, kWave) == __float_as_uint(weight);
       const uint64_t differs = __builtin_amdgcn_ballot_w64(present && !same);
-      reduce_picks<T, KB, VPL>(acc, w.K, row, weight, base, ((no_row >> base) & picks) == 0, vec);
+      reduce_picks<T, KB, VPL>(acc, w.K, row, weight, base, ((no_row >> base) & picks) == 0, at);
       for (uint64_t rest = todo; rest != 0; rest &= rest - 1) {
         const uint32_t head = (uint32_t)__builtin_ctzll(rest);
         if (((differs >> head) & picks) != 0) continue;

@@ -243,6 +243,27 @@ def test_pieces_of_fp32_rows(M, K, H, dp, out_dtype):
     world.destroy()
 
 
+@pytest.mark.parametrize("H", [248, 256, 264, 768, 776])
+@pytest.mark.parametrize("K,dp", [(3, 1), (8, 2)])
+def test_halves_of_an_fp32_piece(H, K, dp):
+    """A lane holds two vectors of four columns, 256 columns apart: rows that end in, at and behind a piece's first half."""
+    M = 70
+    spec = WorkloadSpec(
+        "halves", 80, 4, 16, K, H, M, torch.bfloat16, expert_y_dtype=torch.float32, dp_size=dp, tokens="uniform"
+    )  # fmt: skip
+    groups = generate(spec, seed=H + K)
+    groups[0].n, groups[-1].n = M, 1
+    step = DeviceStep(spec, groups)
+    world = make_world(spec, group_name="halves")
+    step.dispatch_world(world)
+    expected = check_dispatch_against_oracle(step)
+    step.expert_y_all.normal_(generator=torch.Generator(device="cuda").manual_seed(9))
+    step.combine_world(world)
+    check_combine_against_oracle(step, expected.slot_map)
+    assert world.faults() == 0
+    world.destroy()
+
+
 # ---------------------------------------------------------------------------
 # Rows that cut 64-byte half lines, and rows without a register variant: through LDS
 # ---------------------------------------------------------------------------

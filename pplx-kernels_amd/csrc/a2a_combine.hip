@@ -16,7 +16,8 @@ namespace {
 // and takes half of each.  Combine alone on three buffer sets, us, 8 elements in one lane / two vectors apart: 7168 wide, top-8,
 // 8 x 128 tokens 46.0 / 41.5, 8 x 1024 381.8 / 347.4; 512 wide, top-8, 8 x 2048 56.7 / 47.8; 4096 wide, top-2, 8 x 2048
 // 118.1 / 110.0, top-1 72.5 / 66.1; 520 wide, top-6, 8 x 1024 25.7 / 21.4; 2880 wide, top-5, groups of four, 3001 tokens
-// 50.6 / 46.1 (242 MB: 4.8 -> 5.25 TB/s; the stores, 8 bytes a lane, still cover whole lines).
+// 50.6 / 46.1 (242 MB: 4.8 -> 5.25 TB/s).  The stores, 8 bytes a lane, still cover whole lines: lanes that swap halves in
+// pairs to store 16 bytes each measured the same (4200 steps: 1.000).
 template <typename U> struct OutVectors;
 template <> struct OutVectors<__bf16> {
   typedef __bf16 by4 __attribute__((ext_vector_type(4)));
@@ -272,89 +273,133 @@ int launch_combine_v(const WorldDev &w, const CT &tab, bool grouped, hipStream_t
   return (int)hipGetLastError();
 }
 
-// Whether pieces of `length` KiB of a 16-bit row make workgroups that come out even, `least` to four of them to each of the
-// 256 CUs, with at most 1 KiB of padding to a piece.
-bool even_pieces(uint64_t tokens, uint32_t segments, uint32_t length, uint32_t least) {
-  const uint32_t pieces = (segments + length - 1) / length;
-  if (pieces * length - segments > pieces) return false;
+// Whether 8 KiB pieces of a 16-bit row make workgroups that come out even, two to four of them to each of the 256 CUs,
+// with at most 1 KiB of padding to a piece.
+bool even_pieces(uint64_t tokens, uint32_t segments) {
+  const uint32_t pieces = (segments + 7) / 8;
+  if (pieces * 8 - segments > pieces) return false;
   const uint64_t workgroups = (tokens * pieces + kWavesPerBlock - 1) / kWavesPerBlock;
   const uint64_t per_cu = (workgroups + 255) / 256;
-  return per_cu >= least && per_cu <= 4 && 256 * per_cu - workgroups <= 16;
+  return per_cu >= 2 && per_cu <= 4 && 256 * per_cu - workgroups <= 16;
+}
+
+// How pieces of 7 KiB (whole rows of them) or 8 KiB of a 16-bit row fall on the 256 CUs: the most workgroups that one
+// gets, and whether those of all CUs and the padding of the pieces leave less than a quarter of it idle.
+struct LongPieces {
+  uint64_t per_cu;
+  bool even;
+};
+LongPieces long_pieces(uint64_t tokens, uint32_t segments) {
+  const uint32_t length = segments % 7 == 0 ? 7 : 8;
+  const uint32_t pieces = (segments + length - 1) / length;
+  const uint64_t workgroups = (tokens * pieces + kWavesPerBlock - 1) / kWavesPerBlock;
+  const uint64_t per_cu = (workgroups + 255) / 256;
+  return {per_cu, 4 * workgroups * segments >= 3 * 256 * per_cu * pieces * length};
 }
 
 template <typename T, typename U, class CT>
 int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
 #define PPLX_COMBINE(KB, VPL) return launch_combine_v<T, U, CT, KB, VPL>(w, tab, grouped, s)
   const bool grouped = combine_per_group(w, sizeof(T));
-  // Five picks and more are taken up to eight at a time, 1 KiB of a row each -- except for steps of a few
-  // hundred to two thousand tokens, whose waves are all resident at the same moment: there more than four
-  // picks are better taken one after the other in 7 or 8 KiB pieces by a quarter as many waves
-  // (8 x 128 DSv3 tokens, top-8: 23.4 us against 25.3 us; 8 x 256: 45.8 against 46.8; from
-  // 8 x 512 on the wide form wins, 88.7 against 91.5 us, and below 8 x 64 too).  Fewer picks: at the switch below.
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
   const uint64_t tokens = (uint64_t)(grouped ? w.G : w.R) * w.M;
-  if (w.K > 4 && tokens > 384 && tokens <= 2048 && nvec_segments >= 7) {
-    if (nvec_segments % 7 == 0) PPLX_COMBINE(1, 7);
-    PPLX_COMBINE(1, 8);
-  }
-  // fp32 rows are twice as long, and gathering eight of them at a time in 2 KiB pieces leaves each
-  // wave's accesses scattered over too many of them; steps that fill the chip more than once take two
-  // picks in 8 KiB pieces, or three in 4 KiB pieces where the last of the 8 KiB ones would be mostly
-  // padding.  Measured on 8 ranks (us: as before / three in 4 KiB / two in 8 KiB): 1024 tokens a rank,
-  // top-8, 2048 wide 110.3 / 106.8 / 101.8, 4096 wide 217.9 / 214.3 / 204.7; 5120 wide, top-3 111.2 / 107.5
-  // / 106.9; 4096 wide, top-4 112.9 / 110.4 / 108.8; 1024 wide, top-10, 2048 a rank 136.6 / 131.4 / 135.3;
-  // 7168 wide, top-8, 2048 a rank 779 / 773 / 774, 512 and a ragged batch 101.7 / 101.6 / 97.9; 2880 wide,
-  // top-5, dp 4: 2 x 3001 tokens 98.9 / 94.1 / 94.4, ragged 52.0 / 50.6 / 53.0; dp 1, 8 x 1024 98.6 / 96.6 /
-  // 98.0.  Steps of a few hundred tokens lack the waves for it (64 tokens, 7168 wide, top-8: 5.8 / 7.9 /
-  // 11.0; 320 tokens, 1024 wide, top-6: 4.5 / 6.2 / 6.7); 16-bit rows do not care (within 1 %) or lose
-  // (the large ragged prefill of 7168-wide rows: 734 / 761 / 762).  Rows of up to 512 columns are one
-  // 2 KiB piece, and a longer one is only padding: more than four picks of them stay eight at a time
-  // (8 x 2048 tokens, dispatch and combine, eight picks of 2 KiB / three of 4 KiB: 512 wide, top-8 92.7 / 93.8, top-6
-  // 71.8 / 74.0; 256 wide, top-10 62.3 / 66.2; 8 wide, top-8 35.2 / 41.6; 8 x 8192, 512 wide, top-8, combine
-  // alone 221.4 / 226.6).
-  if constexpr (sizeof(T) == 4) {
-    if (w.K > 2 && tokens > 2048 && (w.K <= 4 || nvec_segments > 1)) {
-      const uint32_t padding = (4 - nvec_segments % 4) % 4;
-      if (6 * padding <= nvec_segments) PPLX_COMBINE(2, 4);
-      PPLX_COMBINE(3, 2);
+  // Steps of a few hundred to two thousand tokens have all their waves resident at the same moment.  More than four picks in rows
+  // of 7 KiB and more are best taken one after the other in 7 or 8 KiB pieces there, by a quarter as many waves, but
+  // only where the workgroups of such pieces come out even over the CUs (long_pieces): the CUs that get one more of them
+  // take that much longer.  Dispatch + combine on three buffer sets, top-8, 8 ranks, us, long pieces / three picks in 1
+  // KiB: 7168 wide, 1024 tokens 38.4 / 39.0, 544 25.0 / 23.7, 7136 wide, 528 30.2 / 28.4, 7656 wide, 1048 61.8 / 57.6; 4096 wide, 388
+  // 19.7 / 15.4, 448 20.4 / 17.0, 680 23.7 / 22.7, 784 24.8 / 25.0, 1024 29.9 / 30.3.  (653 steps of that range drawn
+  // at random, against long pieces for all of them: 0.946 of the time, 0.73 to 1.03.)  DP groups, whose waves compare the
+  // members first, take two picks in 2 KiB pieces or, beyond a workgroup to a CU, one in 3 KiB instead (5120 wide, 386
+  // tokens of all groups 20.2 / 17.9; 3696 wide, 596 23.5 / 21.2), fp32 rows two picks in 1 KiB (4608 wide, top-6, 1256
+  // tokens 49.3 / 44.4; 3584 wide, 1152 40.7 / 35.5).
+  const bool middle = tokens > 384 && tokens <= 2048;
+  if (w.K > 4 && middle && nvec_segments >= 7) {
+    const LongPieces pieces = long_pieces(tokens, nvec_segments);
+    if (pieces.even && (grouped || pieces.per_cu > 1)) {
+      if (nvec_segments % 7 == 0) PPLX_COMBINE(1, 7);
+      PPLX_COMBINE(1, 8);
+    }
+    if constexpr (sizeof(T) == 2) {
+      if (!grouped) PPLX_COMBINE(3, 1);
+      if (pieces.per_cu == 1) PPLX_COMBINE(2, 2);
+      PPLX_COMBINE(1, 3);
     }
   }
-  // Of what is left, up to five picks are taken all at once.  One or two leave a wave of 1 KiB with little in flight, so
-  // they read longer pieces: up to 3 KiB of one pick and 2 KiB of two, which is ahead of 8 and of 4 KiB nearly everywhere (dispatch +
-  // combine, 8 ranks, us, long / short pieces: one pick of 16-bit rows, 512 tokens, 2048 wide 8.3 / 7.8, 4096 wide 9.2 /
+  // fp32 rows of three KiB of 16-bit outputs and more.  Two picks at a time beside the above (2048 wide, top-8, 464 tokens
+  // 13.0 / 12.8; 1536 wide, 808 16.3 / 15.6; 2560 wide, 1040 29.8 / 28.7, eight / two).  Larger steps take eight at a time, whose
+  // registers leave room for fewer waves: against two picks of 4 KiB or three of 2 KiB 6656 wide, top-8, 2095 tokens 130.4 / 126.2,
+  // 3588 180.4 / 173.7; 4096 wide, 7168 221.2 / 215.7; top-6, 7680 wide, 5232 279.4 / 271.2; seven KiB and more also with four
+  // picks (6144 wide, 2156 tokens 56.0 / 55.3; 4096 wide, 8 x 1024, combine alone 103.2 / 98.1).  DP groups of that size take three
+  // (2048 wide, 2136 tokens 43.1 / 40.5), rows of two KiB three in pieces of both (eight 1.0 to 1.1 of their time).
+  if constexpr (sizeof(T) == 4) {
+    if (w.K > 4 && middle && nvec_segments >= 3) PPLX_COMBINE(2, 1);
+    if (tokens > 2048) {
+      if (!grouped && w.K > 3 && nvec_segments >= 7) PPLX_COMBINE(8, 1);
+      if (w.K > 4 && nvec_segments == 2) PPLX_COMBINE(3, 2);
+      if (w.K > 4 && nvec_segments >= 3) {
+        if (grouped) PPLX_COMBINE(3, 1);
+        PPLX_COMBINE(8, 1);
+      }
+    }
+  } else if (grouped && nvec_segments > 1) {
+    // Steps of DP groups, 16-bit rows, eight picks / three in pieces of 2 KiB: 5120 wide, top-6, 2888 tokens 86.8 / 84.0;
+    // 1024 wide, top-8, 12268 88.1 / 87.1 (541 steps: 0.983, 0.90 to 1.05); three and four picks, all at once / two:
+    // 1536 wide, top-4, 3260 25.0 / 23.5; 5120 wide, 856 23.5 / 22.9.
+    if (w.K > 4 && tokens > 2048) PPLX_COMBINE(3, 2);
+    if ((w.K == 3 || w.K == 4) && tokens > 600 && nvec_segments > 2) PPLX_COMBINE(2, 2);
+  }
+  // Of what is left, up to five picks are taken all at once, six in two goes of three, nine and ten in two of five, others
+  // up to eight at a time.  One or two leave a wave of 1 KiB with little in flight, so they read longer pieces: up to 3
+  // KiB of one pick and 2 KiB of two, which is ahead of 8 and of 4 KiB nearly everywhere (dispatch + combine, 8 ranks, us,
+  // long / short pieces: one pick of 16-bit rows, 512 tokens, 2048 wide 8.3 / 7.8, 4096 wide 9.2 /
   // 8.8, 8192 wide 12.0 / 11.4; 8192 tokens, 52.3 / 51.0 and 105.9 / 103.6; two picks, 512 tokens, 8.7 / 8.3, 10.0 /
   // 10.0 and 14.1 / 13.9; 8192 tokens, 71.6 / 70.5 and 151.8 / 150.2; not one pick, 1024 tokens, 2560 wide 9.2 / 9.6, 3072
   // 9.6 / 10.1), except
   //  - where the workgroups of the long pieces come out even over the CUs (even_pieces): one pick, 2048 tokens, 3584 wide
   //    15.1 / 15.7, 4096 wide 16.0 / 16.7, 8192 wide 28.9 / 29.5; 4096 tokens of 4096 29.5 / 30.2; 1536 of 7168 19.6 / 20.5 (but
-  //    uneven, 4096 wide, 1536 tokens 15.1 / 14.3, 2560 19.8 / 19.8, 3584 25.1 / 24.6); two picks of fp32 rows only where
-  //    there are four workgroups to a CU: 4096 tokens, 2048 wide 27.9 / 28.8; 2048 tokens, 4096 wide 27.6 / 28.4
-  //    (three, 3072 tokens, 2048 wide 22.8 / 22.9; 3584 tokens 26.2 / 25.4; two, 1024 tokens, 4096 wide 17.2 / 17.1);
+  //    uneven, 4096 wide, 1536 tokens 15.1 / 14.3, 2560 19.8 / 19.8, 3584 25.1 / 24.6);
   //  - for DP groups, whose waves compare the members first.  They keep the long pieces for rows that are longer than half
   //    of one (groups of two, 4 x 512 tokens, one pick, 4096 wide 18.8 / 20.6, 7168 wide 32.1 / 31.4; groups of four, 2 x 512,
   //    15.0 / 15.1 and 22.1 / 24.0; two picks, 25.2 / 25.9 and 44.3 / 44.4, 17.3 / 19.2 and 28.3 / 28.9), one pick also unless
-  //    the last piece would be all but empty (4608 wide, nine KiB, 23.3 / 22.4).
+  //    the last piece would be all but empty (4608 wide, nine KiB, 23.3 / 22.4);
+  //  - fp32 rows, which have twice the bytes: 4 KiB (1 KiB up to 384 tokens) of one pick, 2 KiB of two (one pick, 7168
+  //    wide, 208 tokens 9.0 / 8.4, 4096 wide, 2428 20.4 / 19.6; two picks of 8 KiB / 2 KiB, 7680 wide, 4928 91.6 / 89.2).
   // Picks of one go, against eight places of 1 KiB: top-3 (two picks and then one), 8192 tokens, 2048 wide 57.0 / 52.4, 4096
-  // wide 99.5 / 90.4; top-5 (four and one), 16000 tokens, 512 wide 43.4 / 41.6, 4096 tokens, 7168 wide 124.6 / 122.5.
-  // Top-6 and top-7 in one go measure the same as four picks and the rest (145.0 / 145.9, 165.3 / 165.0).
+  // wide 99.5 / 90.4; top-5 (four and one), 16000 tokens, 512 wide 43.4 / 41.6, 4096 tokens, 7168 wide 124.6 / 122.5.  Four picks
+  // in 2 KiB / 1 KiB: 5120 wide, 88 tokens 8.7 / 8.2, 3584 wide, 2048 25.0 / 24.4, 7680 wide, 1388 43.4 / 42.5 (995 steps: 0.987).
+  // Six, four and two / three and three: 2560 wide, 2792 tokens 32.6 / 31.5, 3072 wide, 3914 50.0 / 48.8 (1 KiB to 6 KiB
+  // wide, beyond 2048 tokens: 0.975; up to 2048 0.99).  Ten, eight and two / five and five: 512 wide, 1160 14.6 / 14.0, 3584
+  // wide, 352 15.5 / 15.2.  Neither in large steps of 16-bit rows of 7 KiB and more (six 0.97 to 1.04, ten 1.012) nor for
+  // DP groups of 16-bit rows.
   switch (w.K) {
     case 1:
       if (nvec_segments == 1) PPLX_COMBINE(1, 1);
       if (nvec_segments == 2) PPLX_COMBINE(1, 2);
+      if (!grouped && sizeof(T) == 4) {
+        if (tokens <= 384) PPLX_COMBINE(1, 1);
+        PPLX_COMBINE(1, 2);
+      }
       if (nvec_segments == 4) PPLX_COMBINE(1, 4);
       if (grouped && nvec_segments > 4 && 8 * ((8 - nvec_segments % 8) % 8) <= 5 * nvec_segments) PPLX_COMBINE(1, 8);
-      if (!grouped && sizeof(T) == 2 && even_pieces(tokens, nvec_segments, 8, 2)) PPLX_COMBINE(1, 8);
+      if (!grouped && sizeof(T) == 2 && even_pieces(tokens, nvec_segments)) PPLX_COMBINE(1, 8);
       PPLX_COMBINE(1, 3);
     case 2:
-      if (nvec_segments == 1) PPLX_COMBINE(2, 1);
-      if (grouped && nvec_segments > 2) PPLX_COMBINE(2, 4);
-      if (!grouped && sizeof(T) == 4 && even_pieces(tokens, nvec_segments, 4, 4)) PPLX_COMBINE(2, 4);
+      if (nvec_segments == 1 || (sizeof(T) == 4 && (!grouped || tokens <= 384))) PPLX_COMBINE(2, 1);
+      if (grouped && sizeof(T) == 2 && nvec_segments > 2) PPLX_COMBINE(2, 4);
       PPLX_COMBINE(2, 2);
     case 3: PPLX_COMBINE(3, 1);
     case 4:
-      if (nvec_segments == 1) PPLX_COMBINE(4, 1);
-      PPLX_COMBINE(4, 2);
+      if (sizeof(T) == 2 && nvec_segments > 1 && (grouped || (nvec_segments == 2 && tokens > 600))) PPLX_COMBINE(4, 2);
+      PPLX_COMBINE(4, 1);
     case 5: PPLX_COMBINE(5, 1);
+    case 6:
+      if (sizeof(T) == 4 || (!grouped && (nvec_segments < 7 || tokens <= 2048))) PPLX_COMBINE(3, 1);
+      PPLX_COMBINE(8, 1);
+    case 9:
+    case 10:
+      if (sizeof(T) == 4 || (!grouped && (nvec_segments < 7 || tokens <= 2048))) PPLX_COMBINE(5, 1);
+      PPLX_COMBINE(8, 1);
     default: PPLX_COMBINE(8, 1);
   }
 #undef PPLX_COMBINE

@@ -479,6 +479,42 @@ def test_pieces_of_few_picks(K, H, dp, y_dtype, out_dtype):
 @pytest.mark.parametrize(
     "K,H,M,y_dtype,dp",
     [
+        (5, 3592, 48, torch.bfloat16, 1),  # 384 tokens, rows of 8 KiB: eight picks at a time still
+        (5, 3592, 49, torch.bfloat16, 1),  # 392: long pieces would leave most CUs without one, three picks and two
+        (8, 4096, 256, torch.float16, 1),  # 2048: long pieces, two workgroups to a CU
+        (8, 4096, 257, torch.float16, 1),  # 2056: eight at a time again
+        (7, 3080, 140, torch.bfloat16, 1),  # seven KiB, the last a single vector; 1120 tokens
+        (8, 3592, 100, torch.bfloat16, 2),  # DP groups: up to a workgroup of long pieces to a CU two picks of 2 KiB
+        (8, 3592, 300, torch.bfloat16, 2),  # ... one of 3 KiB
+        (8, 520, 600, torch.float16, 2),  # ... large steps, three picks of 2 KiB
+        (4, 1032, 151, torch.bfloat16, 2),  # ... two of four picks
+        (9, 1032, 60, torch.bfloat16, 1),  # five picks, then four
+        (10, 3080, 257, torch.bfloat16, 1),  # eight, then two
+        (5, 1032, 60, torch.float32, 1),  # fp32 rows: two at a time
+        (4, 3080, 257, torch.float32, 1),  # ... four in the form that takes eight
+        (7, 1032, 520, torch.float32, 2),  # ... DP groups, three
+    ],
+)
+def test_pieces_of_many_picks(K, H, M, y_dtype, dp):
+    spec = WorkloadSpec(
+        "many-picks", 81, 8, 16, K, H, M, torch.bfloat16, expert_y_dtype=y_dtype, dp_size=dp, tokens="uniform"
+    )  # fmt: skip
+    groups = generate(spec, seed=H + K)
+    groups[0].n, groups[-1].n = M, 1
+    step = DeviceStep(spec, groups)
+    world = make_world(spec, group_name="many-picks")
+    step.dispatch_world(world)
+    expected = check_dispatch_against_oracle(step)
+    step.expert_y_all.normal_(generator=torch.Generator(device="cuda").manual_seed(10))
+    step.combine_world(world)
+    check_combine_against_oracle(step, expected.slot_map)
+    assert world.faults() == 0
+    world.destroy()
+
+
+@pytest.mark.parametrize(
+    "K,H,M,y_dtype,dp",
+    [
         (1, 3584, 256, torch.bfloat16, 1),  # 8 KiB pieces, two workgroups to a CU
         (1, 3208, 250, torch.float16, 1),  # ... a few less, the last of seven KiB a single vector
         (1, 7680, 256, torch.bfloat16, 1),  # ... four workgroups, two pieces to a row

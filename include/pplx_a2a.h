@@ -85,6 +85,7 @@ typedef struct pplx_a2a_world pplx_a2a_world_t;
 typedef struct pplx_a2a pplx_a2a_t;
 /* An instantiated hipGraph. */
 typedef struct pplx_a2a_graph pplx_a2a_graph_t;
+typedef struct pplx_a2a_bound pplx_a2a_bound_t;
 
 /* Arguments of one rank's dispatch: the views built in
  * csrc/bindings/all_to_all_ops.cpp:165-195 for AllToAllIntraNode::dispatch
@@ -257,6 +258,20 @@ int pplx_a2a_plan_on(const pplx_a2a_config_t *cfg, int in_dtype, uint32_t lds_pe
  * process (csrc/core/cuda_utils.h:7-14, csrc/core/utils.h:16-24).  Only host state changes:
  * no allocation, no synchronisation. */
 int pplx_a2a_world_abandon_step(pplx_a2a_world_t *world, uint32_t which, uint32_t *dropped_calls);
+/* A step whose buffers stay where they are: pplx_a2a_bound_create checks the arguments of
+ * pplx_a2a_world_dispatch and pplx_a2a_world_combine once and enqueues the writing of their rank
+ * tables into `device_memory` (pplx_a2a_bound_bytes, 16-byte aligned, the caller's), on `stream`;
+ * pplx_a2a_bound_launch then runs dispatch (op 0) or combine (op 1).  On that stream the kernels
+ * read the tables from there; on another one, or while the stream is captured, they go with the
+ * launch as always (a graph never refers to device_memory).  device_memory is to stay untouched
+ * until the last launch on that stream is done with it; the bound step is to be destroyed before
+ * its world.  The capture of `stream` refuses pplx_a2a_bound_create. */
+int pplx_a2a_bound_bytes(const pplx_a2a_world_t *world, uint64_t *out);
+int pplx_a2a_bound_create(pplx_a2a_world_t *world, const pplx_a2a_dispatch_args_t *dispatch_per_rank,
+                          const pplx_a2a_combine_args_t *combine_per_rank, void *device_memory, void *stream,
+                          pplx_a2a_bound_t **out);
+int pplx_a2a_bound_launch(pplx_a2a_world_t *world, const pplx_a2a_bound_t *bound, int op, void *stream);
+int pplx_a2a_bound_destroy(pplx_a2a_bound_t *bound);
 /* Number of per-rank calls of `op` (0 = dispatch, 1 = combine) in `split_mode` that the world
  * has recorded and not launched yet; 0 once the last rank's call has enqueued the phase.  A
  * binding that keeps the callers' buffers alive for the ranks that called early reads this to

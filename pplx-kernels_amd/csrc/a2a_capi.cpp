@@ -11,6 +11,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -139,6 +140,18 @@ struct pplx_a2a_world {
 struct pplx_a2a {
   pplx_a2a_world *world;
   uint32_t rank;
+};
+
+// A step whose arguments were checked once and whose rank tables lie in device memory of the caller.
+struct pplx_a2a_bound {
+  pplx_a2a_world *world = nullptr;
+  std::vector<DispatchRank> dispatch;
+  std::vector<CombineRank> combine;
+  int in_dtype = -1, out_dtype = -1;
+  uint32_t pick_vector = 1;
+  DispatchRank *drank = nullptr;
+  CombineRank *crank = nullptr;
+  void *stream = nullptr;  // on which the tables were written
 };
 
 struct pplx_a2a_graph {
@@ -338,10 +351,22 @@ void settle_mirror(pplx_a2a_world &w, unsigned long long session, unsigned long 
   last_session = session;
 }
 
-// Makes the device tables equal to `rows`, batch by batch, skipping batches the
+// Writes rows `first`, ... of a step, as many as a batch holds, into a table in HBM.
+template <typename Batch, typename Row, typename Launch>
+int bind_batch(uint32_t R, Row *table, const Row *rows, uint32_t first, Launch launch, void *stream) {
+  Batch b;
+  memset(static_cast<void *>(&b), 0, sizeof(b));
+  b.first = first;
+  b.count = R - first < kBindBatch ? R - first : kBindBatch;
+  memcpy(static_cast<void *>(b.rows), rows + first, sizeof(Row) * b.count);
+  LAUNCH_TRY(launch(table, b, stream));
+  return PPLX_A2A_OK;
+}
+
+// Makes the world's device tables equal to `rows`, batch by batch, skipping batches the
 // tables are known to hold already.
 template <typename Row, typename Batch, typename Launch>
-int flush_table(pplx_a2a_world &w, const std::vector<Row> &rows, std::vector<Row> &bound,
+int flush_table(pplx_a2a_world &w, Row *table, const std::vector<Row> &rows, std::vector<Row> &bound,
                 bool &bound_valid, bool force, Launch launch, void *stream) {
   const uint32_t R = w.dev.R;
   for (uint32_t first = 0; first < R; first += kBindBatch) {
@@ -349,12 +374,8 @@ int flush_table(pplx_a2a_world &w, const std::vector<Row> &rows, std::vector<Row
     bool dirty = force || !bound_valid;
     if (!dirty) dirty = memcmp(&rows[first], &bound[first], sizeof(Row) * count) != 0;
     if (!dirty) continue;
-    Batch b;
-    memset(static_cast<void *>(&b), 0, sizeof(b));
-    b.first = first;
-    b.count = count;
-    memcpy(static_cast<void *>(b.rows), &rows[first], sizeof(Row) * count);
-    LAUNCH_TRY(launch(w.dev, b, stream));
+    const int st = bind_batch<Batch>(R, table, rows.data(), first, launch, stream);
+    if (st) return st;
   }
   bound = rows;
   bound_valid = true;
@@ -451,7 +472,7 @@ int run_dispatch(pplx_a2a_world &w, void *stream) {
     LAUNCH_TRY(launch_dispatch(w.dev, w.pend_dispatch.data(), pick_vector_of(w), stream));
     return PPLX_A2A_OK;
   }
-  st = flush_table<DispatchRank, BindDispatchBatch>(w, w.pend_dispatch, w.bound_dispatch,
+  st = flush_table<DispatchRank, BindDispatchBatch>(w, w.dev.drank, w.pend_dispatch, w.bound_dispatch,
                                                     w.bound_dispatch_valid, false,
                                                     launch_bind_dispatch, stream);
   if (st) return st;
@@ -472,7 +493,7 @@ int run_combine(pplx_a2a_world &w, void *stream) {
                               stream));
     return PPLX_A2A_OK;
   }
-  st = flush_table<CombineRank, BindCombineBatch>(w, w.pend_combine, w.bound_combine,
+  st = flush_table<CombineRank, BindCombineBatch>(w, w.dev.crank, w.pend_combine, w.bound_combine,
                                                   w.bound_combine_valid, false,
                                                   launch_bind_combine, stream);
   if (st) return st;
@@ -574,7 +595,7 @@ int run_split_dispatch(pplx_a2a_world &w, int mode, void *stream) {
   }
   const DispatchRank *inline_rows = d.R <= kInlineRanks ? w.pend_dispatch.data() : nullptr;
   if (!inline_rows) {
-    st = flush_table<DispatchRank, BindDispatchBatch>(w, w.pend_dispatch, w.bound_dispatch,
+    st = flush_table<DispatchRank, BindDispatchBatch>(w, w.dev.drank, w.pend_dispatch, w.bound_dispatch,
                                                       w.bound_dispatch_valid, false, launch_bind_dispatch, stream);
     if (st) return st;
   }
@@ -643,7 +664,7 @@ int run_split_combine(pplx_a2a_world &w, int mode, int in_dtype, int out_dtype, 
   }
   const CombineRank *inline_rows = d.R <= kInlineRanks ? w.pend_combine.data() : nullptr;
   if (!inline_rows) {
-    st = flush_table<CombineRank, BindCombineBatch>(w, w.pend_combine, w.bound_combine, w.bound_combine_valid,
+    st = flush_table<CombineRank, BindCombineBatch>(w, w.dev.crank, w.pend_combine, w.bound_combine, w.bound_combine_valid,
                                                     false, launch_bind_combine, stream);
     if (st) return st;
   }
@@ -964,6 +985,107 @@ int pplx_a2a_world_combine(pplx_a2a_world_t *w, const pplx_a2a_combine_args_t *p
   w->combine_in_dtype = per_rank[0].in_dtype;
   w->combine_out_dtype = per_rank[0].out_dtype;
   return run_combine(*w, stream);
+}
+
+int pplx_a2a_bound_bytes(const pplx_a2a_world_t *w, uint64_t *out) {
+  if (!w || !out) return fail(PPLX_A2A_INVALID_ARGUMENT, "world / out is NULL");
+  *out = (sizeof(DispatchRank) + sizeof(CombineRank)) * (uint64_t)w->dev.R;
+  return PPLX_A2A_OK;
+}
+
+int pplx_a2a_bound_create(pplx_a2a_world_t *w, const pplx_a2a_dispatch_args_t *dispatch_per_rank,
+                          const pplx_a2a_combine_args_t *combine_per_rank, void *device_memory, void *stream,
+                          pplx_a2a_bound_t **out) {
+  if (!w || !dispatch_per_rank || !combine_per_rank || !device_memory || !out)
+    return fail(PPLX_A2A_INVALID_ARGUMENT, "world / arguments / device_memory / out is NULL");
+  *out = nullptr;
+  if (!aligned16(device_memory))
+    return fail(PPLX_A2A_INVALID_ARGUMENT, "device_memory must be 16-byte aligned");
+  const WorldDev &d = w->dev;
+  std::unique_ptr<pplx_a2a_bound> b(new (std::nothrow) pplx_a2a_bound());
+  try {
+    if (b) {
+      b->dispatch.resize(d.R);
+      b->combine.resize(d.R);
+    }
+  } catch (const std::bad_alloc &) {
+    b.reset();
+  }
+  if (!b) return fail(PPLX_A2A_HIP_ERROR, "out of host memory");
+  for (uint32_t r = 0; r < d.R; ++r) {
+    int st = convert_dispatch(d, r, dispatch_per_rank[r], &b->dispatch[r]);
+    if (!st) st = convert_combine(d, r, combine_per_rank[r], &b->combine[r]);
+    if (st) return st;
+    if (combine_per_rank[r].in_dtype != combine_per_rank[0].in_dtype ||
+        combine_per_rank[r].out_dtype != combine_per_rank[0].out_dtype)
+      return fail(PPLX_A2A_UNSUPPORTED, "all ranks of a step must combine with the same dtypes");
+  }
+  int st = check_groups(d, b->dispatch.data());
+  if (st) return st;
+  DeviceScope scope(w->device);
+  if (!scope.ok()) return fail(PPLX_A2A_HIP_ERROR, "cannot select device %d", w->device);
+  unsigned long long session = 0;
+  st = capture_session(stream, &session);
+  if (st) return st;
+  if (session != 0) return fail(PPLX_A2A_INVALID_STATE, "a step cannot be bound while its stream is captured");
+  DispatchRank *drank = static_cast<DispatchRank *>(device_memory);
+  CombineRank *crank = reinterpret_cast<CombineRank *>(drank + d.R);
+  for (uint32_t first = 0; first < d.R; first += kBindBatch) {
+    st = bind_batch<BindDispatchBatch>(d.R, drank, b->dispatch.data(), first, launch_bind_dispatch, stream);
+    if (!st) st = bind_batch<BindCombineBatch>(d.R, crank, b->combine.data(), first, launch_bind_combine, stream);
+    if (st) return st;
+  }
+  b->world = w;
+  b->in_dtype = combine_per_rank[0].in_dtype;
+  b->out_dtype = combine_per_rank[0].out_dtype;
+  b->pick_vector = pick_vector_of(d, b->dispatch.data());
+  b->drank = drank;
+  b->crank = crank;
+  b->stream = stream;
+  *out = b.release();
+  return PPLX_A2A_OK;
+}
+
+int pplx_a2a_bound_launch(pplx_a2a_world_t *w, const pplx_a2a_bound_t *b, int op, void *stream) {
+  if (!w || !b) return fail(PPLX_A2A_INVALID_ARGUMENT, "world / bound is NULL");
+  if (b->world != w) return fail(PPLX_A2A_INVALID_ARGUMENT, "the step was bound for another world");
+  if (op != 0 && op != 1) return fail(PPLX_A2A_INVALID_ARGUMENT, "op must be 0 (dispatch) or 1 (combine)");
+  std::lock_guard<std::mutex> lock(w->mu);
+  if (op == 0 ? w->n_arrived_dispatch != 0 || w->n_dsend != 0 || w->n_drecv != 0
+              : w->n_arrived_combine != 0 || w->n_csend != 0 || w->n_crecv != 0)
+    return fail(PPLX_A2A_INVALID_STATE, "a per-rank %s step is still being assembled", op == 0 ? "dispatch" : "combine");
+  DeviceScope scope(w->device);
+  if (!scope.ok()) return fail(PPLX_A2A_HIP_ERROR, "cannot select device %d", w->device);
+  unsigned long long session = 0;
+  const int st = capture_session(stream, &session);
+  if (st) return st;
+  // The tables in HBM are ordered with their own stream only, and a graph may outlive them: elsewhere they go with
+  // the launch, as those of a step that is not bound.
+  if (stream != b->stream || session != 0) {
+    if (op == 0) {
+      w->pend_dispatch = b->dispatch;
+      return run_dispatch(*w, stream);
+    }
+    w->pend_combine = b->combine;
+    w->combine_in_dtype = b->in_dtype;
+    w->combine_out_dtype = b->out_dtype;
+    return run_combine(*w, stream);
+  }
+  ProfilerRange range(op == 0 ? "dispatch" : "combine");
+  WorldDev d = w->dev;
+  d.drank = b->drank;
+  d.crank = b->crank;
+  if (op == 0) {
+    LAUNCH_TRY(launch_dispatch(d, nullptr, b->pick_vector, stream));
+  } else {
+    LAUNCH_TRY(launch_combine(d, nullptr, b->in_dtype, b->out_dtype, stream));
+  }
+  return PPLX_A2A_OK;
+}
+
+int pplx_a2a_bound_destroy(pplx_a2a_bound_t *b) {
+  delete b;
+  return PPLX_A2A_OK;
 }
 
 int pplx_a2a_world_recorded_calls(pplx_a2a_world_t *w, int op, int split_mode, uint32_t *out) {

@@ -16,13 +16,11 @@ typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-struct InlineDispatch {
-  static constexpr bool kInline = true;  // the table itself is the kernel argument
+struct InlineDispatch {  // the table itself is the kernel argument
   DispatchRank rows[kInlineRanks];
   __device__ __forceinline__ const DispatchRank &at(uint32_t i) const { return rows[i]; }
 };
 struct HbmDispatch {
-  static constexpr bool kInline = false;
   const DispatchRank *rows;
   __device__ __forceinline__ const DispatchRank &at(uint32_t i) const { return rows[i]; }
 };

@@ -188,11 +188,13 @@ inline StageLayout stage_layout(uint32_t row_bytes, uint32_t scales, uint64_t to
   return l;
 }
 
-// Worlds of up to kInlineRanks ranks pass their rank tables to the kernels as
+// A step's rank tables reach the kernels in one of two ways.  Worlds of up to kInlineRanks ranks pass them as
 // kernel arguments (9 KiB for dispatch, 5 KiB for combine; HIP on gfx950 takes kernel
-// arguments well beyond 4 KiB, eagerly and as graph nodes); larger worlds go through the
-// HBM tables (drank / crank), written by bind kernels that take up to kBindBatch rows as
-// arguments each.
+// arguments well beyond 4 KiB, eagerly and as graph nodes).  Larger worlds (drank / crank), and steps that were bound
+// beforehand (pplx_a2a_bound_create), go through tables in HBM, written by bind kernels that take up to kBindBatch rows as
+// arguments each.  Kernels read those faster than their arguments, which no cache holds from one launch to the next.  Us,
+// tables in the arguments / in HBM, dispatch and combine of one buffer set: 1 rank, 32 tokens of 2 KiB 3.77 / 3.50 and
+// 3.27 / 2.87; 64 x 1 DSv3 tokens 5.53 / 5.26 and 4.01 / 3.58; 8 x 128 12.69 / 12.51 and 22.12 / 21.90.
 constexpr uint32_t kInlineRanks = 64;
 constexpr uint32_t kBindBatch = 64;
 // A one-launch dispatch whose rows (all picks of all tokens) stay within this many bytes and go through registers
@@ -239,9 +241,9 @@ struct BindCombineBatch {
 // Launchers implemented in a2a_dispatch.hip, a2a_combine.hip and a2a_split.hip; they return a
 // hipError_t as int.
 // `inline_rows` (world_size rows, host memory) selects the inline-table kernels;
-// NULL selects the HBM tables, which must have been bound.
-int launch_bind_dispatch(const WorldDev &w, const BindDispatchBatch &b, void *stream);
-int launch_bind_combine(const WorldDev &w, const BindCombineBatch &b, void *stream);
+// NULL selects the HBM tables (w.drank / w.crank), which must have been bound.
+int launch_bind_dispatch(DispatchRank *table, const BindDispatchBatch &b, void *stream);
+int launch_bind_combine(CombineRank *table, const BindCombineBatch &b, void *stream);
 // pick_vector: how many expert ids one load may fetch from any rank's indices (4, 2 or 1):
 // K must be a multiple of it and every indices pointer aligned to 4 * pick_vector bytes.
 int launch_dispatch(const WorldDev &w, const DispatchRank *inline_rows, uint32_t pick_vector,

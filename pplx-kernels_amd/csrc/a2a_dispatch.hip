@@ -29,7 +29,7 @@
 //
 // Rank tables reach the kernels either inline, as kernel arguments (worlds of
 // up to kInlineRanks ranks: nothing to bind, nothing to go stale), or through
-// the HBM tables written by bind_rows.
+// HBM tables written by bind_rows (larger worlds, and steps bound beforehand).
 #include "a2a_route.h"
 #include "a2a_rows.h"
 
@@ -291,7 +291,7 @@ __device__ __forceinline__ void count_earlier_picks(const WorldDev &w, const Tab
 // Small steps: one launch does routing and scatter.  A workgroup owns tokens_per_block
 // consecutive virtual tokens; each of them belongs to one wave (or to ksplit waves that share
 // its picks), and lane k of such a row wave is the token's pick k.
-//   0. the rank table (world_size rows of it) is copied from the kernel arguments into LDS with
+//   0. the rank table (world_size rows of it) is copied from the kernel arguments, or from HBM, into LDS with
 //      loads that depend on nothing, so every later lookup is an LDS read and not another trip
 //      to memory behind the one that fetches the geometry;
 //   1. one batch of small loads: every thread fetches the picks of one token before the
@@ -321,12 +321,11 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   extern __shared__ unsigned long long lds_u64[];
   Timeline timeline;
   timeline.mark(0);
-  constexpr bool kStaged = DT::kInline;
   constexpr uint32_t kRowWords = sizeof(DispatchRank) / 8;
-  const uint32_t table_words = kStaged ? w.R * kRowWords : 0;
-  if constexpr (kStaged) {
-    const unsigned long long *args = reinterpret_cast<const unsigned long long *>(&tab);
-    for (uint32_t i = threadIdx.x; i < table_words; i += kFusedThreads) lds_u64[i] = args[i];
+  const uint32_t table_words = w.R * kRowWords;
+  {
+    const unsigned long long *table = reinterpret_cast<const unsigned long long *>(&tab.at(0));
+    for (uint32_t i = threadIdx.x; i < table_words; i += kFusedThreads) lds_u64[i] = table[i];
   }
   uint32_t *hist = reinterpret_cast<uint32_t *>(lds_u64 + table_words);  // [E] tokens before the workgroup's own
   uint32_t *own_mask = hist + w.E;                                       // [E] bit j: own token j goes to e
@@ -336,10 +335,7 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   // Orders the zeroing (and the staged table) before the first counter update of any wave.
   __syncthreads();
   timeline.mark(1);
-  const LdsDispatch staged{reinterpret_cast<const DispatchRank *>(lds_u64)};
-  auto rows = [&]() -> decltype(auto) {
-    if constexpr (kStaged) return (staged); else return (tab);
-  };
+  const LdsDispatch rows{reinterpret_cast<const DispatchRank *>(lds_u64)};
 
   const uint32_t total = w.G * w.M;
   const uint32_t v0 = blockIdx.x * tokens_per_block;
@@ -353,8 +349,8 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   const bool my_in_range = my_j < tokens_per_block && my_v < total;
   const uint32_t my_g = my_in_range ? group_of(w, my_v) : 0;
   const uint32_t my_t = my_in_range ? my_v - my_g * w.M : 0;
-  const DispatchRank &my_head = rows().at(my_g * w.dp);
-  const DispatchRank &my_src = w.dp == 1 ? my_head : rows().at(sender_of(w, my_g, my_t));
+  const DispatchRank &my_head = rows.at(my_g * w.dp);
+  const DispatchRank &my_src = w.dp == 1 ? my_head : rows.at(sender_of(w, my_g, my_t));
   const bool my_row_exists = my_in_range && my_t < my_src.m && my_t < my_head.m;
   const bool my_bounded = my_row_exists && my_head.bound_m != nullptr;
   const uint32_t my_loaded_n = *as_global(my_bounded ? my_head.bound_m : w.faults);
@@ -363,18 +359,18 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
 
   // 2. picks of all earlier tokens
   if constexpr (MANY) {
-    if (pick_vector > 1) count_earlier_picks<2, 16, false, kFusedThreads>(w, rows(), v0, hist);
-    else count_earlier_picks<1, 16, false, kFusedThreads>(w, rows(), v0, hist);
+    if (pick_vector > 1) count_earlier_picks<2, 16, false, kFusedThreads>(w, rows, v0, hist);
+    else count_earlier_picks<1, 16, false, kFusedThreads>(w, rows, v0, hist);
   } else if (w.K > 4) {
-    if (pick_vector == 4) count_earlier_picks<4, 8, true, kFusedThreads>(w, rows(), v0, hist);
-    else if (pick_vector == 2) count_earlier_picks<2, 8, false, kFusedThreads>(w, rows(), v0, hist);
-    else count_earlier_picks<1, 8, false, kFusedThreads>(w, rows(), v0, hist);
+    if (pick_vector == 4) count_earlier_picks<4, 8, true, kFusedThreads>(w, rows, v0, hist);
+    else if (pick_vector == 2) count_earlier_picks<2, 8, false, kFusedThreads>(w, rows, v0, hist);
+    else count_earlier_picks<1, 8, false, kFusedThreads>(w, rows, v0, hist);
   } else if (w.K > 2) {
-    if (pick_vector == 4) count_earlier_picks<4, 4, true, kFusedThreads>(w, rows(), v0, hist);
-    else count_earlier_picks<1, 4, false, kFusedThreads>(w, rows(), v0, hist);
+    if (pick_vector == 4) count_earlier_picks<4, 4, true, kFusedThreads>(w, rows, v0, hist);
+    else count_earlier_picks<1, 4, false, kFusedThreads>(w, rows, v0, hist);
   } else {
-    if (pick_vector == 2) count_earlier_picks<2, 2, true, kFusedThreads>(w, rows(), v0, hist);
-    else count_earlier_picks<1, 2, false, kFusedThreads>(w, rows(), v0, hist);
+    if (pick_vector == 2) count_earlier_picks<2, 2, true, kFusedThreads>(w, rows, v0, hist);
+    else count_earlier_picks<1, 2, false, kFusedThreads>(w, rows, v0, hist);
   }
   timeline.mark(2);
   // ... and the workgroup's own: a pick that names no expert, or repeats an earlier pick of its
@@ -413,7 +409,7 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   Destination dst;
   if (my_in_range && lane < w.K) {
     const size_t pair = (size_t)my_v * w.K + lane;
-    if (my_live) dst = destination_of(w, expert_buffer(w, rows(), my_e), my_slot, my_part == 0);
+    if (my_live) dst = destination_of(w, expert_buffer(w, rows, my_e), my_slot, my_part == 0);
     if (my_live && my_part == 0) {
       as_global(w.slot_map)[pair] = my_slot;
       if (my_e >= w.E) {
@@ -426,7 +422,7 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   if (blockIdx.x == gridDim.x - 1) {
     for (uint32_t e = threadIdx.x; e < w.E; e += kFusedThreads) {
       const uint32_t rows_of_e = hist[e] + __popc(own_mask[e]);
-      const DispatchRank &owner = rows().at(owner_of(w, e));
+      const DispatchRank &owner = rows.at(owner_of(w, e));
       as_global(owner.out_num_tokens)[(int64_t)local_of(w, e) * owner.out_num_tokens_stride] = (int32_t)rows_of_e;
     }
   }
@@ -457,7 +453,7 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
   // A bound_m beyond the limit is reported once, behind the stores (it costs a trip to memory).
   if (blockIdx.x == 0) {
     for (uint32_t g = threadIdx.x; g < w.G; g += kFusedThreads) {
-      if (dispatch_group_overflows(w, rows(), g)) atomicOr(w.faults, kFaultTooManyTokens);
+      if (dispatch_group_overflows(w, rows, g)) atomicOr(w.faults, kFaultTooManyTokens);
     }
   }
 }
@@ -519,11 +515,9 @@ __global__ __launch_bounds__(256) void dispatch_scatter_long(WorldDev w, DT tab)
   }
 }
 
-// LDS of a dispatch_fused workgroup: the rank table (when it came inline), the histogram and
-// the mask of the workgroup's own tokens.
-uint32_t fused_lds_bytes(const WorldDev &w, bool inline_table) {
-  const uint32_t table = inline_table ? w.R * (uint32_t)sizeof(DispatchRank) : 0u;
-  return (table + 2u * w.E * (uint32_t)sizeof(uint32_t) + 15u) & ~15u;
+// LDS of a dispatch_fused workgroup: the rank table, the histogram and the mask of the workgroup's own tokens.
+uint32_t fused_lds_bytes(const WorldDev &w) {
+  return (w.R * (uint32_t)sizeof(DispatchRank) + 2u * w.E * (uint32_t)sizeof(uint32_t) + 15u) & ~15u;
 }
 // Tokens of a dispatch_fused workgroup: as few as still give every CU a workgroup (all of a workgroup's
 // waves help with the counting; only the waves that own a token, or a share of one, load and store
@@ -753,7 +747,7 @@ int launch_fused_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hipSt
   while (ksplit * 2 <= w.K && tokens_per_block * ksplit * 2 <= kWaves && (uint64_t)tokens * ksplit < spread_below) ksplit *= 2;
   const uint32_t kper = (w.K + ksplit - 1) / ksplit;
   const dim3 grid((tokens + tokens_per_block - 1) / tokens_per_block), block(kWaves * kWave);
-  const uint32_t lds = fused_lds_bytes(w, DT::kInline && w.R <= kInlineRanks) + (staged ? tokens_per_block * w.Hb : 0u);
+  const uint32_t lds = fused_lds_bytes(w) + (staged ? tokens_per_block * w.Hb : 0u);
   // Rows that fit the last-level cache with room to spare are written through into it.
   const uint64_t row_bytes = (uint64_t)tokens * w.K * (w.Hb + 4ull * w.S);
   const uint32_t write_through = row_bytes <= (staged ? kLdsWriteThroughMaxBytes : kWriteThroughMaxBytes) ? 1u : 0u;
@@ -814,7 +808,7 @@ uint32_t route_lds_bytes(uint32_t num_experts, uint32_t tile_chunks) {
 }
 
 bool dispatch_is_fused(const WorldDev &w) {
-  if (fused_lds_bytes(w, true) > 60 * 1024) return false;
+  if (fused_lds_bytes(w) > 60 * 1024) return false;
   const bool in_lds = fused_rows_in_lds(w);
   if (in_lds && w.Hb > 16 * 1024) return false;
   // One launch while a workgroup per CU can own all tokens, one wave each: 4096 tokens, or 2048 of
@@ -862,7 +856,7 @@ bool dispatch_is_fused(const WorldDev &w) {
     const uint64_t limit = row_cuts_half_lines(w) ? 180ull << 20 : 128ull << 20;
     // (a device that does not say how much LDS it has is taken to have the 64 KiB of any)
     const uint32_t lds = w.lds_per_cu ? w.lds_per_cu : 64u << 10;
-    return fused_lds_bytes(w, true) + rows <= lds && stored <= limit;
+    return fused_lds_bytes(w) + rows <= lds && stored <= limit;
   }
   if (waves < 16) return true;
   const bool quick_count = w.K % 4 == 0 && w.K <= 8;
@@ -891,15 +885,15 @@ DispatchPlan dispatch_plan(const WorldDev &w) {
   return {form, waves, plan.in_turn && slots != Slots::kMap, scatter_rows_in_lds(w)};
 }
 
-int launch_bind_dispatch(const WorldDev &w, const BindDispatchBatch &b, void *stream) {
+int launch_bind_dispatch(DispatchRank *table, const BindDispatchBatch &b, void *stream) {
   hipLaunchKernelGGL((bind_rows<BindDispatchBatch, DispatchRank>), dim3(1), dim3(256), 0,
-                     (hipStream_t)stream, w.drank, b);
+                     (hipStream_t)stream, table, b);
   return (int)hipGetLastError();
 }
 
-int launch_bind_combine(const WorldDev &w, const BindCombineBatch &b, void *stream) {
+int launch_bind_combine(CombineRank *table, const BindCombineBatch &b, void *stream) {
   hipLaunchKernelGGL((bind_rows<BindCombineBatch, CombineRank>), dim3(1), dim3(256), 0,
-                     (hipStream_t)stream, w.crank, b);
+                     (hipStream_t)stream, table, b);
   return (int)hipGetLastError();
 }
 

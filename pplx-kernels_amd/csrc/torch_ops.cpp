@@ -771,6 +771,58 @@ PyObject *py_world_ptr(PyObject *, PyObject *arg) {
   END_HANDLE_TH_ERRORS
 }
 
+// A bound step with its rank tables in device memory (bind_step).
+void free_plan(PyObject *capsule) {
+  (void)pplx_a2a_bound_destroy(static_cast<pplx_a2a_bound_t *>(PyCapsule_GetPointer(capsule, "pplx_kernels.plan")));
+}
+
+// plan_bytes(world) -> device memory that a bound step's rank tables take
+PyObject *py_plan_bytes(PyObject *, PyObject *arg) {
+  HANDLE_TH_ERRORS
+  uint64_t bytes = 0;
+  A2A_CHECK(pplx_a2a_bound_bytes(world_arg(arg)->ptr, &bytes));
+  return PyLong_FromUnsignedLongLong(bytes);
+  END_HANDLE_TH_ERRORS
+}
+
+// bind_step(world, dispatch_arguments, combine_arguments, device_memory, stream) -> a plan for launch_plan, or None
+// where the arguments are not those of a step that can be launched (its launch says why)
+PyObject *py_bind_step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  arity("bind_step", nargs, 5);
+  const std::shared_ptr<World> world = world_arg(args[0]);
+  const void *dispatch = reinterpret_cast<const void *>((uintptr_t)int_arg(args[1], "dispatch_arguments"));
+  const void *combine = reinterpret_cast<const void *>((uintptr_t)int_arg(args[2], "combine_arguments"));
+  void *memory = reinterpret_cast<void *>((uintptr_t)int_arg(args[3], "device_memory"));
+  void *stream = reinterpret_cast<void *>((uintptr_t)int_arg(args[4], "stream"));
+  pplx_a2a_bound_t *bound = nullptr;
+  const int st = without_gil([&] {
+    return pplx_a2a_bound_create(world->ptr, static_cast<const pplx_a2a_dispatch_args_t *>(dispatch),
+                                 static_cast<const pplx_a2a_combine_args_t *>(combine), memory, stream, &bound);
+  });
+  if (st != PPLX_A2A_OK) Py_RETURN_NONE;
+  PyObject *capsule = PyCapsule_New(bound, "pplx_kernels.plan", free_plan);
+  if (!capsule) (void)pplx_a2a_bound_destroy(bound);
+  return capsule;
+  END_HANDLE_TH_ERRORS
+}
+
+// launch_plan(op, world, plan, device, stream): launch_bound for a step of bind_step
+PyObject *py_launch_plan(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  arity("launch_plan", nargs, 5);
+  const int op = (int)int_arg(args[0], "op");
+  const std::shared_ptr<World> world = world_arg(args[1]);
+  const auto *bound = static_cast<const pplx_a2a_bound_t *>(PyCapsule_GetPointer(args[2], "pplx_kernels.plan"));
+  if (!bound) return nullptr;
+  void *stream = args[4] == Py_None
+                     ? (void *)c10::hip::getCurrentHIPStream((c10::DeviceIndex)int_arg(args[3], "device")).stream()
+                     : reinterpret_cast<void *>((uintptr_t)int_arg(args[4], "stream"));
+  A2A_CHECK(without_gil([&] { return pplx_a2a_bound_launch(world->ptr, bound, op, stream); }));
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
 // world_id(fptr) -> the number of the handle's world, which no other world of the process gets
 PyObject *py_world_id(PyObject *, PyObject *arg) {
   HANDLE_TH_ERRORS
@@ -844,6 +896,11 @@ PyMethodDef kMethods[] = {
     {"launch_bound", (PyCFunction)(void (*)(void))py_launch_bound, METH_FASTCALL,
      "launch_bound(op, world, arguments, device, stream): dispatch (0) or combine (1) of packed arguments on "
      "the stream with this handle, or the device's current one"},
+    {"plan_bytes", py_plan_bytes, METH_O, "plan_bytes(world) -> device memory that bind_step needs"},
+    {"bind_step", (PyCFunction)(void (*)(void))py_bind_step, METH_FASTCALL,
+     "bind_step(world, dispatch_arguments, combine_arguments, device_memory, stream) -> plan for launch_plan, or None"},
+    {"launch_plan", (PyCFunction)(void (*)(void))py_launch_plan, METH_FASTCALL,
+     "launch_plan(op, world, plan, device, stream): dispatch (0) or combine (1) of a step of bind_step"},
     {"world_faults", (PyCFunction)(void (*)(void))py_world_faults, METH_FASTCALL,
      "world_faults(world, stream) -> sticky fault bits since the last call"},
     {"destroy_all", py_destroy_all, METH_NOARGS, "releases every rank handle and world"},

@@ -25,6 +25,7 @@ from . import ops
 from .all_to_all import AllToAll
 
 _launch_bound = ops._C.launch_bound
+_launch_plan = ops._C.launch_plan
 
 
 class Graph:
@@ -61,14 +62,33 @@ class BoundStep:
     def __init__(self, world: "LoopbackWorld", dispatch_args, combine_args, device, keep: tuple) -> None:
         # (what the launches read: packed for this world, which is named by a number of its own)
         self._keep = (dispatch_args, combine_args, keep)
-        self._launch_dispatch = (0, world._world_id, ctypes.addressof(dispatch_args), device.index)
-        self._launch_combine = (1, world._world_id, ctypes.addressof(combine_args), device.index)
+        packed = ctypes.addressof(dispatch_args), ctypes.addressof(combine_args)
+        # The kernels of launches on this stream read the rank tables from device memory, which the allocator gives out
+        # again, to this stream, once the step is gone; launches on others, or under capture, carry the tables along.
+        plan = None
+        if device.type == "cuda" and not torch.cuda.is_current_stream_capturing():
+            try:
+                self._tables = torch.empty(ops._C.plan_bytes(world._world_id), dtype=torch.uint8, device=device)
+            except torch.OutOfMemoryError:
+                self._tables = None
+            if self._tables is not None:
+                plan = ops._C.bind_step(
+                    world._world_id, *packed, self._tables.data_ptr(), torch.cuda.current_stream(device).cuda_stream
+                )
+        if plan is not None:
+            self._launch = _launch_plan
+            self._launch_dispatch = (0, world._world_id, plan, device.index)
+            self._launch_combine = (1, world._world_id, plan, device.index)
+        else:
+            self._launch = _launch_bound
+            self._launch_dispatch = (0, world._world_id, packed[0], device.index)
+            self._launch_combine = (1, world._world_id, packed[1], device.index)
 
     def dispatch(self, stream: torch.cuda.Stream | None = None) -> None:
-        _launch_bound(*self._launch_dispatch, None if stream is None else stream.cuda_stream)
+        self._launch(*self._launch_dispatch, None if stream is None else stream.cuda_stream)
 
     def combine(self, stream: torch.cuda.Stream | None = None) -> None:
-        _launch_bound(*self._launch_combine, None if stream is None else stream.cuda_stream)
+        self._launch(*self._launch_combine, None if stream is None else stream.cuda_stream)
 
 
 class LoopbackWorld:

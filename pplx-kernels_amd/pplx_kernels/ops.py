@@ -9,7 +9,7 @@ Two shared objects sit next to this file (built by ``make -C pplx-kernels_amd/cs
   reference's loader does with ``torch.ops.load_library`` (``src/pplx_kernels/ops.py:8-16``);
   its module functions ``_C.dispatch`` / ``_C.combine`` are the same code without the op
   dispatcher, which ``AllToAll`` uses for eager calls, and ``_C.world_dispatch`` /
-  ``_C.world_combine`` / ``_C.launch_bound`` take a step of all ranks for ``LoopbackWorld``.
+  ``_C.world_combine`` / ``_C.launch_bound`` / ``_C.launch_plan`` take a step of all ranks for ``LoopbackWorld``.
 * ``libpplx_kernels.so`` -- the C ABI of ``include/pplx_a2a.h`` (kernels + host layer, no
   torch types), which ``_C.so`` links against and which ``LoopbackWorld`` (graphs, faults, arguments packed
   once) and the tests also reach through ``ctypes``.
@@ -56,6 +56,10 @@ EXPORTED_SYMBOLS = (
     "pplx_a2a_static_step",
     "pplx_a2a_plan",
     "pplx_a2a_plan_on",
+    "pplx_a2a_bound_bytes",
+    "pplx_a2a_bound_create",
+    "pplx_a2a_bound_launch",
+    "pplx_a2a_bound_destroy",
     "pplx_a2a_world_recorded_calls",
     "pplx_a2a_world_abandon_step",
     "pplx_a2a_world_reserve_split",

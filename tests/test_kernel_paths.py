@@ -538,3 +538,82 @@ def test_long_pieces_of_few_picks(K, H, M, y_dtype, dp):
     check_combine_against_oracle(step, expected.slot_map)
     assert world.faults() == 0
     world.destroy()
+
+
+# ---------------------------------------------------------------------------
+# Bound steps: rank tables in device memory on the stream that bound them, with the launch elsewhere
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize(
+    "R,L,M,row_bytes,K",
+    [
+        (1, 8, 5, 1024, 2),  # one launch
+        (8, 4, 90, 5264, 4),  # ... rows in LDS
+        (64, 1, 3, 2048, 8),  # the most ranks whose tables fit the arguments
+        (72, 1, 3, 1040, 3),  # ... and beyond
+        (8, 1, 900, 2064, 3),  # routing and scatter
+        (2, 8, 300, 16400, 2),  # ... with the slots in a launch of their own
+    ],
+)
+def test_bound_step_on_its_stream_on_another_and_in_a_graph(R, L, M, row_bytes, K):
+    spec = WorkloadSpec("bound", 82, R, R * L, K, row_bytes // 2, M, torch.bfloat16, tokens="uniform")
+    step = DeviceStep(spec, generate(spec, seed=1), cap=R * M)
+    world = make_world(spec, group_name="bound")
+    step.expert_y_all.normal_(generator=torch.Generator(device="cuda").manual_seed(11))
+    stream, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        bound = step.bind_world(world)
+        bound.dispatch()
+        bound.combine()
+        stream.synchronize()
+        with world.capture() as cap:
+            bound.dispatch()
+            bound.combine()
+
+    def check(seed, launch):
+        new = generate(spec, seed=seed)
+        new[-1].n = 0
+        for r, g in enumerate(new):
+            step.dp_x[r].copy_(g.x)
+            step.indices[r].copy_(g.indices.to(torch.uint32))
+            step.weights[r].copy_(g.weights)
+            step.bound_m[r].copy_(torch.tensor([g.n], dtype=torch.uint32))
+            step.out_tokens[r].fill_(float("nan"))
+        step.groups = new
+        torch.cuda.synchronize()
+        launch()
+        torch.cuda.synchronize()
+        expected = check_dispatch_against_oracle(step)
+        check_combine_against_oracle(step, expected.slot_map)
+
+    def launch_on(s):
+        bound.dispatch(stream=s)
+        bound.combine(stream=s)
+
+    for seed in (2, 3):
+        check(seed, lambda: launch_on(stream))
+        check(seed + 10, lambda: launch_on(other))
+        check(seed + 20, lambda: cap.graph.replay(stream))
+    # the graph outlives the bound step, and what its tables were in
+    del bound, launch_on
+    with torch.cuda.stream(stream):
+        reused = [torch.full((1 << 14,), 0x5A, dtype=torch.uint8, device="cuda") for _ in range(8)]
+    check(30, lambda: cap.graph.replay(stream))
+    assert all((t == 0x5A).all() for t in reused)
+    with torch.cuda.stream(stream):
+        again = step.bind_world(world)
+    check(31, lambda: (again.dispatch(stream), again.combine(stream)))
+    assert world.faults() == 0
+    cap.graph.destroy()
+    world.destroy()
+
+
+def test_bound_step_that_cannot_be_launched_says_so_at_its_launch():
+    spec = WorkloadSpec("bound", 83, 4, 8, 2, 512, 6, torch.bfloat16, dp_size=2, tokens="uniform")
+    step = DeviceStep(spec, generate(spec, seed=1))
+    world = make_world(spec, group_name="bound-bad")
+    step.bound_m[1] = None  # (its group's first rank has one)
+    bound = step.bind_world(world)
+    with pytest.raises(RuntimeError, match="share a DP group"):
+        bound.dispatch()
+    world.destroy()

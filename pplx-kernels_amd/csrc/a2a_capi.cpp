@@ -102,7 +102,7 @@ class DeviceScope {
 struct pplx_a2a_world {
   pplx_a2a_config_t cfg;
   int device = 0;
-  WorldDev dev{};
+  WorldHost dev{};
   std::mutex mu;
   int attached = 0;
 
@@ -209,8 +209,9 @@ uint32_t lds_per_cu_of(int device) {
   return (uint32_t)cached[device];
 }
 
-// The geometry part of a WorldDev (everything but the pointers) for a checked configuration.
-void fill_geometry(const pplx_a2a_config_t &cfg, WorldDev &d) {
+// The geometry part of a WorldHost (everything but the pointers) for a checked configuration.
+void fill_geometry(const pplx_a2a_config_t &cfg, WorldHost &d) {
+  // (check_config: experts up to 5461, no more ranks than experts, 64 picks)
   d.R = cfg.world_size;
   d.dp = cfg.dp_size;
   d.G = d.R / d.dp;
@@ -241,7 +242,7 @@ void fill_geometry(const pplx_a2a_config_t &cfg, WorldDev &d) {
   d.num_tiles = (uint32_t)(((uint64_t)d.G * d.M + tile_tokens - 1) / tile_tokens);
 }
 
-int convert_dispatch(const WorldDev &geo, uint32_t rank, const pplx_a2a_dispatch_args_t &a,
+int convert_dispatch(const WorldHost &geo, uint32_t rank, const pplx_a2a_dispatch_args_t &a,
                      DispatchRank *out) {
   const uint32_t S = geo.S;
   if (!a.out_expert_num_tokens)
@@ -289,7 +290,7 @@ int convert_dispatch(const WorldDev &geo, uint32_t rank, const pplx_a2a_dispatch
 
 size_t dtype_size(int dt) { return dt == PPLX_A2A_F32 ? 4 : 2; }
 
-int convert_combine(const WorldDev &geo, uint32_t rank, const pplx_a2a_combine_args_t &a,
+int convert_combine(const WorldHost &geo, uint32_t rank, const pplx_a2a_combine_args_t &a,
                     CombineRank *out) {
   // csrc/bindings/all_to_all_ops.cpp:265-310
   if (a.in_dtype != PPLX_A2A_F32 && a.in_dtype != PPLX_A2A_BF16 && a.in_dtype != PPLX_A2A_F16)
@@ -392,7 +393,7 @@ uint32_t pick_vector_for(uint32_t K, const uint32_t *indices, uint32_t at_most =
 }
 
 // ... that suits the indices of every rank of the pending step.
-uint32_t pick_vector_of(const WorldDev &d, const DispatchRank *rows) {
+uint32_t pick_vector_of(const WorldHost &d, const DispatchRank *rows) {
   uint32_t pv = 4;
   for (uint32_t r = 0; r < d.R; ++r) pv = pick_vector_for(d.K, rows[r].indices, pv);
   return pv;
@@ -402,7 +403,7 @@ uint32_t pick_vector_of(const pplx_a2a_world &w) { return pick_vector_of(w.dev, 
 // The members of a DP group hold the same tokens (csrc/all_to_all/intranode_dispatch.cu:97
 // strides one token list over them), so they must agree on how many rows there are: the
 // kernels take the count from the group's first member and read every member's rows.
-int check_groups(const WorldDev &d, const DispatchRank *rows) {
+int check_groups(const WorldHost &d, const DispatchRank *rows) {
   const uint32_t dp = d.dp;
   if (dp == 1) return PPLX_A2A_OK;
   for (uint32_t g = 0; g < d.G; ++g) {
@@ -517,7 +518,7 @@ int reserve_split(pplx_a2a_world &w, uint32_t y_elem_bytes) {
     return fail(PPLX_A2A_INVALID_ARGUMENT, "expert_y_elem_bytes must be 0, 2 or 4");
   DeviceScope scope(w.device);
   if (!scope.ok()) return fail(PPLX_A2A_HIP_ERROR, "cannot select device %d", w.device);
-  const WorldDev &d = w.dev;
+  const WorldHost &d = w.dev;
   SplitDev &sp = w.split;
   if (!w.split_ready) {
     if (w.n_arrived_dispatch != 0 || w.n_arrived_combine != 0)
@@ -571,7 +572,7 @@ int run_split_dispatch(pplx_a2a_world &w, int mode, void *stream) {
   int st = capture_session(stream, &session);
   if (st) return st;
   settle_mirror(w, session, w.bind_capture_dispatch, w.bound_dispatch_valid);
-  const WorldDev &d = w.dev;
+  const WorldHost &d = w.dev;
   if (mode == PPLX_A2A_SPLIT_SEND) {
     st = check_groups(d, w.pend_dispatch.data());
     if (st) return st;
@@ -653,7 +654,7 @@ int run_split_combine(pplx_a2a_world &w, int mode, int in_dtype, int out_dtype, 
   int st = capture_session(stream, &session);
   if (st) return st;
   settle_mirror(w, session, w.bind_capture_combine, w.bound_combine_valid);
-  const WorldDev &d = w.dev;
+  const WorldHost &d = w.dev;
   if (mode == PPLX_A2A_SPLIT_SEND) {
     // SEND is the one-call combine with every rank's output rows in the staging area.
     for (uint32_t r = 0; r < d.R; ++r) {
@@ -772,7 +773,7 @@ int pplx_a2a_world_create(const pplx_a2a_config_t *cfg, int device, pplx_a2a_wor
   if (!w) return fail(PPLX_A2A_HIP_ERROR, "out of host memory");
   w->cfg = *cfg;
   w->device = device;
-  WorldDev &d = w->dev;
+  WorldHost &d = w->dev;
   fill_geometry(*cfg, d);
   d.lds_per_cu = lds_per_cu_of(device);
 
@@ -1001,7 +1002,7 @@ int pplx_a2a_bound_create(pplx_a2a_world_t *w, const pplx_a2a_dispatch_args_t *d
   *out = nullptr;
   if (!aligned16(device_memory))
     return fail(PPLX_A2A_INVALID_ARGUMENT, "device_memory must be 16-byte aligned");
-  const WorldDev &d = w->dev;
+  const WorldHost &d = w->dev;
   std::unique_ptr<pplx_a2a_bound> b(new (std::nothrow) pplx_a2a_bound());
   try {
     if (b) {
@@ -1072,7 +1073,7 @@ int pplx_a2a_bound_launch(pplx_a2a_world_t *w, const pplx_a2a_bound_t *b, int op
     return run_combine(*w, stream);
   }
   ProfilerRange range(op == 0 ? "dispatch" : "combine");
-  WorldDev d = w->dev;
+  WorldHost d = w->dev;
   d.drank = b->drank;
   d.crank = b->crank;
   if (op == 0) {
@@ -1158,7 +1159,7 @@ int pplx_a2a_static_step(const pplx_a2a_config_t *cfg, int device,
   if (cfg->world_size > kInlineRanks)
     return fail(PPLX_A2A_UNSUPPORTED, "the static step serves worlds of up to %u ranks, not %u", kInlineRanks,
                 cfg->world_size);
-  WorldDev d{};
+  WorldHost d{};
   fill_geometry(*cfg, d);
   // Scratch layout: the fault word, the slot map (the hand-off from dispatch to combine, kept
   // from one call to the next), the routing tiles' counts and masks.
@@ -1229,7 +1230,7 @@ int pplx_a2a_plan_on(const pplx_a2a_config_t *cfg, int in_dtype, uint32_t lds_pe
                      int32_t *rows_in_lds) {
   if (!cfg || !out) return fail(PPLX_A2A_INVALID_ARGUMENT, "cfg / out is NULL");
   if (int st = check_config(*cfg)) return st;
-  WorldDev d{};
+  WorldHost d{};
   fill_geometry(*cfg, d);
   d.lds_per_cu = lds_per_cu;
   const DispatchPlan dispatch = dispatch_plan(d);

@@ -252,13 +252,13 @@ __global__ __launch_bounds__(kWavesPerBlock * kWave) void combine_gather(WorldDe
 // 3.5 10.3 / 10.7, 19 14.3 / 12.8; 1024-wide f16, top-4: 8 10.2 / 11.1, 14 11.5 / 11.8, 32 14.6 / 13.9; 2880-wide
 // fp32, top-5: 7 11.0 / 11.8, 14 13.9 / 12.6; 64 ranks in groups of four, 10 13.8 / 12.6.
 constexpr uint64_t kGroupGatherMinBytes = 10ull << 20;
-bool combine_per_group(const WorldDev &w, size_t elem_bytes) {
+bool combine_per_group(const WorldHost &w, size_t elem_bytes) {
   return w.dp > 1 && w.dp * w.K <= kWave &&
          (uint64_t)w.R * w.M * w.K * w.H * elem_bytes > kGroupGatherMinBytes;
 }
 
 template <typename T, typename U, class CT, int KB, int VPL>
-int launch_combine_v(const WorldDev &w, const CT &tab, bool grouped, hipStream_t s) {
+int launch_combine_v(const WorldHost &w, const CT &tab, bool grouped, hipStream_t s) {
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
   const uint32_t segments = (nvec_segments + VPL - 1) / VPL;
   const uint64_t waves = (uint64_t)(grouped ? w.G : w.R) * w.M * segments;
@@ -298,7 +298,7 @@ LongPieces long_pieces(uint64_t tokens, uint32_t segments) {
 }
 
 template <typename T, typename U, class CT>
-int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
+int launch_combine_k(const WorldHost &w, const CT &tab, hipStream_t s) {
 #define PPLX_COMBINE(KB, VPL) return launch_combine_v<T, U, CT, KB, VPL>(w, tab, grouped, s)
   const bool grouped = combine_per_group(w, sizeof(T));
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
@@ -406,7 +406,7 @@ int launch_combine_k(const WorldDev &w, const CT &tab, hipStream_t s) {
 }
 
 template <class CT>
-int launch_combine_t(const WorldDev &w, const CT &tab, int in_dtype, int out_dtype, hipStream_t s) {
+int launch_combine_t(const WorldHost &w, const CT &tab, int in_dtype, int out_dtype, hipStream_t s) {
   // dtype codes follow pplx_a2a_dtype: 0 = f32, 1 = bf16, 2 = f16.
   switch (in_dtype * 4 + out_dtype) {
     case 0 * 4 + 1: return launch_combine_k<float, __bf16>(w, tab, s);
@@ -421,11 +421,11 @@ int launch_combine_t(const WorldDev &w, const CT &tab, int in_dtype, int out_dty
 
 }  // namespace
 
-bool combine_gathers_per_group(const WorldDev &w, int in_dtype) {
+bool combine_gathers_per_group(const WorldHost &w, int in_dtype) {
   return combine_per_group(w, in_dtype == 0 ? 4 : 2);
 }
 
-int launch_combine(const WorldDev &w, const CombineRank *inline_rows, int in_dtype, int out_dtype,
+int launch_combine(const WorldHost &w, const CombineRank *inline_rows, int in_dtype, int out_dtype,
                    void *stream) {
   if (inline_rows)
     return launch_combine_t(w, make_inline(w, inline_rows), in_dtype, out_dtype, (hipStream_t)stream);

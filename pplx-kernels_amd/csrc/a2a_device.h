@@ -84,29 +84,37 @@ struct alignas(16) CombineRank {
 };
 static_assert(sizeof(CombineRank) == 80, "CombineRank layout");
 
-// Geometry + scratch of a world; passed to every kernel by value.
+// Geometry + scratch of a world; passed to every kernel by value, and kept short: in some processes a launch with more
+// than 112 bytes of arguments costs the host 3.4 to 4 us instead of 2.6 (9 KiB no more than 1 KiB), and the tables of bound
+// steps, which are in HBM, leave room for this.
 struct WorldDev {
-  uint32_t R;        // simulated ranks
-  uint32_t dp;       // ranks per DP group
-  uint32_t G;        // DP groups = R / dp
   uint32_t M;        // max tokens per DP group
-  uint32_t E;        // experts
-  uint32_t L;        // experts per rank
-  uint32_t K;        // experts per token
   uint32_t H;        // elements per row
   uint32_t Hb;       // bytes per dispatched row
   uint32_t S;        // fp32 scales per row
-  uint32_t tile_chunks;  // 64-token chunks per routing tile of a whole-step dispatch
   uint32_t num_tiles;    // ceil(G * M / (64 * tile_chunks))
-  uint32_t lds_per_cu;   // bytes of LDS a CU has (0 = unknown): caps residency, and rows in LDS have to fit it
+  // (bits of words, which scalar loads fetch, and not shorter integers, which they do not)
+  uint32_t R : 16;   // simulated ranks (no more than experts)
+  uint32_t dp : 16;  // ranks per DP group
+  uint32_t G : 16;   // DP groups = R / dp
+  uint32_t E : 16;   // experts (check_config: up to 5461)
+  uint32_t L : 16;   // experts per rank
+  uint32_t K : 8;    // experts per token (up to 64)
+  uint32_t tile_chunks : 8;  // 64-token chunks per routing tile of a whole-step dispatch (up to 16)
   FastDiv by_M, by_dp, by_L, by_K;  // fast_div(n, by_X) == n / X
-  DispatchRank *drank;   // [R]
-  CombineRank *crank;    // [R]
   uint32_t *tile_cnt;    // tokens routed to each expert inside each tile, and behind them
                          // (route_tables) [num_tiles * tile_chunks][E] 64-bit masks, one bit per
                          // token of a chunk
   uint32_t *slot_map;    // [G * M][K] row of (token, pick) inside its expert
   uint32_t *faults;      // [1] sticky fault bits
+};
+static_assert(sizeof(WorldDev) == 88, "a kernel's arguments beside a table in HBM fit 112 bytes");
+
+// ... and what only the host needs of it.
+struct WorldHost : WorldDev {
+  uint32_t lds_per_cu;   // bytes of LDS a CU has (0 = unknown): caps residency, and rows in LDS have to fit it
+  DispatchRank *drank;   // [R]
+  CombineRank *crank;    // [R]
 };
 
 // The routing scratch of a world is one block: the tiles' counts, the chunks' masks, and for each
@@ -246,19 +254,19 @@ int launch_bind_dispatch(DispatchRank *table, const BindDispatchBatch &b, void *
 int launch_bind_combine(CombineRank *table, const BindCombineBatch &b, void *stream);
 // pick_vector: how many expert ids one load may fetch from any rank's indices (4, 2 or 1):
 // K must be a multiple of it and every indices pointer aligned to 4 * pick_vector bytes.
-int launch_dispatch(const WorldDev &w, const DispatchRank *inline_rows, uint32_t pick_vector,
+int launch_dispatch(const WorldHost &w, const DispatchRank *inline_rows, uint32_t pick_vector,
                     void *stream);
-int launch_combine(const WorldDev &w, const CombineRank *inline_rows, int in_dtype, int out_dtype,
+int launch_combine(const WorldHost &w, const CombineRank *inline_rows, int in_dtype, int out_dtype,
                    void *stream);
 // Split mode's own launches, each for all ranks at once (`inline_rows` as above): dispatch SEND
 // stages the tokens, combine RECV delivers the combined rows (`elem_bytes` of out_tokens).
 // dispatch RECV and combine SEND are launch_dispatch / launch_combine on rows that point into
 // the staging area.
-int launch_split_stage_tokens(const WorldDev &w, const SplitDev &sp, const DispatchRank *inline_rows,
+int launch_split_stage_tokens(const WorldHost &w, const SplitDev &sp, const DispatchRank *inline_rows,
                               void *stream);
-int launch_split_deliver(const WorldDev &w, const SplitDev &sp, const CombineRank *inline_rows, void *stream);
+int launch_split_deliver(const WorldHost &w, const SplitDev &sp, const CombineRank *inline_rows, void *stream);
 // True when dispatch runs as the single fused launch for this geometry.
-bool dispatch_is_fused(const WorldDev &w);
+bool dispatch_is_fused(const WorldHost &w);
 // What launch_dispatch does with this geometry (the values of pplx_a2a_plan_t).
 enum class DispatchForm : uint32_t { kOneLaunch = 0, kSlotMap = 1, kTables = 2, kScannedTables = 3 };
 struct DispatchPlan {
@@ -267,9 +275,9 @@ struct DispatchPlan {
   bool scatter_in_turn;
   bool rows_in_lds;
 };
-DispatchPlan dispatch_plan(const WorldDev &w);
+DispatchPlan dispatch_plan(const WorldHost &w);
 // True when combine gathers the rows of a DP group once for its ranks (in_dtype: pplx_a2a_dtype).
-bool combine_gathers_per_group(const WorldDev &w, int in_dtype);
+bool combine_gathers_per_group(const WorldHost &w, int in_dtype);
 // LDS bytes the routing kernels need for a given geometry.
 uint32_t route_lds_bytes(uint32_t num_experts, uint32_t tile_chunks);
 

@@ -170,6 +170,14 @@ __global__ __launch_bounds__(kWave) void dispatch_scatter_slots(WorldDev w, DT t
 // A compile-time size also keeps the kernel's first loads free of any wait.
 constexpr uint32_t fused_threads(int nv) { return nv > 8 ? 512u : 1024u; }
 
+// How a launch of dispatch_fused goes about its tokens.
+struct FusedShape {
+  uint32_t ksplit : 8, kper : 8;  // waves that share a token's picks, picks of each
+  uint32_t tokens_per_block : 8;
+  uint32_t pick_vector : 4;       // expert ids one load may fetch
+  uint32_t write_through : 1;
+};
+
 // A rank table that dispatch_fused has copied into LDS.
 struct LdsDispatch {
   const DispatchRank *rows;
@@ -314,9 +322,9 @@ __device__ __forceinline__ void count_earlier_picks(const WorldDev &w, const Tab
 // numbers of picks in one kernel / apart, medians of two runs of 360 launches: 512-byte rows, 8 x 128 tokens, top-8 6.28 6.36 /
 // 6.12 6.24, 8 x 512, top-4 7.64 7.72 / 7.44 7.64; 1 KiB rows, 8 x 128, top-8 level at 6.20 - 6.32).
 template <int NV, bool EXACT, class DT, bool MANY>
-__global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, DT tab, uint32_t ksplit,
-                                                                  uint32_t kper, uint32_t tokens_per_block,
-                                                                  uint32_t pick_vector, uint32_t write_through) {
+__global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, DT tab, FusedShape shape) {
+  const uint32_t ksplit = shape.ksplit, kper = shape.kper, tokens_per_block = shape.tokens_per_block;
+  const uint32_t pick_vector = shape.pick_vector, write_through = shape.write_through;
   constexpr uint32_t kFusedThreads = fused_threads(NV);
   extern __shared__ unsigned long long lds_u64[];
   Timeline timeline;
@@ -419,7 +427,7 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
       }
     }
   }
-  if (blockIdx.x == gridDim.x - 1) {
+  if (v0 + tokens_per_block >= total) {  // (and not by gridDim, which is an argument of its own)
     for (uint32_t e = threadIdx.x; e < w.E; e += kFusedThreads) {
       const uint32_t rows_of_e = hist[e] + __popc(own_mask[e]);
       const DispatchRank &owner = rows.at(owner_of(w, e));
@@ -516,7 +524,7 @@ __global__ __launch_bounds__(256) void dispatch_scatter_long(WorldDev w, DT tab)
 }
 
 // LDS of a dispatch_fused workgroup: the rank table, the histogram and the mask of the workgroup's own tokens.
-uint32_t fused_lds_bytes(const WorldDev &w) {
+uint32_t fused_lds_bytes(const WorldHost &w) {
   return (w.R * (uint32_t)sizeof(DispatchRank) + 2u * w.E * (uint32_t)sizeof(uint32_t) + 15u) & ~15u;
 }
 // Tokens of a dispatch_fused workgroup: as few as still give every CU a workgroup (all of a workgroup's
@@ -545,13 +553,13 @@ uint32_t fused_tokens_per_block(uint32_t tokens, uint32_t waves) {
 // (* below 64 MiB these two stay in registers.)  Rows without a register variant took two launches; dispatch, two
 // launches / one: 12016 bytes, top-8 0.7 MiB 8.8 / 6.4, 46 27.6 / 13.5, 93 41.5 / 23.6; 13312 bytes, top-5 32 23.8 / 10.8;
 // 9216 bytes, top-4 18 12.8 / 7.7.
-bool fused_rows_in_lds(const WorldDev &w) {
+bool fused_rows_in_lds(const WorldHost &w) {
   if (!row_has_register_variant(w)) return true;
   if (!row_cuts_half_lines(w)) return false;
   const uint64_t stored = (uint64_t)w.G * w.M * w.K * (w.Hb + 4ull * w.S);
   return w.Hb >= 3072 ? stored > 16ull << 20 : w.Hb >= 2048 && stored > 64ull << 20;
 }
-uint32_t fused_waves(const WorldDev &w) {
+uint32_t fused_waves(const WorldHost &w) {
   const uint32_t per_lane = (w.Hb / 16 + kWave - 1) / kWave;
   return fused_threads(fused_rows_in_lds(w) ? 0 : (int)per_lane) / kWave;
 }
@@ -561,7 +569,7 @@ uint32_t fused_waves(const WorldDev &w) {
 // runs of stores (8 ranks, us in this form at one / two / four waves per token: 14 KiB rows, top-8, 1280 tokens
 // 38.8 / 36.4 / 38.6; 7 KiB rows, top-8, 2048 tokens 29.9 / 29.8 / 35.2; 4 KiB rows, top-8, 3072 tokens
 // 25.1 / 28.3 / 30.6; 8 KiB rows, top-2, 3072 tokens 18.1 / 20.4 / 30.6).
-uint32_t pick_ksplit(const WorldDev &w, uint32_t max_split) {
+uint32_t pick_ksplit(const WorldHost &w, uint32_t max_split) {
   const uint64_t tokens = (uint64_t)w.G * w.M;
   const uint64_t stored = w.K * (w.Hb + 4ull * w.S);
   uint32_t ksplit = 1;
@@ -583,7 +591,7 @@ uint32_t pick_ksplit(const WorldDev &w, uint32_t max_split) {
 // The two are level where the step's rows, read once, come to 2 MiB, or what it stores to 24.  Rows of 96 bytes and
 // less lose (16 bytes 1.03 - 1.44, 48 bytes 1.0 - 1.26, 64 bytes, which cut no line, 1.20 - 1.44, 96 bytes 1.0 - 1.12)
 // except for some steps of 64 picks (80 and 96 bytes 0.85 - 0.91).
-bool scatter_rows_in_lds(const WorldDev &w) {
+bool scatter_rows_in_lds(const WorldHost &w) {
   if (!row_cuts_half_lines(w) || w.Hb < 112) return false;
   const uint64_t read = (uint64_t)w.G * w.M * w.Hb;
   return w.Hb >= 1024 || read >= 2u << 20 || read * w.K >= 24u << 20;
@@ -641,7 +649,7 @@ struct ScatterPlan {
   bool in_turn;
 };
 
-ScatterPlan scatter_plan(const WorldDev &w, uint32_t picks_per_wave) {
+ScatterPlan scatter_plan(const WorldHost &w, uint32_t picks_per_wave) {
   if (w.lds_per_cu == 0) return {0, false};
   const uint64_t tokens = (uint64_t)w.G * w.M;
   const uint64_t row = w.Hb + 4ull * w.S;
@@ -667,16 +675,16 @@ ScatterPlan scatter_plan(const WorldDev &w, uint32_t picks_per_wave) {
 // many fit as the plan wants.  LDS is handed out in blocks of 1280 bytes, 128 to a CU (one-wave workgroups that hold 16384
 // bytes run nine to a CU, with 15360 ten; 12288 and 12800 twelve).
 constexpr uint32_t kLdsBlock = 1280;
-uint32_t scatter_lds(const WorldDev &w, const ScatterPlan &plan) {
+uint32_t scatter_lds(const WorldHost &w, const ScatterPlan &plan) {
   const uint32_t share = plan.waves_per_cu ? w.lds_per_cu / kLdsBlock / plan.waves_per_cu * kLdsBlock : 0;
   return scatter_rows_in_lds(w) && share < w.Hb ? w.Hb : share;
 }
 
 // Rows that dispatch_scatter holds in registers (longer ones stream through dispatch_scatter_long).
-bool scatter_has_register_rows(const WorldDev &w) { return (w.Hb / 16 + kWave - 1) / kWave <= 32; }
+bool scatter_has_register_rows(const WorldHost &w) { return (w.Hb / 16 + kWave - 1) / kWave <= 32; }
 
 template <class DT>
-int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t s) {
+int launch_scatter_t(const WorldHost &w, const DT &tab, Slots slots, hipStream_t s) {
   const uint32_t tokens = w.G * w.M;
   if (!scatter_has_register_rows(w)) {
     hipLaunchKernelGGL(dispatch_scatter_long<DT>, dim3(tokens), dim3(256), 0, s, w, tab);
@@ -734,7 +742,7 @@ int launch_scatter_t(const WorldDev &w, const DT &tab, Slots slots, hipStream_t 
 }
 
 template <class DT>
-int launch_fused_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hipStream_t s) {
+int launch_fused_t(const WorldHost &w, const DT &tab, uint32_t pick_vector, hipStream_t s) {
   const uint32_t tokens = w.G * w.M;
   const uint32_t kWaves = fused_waves(w);
   const uint32_t tokens_per_block = fused_tokens_per_block(tokens, kWaves);
@@ -751,7 +759,8 @@ int launch_fused_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hipSt
   // Rows that fit the last-level cache with room to spare are written through into it.
   const uint64_t row_bytes = (uint64_t)tokens * w.K * (w.Hb + 4ull * w.S);
   const uint32_t write_through = row_bytes <= (staged ? kLdsWriteThroughMaxBytes : kWriteThroughMaxBytes) ? 1u : 0u;
-#define PPLX_ROW_KERNEL_ARGS ksplit, kper, tokens_per_block, pick_vector, write_through
+  const FusedShape shape{ksplit, kper, tokens_per_block, pick_vector, write_through};
+#define PPLX_ROW_KERNEL_ARGS shape
 #define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                                                       \
   do {                                                                                                                   \
     if (w.K > 8)                                                                                                         \
@@ -770,13 +779,13 @@ int launch_fused_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hipSt
 
 // Steps of several tiles leave the last routing launch out (the scatter's waves work their own
 // slots out of the tiles' tables), and the scan too as long as an expert's counts are one line.
-Slots slots_of(const WorldDev &w) {
+Slots slots_of(const WorldHost &w) {
   if (w.num_tiles == 1 || (w.Hb / 16 + kWave - 1) / kWave > 16) return Slots::kMap;
   return w.num_tiles <= kScanFreeTiles ? Slots::kTables : Slots::kScanned;
 }
 
 template <class DT>
-int launch_dispatch_t(const WorldDev &w, const DT &tab, uint32_t pick_vector, hipStream_t s) {
+int launch_dispatch_t(const WorldHost &w, const DT &tab, uint32_t pick_vector, hipStream_t s) {
   if (dispatch_is_fused(w)) return launch_fused_t(w, tab, pick_vector, s);
   RouteSpan span{};
   span.v_begin = 0;
@@ -807,7 +816,7 @@ uint32_t route_lds_bytes(uint32_t num_experts, uint32_t tile_chunks) {
   return tile_chunks * num_experts * (uint32_t)(sizeof(unsigned long long) + sizeof(uint32_t));
 }
 
-bool dispatch_is_fused(const WorldDev &w) {
+bool dispatch_is_fused(const WorldHost &w) {
   if (fused_lds_bytes(w) > 60 * 1024) return false;
   const bool in_lds = fused_rows_in_lds(w);
   if (in_lds && w.Hb > 16 * 1024) return false;
@@ -867,7 +876,7 @@ bool dispatch_is_fused(const WorldDev &w) {
   return stored <= limit;
 }
 
-DispatchPlan dispatch_plan(const WorldDev &w) {
+DispatchPlan dispatch_plan(const WorldHost &w) {
   if (dispatch_is_fused(w)) return {DispatchForm::kOneLaunch, 0, false, fused_rows_in_lds(w)};
   const Slots slots = slots_of(w);
   const DispatchForm form = slots == Slots::kMap      ? DispatchForm::kSlotMap
@@ -897,7 +906,7 @@ int launch_bind_combine(CombineRank *table, const BindCombineBatch &b, void *str
   return (int)hipGetLastError();
 }
 
-int launch_dispatch(const WorldDev &w, const DispatchRank *inline_rows, uint32_t pick_vector, void *stream) {
+int launch_dispatch(const WorldHost &w, const DispatchRank *inline_rows, uint32_t pick_vector, void *stream) {
   if (pick_vector != 4 && pick_vector != 2) pick_vector = 1;
   if (inline_rows) return launch_dispatch_t(w, make_inline(w, inline_rows), pick_vector, (hipStream_t)stream);
   return launch_dispatch_t(w, HbmDispatch{w.drank}, pick_vector, (hipStream_t)stream);

@@ -143,7 +143,7 @@ __global__ __launch_bounds__(256) void split_deliver(WorldDev w, CT tab, SplitDe
 }
 
 template <class DT>
-int launch_split_stage_tokens_t(const WorldDev &w, const SplitDev &sp, const DT &tab, hipStream_t s) {
+int launch_split_stage_tokens_t(const WorldHost &w, const SplitDev &sp, const DT &tab, hipStream_t s) {
   const uint32_t lds = 0;
   const uint32_t tokens = w.G * w.M;
   if (!row_has_register_variant(w)) {
@@ -162,7 +162,7 @@ int launch_split_stage_tokens_t(const WorldDev &w, const SplitDev &sp, const DT 
 }
 
 template <class CT>
-int launch_split_deliver_t(const WorldDev &w, const SplitDev &sp, const CT &tab, hipStream_t s) {
+int launch_split_deliver_t(const WorldHost &w, const SplitDev &sp, const CT &tab, hipStream_t s) {
   const uint32_t nvec = w.H / 8;
   const uint32_t segments = (nvec + 8 * kWave - 1) / (8 * kWave);
   const uint64_t waves = (uint64_t)w.R * w.M * segments;
@@ -173,13 +173,13 @@ int launch_split_deliver_t(const WorldDev &w, const SplitDev &sp, const CT &tab,
 
 }  // namespace
 
-int launch_split_stage_tokens(const WorldDev &w, const SplitDev &sp, const DispatchRank *inline_rows,
+int launch_split_stage_tokens(const WorldHost &w, const SplitDev &sp, const DispatchRank *inline_rows,
                               void *stream) {
   if (inline_rows) return launch_split_stage_tokens_t(w, sp, make_inline(w, inline_rows), (hipStream_t)stream);
   return launch_split_stage_tokens_t(w, sp, HbmDispatch{w.drank}, (hipStream_t)stream);
 }
 
-int launch_split_deliver(const WorldDev &w, const SplitDev &sp, const CombineRank *inline_rows, void *stream) {
+int launch_split_deliver(const WorldHost &w, const SplitDev &sp, const CombineRank *inline_rows, void *stream) {
   if (inline_rows) return launch_split_deliver_t(w, sp, make_inline(w, inline_rows), (hipStream_t)stream);
   return launch_split_deliver_t(w, sp, HbmCombine{w.crank}, (hipStream_t)stream);
 }

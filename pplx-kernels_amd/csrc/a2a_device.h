@@ -46,9 +46,10 @@ inline uint32_t fast_div(uint32_t n, const FastDiv &f) {
   return (t + ((n - t) >> (f.shifts & 1u))) >> (f.shifts >> 8);
 }
 
+// (The buffers of a rank's experts come first, together: every pick of a token looks its expert's up, in three loads out of
+// two lines before, in two out of mostly one now.  Combine with the tables in the arguments, us: 1 rank, 32 tokens 3.30 /
+// 2.93, 4 ranks in groups of two, 20 tokens 3.29 / 3.13.)
 struct alignas(16) DispatchRank {
-  int32_t *out_num_tokens;
-  int64_t out_num_tokens_stride;
   uint8_t *expert_x;
   int64_t x_stride_row;     // bytes
   int64_t x_stride_expert;  // bytes
@@ -56,6 +57,8 @@ struct alignas(16) DispatchRank {
   int64_t xs_stride_elem;   // floats
   int64_t xs_stride_row;
   int64_t xs_stride_expert;
+  uint32_t x_rows;
+  uint32_t m;
   const uint8_t *dp_x;
   int64_t dp_x_stride_row;  // bytes
   const float *dp_xs;
@@ -63,24 +66,24 @@ struct alignas(16) DispatchRank {
   int64_t dp_xs_stride_row;
   const uint32_t *indices;
   const uint32_t *bound_m;
-  uint32_t m;
-  uint32_t x_rows;
+  int32_t *out_num_tokens;
+  int64_t out_num_tokens_stride;
   uint64_t pad_;
 };
 static_assert(sizeof(DispatchRank) == 144, "DispatchRank layout");
 
 struct alignas(16) CombineRank {
-  void *out_tokens;
-  int64_t out_stride_row;   // elements
-  const uint32_t *indices;
-  const float *weights;
-  int64_t w_stride_row;
   const void *expert_y;
   int64_t y_stride_row;     // elements
   int64_t y_stride_expert;
-  const uint32_t *bound_m;
-  uint32_t m;
   uint32_t y_rows;
+  uint32_t m;
+  const uint32_t *bound_m;
+  const uint32_t *indices;
+  const float *weights;
+  int64_t w_stride_row;
+  void *out_tokens;
+  int64_t out_stride_row;   // elements
 };
 static_assert(sizeof(CombineRank) == 80, "CombineRank layout");
 

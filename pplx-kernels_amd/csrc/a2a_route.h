@@ -43,11 +43,11 @@ struct RouteToken {
 template <class DT>
 __device__ __forceinline__ RouteToken route_token(const WorldDev &w, const DT &tab, const RouteSpan &span) {
   RouteToken r;
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = blockIdx.x * span.tile_chunks * kWave + threadIdx.x;
   r.v = span.v_begin + i;
   r.g = group_of(w, r.v);
   r.t = r.v - r.g * w.M;
-  r.in_span = i < span.v_count && r.g < w.G;
+  r.in_span = threadIdx.x < span.tile_chunks * kWave && i < span.v_count && r.g < w.G;
   const DispatchRank &src = tab.at(r.in_span ? sender_of(w, r.g, r.t) : 0);
   r.row_exists = r.in_span && r.t < src.m;
   r.n_group = r.in_span ? dispatch_group_tokens(w, tab, r.g) : 0;
@@ -55,11 +55,18 @@ __device__ __forceinline__ RouteToken route_token(const WorldDev &w, const DT &t
   return r;
 }
 
+// Threads of a routing workgroup: one for each token of the tile, and enough to go over the experts (dispatch, us, one for
+// each token only / at least 256: 8 x 509 DSv3 tokens, tiles of one chunk, 51.1 / 50.4; 8 x 1024 of 2 KiB, top-6, two chunks,
+// 26.7 / 26.3; groups of four, 6002 of 5760 bytes 23.7 / 23.4; sixteen chunks the same).
+__host__ __device__ constexpr uint32_t route_threads(uint32_t tile_chunks) {
+  return tile_chunks * kWave < 256 ? 256 : tile_chunks * kWave;
+}
+
 template <class DT, int PV>
 __global__ __launch_bounds__(1024) void route_count(WorldDev w, DT tab, RouteSpan span) {
   extern __shared__ unsigned long long lds_mask[];
-  const uint32_t chunks = span.tile_chunks;
-  for (uint32_t i = threadIdx.x; i < chunks * w.E; i += blockDim.x) lds_mask[i] = 0ull;
+  const uint32_t chunks = span.tile_chunks, threads = route_threads(chunks);
+  for (uint32_t i = threadIdx.x; i < chunks * w.E; i += threads) lds_mask[i] = 0ull;
   __syncthreads();
 
   const uint32_t lane = threadIdx.x & (kWave - 1);
@@ -78,7 +85,7 @@ __global__ __launch_bounds__(1024) void route_count(WorldDev w, DT tab, RouteSpa
     }).codes;
   }
   __syncthreads();
-  for (uint32_t e = threadIdx.x; e < w.E; e += blockDim.x) {
+  for (uint32_t e = threadIdx.x; e < w.E; e += threads) {
     uint32_t rows = 0;
     for (uint32_t c = 0; c < chunks; ++c) {
       if (span.tile_mask != nullptr) span.chunk_base[((size_t)blockIdx.x * chunks + c) * w.E + e] = (uint16_t)rows;
@@ -92,7 +99,7 @@ __global__ __launch_bounds__(1024) void route_count(WorldDev w, DT tab, RouteSpa
   }
   if (span.tile_mask != nullptr) {
     unsigned long long *keep = span.tile_mask + (size_t)blockIdx.x * chunks * w.E;
-    for (uint32_t i = threadIdx.x; i < chunks * w.E; i += blockDim.x) keep[i] = lds_mask[i];
+    for (uint32_t i = threadIdx.x; i < chunks * w.E; i += threads) keep[i] = lds_mask[i];
     if (codes) atomicOr(w.faults, codes);
     if (tok.in_span && tok.t == 0 && dispatch_group_overflows(w, tab, tok.g)) {
       atomicOr(w.faults, kFaultTooManyTokens);
@@ -222,13 +229,13 @@ __global__ __launch_bounds__(1024) void route_slots(WorldDev w, DT tab, RouteSpa
   // LDS: mask[chunks][E] (one bit per token of the chunk routed to e),
   //      then base[chunks][E] (rows of e taken before the chunk starts).
   extern __shared__ unsigned long long lds_mask[];
-  const uint32_t chunks = span.tile_chunks;
+  const uint32_t chunks = span.tile_chunks, threads = route_threads(chunks);
   uint32_t *lds_base = reinterpret_cast<uint32_t *>(lds_mask + (size_t)chunks * w.E);
 
-  for (uint32_t i = threadIdx.x; i < chunks * w.E; i += blockDim.x) lds_mask[i] = 0ull;
+  for (uint32_t i = threadIdx.x; i < chunks * w.E; i += threads) lds_mask[i] = 0ull;
   {
     const uint32_t *earlier = span.tile_cnt + (size_t)blockIdx.x * w.E;
-    for (uint32_t e = threadIdx.x; e < w.E; e += blockDim.x) lds_base[e] = scanned ? earlier[e] : 0u;
+    for (uint32_t e = threadIdx.x; e < w.E; e += threads) lds_base[e] = scanned ? earlier[e] : 0u;
   }
   __syncthreads();
 
@@ -249,7 +256,7 @@ __global__ __launch_bounds__(1024) void route_slots(WorldDev w, DT tab, RouteSpa
   __syncthreads();
 
   // Per expert: running prefix over chunks, starting from the rows of earlier tiles.
-  for (uint32_t e = threadIdx.x; e < w.E; e += blockDim.x) {
+  for (uint32_t e = threadIdx.x; e < w.E; e += threads) {
     uint32_t running = lds_base[e];
     for (uint32_t c = 0; c < chunks; ++c) {
       lds_base[c * w.E + e] = running;
@@ -282,8 +289,8 @@ __global__ __launch_bounds__(1024) void route_slots(WorldDev w, DT tab, RouteSpa
 
 template <class DT, int PV>
 int launch_route_pv(const WorldDev &w, const DT &tab, const RouteSpan &span, hipStream_t s) {
-  const uint32_t block = span.tile_chunks * kWave;
-  const uint32_t tiles = (span.v_count + block - 1) / block;
+  const uint32_t tile = span.tile_chunks * kWave, block = route_threads(span.tile_chunks);
+  const uint32_t tiles = (span.v_count + tile - 1) / tile;
   const uint32_t lds = route_lds_bytes(w.E, span.tile_chunks);
   if (tiles > 1) {
     hipLaunchKernelGGL((route_count<DT, PV>), dim3(tiles), dim3(block),

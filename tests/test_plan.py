@@ -64,6 +64,22 @@ def test_scatter(tokens, row, scales, topk, waves, in_turn):
 
 
 @pytest.mark.parametrize(
+    "tokens,row,scales,topk,waves",
+    [
+        (8192, 7168, 56, 2, 4),
+        (8200, 7168, 56, 2, 9),
+        (8200, 7168, 0, 2, 4),
+        (8200, 3584, 28, 4, 9),  # shorter rows: nine with and without
+        (8200, 3584, 0, 4, 9),
+        (8200, 7168, 56, 4, 4),  # beyond 24 KiB
+    ],
+)
+def test_scatter_of_rows_with_scales(tokens, row, scales, topk, waves):
+    p = plan(tokens, row, topk, scales=scales)
+    assert (p.dispatch_form, p.scatter_waves_per_cu, bool(p.scatter_in_turn)) == (TABLES, waves, False)
+
+
+@pytest.mark.parametrize(
     "tokens,row,scales,topk,one_launch",
     [
         # a wave per token in a workgroup per CU

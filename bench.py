@@ -209,7 +209,9 @@ def measure_workload(name, spec, steps_k, warmup):
     order = [i % n_sets for i in range(steps_k)]
 
     # 1. eager launches of steps packed once (LoopbackWorld.bind): two library calls per step
-    bound = [st.bind_world(world) for st in steps]
+    # (on the stream of their launches: these read the rank tables from device memory, launches elsewhere carry them)
+    with torch.cuda.stream(stream):
+        bound = [st.bind_world(world) for st in steps]
     bound_us = time_steps(lambda i: (bound[i].dispatch(stream), bound[i].combine(stream)), order, stream, warmup)
     more = [
         time_steps(lambda i: (bound[i].dispatch(stream), bound[i].combine(stream)), order, stream, 0)

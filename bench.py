@@ -568,7 +568,7 @@ def main() -> None:
             del grp
 
     form = (
-        "eager launches of a bound step (LoopbackWorld.bind: pplx_a2a_world_dispatch + _combine on arguments "
+        "eager launches of a bound step (LoopbackWorld.bind: pplx_a2a_bound_launch twice, on arguments "
         "packed once)"
     )
     result = {

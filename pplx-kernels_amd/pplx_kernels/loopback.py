@@ -164,7 +164,8 @@ class LoopbackWorld:
         expert_y: Sequence[torch.Tensor],
     ) -> BoundStep:
         """Checks and packs the arguments of :meth:`dispatch` and :meth:`combine` once and
-        returns a :class:`BoundStep` that launches them as often as wanted."""
+        returns a :class:`BoundStep` that launches them as often as wanted, fastest on the stream
+        that is current now."""
         d_args = (ops.DispatchArgs * self.world_size)()
         c_args = (ops.CombineArgs * self.world_size)()
         for r in range(self.world_size):

@@ -262,8 +262,8 @@ int pplx_a2a_world_abandon_step(pplx_a2a_world_t *world, uint32_t which, uint32_
  * pplx_a2a_world_dispatch and pplx_a2a_world_combine once and enqueues the writing of their rank
  * tables into `device_memory` (pplx_a2a_bound_bytes, 16-byte aligned, the caller's), on `stream`;
  * pplx_a2a_bound_launch then runs dispatch (op 0) or combine (op 1).  On that stream the kernels
- * read the tables from there; on another one, or while the stream is captured, they go with the
- * launch as always (a graph never refers to device_memory).  device_memory is to stay untouched
+ * read the tables from there; on another one, on hipStreamPerThread, or while the stream is captured, they
+ * go with the launch as always (a graph never refers to device_memory).  device_memory is to stay untouched
  * until the last launch on that stream is done with it; the bound step is to be destroyed before
  * its world.  The capture of `stream` refuses pplx_a2a_bound_create. */
 int pplx_a2a_bound_bytes(const pplx_a2a_world_t *world, uint64_t *out);

@@ -1061,8 +1061,8 @@ int pplx_a2a_bound_launch(pplx_a2a_world_t *w, const pplx_a2a_bound_t *b, int op
   const int st = capture_session(stream, &session);
   if (st) return st;
   // The tables in HBM are ordered with their own stream only, and a graph may outlive them: elsewhere they go with
-  // the launch, as those of a step that is not bound.
-  if (stream != b->stream || session != 0) {
+  // the launch, as those of a step that is not bound.  (hipStreamPerThread is another stream in every thread.)
+  if (stream != b->stream || stream == hipStreamPerThread || session != 0) {
     if (op == 0) {
       w->pend_dispatch = b->dispatch;
       return run_dispatch(*w, stream);

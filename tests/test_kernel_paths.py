@@ -608,6 +608,30 @@ def test_bound_step_on_its_stream_on_another_and_in_a_graph(R, L, M, row_bytes, 
     world.destroy()
 
 
+def test_bound_step_on_the_stream_per_thread_takes_its_tables_along():
+    spec = WorkloadSpec("bound", 84, 4, 16, 2, 512, 20, torch.bfloat16, tokens="uniform")
+    groups = generate(spec, seed=1)
+    mine, others = DeviceStep(spec, groups), DeviceStep(spec, groups)
+    world = make_world(spec, group_name="bound-per-thread")
+    bound, other = mine.bind_world(world), others.bind_world(world)
+    packed = [ctypes.addressof(args) for args in bound._keep[:2]]
+    tables = torch.empty_like(bound._tables)
+    torch.cuda.synchronize()
+    per_thread = 2  # hipStreamPerThread: one handle, another stream in every thread
+    plan = ops._C.bind_step(world._world_id, *packed, tables.data_ptr(), per_thread)
+    torch.cuda.synchronize()
+    tables.copy_(other._tables)  # what an unordered launch might see: here the tables of a step on other buffers
+    torch.cuda.synchronize()
+    for op in (0, 1):
+        ops._C.launch_plan(op, world._world_id, plan, 0, per_thread)
+    torch.cuda.synchronize()
+    expected = check_dispatch_against_oracle(mine)
+    check_combine_against_oracle(mine, expected.slot_map)
+    assert world.faults() == 0
+    del plan
+    world.destroy()
+
+
 def test_bound_step_that_cannot_be_launched_says_so_at_its_launch():
     spec = WorkloadSpec("bound", 83, 4, 8, 2, 512, 6, torch.bfloat16, dp_size=2, tokens="uniform")
     step = DeviceStep(spec, generate(spec, seed=1))

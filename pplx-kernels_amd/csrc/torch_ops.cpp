@@ -16,11 +16,14 @@
 #include <Python.h>
 
 #include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/util/Exception.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/disable_torch_function.h>
 #include <torch/library.h>
 
 #include <array>
@@ -776,12 +779,42 @@ void free_plan(PyObject *capsule) {
   (void)pplx_a2a_bound_destroy(static_cast<pplx_a2a_bound_t *>(PyCapsule_GetPointer(capsule, "pplx_kernels.plan")));
 }
 
-// plan_bytes(world) -> device memory that a bound step's rank tables take
-PyObject *py_plan_bytes(PyObject *, PyObject *arg) {
+// What a thread may not do while streams are captured, by it or by others, it may within this scope.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// step_tables(world, device) -> memory for a bound step's rank tables, to be used on the device's current stream, or
+// None where launches on that stream have to carry them: it is captured (what a capture allocates belongs to its
+// graph), or cannot be told to be, or there is no memory.  Memory may come from the device here, which spoils the
+// capture of any other stream unless this thread is exempt from it; torch's allocator sees to that for itself only
+// on the captured stream.
+PyObject *py_step_tables(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
+  arity("step_tables", nargs, 2);
   uint64_t bytes = 0;
-  A2A_CHECK(pplx_a2a_bound_bytes(world_arg(arg)->ptr, &bytes));
-  return PyLong_FromUnsignedLongLong(bytes);
+  A2A_CHECK(pplx_a2a_bound_bytes(world_arg(args[0])->ptr, &bytes));
+  const c10::Device device(c10::kCUDA, (c10::DeviceIndex)int_arg(args[1], "device"));
+  const c10::DeviceGuard guard(device);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c10::hip::getCurrentHIPStream(device.index()).stream(), &capture) != hipSuccess) {
+    (void)hipGetLastError();
+    Py_RETURN_NONE;
+  }
+  if (capture != hipStreamCaptureStatusNone) Py_RETURN_NONE;
+  at::Tensor tables;
+  try {
+    const WithoutGil released;
+    const RelaxedCapture relaxed;
+    // (memory, whatever modes tensors are made under)
+    const torch::DisableTorchDispatch plain;
+    tables = at::empty({(int64_t)bytes}, at::TensorOptions(device).dtype(at::kByte));
+  } catch (const c10::OutOfMemoryError &) {
+    Py_RETURN_NONE;
+  }
+  return THPVariable_Wrap(tables);
   END_HANDLE_TH_ERRORS
 }
 
@@ -896,7 +929,8 @@ PyMethodDef kMethods[] = {
     {"launch_bound", (PyCFunction)(void (*)(void))py_launch_bound, METH_FASTCALL,
      "launch_bound(op, world, arguments, device, stream): dispatch (0) or combine (1) of packed arguments on "
      "the stream with this handle, or the device's current one"},
-    {"plan_bytes", py_plan_bytes, METH_O, "plan_bytes(world) -> device memory that bind_step needs"},
+    {"step_tables", (PyCFunction)(void (*)(void))py_step_tables, METH_FASTCALL,
+     "step_tables(world, device) -> device memory for bind_step on the device's current stream, or None"},
     {"bind_step", (PyCFunction)(void (*)(void))py_bind_step, METH_FASTCALL,
      "bind_step(world, dispatch_arguments, combine_arguments, device_memory, stream) -> plan for launch_plan, or None"},
     {"launch_plan", (PyCFunction)(void (*)(void))py_launch_plan, METH_FASTCALL,

@@ -65,16 +65,13 @@ class BoundStep:
         packed = ctypes.addressof(dispatch_args), ctypes.addressof(combine_args)
         # From the second launch on this stream its kernels read the rank tables from device memory, which the allocator
         # gives out again, to this stream, once the step is gone; launches on others, or under capture, carry the tables along.
-        plan = None
-        if device.type == "cuda" and not torch.cuda.is_current_stream_capturing():
-            try:
-                self._tables = torch.empty(ops._C.plan_bytes(world._world_id), dtype=torch.uint8, device=device)
-            except torch.OutOfMemoryError:
-                self._tables = None
-            if self._tables is not None:
-                plan = ops._C.bind_step(
-                    world._world_id, *packed, self._tables.data_ptr(), torch.cuda.current_stream(device).cuda_stream
-                )
+        self._tables = plan = None
+        if device.type == "cuda":
+            self._tables = ops._C.step_tables(world._world_id, device.index)
+        if self._tables is not None:
+            plan = ops._C.bind_step(
+                world._world_id, *packed, self._tables.data_ptr(), torch.cuda.current_stream(device).cuda_stream
+            )
         if plan is not None:
             self._launch = _launch_plan
             self._launch_dispatch = (0, world._world_id, plan, device.index)

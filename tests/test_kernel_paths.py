@@ -3,6 +3,7 @@ can go wrong, against the CPU oracle."""
 
 from __future__ import annotations
 
+import concurrent.futures
 import ctypes
 import dataclasses
 
@@ -656,6 +657,54 @@ def test_binding_enqueues_nothing_and_a_launch_writes_the_tables(R, written_by):
         check_combine_against_oracle(step, expected.slot_map)
     assert world.faults() == 0
     del plan
+    world.destroy()
+
+
+@pytest.mark.parametrize("which", ["another thread, global", "this thread", "a blocking stream"])
+def test_binding_leaves_captures_alone(which):
+    """Where the memory for the tables has to come from the device, and on a stream that a capture keeps launches from."""
+    spec = WorkloadSpec("bound", 86, 4, 16, 2, 512, 6, torch.bfloat16, tokens="uniform")
+    step = DeviceStep(spec, generate(spec, seed=1))
+    step.expert_y_all.normal_(generator=torch.Generator(device="cuda").manual_seed(13))
+    world = make_world(spec, group_name="bound-capture")
+    captured, fresh = torch.cuda.Stream(), torch.cuda.Stream()
+    counter = torch.zeros(1, device="cuda")
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()  # nothing is left that the new stream could take memory from
+
+    def bind_on(stream):
+        with torch.cuda.stream(stream):
+            return step.bind_world(world)
+
+    if which == "another thread, global":
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=captured, capture_error_mode="global"):
+            counter.add_(1)
+            with concurrent.futures.ThreadPoolExecutor(1) as other:
+                bound = other.submit(bind_on, fresh).result(timeout=60)
+        replay = graph.replay
+    else:
+        lib = ops.load_library()
+        handle = ctypes.c_void_p(captured.cuda_stream)
+        if which == "a blocking stream":  # (torch's are not): the default stream takes no launches meanwhile
+            assert lib.hipStreamCreate(ctypes.byref(handle)) == 0
+        recorded = torch.cuda.ExternalStream(handle.value)
+        with torch.cuda.stream(recorded), world.capture() as cap:
+            counter.add_(1)
+            bound = bind_on(fresh if which == "this thread" else torch.cuda.default_stream())
+        replay = lambda: cap.graph.replay(recorded)  # noqa: E731
+    for launches in range(1, 4):
+        replay()
+        torch.cuda.synchronize()
+        assert counter.item() == launches
+        bound.dispatch(fresh)
+        bound.combine(fresh)
+        torch.cuda.synchronize()
+        expected = check_dispatch_against_oracle(step)
+        check_combine_against_oracle(step, expected.slot_map)
+    assert world.faults() == 0
+    if which != "another thread, global":
+        cap.graph.destroy()
     world.destroy()
 
 

@@ -98,11 +98,16 @@ std::mutex g_live_mu;
 std::unordered_map<uint64_t, std::shared_ptr<World>> g_live;
 uint64_t g_last_id = 0;
 
-std::shared_ptr<World> live_world(uint64_t id) {
+std::shared_ptr<World> live_world_or_null(uint64_t id) {
   std::lock_guard<std::mutex> lock(g_live_mu);
   auto it = g_live.find(id);
-  TORCH_CHECK(it != g_live.end(), "pplx_kernels: invalid state: the world has been destroyed");
-  return it->second;
+  return it == g_live.end() ? nullptr : it->second;
+}
+
+std::shared_ptr<World> live_world(uint64_t id) {
+  std::shared_ptr<World> world = live_world_or_null(id);
+  TORCH_CHECK(world, "pplx_kernels: invalid state: the world has been destroyed");
+  return world;
 }
 
 bool same_config(const pplx_a2a_config_t &a, const pplx_a2a_config_t &b) {
@@ -788,14 +793,16 @@ struct RelaxedCapture {
 
 // step_tables(world, device) -> memory for a bound step's rank tables, to be used on the device's current stream, or
 // None where launches on that stream have to carry them: it is captured (what a capture allocates belongs to its
-// graph), or cannot be told to be, or there is no memory.  Memory may come from the device here, which spoils the
-// capture of any other stream unless this thread is exempt from it; torch's allocator sees to that for itself only
-// on the captured stream.
+// graph), or cannot be told to be, or there is no memory, or no such world any more (the step's launch says so).
+// Memory may come from the device here, which spoils the capture of any other stream unless this thread is exempt
+// from it; torch's allocator sees to that for itself only on the captured stream.
 PyObject *py_step_tables(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   arity("step_tables", nargs, 2);
+  const std::shared_ptr<World> world = live_world_or_null((uint64_t)int_arg(args[0], "world"));
+  if (!world) Py_RETURN_NONE;
   uint64_t bytes = 0;
-  A2A_CHECK(pplx_a2a_bound_bytes(world_arg(args[0])->ptr, &bytes));
+  A2A_CHECK(pplx_a2a_bound_bytes(world->ptr, &bytes));
   const c10::Device device(c10::kCUDA, (c10::DeviceIndex)int_arg(args[1], "device"));
   const c10::DeviceGuard guard(device);
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
@@ -819,7 +826,8 @@ PyObject *py_step_tables(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 }
 
 // bind_step(world, dispatch_arguments, combine_arguments, device_memory, stream) -> a plan for launch_plan, or None
-// where the arguments are not those of a step that can be launched (its launch says why)
+// where the arguments are not those of a step that can be launched (its launch says why).  Host work alone: an error of
+// HIP can only come from the launches, which raise it.
 PyObject *py_bind_step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   arity("bind_step", nargs, 5);

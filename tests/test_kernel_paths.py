@@ -717,3 +717,14 @@ def test_bound_step_that_cannot_be_launched_says_so_at_its_launch():
     with pytest.raises(RuntimeError, match="share a DP group"):
         bound.dispatch()
     world.destroy()
+
+
+def test_binding_for_a_destroyed_world_fails_at_the_launch():
+    spec = WorkloadSpec("bound", 87, 2, 8, 2, 512, 6, torch.bfloat16, tokens="uniform")
+    step = DeviceStep(spec, generate(spec, seed=1))
+    world = make_world(spec, group_name="bound-gone")
+    world.destroy()
+    bound = step.bind_world(world)
+    for launch in (bound.dispatch, bound.combine):
+        with pytest.raises(RuntimeError, match="the world has been destroyed"):
+            launch()

@@ -243,6 +243,15 @@ int pplx_a2a_plan(const pplx_a2a_config_t *cfg, int in_dtype, pplx_a2a_plan_t *o
 int pplx_a2a_plan_on(const pplx_a2a_config_t *cfg, int in_dtype, uint32_t lds_per_cu, pplx_a2a_plan_t *out,
                      int32_t *rows_in_lds);
 
+/* How combine takes a step: `picks` rows of a token at a time, `pieces` times 512 elements of each (1 KiB of
+ * a 16-bit row, 2 KiB of an fp32 one), once for all ranks of a DP group when per_group is 1. */
+typedef struct pplx_a2a_combine_plan {
+  uint32_t picks;
+  uint32_t pieces;
+  int32_t per_group;
+} pplx_a2a_combine_plan_t;
+int pplx_a2a_combine_plan(const pplx_a2a_config_t *cfg, int in_dtype, pplx_a2a_combine_plan_t *out);
+
 /* Parts of a step for pplx_a2a_world_abandon_step. */
 #define PPLX_A2A_ABANDON_DISPATCH 1u
 #define PPLX_A2A_ABANDON_COMBINE 2u

@@ -1240,9 +1240,21 @@ int pplx_a2a_plan_on(const pplx_a2a_config_t *cfg, int in_dtype, uint32_t lds_pe
   plan.routing_tiles = d.num_tiles;
   plan.scatter_waves_per_cu = dispatch.scatter_waves_per_cu;
   plan.scatter_in_turn = dispatch.scatter_in_turn;
-  plan.combine_per_group = combine_gathers_per_group(d, in_dtype);
+  plan.combine_per_group = combine_form(d, in_dtype).per_group;
   *out = plan;
   if (rows_in_lds) *rows_in_lds = dispatch.rows_in_lds;
+  return PPLX_A2A_OK;
+}
+
+int pplx_a2a_combine_plan(const pplx_a2a_config_t *cfg, int in_dtype, pplx_a2a_combine_plan_t *out) {
+  if (!cfg || !out) return fail(PPLX_A2A_INVALID_ARGUMENT, "cfg / out is NULL");
+  if (in_dtype != PPLX_A2A_F32 && in_dtype != PPLX_A2A_BF16 && in_dtype != PPLX_A2A_F16)
+    return fail(PPLX_A2A_UNSUPPORTED, "expert_y must be fp32, bf16 or fp16");
+  if (int st = check_config(*cfg)) return st;
+  WorldHost d{};
+  fill_geometry(*cfg, d);
+  const CombineForm form = combine_form(d, in_dtype);
+  *out = pplx_a2a_combine_plan_t{form.picks, form.pieces, form.per_group};
   return PPLX_A2A_OK;
 }
 

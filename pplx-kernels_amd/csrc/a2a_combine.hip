@@ -297,10 +297,10 @@ LongPieces long_pieces(uint64_t tokens, uint32_t segments) {
   return {per_cu, 4 * workgroups * segments >= 3 * 256 * per_cu * pieces * length};
 }
 
-template <typename T, typename U, class CT>
-int launch_combine_k(const WorldHost &w, const CT &tab, hipStream_t s) {
-#define PPLX_COMBINE(KB, VPL) return launch_combine_v<T, U, CT, KB, VPL>(w, tab, grouped, s)
-  const bool grouped = combine_per_group(w, sizeof(T));
+// The form of combine_gather that a step takes, for rows of `elem_bytes` (2 or 4) an element.
+CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
+  const bool grouped = combine_per_group(w, elem_bytes);
+  auto form = [grouped](uint32_t picks, uint32_t pieces) { return CombineForm{picks, pieces, grouped}; };
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
   const uint64_t tokens = (uint64_t)(grouped ? w.G : w.R) * w.M;
   // Steps of a few hundred to two thousand tokens have all their waves resident at the same moment.  More than four picks in rows
@@ -317,13 +317,13 @@ int launch_combine_k(const WorldHost &w, const CT &tab, hipStream_t s) {
   if (w.K > 4 && middle && nvec_segments >= 7) {
     const LongPieces pieces = long_pieces(tokens, nvec_segments);
     if (pieces.even && (grouped || pieces.per_cu > 1)) {
-      if (nvec_segments % 7 == 0) PPLX_COMBINE(1, 7);
-      PPLX_COMBINE(1, 8);
+      if (nvec_segments % 7 == 0) return form(1, 7);
+      return form(1, 8);
     }
-    if constexpr (sizeof(T) == 2) {
-      if (!grouped) PPLX_COMBINE(3, 1);
-      if (pieces.per_cu == 1) PPLX_COMBINE(2, 2);
-      PPLX_COMBINE(1, 3);
+    if (elem_bytes == 2) {
+      if (!grouped) return form(3, 1);
+      if (pieces.per_cu == 1) return form(2, 2);
+      return form(1, 3);
     }
   }
   // fp32 rows of three KiB of 16-bit outputs and more.  Two picks at a time beside the above (2048 wide, top-8, 464 tokens
@@ -332,22 +332,22 @@ int launch_combine_k(const WorldHost &w, const CT &tab, hipStream_t s) {
   // 3588 180.4 / 173.7; 4096 wide, 7168 221.2 / 215.7; top-6, 7680 wide, 5232 279.4 / 271.2; seven KiB and more also with four
   // picks (6144 wide, 2156 tokens 56.0 / 55.3; 4096 wide, 8 x 1024, combine alone 103.2 / 98.1).  DP groups of that size take three
   // (2048 wide, 2136 tokens 43.1 / 40.5), rows of two KiB three in pieces of both (eight 1.0 to 1.1 of their time).
-  if constexpr (sizeof(T) == 4) {
-    if (w.K > 4 && middle && nvec_segments >= 3) PPLX_COMBINE(2, 1);
+  if (elem_bytes == 4) {
+    if (w.K > 4 && middle && nvec_segments >= 3) return form(2, 1);
     if (tokens > 2048) {
-      if (!grouped && w.K > 3 && nvec_segments >= 7) PPLX_COMBINE(8, 1);
-      if (w.K > 4 && nvec_segments == 2) PPLX_COMBINE(3, 2);
+      if (!grouped && w.K > 3 && nvec_segments >= 7) return form(8, 1);
+      if (w.K > 4 && nvec_segments == 2) return form(3, 2);
       if (w.K > 4 && nvec_segments >= 3) {
-        if (grouped) PPLX_COMBINE(3, 1);
-        PPLX_COMBINE(8, 1);
+        if (grouped) return form(3, 1);
+        return form(8, 1);
       }
     }
   } else if (grouped && nvec_segments > 1) {
     // Steps of DP groups, 16-bit rows, eight picks / three in pieces of 2 KiB: 5120 wide, top-6, 2888 tokens 86.8 / 84.0;
     // 1024 wide, top-8, 12268 88.1 / 87.1 (541 steps: 0.983, 0.90 to 1.05); three and four picks, all at once / two:
     // 1536 wide, top-4, 3260 25.0 / 23.5; 5120 wide, 856 23.5 / 22.9.
-    if (w.K > 4 && tokens > 2048) PPLX_COMBINE(3, 2);
-    if ((w.K == 3 || w.K == 4) && tokens > 600 && nvec_segments > 2) PPLX_COMBINE(2, 2);
+    if (w.K > 4 && tokens > 2048) return form(3, 2);
+    if ((w.K == 3 || w.K == 4) && tokens > 600 && nvec_segments > 2) return form(2, 2);
   }
   // Of what is left, up to five picks are taken all at once, six in two goes of three, nine and ten in two of five, others
   // up to eight at a time.  One or two leave a wave of 1 KiB with little in flight, so they read longer pieces: up to 3
@@ -374,35 +374,60 @@ int launch_combine_k(const WorldHost &w, const CT &tab, hipStream_t s) {
   // DP groups of 16-bit rows.
   switch (w.K) {
     case 1:
-      if (nvec_segments == 1) PPLX_COMBINE(1, 1);
-      if (nvec_segments == 2) PPLX_COMBINE(1, 2);
-      if (!grouped && sizeof(T) == 4) {
-        if (tokens <= 384) PPLX_COMBINE(1, 1);
-        PPLX_COMBINE(1, 2);
+      if (nvec_segments == 1) return form(1, 1);
+      if (nvec_segments == 2) return form(1, 2);
+      if (!grouped && elem_bytes == 4) {
+        if (tokens <= 384) return form(1, 1);
+        return form(1, 2);
       }
-      if (nvec_segments == 4) PPLX_COMBINE(1, 4);
-      if (grouped && nvec_segments > 4 && 8 * ((8 - nvec_segments % 8) % 8) <= 5 * nvec_segments) PPLX_COMBINE(1, 8);
-      if (!grouped && sizeof(T) == 2 && even_pieces(tokens, nvec_segments)) PPLX_COMBINE(1, 8);
-      PPLX_COMBINE(1, 3);
+      if (nvec_segments == 4) return form(1, 4);
+      if (grouped && nvec_segments > 4 && 8 * ((8 - nvec_segments % 8) % 8) <= 5 * nvec_segments) return form(1, 8);
+      if (!grouped && elem_bytes == 2 && even_pieces(tokens, nvec_segments)) return form(1, 8);
+      return form(1, 3);
     case 2:
-      if (nvec_segments == 1 || (sizeof(T) == 4 && (!grouped || tokens <= 384))) PPLX_COMBINE(2, 1);
-      if (grouped && sizeof(T) == 2 && nvec_segments > 2) PPLX_COMBINE(2, 4);
-      PPLX_COMBINE(2, 2);
-    case 3: PPLX_COMBINE(3, 1);
+      if (nvec_segments == 1 || (elem_bytes == 4 && (!grouped || tokens <= 384))) return form(2, 1);
+      if (grouped && elem_bytes == 2 && nvec_segments > 2) return form(2, 4);
+      return form(2, 2);
+    case 3: return form(3, 1);
     case 4:
-      if (sizeof(T) == 2 && nvec_segments > 1 && (grouped || (nvec_segments == 2 && tokens > 600))) PPLX_COMBINE(4, 2);
-      PPLX_COMBINE(4, 1);
-    case 5: PPLX_COMBINE(5, 1);
+      if (elem_bytes == 2 && nvec_segments > 1 && (grouped || (nvec_segments == 2 && tokens > 600))) return form(4, 2);
+      return form(4, 1);
+    case 5: return form(5, 1);
     case 6:
-      if (sizeof(T) == 4 || (!grouped && (nvec_segments < 7 || tokens <= 2048))) PPLX_COMBINE(3, 1);
-      PPLX_COMBINE(8, 1);
+      if (elem_bytes == 4 || (!grouped && (nvec_segments < 7 || tokens <= 2048))) return form(3, 1);
+      return form(8, 1);
     case 9:
     case 10:
-      if (sizeof(T) == 4 || (!grouped && (nvec_segments < 7 || tokens <= 2048))) PPLX_COMBINE(5, 1);
-      PPLX_COMBINE(8, 1);
-    default: PPLX_COMBINE(8, 1);
+      if (elem_bytes == 4 || (!grouped && (nvec_segments < 7 || tokens <= 2048))) return form(5, 1);
+      return form(8, 1);
+    default: return form(8, 1);
   }
+}
+
+template <typename T, typename U, class CT>
+int launch_combine_k(const WorldHost &w, const CT &tab, hipStream_t s) {
+  const CombineForm form = combine_form_of(w, sizeof(T));
+  switch (form.picks * 16 + form.pieces) {
+#define PPLX_COMBINE(KB, VPL) \
+  case KB * 16 + VPL: return launch_combine_v<T, U, CT, KB, VPL>(w, tab, form.per_group, s)
+    PPLX_COMBINE(1, 1);
+    PPLX_COMBINE(1, 2);
+    PPLX_COMBINE(1, 3);
+    PPLX_COMBINE(1, 4);
+    PPLX_COMBINE(1, 7);
+    PPLX_COMBINE(1, 8);
+    PPLX_COMBINE(2, 1);
+    PPLX_COMBINE(2, 2);
+    PPLX_COMBINE(2, 4);
+    PPLX_COMBINE(3, 1);
+    PPLX_COMBINE(3, 2);
+    PPLX_COMBINE(4, 1);
+    PPLX_COMBINE(4, 2);
+    PPLX_COMBINE(5, 1);
+    PPLX_COMBINE(8, 1);
 #undef PPLX_COMBINE
+    default: return (int)hipErrorInvalidValue;
+  }
 }
 
 template <class CT>
@@ -421,9 +446,7 @@ int launch_combine_t(const WorldHost &w, const CT &tab, int in_dtype, int out_dt
 
 }  // namespace
 
-bool combine_gathers_per_group(const WorldHost &w, int in_dtype) {
-  return combine_per_group(w, in_dtype == 0 ? 4 : 2);
-}
+CombineForm combine_form(const WorldHost &w, int in_dtype) { return combine_form_of(w, in_dtype == 0 ? 4 : 2); }
 
 int launch_combine(const WorldHost &w, const CombineRank *inline_rows, int in_dtype, int out_dtype,
                    void *stream) {

@@ -279,8 +279,13 @@ struct DispatchPlan {
   bool rows_in_lds;
 };
 DispatchPlan dispatch_plan(const WorldHost &w);
-// True when combine gathers the rows of a DP group once for its ranks (in_dtype: pplx_a2a_dtype).
-bool combine_gathers_per_group(const WorldHost &w, int in_dtype);
+// What launch_combine does with this geometry (in_dtype: pplx_a2a_dtype): the picks that a wave takes at a time, the
+// pieces of 64 x 8 elements that it reads of each, and whether it gathers once for the ranks of a DP group.
+struct CombineForm {
+  uint32_t picks, pieces;
+  bool per_group;
+};
+CombineForm combine_form(const WorldHost &w, int in_dtype);
 // LDS bytes the routing kernels need for a given geometry.
 uint32_t route_lds_bytes(uint32_t num_experts, uint32_t tile_chunks);
 

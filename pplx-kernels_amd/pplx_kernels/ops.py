@@ -56,6 +56,7 @@ EXPORTED_SYMBOLS = (
     "pplx_a2a_static_step",
     "pplx_a2a_plan",
     "pplx_a2a_plan_on",
+    "pplx_a2a_combine_plan",
     "pplx_a2a_bound_bytes",
     "pplx_a2a_bound_create",
     "pplx_a2a_bound_launch",
@@ -98,6 +99,16 @@ class Plan(ctypes.Structure):
         ("scatter_waves_per_cu", ctypes.c_uint32),
         ("scatter_in_turn", ctypes.c_int32),
         ("combine_per_group", ctypes.c_int32),
+    ]
+
+
+class CombinePlan(ctypes.Structure):
+    """pplx_a2a_combine_plan_t"""
+
+    _fields_ = [
+        ("picks", ctypes.c_uint32),
+        ("pieces", ctypes.c_uint32),
+        ("per_group", ctypes.c_int32),
     ]
 
 
@@ -187,6 +198,7 @@ def load_library() -> ctypes.CDLL:
         lib.pplx_a2a_plan_on.argtypes = [
             ctypes.POINTER(Config), i32, u32, ctypes.POINTER(Plan), ctypes.POINTER(i32),
         ]  # fmt: skip
+        lib.pplx_a2a_combine_plan.argtypes = [ctypes.POINTER(Config), i32, ctypes.POINTER(CombinePlan)]
         lib.pplx_a2a_world_of.argtypes = [vp]
         lib.pplx_a2a_world_of.restype = vp
         lib.pplx_a2a_world_recorded_calls.argtypes = [vp, i32, i32, ctypes.POINTER(u32)]
@@ -223,6 +235,16 @@ def plan_on(config: Config, lds_per_cu: int = 160 << 10, in_dtype: torch.dtype =
         )
     )
     return plan, bool(rows_in_lds.value)
+
+
+def combine_plan_of(config: Config, y_dtype: torch.dtype = torch.bfloat16) -> tuple[int, int, bool]:
+    """How combine takes a step of this geometry with expert outputs of ``y_dtype``: how many picks at a time, how many
+    times 512 elements of each, and whether once for all ranks of a DP group (no GPU needed)."""
+    plan = CombinePlan()
+    check_status(
+        load_library().pplx_a2a_combine_plan(ctypes.byref(config), DTYPE_CODE[y_dtype], ctypes.byref(plan))
+    )
+    return plan.picks, plan.pieces, bool(plan.per_group)
 
 
 def check_status(status: int) -> None:

@@ -125,6 +125,20 @@ def check_dispatch_against_oracle(step: DeviceStep, expected=None):
     return expected
 
 
+def combine_form(spec: WorkloadSpec) -> tuple[int, int, bool]:
+    """The form of the combine kernel that a step of this workload takes: picks at a time, times 512 elements of each,
+    once for all ranks of a DP group."""
+    from pplx_kernels import ops
+
+    return ops.combine_plan_of(
+        ops.Config(
+            spec.max_num_tokens, spec.num_experts, spec.experts_per_token, spec.world_size, spec.dp_size,
+            spec.hidden_dim, spec.hidden_dim_bytes, spec.hidden_dim_scale_bytes,
+        ),
+        spec.expert_y_dtype,
+    )  # fmt: skip
+
+
 COMBINE_RTOL = 1e-2  # bf16 tolerance of the fp32-accumulated reference
 COMBINE_ATOL = 1e-2
 

@@ -29,6 +29,7 @@ from tests.all_to_all_utils import (
     baseline_configs,
     check_combine_against_oracle,
     check_dispatch_against_oracle,
+    combine_form,
     expert_counts,
     generate,
     make_world,
@@ -457,25 +458,31 @@ def test_combine_dtype_matrix(y_dtype, out_dtype):
 
 
 @pytest.mark.parametrize(
-    "hidden,y_dtype,out_dtype",
+    "hidden,tokens,y_dtype,out_dtype,form",
     [
-        (7168, torch.float16, torch.bfloat16),
-        (4096, torch.float32, torch.float16),
-        (3600, torch.bfloat16, torch.bfloat16),  # the last 1 KiB piece of a row is partial
-        (8192 + 512, torch.bfloat16, torch.float16),
+        (7168, 128, torch.float16, torch.bfloat16, (1, 7, False)),
+        (7168, 128, torch.float32, torch.bfloat16, (1, 7, False)),
+        (7160, 128, torch.float32, torch.float16, (1, 7, False)),  # a vector short of the last KiB
+        (4096, 256, torch.float32, torch.float16, (1, 8, False)),
+        (4088, 256, torch.bfloat16, torch.bfloat16, (1, 8, False)),
+        (3600, 256, torch.bfloat16, torch.bfloat16, (1, 8, False)),  # the last 1 KiB piece of a row is partial
+        (7176, 126, torch.bfloat16, torch.float16, (1, 8, False)),  # a second 8 KiB piece, of six KiB and a vector
+        (7176, 126, torch.float32, torch.bfloat16, (1, 8, False)),
+        (8192 + 512, 130, torch.bfloat16, torch.float16, (3, 1, False)),  # the third 8 KiB piece would hold one
     ],
 )
-def test_combine_of_mid_size_steps(hidden, y_dtype, out_dtype):
+def test_combine_of_mid_size_steps(hidden, tokens, y_dtype, out_dtype, form):
     """Steps of a few hundred to two thousand tokens with more than four picks take the combine
-    variant that reads one pick at a time in 7 or 8 KiB pieces."""
+    variant that reads one pick at a time in 7 or 8 KiB pieces where those come out even over the CUs."""
     spec = _small_spec(
-        name=f"mid{hidden}", world_size=4, num_experts=32, experts_per_token=6, max_num_tokens=130,
+        name=f"mid{hidden}", world_size=8, num_experts=32, experts_per_token=6, max_num_tokens=tokens,
         hidden_dim=hidden, expert_y_dtype=y_dtype, out_dtype=out_dtype, tokens="uniform",
     )  # fmt: skip
+    assert combine_form(spec) == form
     groups = generate(spec)
     groups[0].n = spec.max_num_tokens
     groups[1].n = 0
-    run_and_check(spec, groups, use_numpy=True)
+    run_and_check(spec, groups, cap=max(int(expert_counts(groups, spec.num_experts).max()), 1))
 
 
 @pytest.mark.parametrize(

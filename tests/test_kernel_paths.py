@@ -21,6 +21,7 @@ from tests.all_to_all_utils import (
     WorkloadSpec,
     check_combine_against_oracle,
     check_dispatch_against_oracle,
+    combine_form,
     generate,
     make_world,
     to_oracle_groups,
@@ -207,28 +208,29 @@ def test_both_sides_of_the_one_launch_limit(M, topk, hidden, in_dtype, form):
 
 
 # ---------------------------------------------------------------------------
-# Expert outputs in fp32: pieces of 2 KiB (up to 2048 tokens), 4 and 8 KiB of a row
+# Expert outputs in fp32: how many picks at a time, in pieces of 2 and 4 KiB of a row
 # ---------------------------------------------------------------------------
 @pytest.mark.parametrize(
-    "M,K,H,dp,out_dtype",
+    "M,K,H,dp,out_dtype,form",
     [
-        (1024, 5, 2048, 1, torch.bfloat16),  # eight picks at a time still
-        (1025, 3, 2048, 1, torch.bfloat16),  # two picks of 8 KiB, the third by itself
-        (1025, 8, 3592, 1, torch.float16),  # 8 segments, one vector in the last
-        (1025, 5, 2056, 1, torch.bfloat16),  # 5 segments: three picks of 4 KiB, then two
-        (1025, 10, 520, 1, torch.bfloat16),  # one vector beyond a segment; three times three picks, then one
-        (1025, 10, 8, 1, torch.bfloat16),  # one segment, of one vector: eight picks, then two
-        (1025, 5, 512, 1, torch.float16),  # a full segment: four picks, then one
-        (1025, 4, 512, 1, torch.bfloat16),  # three picks, then one
-        (1025, 7, 1536, 2, torch.float16),  # the same for DP groups
-        (1025, 3, 2880, 4, torch.float16),
+        (1024, 5, 2048, 1, torch.bfloat16, (2, 1, False)),  # up to 2048 tokens: two, two and one
+        (1025, 3, 2048, 1, torch.bfloat16, (3, 1, False)),
+        (1025, 8, 3592, 1, torch.float16, (8, 1, False)),  # one vector in the last of eight pieces
+        (1025, 5, 2056, 1, torch.bfloat16, (8, 1, False)),  # five pieces: four picks, then one
+        (1025, 10, 520, 1, torch.bfloat16, (3, 2, False)),  # one vector beyond a piece; three times three picks, then one
+        (1025, 10, 8, 1, torch.bfloat16, (5, 1, False)),  # one piece, of one vector: twice five picks
+        (1025, 5, 512, 1, torch.float16, (5, 1, False)),  # a full piece
+        (1025, 4, 512, 1, torch.bfloat16, (4, 1, False)),
+        (1025, 7, 1536, 2, torch.float16, (3, 1, True)),  # DP groups
+        (1025, 3, 2880, 4, torch.float16, (3, 1, True)),
     ],
 )
-def test_pieces_of_fp32_rows(M, K, H, dp, out_dtype):
+def test_pieces_of_fp32_rows(M, K, H, dp, out_dtype, form):
     spec = WorkloadSpec(
         "pieces", 74, 2 * dp, 8 * dp if dp > 1 else 16, K, H, M, torch.bfloat16, out_dtype=out_dtype,
         expert_y_dtype=torch.float32, dp_size=dp,
     )  # fmt: skip
+    assert combine_form(spec) == form
     groups = generate(spec, seed=H + K)
     groups[0].n, groups[1].n = M, M - 3
     experts = np.concatenate([g.indices[: g.n].reshape(-1).numpy() for g in groups])
@@ -445,25 +447,27 @@ def test_one_launch_with_many_picks_and_rank_tables_in_hbm(row_bytes):
 # ---------------------------------------------------------------------------
 @pytest.mark.parametrize("K", [1, 2, 3, 4, 5, 6])
 @pytest.mark.parametrize(
-    "H,dp,y_dtype,out_dtype",
+    "H,dp,y_dtype,out_dtype,forms",  # picks and pieces of one to six picks
     [
-        (8, 1, torch.bfloat16, torch.bfloat16),  # one vector
-        (512, 1, torch.float16, torch.float16),  # a full segment
-        (520, 1, torch.bfloat16, torch.bfloat16),  # one vector in the second
-        (1032, 1, torch.bfloat16, torch.float16),  # one vector in the third
-        (1536, 2, torch.float16, torch.bfloat16),  # three segments
-        (1544, 1, torch.bfloat16, torch.bfloat16),  # a second piece of one vector
-        (4096, 2, torch.bfloat16, torch.bfloat16),
-        (1032, 1, torch.float32, torch.bfloat16),
-        (504, 4, torch.float32, torch.float16),
+        (8, 1, torch.bfloat16, torch.bfloat16, "11 21 31 41 51 31"),  # one vector
+        (512, 1, torch.float16, torch.float16, "11 21 31 41 51 31"),  # a full segment
+        (520, 1, torch.bfloat16, torch.bfloat16, "12 22 31 42 51 31"),  # one vector in the second
+        (1032, 1, torch.bfloat16, torch.float16, "13 22 31 41 51 31"),  # one vector in the third
+        (1536, 2, torch.float16, torch.bfloat16, "13 22 31 41 51g 81g"),  # three segments; g: once per group
+        (1544, 1, torch.bfloat16, torch.bfloat16, "14 22 31 41 51 31"),  # one vector in the fourth
+        (4096, 2, torch.bfloat16, torch.bfloat16, "13 24g 31g 42g 51g 81g"),
+        (1032, 1, torch.float32, torch.bfloat16, "12 21 31 41 21 21"),
+        (504, 4, torch.float32, torch.float16, "11 21 31 41 51 31"),
     ],
 )
-def test_pieces_of_few_picks(K, H, dp, y_dtype, out_dtype):
+def test_pieces_of_few_picks(K, H, dp, y_dtype, out_dtype, forms):
     M = 90
     spec = WorkloadSpec(
         "few-picks", 78, 8, 16, K, H, M, torch.bfloat16, out_dtype=out_dtype, expert_y_dtype=y_dtype, dp_size=dp,
         tokens="uniform",
     )  # fmt: skip
+    picks, pieces, per_group = combine_form(spec)
+    assert f"{picks}{pieces}{'g' if per_group else ''}" == forms.split()[K - 1]
     groups = generate(spec, seed=H + K)
     groups[0].n, groups[-1].n = M, 1
     step = DeviceStep(spec, groups)
@@ -478,28 +482,29 @@ def test_pieces_of_few_picks(K, H, dp, y_dtype, out_dtype):
 
 
 @pytest.mark.parametrize(
-    "K,H,M,y_dtype,dp",
+    "K,H,M,y_dtype,dp,form",
     [
-        (5, 3592, 48, torch.bfloat16, 1),  # 384 tokens, rows of 8 KiB: eight picks at a time still
-        (5, 3592, 49, torch.bfloat16, 1),  # 392: long pieces would leave most CUs without one, three picks and two
-        (8, 4096, 256, torch.float16, 1),  # 2048: long pieces, two workgroups to a CU
-        (8, 4096, 257, torch.float16, 1),  # 2056: eight at a time again
-        (7, 3080, 140, torch.bfloat16, 1),  # seven KiB, the last a single vector; 1120 tokens
-        (8, 3592, 100, torch.bfloat16, 2),  # DP groups: up to a workgroup of long pieces to a CU two picks of 2 KiB
-        (8, 3592, 300, torch.bfloat16, 2),  # ... one of 3 KiB
-        (8, 520, 600, torch.float16, 2),  # ... large steps, three picks of 2 KiB
-        (4, 1032, 151, torch.bfloat16, 2),  # ... two of four picks
-        (9, 1032, 60, torch.bfloat16, 1),  # five picks, then four
-        (10, 3080, 257, torch.bfloat16, 1),  # eight, then two
-        (5, 1032, 60, torch.float32, 1),  # fp32 rows: two at a time
-        (4, 3080, 257, torch.float32, 1),  # ... four in the form that takes eight
-        (7, 1032, 520, torch.float32, 2),  # ... DP groups, three
+        (5, 3592, 48, torch.bfloat16, 1, (5, 1, False)),  # 384 tokens, rows of 8 KiB
+        (5, 3592, 49, torch.bfloat16, 1, (3, 1, False)),  # 392: long pieces would leave most CUs without one
+        (8, 4096, 256, torch.float16, 1, (1, 8, False)),  # 2048: long pieces, two workgroups to a CU
+        (8, 4096, 257, torch.float16, 1, (8, 1, False)),  # 2056
+        (7, 3080, 140, torch.bfloat16, 1, (3, 1, False)),  # seven KiB, the last a single vector; 1120 tokens
+        (8, 3592, 100, torch.bfloat16, 2, (2, 2, True)),  # DP groups: up to a workgroup of long pieces to a CU
+        (8, 3592, 300, torch.bfloat16, 2, (1, 3, True)),  # ... beyond
+        (8, 520, 600, torch.float16, 2, (3, 2, True)),  # ... large steps
+        (4, 1032, 160, torch.bfloat16, 2, (2, 2, True)),  # ... four picks
+        (9, 1032, 60, torch.bfloat16, 1, (5, 1, False)),  # five picks, then four
+        (10, 3080, 257, torch.bfloat16, 1, (8, 1, False)),  # eight, then two
+        (5, 1032, 60, torch.float32, 1, (2, 1, False)),
+        (4, 3080, 257, torch.float32, 1, (8, 1, False)),  # four picks in the form that takes up to eight
+        (7, 1032, 520, torch.float32, 2, (3, 1, True)),
     ],
 )
-def test_pieces_of_many_picks(K, H, M, y_dtype, dp):
+def test_pieces_of_many_picks(K, H, M, y_dtype, dp, form):
     spec = WorkloadSpec(
         "many-picks", 81, 8, 16, K, H, M, torch.bfloat16, expert_y_dtype=y_dtype, dp_size=dp, tokens="uniform"
     )  # fmt: skip
+    assert combine_form(spec) == form
     groups = generate(spec, seed=H + K)
     groups[0].n, groups[-1].n = M, 1
     step = DeviceStep(spec, groups)
@@ -514,20 +519,21 @@ def test_pieces_of_many_picks(K, H, M, y_dtype, dp):
 
 
 @pytest.mark.parametrize(
-    "K,H,M,y_dtype,dp",
+    "K,H,M,y_dtype,dp,form",
     [
-        (1, 3584, 256, torch.bfloat16, 1),  # 8 KiB pieces, two workgroups to a CU
-        (1, 3208, 250, torch.float16, 1),  # ... a few less, the last of seven KiB a single vector
-        (1, 7680, 256, torch.bfloat16, 1),  # ... four workgroups, two pieces to a row
-        (2, 1544, 512, torch.float32, 1),  # 4 KiB pieces, four workgroups
-        (2, 2560, 300, torch.bfloat16, 2),  # five KiB of a DP group's rows
-        (2, 1032, 300, torch.float16, 4),  # a single vector in the third
+        (1, 3584, 256, torch.bfloat16, 1, (1, 8, False)),  # two workgroups to a CU
+        (1, 3208, 250, torch.float16, 1, (1, 8, False)),  # ... a few less, the last of seven KiB a single vector
+        (1, 7680, 256, torch.bfloat16, 1, (1, 8, False)),  # ... four workgroups, two pieces to a row
+        (2, 1544, 512, torch.float32, 1, (2, 1, False)),  # pieces of 2 KiB, the last a single vector
+        (2, 2560, 300, torch.bfloat16, 2, (2, 4, True)),  # five KiB of a DP group's rows
+        (2, 1032, 320, torch.float16, 4, (2, 4, True)),  # a single vector in the third
     ],
 )
-def test_long_pieces_of_few_picks(K, H, M, y_dtype, dp):
+def test_long_pieces_of_few_picks(K, H, M, y_dtype, dp, form):
     spec = WorkloadSpec(
         "long-pieces", 79, 8, 16, K, H, M, torch.bfloat16, expert_y_dtype=y_dtype, dp_size=dp, tokens="uniform"
     )  # fmt: skip
+    assert combine_form(spec) == form
     groups = generate(spec, seed=H + K)
     groups[0].n, groups[-1].n = M, 1
     step = DeviceStep(spec, groups)

@@ -156,6 +156,78 @@ def test_combine_per_group(ranks, dp, max_tokens, topk, hidden, dtype, per_group
 
 
 @pytest.mark.parametrize(
+    "tokens,topk,hidden,dtype,dp,picks,pieces",  # tokens of all groups
+    [
+        # one and two picks
+        (4096, 1, 512, torch.bfloat16, 1, 1, 1),
+        (4096, 1, 1024, torch.bfloat16, 1, 1, 2),
+        (4096, 1, 2048, torch.bfloat16, 1, 1, 4),
+        (4096, 1, 2560, torch.bfloat16, 1, 1, 3),
+        (2048, 1, 4096, torch.bfloat16, 1, 1, 8),  # 512 workgroups of 8 KiB pieces
+        (1976, 1, 4096, torch.bfloat16, 1, 1, 3),  # 494
+        (384, 1, 4096, torch.float32, 1, 1, 1),
+        (392, 1, 4096, torch.float32, 1, 1, 2),
+        (4096, 1, 4608, torch.bfloat16, 2, 1, 3),
+        (4096, 1, 5120, torch.bfloat16, 2, 1, 8),
+        (4096, 2, 512, torch.bfloat16, 1, 2, 1),
+        (4096, 2, 4096, torch.bfloat16, 1, 2, 2),
+        (4096, 2, 4096, torch.float32, 1, 2, 1),
+        (4096, 2, 4096, torch.bfloat16, 2, 2, 4),
+        (4096, 2, 4096, torch.float32, 2, 2, 2),
+        # three and four
+        (4096, 3, 4096, torch.bfloat16, 1, 3, 1),
+        (600, 3, 4096, torch.bfloat16, 2, 3, 1),
+        (608, 3, 4096, torch.bfloat16, 2, 2, 2),
+        (4096, 3, 1024, torch.bfloat16, 2, 3, 1),
+        (600, 4, 1024, torch.bfloat16, 1, 4, 1),
+        (608, 4, 1024, torch.bfloat16, 1, 4, 2),
+        (4096, 4, 4096, torch.bfloat16, 1, 4, 1),
+        (600, 4, 4096, torch.bfloat16, 2, 4, 2),
+        (608, 4, 4096, torch.bfloat16, 2, 2, 2),
+        (2048, 4, 3584, torch.float32, 1, 4, 1),
+        (2056, 4, 3584, torch.float32, 1, 8, 1),
+        (2056, 4, 3072, torch.float32, 1, 4, 1),
+        # more, steps of a few hundred to two thousand tokens
+        (384, 8, 7168, torch.bfloat16, 1, 8, 1),
+        (392, 8, 7168, torch.bfloat16, 1, 3, 1),  # 196 workgroups of 7 KiB pieces
+        (760, 8, 7168, torch.bfloat16, 1, 3, 1),  # 380
+        (768, 8, 7168, torch.bfloat16, 1, 1, 7),  # 384, three quarters of two to a CU
+        (1024, 8, 4096, torch.bfloat16, 1, 3, 1),  # one to a CU
+        (1528, 8, 4096, torch.bfloat16, 1, 3, 1),  # 382
+        (1536, 8, 4096, torch.bfloat16, 1, 1, 8),
+        (2048, 8, 4608, torch.bfloat16, 1, 3, 1),  # the second piece one KiB
+        (2056, 8, 4096, torch.bfloat16, 1, 8, 1),
+        (2048, 8, 3072, torch.bfloat16, 1, 8, 1),
+        (512, 8, 4096, torch.bfloat16, 2, 2, 2),
+        (1024, 8, 4096, torch.bfloat16, 2, 1, 8),  # one to a CU
+        (1152, 8, 4096, torch.bfloat16, 2, 1, 3),
+        (392, 8, 2048, torch.float32, 1, 2, 1),
+        (384, 8, 2048, torch.float32, 1, 8, 1),
+        (2048, 8, 1024, torch.float32, 1, 8, 1),
+        # ... large ones
+        (2056, 8, 1024, torch.float32, 1, 3, 2),
+        (2056, 8, 1536, torch.float32, 1, 8, 1),
+        (2056, 8, 1536, torch.float32, 2, 3, 1),
+        (2056, 8, 512, torch.float32, 1, 8, 1),
+        (2056, 5, 4096, torch.bfloat16, 2, 3, 2),
+        (2056, 8, 512, torch.bfloat16, 2, 8, 1),
+        (2056, 5, 4096, torch.bfloat16, 1, 5, 1),
+        (2056, 6, 3072, torch.bfloat16, 1, 3, 1),
+        (2056, 6, 3584, torch.bfloat16, 1, 8, 1),
+        (384, 6, 3584, torch.bfloat16, 1, 3, 1),
+        (2056, 10, 3072, torch.bfloat16, 1, 5, 1),
+        (2056, 10, 3584, torch.bfloat16, 1, 8, 1),
+        (2056, 9, 512, torch.float32, 1, 5, 1),
+        (2056, 7, 3072, torch.bfloat16, 1, 8, 1),
+    ],
+)
+def test_pieces_of_combine(tokens, topk, hidden, dtype, dp, picks, pieces):
+    assert tokens % 8 == 0
+    p = ops.combine_plan_of(ops.Config(tokens * dp // 8, 64, topk, 8, dp, hidden, 2 * hidden, 0), dtype)
+    assert p == (picks, pieces, dp > 1)
+
+
+@pytest.mark.parametrize(
     "lds,tokens,row,topk,one_launch",
     [
         # 8 x 2 rows of 12 KiB and the tables beside them fit any device's LDS, sixteen rows of 10128 bytes only

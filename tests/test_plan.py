@@ -219,6 +219,17 @@ def test_combine_per_group(ranks, dp, max_tokens, topk, hidden, dtype, per_group
         (2056, 10, 3584, torch.bfloat16, 1, 8, 1),
         (2056, 9, 512, torch.float32, 1, 5, 1),
         (2056, 7, 3072, torch.bfloat16, 1, 8, 1),
+        # ... of more than 512 MiB, or 1 GiB of DP groups
+        (43688, 6, 1024, torch.bfloat16, 1, 3, 1),
+        (43696, 6, 1024, torch.bfloat16, 1, 8, 1),
+        (26208, 10, 1024, torch.bfloat16, 1, 5, 1),
+        (26216, 10, 1024, torch.bfloat16, 1, 8, 1),
+        (43696, 6, 1024, torch.float32, 1, 3, 2),
+        (16384, 8, 4096, torch.bfloat16, 2, 3, 2),
+        (16392, 8, 4096, torch.bfloat16, 2, 8, 1),
+        (13104, 10, 4096, torch.bfloat16, 2, 3, 2),
+        (13112, 10, 4096, torch.bfloat16, 2, 8, 1),
+        (32768, 7, 4096, torch.bfloat16, 2, 3, 2),
     ],
 )
 def test_pieces_of_combine(tokens, topk, hidden, dtype, dp, picks, pieces):

@@ -365,7 +365,8 @@ CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
   //  - for DP groups, whose waves compare the members first.  They keep the long pieces for rows that are longer than half
   //    of one (groups of two, 4 x 512 tokens, one pick, 4096 wide 18.8 / 20.6, 7168 wide 32.1 / 31.4; groups of four, 2 x 512,
   //    15.0 / 15.1 and 22.1 / 24.0; two picks, 25.2 / 25.9 and 44.3 / 44.4, 17.3 / 19.2 and 28.3 / 28.9), one pick also unless
-  //    the last piece would be all but empty (4608 wide, nine KiB, 23.3 / 22.4);
+  //    the last piece would be all but empty (4608 wide, nine KiB, 23.3 / 22.4), but not of fp32 rows (combine, 16 / 6 KiB: 6880 wide,
+  //    17562 tokens 295 / 265, 6600 wide, 20950 345 / 322; 2560 wide, 1198 10.6 / 9.1; 30 steps 0.96 of the time);
   //  - fp32 rows, which have twice the bytes: 4 KiB (1 KiB up to 384 tokens) of one pick, 2 KiB of two (one pick, 7168
   //    wide, 208 tokens 9.0 / 8.4, 4096 wide, 2428 20.4 / 19.6; two picks of 8 KiB / 2 KiB, 7680 wide, 4928 91.6 / 89.2).
   // Picks of one go, against eight places of 1 KiB: top-3 (two picks and then one), 8192 tokens, 2048 wide 57.0 / 52.4, 4096
@@ -386,7 +387,8 @@ CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
         return form(1, 2);
       }
       if (nvec_segments == 4) return form(1, 4);
-      if (grouped && nvec_segments > 4 && 8 * ((8 - nvec_segments % 8) % 8) <= 5 * nvec_segments) return form(1, 8);
+      if (grouped && elem_bytes == 2 && nvec_segments > 4 && 8 * ((8 - nvec_segments % 8) % 8) <= 5 * nvec_segments)
+        return form(1, 8);
       if (!grouped && elem_bytes == 2 && even_pieces(tokens, nvec_segments)) return form(1, 8);
       return form(1, 3);
     case 2:

@@ -527,6 +527,7 @@ def test_pieces_of_many_picks(K, H, M, y_dtype, dp, form):
         (2, 1544, 512, torch.float32, 1, (2, 1, False)),  # pieces of 2 KiB, the last a single vector
         (2, 2560, 300, torch.bfloat16, 2, (2, 4, True)),  # five KiB of a DP group's rows
         (2, 1032, 320, torch.float16, 4, (2, 4, True)),  # a single vector in the third
+        (1, 2568, 150, torch.float32, 2, (1, 3, True)),  # a single vector in the sixth piece of 2 KiB
     ],
 )
 def test_long_pieces_of_few_picks(K, H, M, y_dtype, dp, form):

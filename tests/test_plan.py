@@ -169,6 +169,7 @@ def test_combine_per_group(ranks, dp, max_tokens, topk, hidden, dtype, per_group
         (392, 1, 4096, torch.float32, 1, 1, 2),
         (4096, 1, 4608, torch.bfloat16, 2, 1, 3),
         (4096, 1, 5120, torch.bfloat16, 2, 1, 8),
+        (4096, 1, 5120, torch.float32, 2, 1, 3),
         (4096, 2, 512, torch.bfloat16, 1, 2, 1),
         (4096, 2, 4096, torch.bfloat16, 1, 2, 2),
         (4096, 2, 4096, torch.float32, 1, 2, 1),

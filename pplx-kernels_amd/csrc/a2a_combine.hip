@@ -304,6 +304,7 @@ CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
   const uint64_t tokens = (uint64_t)(grouped ? w.G : w.R) * w.M;
   const uint64_t gathered = tokens * w.K * w.H * elem_bytes;
+  const bool whole_pieces = w.H % (8 * kWave) == 0;
   // Steps of a few hundred to two thousand tokens have all their waves resident at the same moment.  More than four picks in rows
   // of 7 KiB and more are best taken one after the other in 7 or 8 KiB pieces there, by a quarter as many waves, but
   // only where the workgroups of such pieces come out even over the CUs (long_pieces): the CUs that get one more of them
@@ -346,10 +347,11 @@ CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
   } else if (grouped && nvec_segments > 1) {
     // Steps of DP groups, 16-bit rows, eight picks / three in pieces of 2 KiB: 5120 wide, top-6, 2888 tokens 86.8 / 84.0;
     // 1024 wide, top-8, 12268 88.1 / 87.1 (541 steps: 0.983, 0.90 to 1.05).  Eight and more are eight at a time again where the
-    // rows are more than 1 GiB (combine, eight / three: 6144 wide, top-8, 25012 tokens 611 / 640, 5120 wide, 25104 423 / 445;
-    // 4608 wide, top-10, 19340 419 / 439; 28 steps of that size 0.99 of the time, 65 smaller ones 1.01).  Three and four picks,
-    // all at once / two: 1536 wide, top-4, 3260 25.0 / 23.5; 5120 wide, 856 23.5 / 22.9.
-    if (w.K > 4 && tokens > 2048 && (w.K < 8 || gathered <= 1ull << 30)) return form(3, 2);
+    // rows are more than 1 GiB of whole KiB (combine, eight / three: 6144 wide, top-8, 25012 tokens 611 / 640, 5120 wide, 25104 423 /
+    // 445; 4608 wide, top-10, 19340 419 / 439; 28 steps of that size 0.99 of the time, 65 smaller ones 1.01, 31 of rows with a
+    // partial KiB 1.02: 3784 wide, top-8, 29830 537 / 491).  Three and four picks, all at once / two: 1536 wide, top-4, 3260
+    // 25.0 / 23.5; 5120 wide, 856 23.5 / 22.9.
+    if (w.K > 4 && tokens > 2048 && (w.K < 8 || !whole_pieces || gathered <= 1ull << 30)) return form(3, 2);
     if ((w.K == 3 || w.K == 4) && tokens > 600 && nvec_segments > 2) return form(2, 2);
   }
   // Of what is left, up to five picks are taken all at once, six in two goes of three, nine and ten in two of five, others
@@ -376,8 +378,10 @@ CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
   // wide, beyond 2048 tokens: 0.975; up to 2048 0.99).  Ten, eight and two / five and five: 512 wide, 1160 14.6 / 14.0, 3584
   // wide, 352 15.5 / 15.2.  Of 16-bit rows neither in large steps of 7 KiB and more (six 0.97 to 1.04, ten 1.012), nor where the
   // rows are more than 512 MiB (combine, six, 2560 wide, 50368 tokens 298 / 312, 2048 wide, 52608 252 / 263; ten, 2048 wide, 50224
-  // 364 / 384; 35 steps of that size 0.98 of the time, 69 smaller ones 1.03), nor for DP groups.
-  const bool halves = elem_bytes == 4 || (!grouped && (tokens <= 2048 || (nvec_segments < 7 && gathered <= 512ull << 20)));
+  // 364 / 384; 35 steps of that size 0.98 of the time, 69 smaller ones 1.03), but six also there if the last KiB is partial
+  // (1048 wide, 46064 tokens 131 / 117, 1544 wide, 38208 151 / 141), nor for DP groups.
+  const bool large = gathered > 512ull << 20 && (w.K > 6 || whole_pieces);
+  const bool halves = elem_bytes == 4 || (!grouped && (tokens <= 2048 || (nvec_segments < 7 && !large)));
   switch (w.K) {
     case 1:
       if (nvec_segments == 1) return form(1, 1);

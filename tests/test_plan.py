@@ -228,6 +228,9 @@ def test_combine_per_group(ranks, dp, max_tokens, topk, hidden, dtype, per_group
         (43696, 6, 1024, torch.bfloat16, 1, 8, 1),
         (26208, 10, 1024, torch.bfloat16, 1, 5, 1),
         (26216, 10, 1024, torch.bfloat16, 1, 8, 1),
+        (43696, 6, 1032, torch.bfloat16, 1, 3, 1),  # ... and a partial KiB
+        (26216, 10, 1032, torch.bfloat16, 1, 8, 1),
+        (16392, 8, 4104, torch.bfloat16, 2, 3, 2),
         (43696, 6, 1024, torch.float32, 1, 3, 2),
         (16384, 8, 4096, torch.bfloat16, 2, 3, 2),
         (16392, 8, 4096, torch.bfloat16, 2, 8, 1),

@@ -259,6 +259,8 @@ bool combine_per_group(const WorldHost &w, size_t elem_bytes) {
 
 template <typename T, typename U, class CT, int KB, int VPL>
 int launch_combine_v(const WorldHost &w, const CT &tab, bool grouped, hipStream_t s) {
+  static_assert(sizeof(WorldDev) + sizeof(HbmCombine) + sizeof(uint32_t) + sizeof(FastDiv) <= kShortArguments,
+                "arguments of combine_gather");
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
   const uint32_t segments = (nvec_segments + VPL - 1) / VPL;
   const uint64_t waves = (uint64_t)(grouped ? w.G : w.R) * w.M * segments;
@@ -297,7 +299,8 @@ LongPieces long_pieces(uint64_t tokens, uint32_t segments) {
   return {per_cu, 4 * workgroups * segments >= 3 * 256 * per_cu * pieces * length};
 }
 
-// The form of combine_gather that a step takes, for rows of `elem_bytes` (2 or 4) an element.
+// The form of combine_gather that a step takes, for rows of `elem_bytes` (2 or 4) an element: form(picks, pieces).  A piece is
+// 512 elements, 1 KiB of a 16-bit row and 2 KiB of an fp32 one; KiB are those of the rows that are read.
 CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
   const bool grouped = combine_per_group(w, elem_bytes);
   auto form = [grouped](uint32_t picks, uint32_t pieces) { return CombineForm{picks, pieces, grouped}; };
@@ -306,15 +309,15 @@ CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
   const uint64_t gathered = tokens * w.K * w.H * elem_bytes;
   const bool whole_pieces = w.H % (8 * kWave) == 0;
   // Steps of a few hundred to two thousand tokens have all their waves resident at the same moment.  More than four picks in rows
-  // of 7 KiB and more are best taken one after the other in 7 or 8 KiB pieces there, by a quarter as many waves, but
+  // of seven pieces and more are best taken one after the other in 7 or 8 KiB pieces there, by a quarter as many waves, but
   // only where the workgroups of such pieces come out even over the CUs (long_pieces): the CUs that get one more of them
   // take that much longer.  Dispatch + combine on three buffer sets, top-8, 8 ranks, us, long pieces / three picks in 1
   // KiB: 7168 wide, 1024 tokens 38.4 / 39.0, 544 25.0 / 23.7, 7136 wide, 528 30.2 / 28.4, 7656 wide, 1048 61.8 / 57.6; 4096 wide, 388
   // 19.7 / 15.4, 448 20.4 / 17.0, 680 23.7 / 22.7, 784 24.8 / 25.0, 1024 29.9 / 30.3.  (653 steps of that range drawn
   // at random, against long pieces for all of them: 0.946 of the time, 0.73 to 1.03.)  DP groups, whose waves compare the
   // members first, take two picks in 2 KiB pieces or, beyond a workgroup to a CU, one in 3 KiB instead (5120 wide, 386
-  // tokens of all groups 20.2 / 17.9; 3696 wide, 596 23.5 / 21.2), fp32 rows two picks in 1 KiB (4608 wide, top-6, 1256
-  // tokens 49.3 / 44.4; 3584 wide, 1152 40.7 / 35.5).
+  // tokens of all groups 20.2 / 17.9; 3696 wide, 596 23.5 / 21.2), fp32 rows two picks in 2 KiB (4608 wide, top-6, 1256
+  // tokens 49.3 / 44.4; 3584 wide, 1152 40.7 / 35.5; their long pieces are 14 and 16 KiB).
   const bool middle = tokens > 384 && tokens <= 2048;
   if (w.K > 4 && middle && nvec_segments >= 7) {
     const LongPieces pieces = long_pieces(tokens, nvec_segments);
@@ -328,12 +331,12 @@ CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
       return form(1, 3);
     }
   }
-  // fp32 rows of three KiB of 16-bit outputs and more.  Two picks at a time beside the above (2048 wide, top-8, 464 tokens
+  // fp32 rows of three pieces (6 KiB) and more.  Two picks at a time beside the above (2048 wide, top-8, 464 tokens
   // 13.0 / 12.8; 1536 wide, 808 16.3 / 15.6; 2560 wide, 1040 29.8 / 28.7, eight / two).  Larger steps take eight at a time, whose
-  // registers leave room for fewer waves: against two picks of 4 KiB or three of 2 KiB 6656 wide, top-8, 2095 tokens 130.4 / 126.2,
-  // 3588 180.4 / 173.7; 4096 wide, 7168 221.2 / 215.7; top-6, 7680 wide, 5232 279.4 / 271.2; seven KiB and more also with four
+  // registers leave room for fewer waves: against two picks of 8 KiB or three of 4 KiB 6656 wide, top-8, 2095 tokens 130.4 / 126.2,
+  // 3588 180.4 / 173.7; 4096 wide, 7168 221.2 / 215.7; top-6, 7680 wide, 5232 279.4 / 271.2; seven pieces and more also with four
   // picks (6144 wide, 2156 tokens 56.0 / 55.3; 4096 wide, 8 x 1024, combine alone 103.2 / 98.1).  DP groups of that size take three
-  // (2048 wide, 2136 tokens 43.1 / 40.5), rows of two KiB three in pieces of both (eight 1.0 to 1.1 of their time).
+  // (2048 wide, 2136 tokens 43.1 / 40.5), rows of two pieces three of both (eight 1.0 to 1.1 of their time).
   if (elem_bytes == 4) {
     if (w.K > 4 && middle && nvec_segments >= 3) return form(2, 1);
     if (tokens > 2048) {
@@ -369,8 +372,9 @@ CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
   //    15.0 / 15.1 and 22.1 / 24.0; two picks, 25.2 / 25.9 and 44.3 / 44.4, 17.3 / 19.2 and 28.3 / 28.9), one pick also unless
   //    the last piece would be all but empty (4608 wide, nine KiB, 23.3 / 22.4), but not of fp32 rows (combine, 16 / 6 KiB: 6880 wide,
   //    17562 tokens 295 / 265, 6600 wide, 20950 345 / 322; 2560 wide, 1198 10.6 / 9.1; 30 steps 0.96 of the time);
-  //  - fp32 rows, which have twice the bytes: 4 KiB (1 KiB up to 384 tokens) of one pick, 2 KiB of two (one pick, 7168
-  //    wide, 208 tokens 9.0 / 8.4, 4096 wide, 2428 20.4 / 19.6; two picks of 8 KiB / 2 KiB, 7680 wide, 4928 91.6 / 89.2).
+  //  - fp32 rows, which have twice the bytes, outside DP groups: 4 KiB of one pick (2 KiB up to 384 tokens, unless the row
+  //    has two pieces), 2 KiB of two (one pick, 7168 wide, 208 tokens 9.0 / 8.4, 4096 wide, 2428 20.4 / 19.6; two picks of
+  //    8 KiB / 2 KiB, 7680 wide, 4928 91.6 / 89.2).
   // Picks of one go, against eight places of 1 KiB: top-3 (two picks and then one), 8192 tokens, 2048 wide 57.0 / 52.4, 4096
   // wide 99.5 / 90.4; top-5 (four and one), 16000 tokens, 512 wide 43.4 / 41.6, 4096 tokens, 7168 wide 124.6 / 122.5.  Four picks
   // in 2 KiB / 1 KiB: 5120 wide, 88 tokens 8.7 / 8.2, 3584 wide, 2048 25.0 / 24.4, 7680 wide, 1388 43.4 / 42.5 (995 steps: 0.987).

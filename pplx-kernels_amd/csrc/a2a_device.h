@@ -88,8 +88,10 @@ struct alignas(16) CombineRank {
 static_assert(sizeof(CombineRank) == 80, "CombineRank layout");
 
 // Geometry + scratch of a world; passed to every kernel by value, and kept short: in some processes a launch with more
-// than 112 bytes of arguments costs the host 3.4 to 4 us instead of 2.6 (9 KiB no more than 1 KiB), and the tables of bound
-// steps, which are in HBM, leave room for this.
+// than kShortArguments bytes of arguments costs the host 3.4 to 4 us instead of 2.6 (9 KiB no more than 1 KiB).  Beside a
+// table in HBM the one-launch dispatch, the scatters and the gather of combine stay within them; the routing kernels, whose
+// RouteSpan alone is 56 bytes, do not.
+constexpr size_t kShortArguments = 112;
 struct WorldDev {
   uint32_t M;        // max tokens per DP group
   uint32_t H;        // elements per row
@@ -111,7 +113,7 @@ struct WorldDev {
   uint32_t *slot_map;    // [G * M][K] row of (token, pick) inside its expert
   uint32_t *faults;      // [1] sticky fault bits
 };
-static_assert(sizeof(WorldDev) == 88, "a kernel's arguments beside a table in HBM fit 112 bytes");
+static_assert(sizeof(WorldDev) == 88, "WorldDev layout");
 
 // ... and what only the host needs of it.
 struct WorldHost : WorldDev {

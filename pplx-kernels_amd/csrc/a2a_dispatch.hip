@@ -177,6 +177,8 @@ struct FusedShape {
   uint32_t pick_vector : 4;       // expert ids one load may fetch
   uint32_t write_through : 1;
 };
+static_assert(sizeof(WorldDev) + sizeof(HbmDispatch) + sizeof(FusedShape) <= kShortArguments, "arguments of dispatch_fused");
+static_assert(sizeof(WorldDev) + sizeof(HbmDispatch) + 2 * sizeof(uint32_t) <= kShortArguments, "arguments of the scatters");
 
 // A rank table that dispatch_fused has copied into LDS.
 struct LdsDispatch {
@@ -301,7 +303,9 @@ __device__ __forceinline__ void count_earlier_picks(const WorldDev &w, const Tab
 // its picks), and lane k of such a row wave is the token's pick k.
 //   0. the rank table (world_size rows of it) is copied from the kernel arguments, or from HBM, into LDS with
 //      loads that depend on nothing, so every later lookup is an LDS read and not another trip
-//      to memory behind the one that fetches the geometry;
+//      to memory behind the one that fetches the geometry (tables of more than 64 ranks too, up to 56 KiB for 384:
+//      dispatch, us, looked up in HBM / copied: 72 ranks x 1 token, top-8, 2 KiB fp8 rows 4.96 / 4.51, 256 x 1 5.65 / 5.23, 384 x
+//      10, 512 wide, top-2 7.50 / 6.11; 60 shapes of 72 to 384 ranks 0.94 of the time, at worst, 384 x 4 rows of 14 KiB, 1.03);
 //   1. one batch of small loads: every thread fetches the picks of one token before the
 //      workgroup's own (and its group's token count), the row waves their own picks;
 //   2. the picks of the earlier tokens are counted per expert in an LDS histogram (every

@@ -268,13 +268,13 @@ int pplx_a2a_combine_plan(const pplx_a2a_config_t *cfg, int in_dtype, pplx_a2a_c
  * no allocation, no synchronisation. */
 int pplx_a2a_world_abandon_step(pplx_a2a_world_t *world, uint32_t which, uint32_t *dropped_calls);
 /* A step whose buffers stay where they are: pplx_a2a_bound_create checks the arguments of
- * pplx_a2a_world_dispatch and pplx_a2a_world_combine once (host work alone: nothing is enqueued);
- * pplx_a2a_bound_launch then runs dispatch (op 0) or combine (op 1).  The first launch on `stream` carries the
- * rank tables along as always (up to 64 ranks), the second writes them into `device_memory`
- * (pplx_a2a_bound_bytes, 16-byte aligned, the caller's), and from then on the kernels of launches there read
- * them.  On another stream, on hipStreamPerThread, or while the stream is captured, they always go with the
- * launch (a graph never refers to device_memory).  device_memory is to stay untouched from the first launch
- * on that stream until the last one is done with it; the bound step is to be destroyed before its world. */
+ * pplx_a2a_world_dispatch and pplx_a2a_world_combine once and enqueues the writing of their rank
+ * tables into `device_memory` (pplx_a2a_bound_bytes, 16-byte aligned, the caller's), on `stream`;
+ * pplx_a2a_bound_launch then runs dispatch (op 0) or combine (op 1).  On that stream the kernels
+ * read the tables from there; on another one, on hipStreamPerThread, or while the stream is captured, they
+ * go with the launch as always (a graph never refers to device_memory).  device_memory is to stay untouched
+ * until the last launch on that stream is done with it; the bound step is to be destroyed before
+ * its world.  The capture of `stream` refuses pplx_a2a_bound_create. */
 int pplx_a2a_bound_bytes(const pplx_a2a_world_t *world, uint64_t *out);
 int pplx_a2a_bound_create(pplx_a2a_world_t *world, const pplx_a2a_dispatch_args_t *dispatch_per_rank,
                           const pplx_a2a_combine_args_t *combine_per_rank, void *device_memory, void *stream,

@@ -142,7 +142,7 @@ struct pplx_a2a {
   uint32_t rank;
 };
 
-// A step whose arguments were checked once and whose rank tables get a place in device memory of the caller.
+// A step whose arguments were checked once and whose rank tables lie in device memory of the caller.
 struct pplx_a2a_bound {
   pplx_a2a_world *world = nullptr;
   std::vector<DispatchRank> dispatch;
@@ -151,9 +151,7 @@ struct pplx_a2a_bound {
   uint32_t pick_vector = 1;
   DispatchRank *drank = nullptr;
   CombineRank *crank = nullptr;
-  void *stream = nullptr;  // whose launches read the tables
-  // Of dispatch and of combine, under the world's lock: a launch on `stream` has gone by, the table is written.
-  mutable bool launched[2] = {false, false}, written[2] = {false, false};
+  void *stream = nullptr;  // on which the tables were written
 };
 
 struct pplx_a2a_graph {
@@ -1025,12 +1023,25 @@ int pplx_a2a_bound_create(pplx_a2a_world_t *w, const pplx_a2a_dispatch_args_t *d
   }
   int st = check_groups(d, b->dispatch.data());
   if (st) return st;
+  DeviceScope scope(w->device);
+  if (!scope.ok()) return fail(PPLX_A2A_HIP_ERROR, "cannot select device %d", w->device);
+  unsigned long long session = 0;
+  st = capture_session(stream, &session);
+  if (st) return st;
+  if (session != 0) return fail(PPLX_A2A_INVALID_STATE, "a step cannot be bound while its stream is captured");
+  DispatchRank *drank = static_cast<DispatchRank *>(device_memory);
+  CombineRank *crank = reinterpret_cast<CombineRank *>(drank + d.R);
+  for (uint32_t first = 0; first < d.R; first += kBindBatch) {
+    st = bind_batch<BindDispatchBatch>(d.R, drank, b->dispatch.data(), first, launch_bind_dispatch, stream);
+    if (!st) st = bind_batch<BindCombineBatch>(d.R, crank, b->combine.data(), first, launch_bind_combine, stream);
+    if (st) return st;
+  }
   b->world = w;
   b->in_dtype = combine_per_rank[0].in_dtype;
   b->out_dtype = combine_per_rank[0].out_dtype;
   b->pick_vector = pick_vector_of(d, b->dispatch.data());
-  b->drank = static_cast<DispatchRank *>(device_memory);
-  b->crank = reinterpret_cast<CombineRank *>(b->drank + d.R);
+  b->drank = drank;
+  b->crank = crank;
   b->stream = stream;
   *out = b.release();
   return PPLX_A2A_OK;
@@ -1047,36 +1058,24 @@ int pplx_a2a_bound_launch(pplx_a2a_world_t *w, const pplx_a2a_bound_t *b, int op
   DeviceScope scope(w->device);
   if (!scope.ok()) return fail(PPLX_A2A_HIP_ERROR, "cannot select device %d", w->device);
   unsigned long long session = 0;
-  int st = capture_session(stream, &session);
+  const int st = capture_session(stream, &session);
   if (st) return st;
   // The tables in HBM are ordered with their own stream only, and a graph may outlive them: elsewhere they go with
   // the launch, as those of a step that is not bound.  (hipStreamPerThread is another stream in every thread.)
-  const bool on_its_stream = stream == b->stream && stream != hipStreamPerThread && session == 0;
-  // So they do in the first launch: writing a table takes a launch of its own, which only a second one pays back.
-  // (Tables that do not fit the arguments are written either way.)
-  if (!on_its_stream || (!b->launched[op] && w->dev.R <= kInlineRanks)) {
+  if (stream != b->stream || stream == hipStreamPerThread || session != 0) {
     if (op == 0) {
       w->pend_dispatch = b->dispatch;
-      st = run_dispatch(*w, stream);
-    } else {
-      w->pend_combine = b->combine;
-      w->combine_in_dtype = b->in_dtype;
-      w->combine_out_dtype = b->out_dtype;
-      st = run_combine(*w, stream);
+      return run_dispatch(*w, stream);
     }
-    if (!st && on_its_stream) b->launched[op] = true;
-    return st;
+    w->pend_combine = b->combine;
+    w->combine_in_dtype = b->in_dtype;
+    w->combine_out_dtype = b->out_dtype;
+    return run_combine(*w, stream);
   }
   ProfilerRange range(op == 0 ? "dispatch" : "combine");
   WorldHost d = w->dev;
   d.drank = b->drank;
   d.crank = b->crank;
-  for (uint32_t first = 0; first < d.R && !b->written[op]; first += kBindBatch) {
-    st = op == 0 ? bind_batch<BindDispatchBatch>(d.R, d.drank, b->dispatch.data(), first, launch_bind_dispatch, stream)
-                 : bind_batch<BindCombineBatch>(d.R, d.crank, b->combine.data(), first, launch_bind_combine, stream);
-    if (st) return st;
-  }
-  b->written[op] = true;
   if (op == 0) {
     LAUNCH_TRY(launch_dispatch(d, nullptr, b->pick_vector, stream));
   } else {

@@ -826,8 +826,7 @@ PyObject *py_step_tables(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 }
 
 // bind_step(world, dispatch_arguments, combine_arguments, device_memory, stream) -> a plan for launch_plan, or None
-// where the arguments are not those of a step that can be launched (its launch says why).  Host work alone: an error of
-// HIP can only come from the launches, which raise it.
+// where the arguments are not those of a step that can be launched (its launch says why)
 PyObject *py_bind_step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   arity("bind_step", nargs, 5);

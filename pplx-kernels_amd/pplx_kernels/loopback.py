@@ -63,8 +63,8 @@ class BoundStep:
         # (what the launches read: packed for this world, which is named by a number of its own)
         self._keep = (dispatch_args, combine_args, keep)
         packed = ctypes.addressof(dispatch_args), ctypes.addressof(combine_args)
-        # From the second launch on this stream its kernels read the rank tables from device memory, which the allocator
-        # gives out again, to this stream, once the step is gone; launches on others, or under capture, carry the tables along.
+        # The kernels of launches on this stream read the rank tables from device memory, which the allocator gives out
+        # again, to this stream, once the step is gone; launches on others, or under capture, carry the tables along.
         self._tables = plan = None
         if device.type == "cuda":
             self._tables = ops._C.step_tables(world._world_id, device.index)

@@ -640,33 +640,6 @@ def test_bound_step_on_the_stream_per_thread_takes_its_tables_along():
     world.destroy()
 
 
-@pytest.mark.parametrize("R,written_by", [(4, 2), (72, 1)], ids=["4-ranks", "72-ranks"])
-def test_binding_enqueues_nothing_and_a_launch_writes_the_tables(R, written_by):
-    """The second launch, or the first where the tables do not fit a kernel's arguments."""
-    spec = WorkloadSpec("bound", 85, R, R, 2, 512, 6, torch.bfloat16, tokens="uniform")
-    step = DeviceStep(spec, generate(spec, seed=1))
-    step.expert_y_all.normal_(generator=torch.Generator(device="cuda").manual_seed(12))
-    world = make_world(spec, group_name="bound-late")
-    bound = step.bind_world(world)
-    packed = [ctypes.addressof(args) for args in bound._keep[:2]]
-    tables = torch.full_like(bound._tables, 0x5A)
-    stream = torch.cuda.current_stream().cuda_stream
-    plan = ops._C.bind_step(world._world_id, *packed, tables.data_ptr(), stream)
-    torch.cuda.synchronize()
-    assert (tables == 0x5A).all()
-    of_dispatch, of_combine = tables[: 144 * R], tables[144 * R :]
-    for launch in range(1, 4):
-        for op, table in enumerate((of_dispatch, of_combine)):
-            ops._C.launch_plan(op, world._world_id, plan, 0, stream)
-            torch.cuda.synchronize()
-            assert bool((table == 0x5A).all()) == (launch < written_by)
-        expected = check_dispatch_against_oracle(step)
-        check_combine_against_oracle(step, expected.slot_map)
-    assert world.faults() == 0
-    del plan
-    world.destroy()
-
-
 @pytest.mark.parametrize("which", ["another thread, global", "this thread", "a blocking stream"])
 def test_binding_leaves_captures_alone(which):
     """Where the memory for the tables has to come from the device, and on a stream that a capture keeps launches from."""

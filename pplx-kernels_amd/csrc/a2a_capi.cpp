@@ -43,11 +43,14 @@ int fail(int status, const char *fmt, ...) {
   return status;
 }
 
+// (hipGetLastError: an error that is returned here is not reported once more by whoever asks for the last one)
 #define HIP_TRY(expr)                                                                        \
   do {                                                                                       \
     hipError_t err_ = (expr);                                                                \
-    if (err_ != hipSuccess)                                                                  \
+    if (err_ != hipSuccess) {                                                                \
+      (void)hipGetLastError();                                                               \
       return fail(PPLX_A2A_HIP_ERROR, "%s failed: %s", #expr, hipGetErrorString(err_));      \
+    }                                                                                        \
   } while (0)
 
 #define LAUNCH_TRY(expr)                                                                     \

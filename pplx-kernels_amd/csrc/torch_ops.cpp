@@ -840,6 +840,7 @@ PyObject *py_bind_step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     return pplx_a2a_bound_create(world->ptr, static_cast<const pplx_a2a_dispatch_args_t *>(dispatch),
                                  static_cast<const pplx_a2a_combine_args_t *>(combine), memory, stream, &bound);
   });
+  if (st == PPLX_A2A_HIP_ERROR) A2A_CHECK(st);
   if (st != PPLX_A2A_OK) Py_RETURN_NONE;
   PyObject *capsule = PyCapsule_New(bound, "pplx_kernels.plan", free_plan);
   if (!capsule) (void)pplx_a2a_bound_destroy(bound);

@@ -688,6 +688,30 @@ def test_binding_leaves_captures_alone(which):
     world.destroy()
 
 
+def test_an_error_of_hip_at_the_binding_is_raised():
+    """Here the one that the default stream reports while a blocking stream is captured."""
+    spec = WorkloadSpec("bound", 88, 2, 8, 2, 512, 6, torch.bfloat16, tokens="uniform")
+    step = DeviceStep(spec, generate(spec, seed=1))
+    world = make_world(spec, group_name="bound-error")
+    bound = step.bind_world(world)
+    packed = [ctypes.addressof(args) for args in bound._keep[:2]]
+    tables = torch.zeros_like(bound._tables)
+    torch.cuda.synchronize()
+    handle = ctypes.c_void_p()
+    assert ops.load_library().hipStreamCreate(ctypes.byref(handle)) == 0
+    recorded = torch.cuda.ExternalStream(handle.value)
+    with torch.cuda.stream(recorded), world.capture() as cap:
+        bound.dispatch()
+        with pytest.raises(RuntimeError, match="HIP error"):
+            ops._C.bind_step(world._world_id, *packed, tables.data_ptr(), 0)
+    cap.graph.replay(recorded)
+    torch.cuda.synchronize()
+    check_dispatch_against_oracle(step)
+    assert world.faults() == 0 and not tables.any()
+    cap.graph.destroy()
+    world.destroy()
+
+
 def test_bound_step_that_cannot_be_launched_says_so_at_its_launch():
     spec = WorkloadSpec("bound", 83, 4, 8, 2, 512, 6, torch.bfloat16, dp_size=2, tokens="uniform")
     step = DeviceStep(spec, generate(spec, seed=1))

@@ -162,7 +162,10 @@ class LoopbackWorld:
     ) -> BoundStep:
         """Checks and packs the arguments of :meth:`dispatch` and :meth:`combine` once and
         returns a :class:`BoundStep` that launches them as often as wanted, fastest on the stream
-        that is current now."""
+        that is current now: the rank tables are written to device memory there (by two small kernels,
+        unless the stream is captured), and the step's kernels read them.  Binding takes 18 us of the
+        host for one rank, 60 for 8 and 390 for 64, 10 of them for the tables, which save 1 to 2 us a
+        step: a step that is bound for fewer than some ten launches loses by them."""
         d_args = (ops.DispatchArgs * self.world_size)()
         c_args = (ops.CombineArgs * self.world_size)()
         for r in range(self.world_size):

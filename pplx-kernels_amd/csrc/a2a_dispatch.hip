@@ -632,11 +632,10 @@ bool scatter_rows_in_lds(const WorldHost &w) {
 // 13 KiB, step 67.9 at nine, 68.3 at ten)
 // What a wave stores between 12 and 24 KiB of in rows of 4 KiB and more depends on the rows: those with scales, whose short
 // stores hold a wave up, want nine waves from 8192 tokens on, the others four (steps on three buffer sets, four / nine: 4608-byte
-// rows with scales, top-3, 46000 tokens 247.9 / 224.2, 20000 203.2 / 184.2, top-4, 39000 263.8 / 238.7; 8 KiB rows without,
-// top-2, 8 x 4096 tokens, skewed 266 / 278), but rows of 7 KiB and more with scales four again beyond 16384 tokens (dispatch: 7392
-// bytes, top-2, 47992 tokens 193 / 208, top-3, 56896 160 / 169; 8448 bytes, top-2, 54243 233 / 253, 47764 223 / 237; 40 drawn steps
-// of these 0.97 of the time, 21 of up to 16384 tokens 1.03, 51 of shorter rows 1.07; steps with half of their tokens absent
-// are as the smaller ones, which the host does not see: 7920 bytes, top-2, 24732 tokens 61.0 / 54.9).
+// rows with scales, top-3, 46000 tokens 247.9 / 224.2, 20000 203.2 / 184.2, top-4, 39000 263.8 / 238.7; drawn ones with
+// scales of more than 16384 tokens 0.965, of more than 8192 0.984, of up to 8192 0.998 of the time; 8 KiB rows without, top-2, 8 x
+// 4096 tokens, skewed 266 / 278; rows of 7 KiB and more with scales beyond 16384 tokens, which in dispatches back to back are up
+// to 8 % ahead with four, are level in steps: 1.00 over 59 drawn ones, 1.02 where tokens are absent).
 // (one behind the other they lose: 8 x 4096 tokens of 8 KiB, top-2, skewed: 123 and 130; 2 KiB rows,
 // top-6, 8 x 1024: 26.2 and 27.5).
 // Rows in LDS (a2a_rows.h) spend more time in front of and between their stores and want more waves.  Us at 6 / 8 / 12 /
@@ -678,10 +677,7 @@ ScatterPlan scatter_plan(const WorldHost &w, uint32_t picks_per_wave) {
     if (stored >= 48 * 1024 || (stored >= 32 * 1024 && (row >= 8192 || tokens <= 32768))) return {3, true};
     return {stored >= 32 * 1024 || tokens <= 32768 ? 4u : 9u, false};
   }
-  if (stored >= 12 * 1024) {
-    const bool nine = row < 4096 || (w.S != 0 && tokens > 8192 && (row < 7168 || tokens <= 16384));
-    return {nine ? 9u : 4u, false};
-  }
+  if (stored >= 12 * 1024) return {row >= 4096 && (w.S == 0 || tokens <= 8192) ? 4u : 9u, false};
   return {stored >= 6 * 1024 ? 12u : 0u, false};
 }
 

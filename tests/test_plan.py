@@ -72,9 +72,6 @@ def test_scatter(tokens, row, scales, topk, waves, in_turn):
         (8200, 3584, 28, 4, 9),  # shorter rows: nine with and without
         (8200, 3584, 0, 4, 9),
         (8200, 7168, 56, 4, 4),  # beyond 24 KiB
-        (16384, 7168, 56, 2, 9),
-        (16392, 7168, 56, 2, 4),  # 7 KiB and more
-        (16392, 6656, 52, 2, 9),
     ],
 )
 def test_scatter_of_rows_with_scales(tokens, row, scales, topk, waves):

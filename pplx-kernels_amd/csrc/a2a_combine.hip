@@ -352,8 +352,8 @@ CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
     // 1024 wide, top-8, 12268 88.1 / 87.1 (541 steps: 0.983, 0.90 to 1.05).  Eight and more are eight at a time again where the
     // rows are more than 1 GiB of whole KiB (combine, eight / three: 6144 wide, top-8, 25012 tokens 611 / 640, 5120 wide, 25104 423 /
     // 445; 4608 wide, top-10, 19340 419 / 439; 28 steps of that size 0.99 of the time, 65 smaller ones 1.01, 31 of rows with a
-    // partial KiB 1.02: 3784 wide, top-8, 29830 537 / 491; dispatch + combine 0.98, 1.01 where tokens are absent).  Three and four picks, all at once / two: 1536 wide, top-4, 3260
-    // 25.0 / 23.5; 5120 wide, 856 23.5 / 22.9.
+    // partial KiB 1.02: 3784 wide, top-8, 29830 537 / 491; dispatch + combine 0.98, 1.01 where tokens are absent).  Three and
+    // four picks, all at once / two: 1536 wide, top-4, 3260 25.0 / 23.5; 5120 wide, 856 23.5 / 22.9.
     if (w.K > 4 && tokens > 2048 && (w.K < 8 || !whole_pieces || gathered <= 1ull << 30)) return form(3, 2);
     if ((w.K == 3 || w.K == 4) && tokens > 600 && nvec_segments > 2) return form(2, 2);
   }
@@ -371,7 +371,8 @@ CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
   //    of one (groups of two, 4 x 512 tokens, one pick, 4096 wide 18.8 / 20.6, 7168 wide 32.1 / 31.4; groups of four, 2 x 512,
   //    15.0 / 15.1 and 22.1 / 24.0; two picks, 25.2 / 25.9 and 44.3 / 44.4, 17.3 / 19.2 and 28.3 / 28.9), one pick also unless
   //    the last piece would be all but empty (4608 wide, nine KiB, 23.3 / 22.4), but not of fp32 rows (combine, 16 / 6 KiB: 6880 wide,
-  //    17562 tokens 295 / 265, 6600 wide, 20950 345 / 322; 2560 wide, 1198 10.6 / 9.1; 30 steps 0.96 of the time, 30 of dispatch + combine 0.97);
+  //    17562 tokens 295 / 265, 6600 wide, 20950 345 / 322; 2560 wide, 1198 10.6 / 9.1; 30 steps 0.96 of the time, 30 of
+  //    dispatch + combine 0.97);
   //  - fp32 rows, which have twice the bytes, outside DP groups: 4 KiB of one pick (2 KiB up to 384 tokens, unless the row
   //    has two pieces), 2 KiB of two (one pick, 7168 wide, 208 tokens 9.0 / 8.4, 4096 wide, 2428 20.4 / 19.6; two picks of
   //    8 KiB / 2 KiB, 7680 wide, 4928 91.6 / 89.2).
@@ -382,8 +383,8 @@ CombineForm combine_form_of(const WorldHost &w, uint32_t elem_bytes) {
   // wide, beyond 2048 tokens: 0.975; up to 2048 0.99).  Ten, eight and two / five and five: 512 wide, 1160 14.6 / 14.0, 3584
   // wide, 352 15.5 / 15.2.  Of 16-bit rows neither in large steps of 7 KiB and more (six 0.97 to 1.04, ten 1.012), nor where the
   // rows are more than 512 MiB (combine, six, 2560 wide, 50368 tokens 298 / 312, 2048 wide, 52608 252 / 263; ten, 2048 wide, 50224
-  // 364 / 384; 35 steps of that size 0.98 of the time, 69 smaller ones 1.03; dispatch + combine 0.98), but six also there if the last KiB is partial
-  // (1048 wide, 46064 tokens 131 / 117, 1544 wide, 38208 151 / 141), nor for DP groups.
+  // 364 / 384; 35 steps of that size 0.98 of the time, 69 smaller ones 1.03; dispatch + combine 0.98), but six also there if the
+  // last KiB is partial (1048 wide, 46064 tokens 131 / 117, 1544 wide, 38208 151 / 141), nor for DP groups.
   const bool large = gathered > 512ull << 20 && (w.K > 6 || whole_pieces);
   const bool halves = elem_bytes == 4 || (!grouped && (tokens <= 2048 || (nvec_segments < 7 && !large)));
   switch (w.K) {

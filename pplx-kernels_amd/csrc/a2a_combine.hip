@@ -265,14 +265,9 @@ int launch_combine_v(const WorldHost &w, const CT &tab, bool grouped, hipStream_
   const uint32_t segments = (nvec_segments + VPL - 1) / VPL;
   const uint64_t waves = (uint64_t)(grouped ? w.G : w.R) * w.M * segments;
   const dim3 grid((uint32_t)((waves + kWavesPerBlock - 1) / kWavesPerBlock)), block(kWavesPerBlock * kWave);
-  if (grouped) {
-    hipLaunchKernelGGL((combine_gather<T, U, CT, KB, VPL, true>), grid, block, 0, s, w, tab, segments,
-                       make_fast_div(segments));
-  } else {
-    hipLaunchKernelGGL((combine_gather<T, U, CT, KB, VPL, false>), grid, block, 0, s, w, tab, segments,
-                       make_fast_div(segments));
-  }
-  return (int)hipGetLastError();
+  const FastDiv by_segments = make_fast_div(segments);
+  if (grouped) return launch_kernel(combine_gather<T, U, CT, KB, VPL, true>, grid, block, 0, s, w, tab, segments, by_segments);
+  return launch_kernel(combine_gather<T, U, CT, KB, VPL, false>, grid, block, 0, s, w, tab, segments, by_segments);
 }
 
 // Whether 8 KiB pieces of a 16-bit row make workgroups that come out even, two to four of them to each of the 256 CUs,

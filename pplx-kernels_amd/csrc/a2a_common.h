@@ -5,10 +5,29 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "a2a_device.h"
 
 namespace pplx_amd {
 namespace {
+
+// Launches `kernel` on arguments of its parameters' own types (or types derived from them) and returns a hipError_t as
+// int.  By hipLaunchKernel, which takes the addresses of the arguments, and not by <<<>>>: that copies every argument into
+// its stub, a rank table of 9 KiB twice, and passes the launch's shape by a stack of the thread's.  Host time of a launch,
+// us, <<<>>> / this: 104 bytes of arguments 2.45 / 2.25, 176 bytes 2.97 / 2.76, 9 KiB 3.41 / 3.16.
+template <typename P, typename A> const void *argument(const A &a) {
+  static_assert(std::is_same_v<P, A> || std::is_base_of_v<P, A>, "an argument that would be converted");
+  return static_cast<const P *>(&a);
+}
+template <typename... P, typename... A>
+int launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, uint32_t lds, hipStream_t s, const A &...a) {
+  const void *args[] = {argument<P>(a)...};
+  const hipError_t err =
+      hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, const_cast<void **>(args), lds, s);
+  if (err != hipSuccess) (void)hipGetLastError();  // (reported here, and not once more by whoever asks for the last one)
+  return (int)err;
+}
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));

@@ -697,8 +697,7 @@ template <class DT>
 int launch_scatter_t(const WorldHost &w, const DT &tab, Slots slots, hipStream_t s) {
   const uint32_t tokens = w.G * w.M;
   if (!scatter_has_register_rows(w)) {
-    hipLaunchKernelGGL(dispatch_scatter_long<DT>, dim3(tokens), dim3(256), 0, s, w, tab);
-    return (int)hipGetLastError();
+    return launch_kernel(dispatch_scatter_long<DT>, dim3(tokens), dim3(256), 0, s, w, tab);
   }
   const uint32_t ksplit = pick_ksplit(w, kWave);
   const uint32_t kper = (w.K + ksplit - 1) / ksplit;
@@ -733,10 +732,8 @@ int launch_scatter_t(const WorldHost &w, const DT &tab, Slots slots, hipStream_t
 #undef PPLX_LAUNCH_ROW_VARIANT
 #define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                               \
   do {                                                                                           \
-    if (plan.in_turn)                                                                       \
-      hipLaunchKernelGGL((KERNEL<NV, EXACT, DT, true>), grid, block, lds, s, w, tab, ksplit, kper);  \
-    else                                                                                         \
-      hipLaunchKernelGGL((KERNEL<NV, EXACT, DT, false>), grid, block, lds, s, w, tab, ksplit, kper); \
+    if (plan.in_turn) return launch_kernel(KERNEL<NV, EXACT, DT, true>, grid, block, lds, s, w, tab, ksplit, kper); \
+    return launch_kernel(KERNEL<NV, EXACT, DT, false>, grid, block, lds, s, w, tab, ksplit, kper); \
   } while (0)
   if (slots == Slots::kScanned) {
     if (staged) PPLX_LAUNCH_ROW_VARIANT(dispatch_scatter_scanned, 0, false);
@@ -748,7 +745,7 @@ int launch_scatter_t(const WorldHost &w, const DT &tab, Slots slots, hipStream_t
 #undef PPLX_LAUNCH_ROW_VARIANT
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
 #undef PPLX_ROW_KERNEL_ARGS
-  return (int)hipGetLastError();
+  return (int)hipErrorInvalidValue;
 }
 
 template <class DT>
@@ -773,10 +770,8 @@ int launch_fused_t(const WorldHost &w, const DT &tab, uint32_t pick_vector, hipS
 #define PPLX_ROW_KERNEL_ARGS shape
 #define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                                                       \
   do {                                                                                                                   \
-    if (w.K > 8)                                                                                                         \
-      hipLaunchKernelGGL((KERNEL<NV, EXACT, DT, true>), grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS);              \
-    else                                                                                                                 \
-      hipLaunchKernelGGL((KERNEL<NV, EXACT, DT, false>), grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS);             \
+    if (w.K > 8) return launch_kernel(KERNEL<NV, EXACT, DT, true>, grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS);   \
+    return launch_kernel(KERNEL<NV, EXACT, DT, false>, grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS);               \
   } while (0)
 #define PPLX_LAUNCH_LARGE_ROW_VARIANT(KERNEL) return (int)hipErrorInvalidValue
   if (staged) PPLX_LAUNCH_ROW_VARIANT(dispatch_fused, 0, false);
@@ -784,7 +779,7 @@ int launch_fused_t(const WorldHost &w, const DT &tab, uint32_t pick_vector, hipS
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
 #undef PPLX_LAUNCH_ROW_VARIANT
 #undef PPLX_ROW_KERNEL_ARGS
-  return (int)hipGetLastError();
+  return (int)hipErrorInvalidValue;
 }
 
 // Steps of several tiles leave the last routing launch out (the scatter's waves work their own
@@ -905,15 +900,11 @@ DispatchPlan dispatch_plan(const WorldHost &w) {
 }
 
 int launch_bind_dispatch(DispatchRank *table, const BindDispatchBatch &b, void *stream) {
-  hipLaunchKernelGGL((bind_rows<BindDispatchBatch, DispatchRank>), dim3(1), dim3(256), 0,
-                     (hipStream_t)stream, table, b);
-  return (int)hipGetLastError();
+  return launch_kernel(bind_rows<BindDispatchBatch, DispatchRank>, dim3(1), dim3(256), 0, (hipStream_t)stream, table, b);
 }
 
 int launch_bind_combine(CombineRank *table, const BindCombineBatch &b, void *stream) {
-  hipLaunchKernelGGL((bind_rows<BindCombineBatch, CombineRank>), dim3(1), dim3(256), 0,
-                     (hipStream_t)stream, table, b);
-  return (int)hipGetLastError();
+  return launch_kernel(bind_rows<BindCombineBatch, CombineRank>, dim3(1), dim3(256), 0, (hipStream_t)stream, table, b);
 }
 
 int launch_dispatch(const WorldHost &w, const DispatchRank *inline_rows, uint32_t pick_vector, void *stream) {

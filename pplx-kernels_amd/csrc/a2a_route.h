@@ -293,17 +293,17 @@ int launch_route_pv(const WorldDev &w, const DT &tab, const RouteSpan &span, hip
   const uint32_t tiles = (span.v_count + tile - 1) / tile;
   const uint32_t lds = route_lds_bytes(w.E, span.tile_chunks);
   if (tiles > 1) {
-    hipLaunchKernelGGL((route_count<DT, PV>), dim3(tiles), dim3(block),
-                       span.tile_chunks * w.E * sizeof(unsigned long long), s, w, tab, span);
-    if (span.tile_row == nullptr)
-      hipLaunchKernelGGL((route_scan<DT>), dim3((w.E + 3) / 4), dim3(256), 0, s, w, tab, span, tiles);
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return (int)err;
+    int err = launch_kernel(route_count<DT, PV>, dim3(tiles), dim3(block),
+                            span.tile_chunks * w.E * (uint32_t)sizeof(unsigned long long), s, w, tab, span);
+    if (err) return err;
+    if (span.tile_row == nullptr) {
+      err = launch_kernel(route_scan<DT>, dim3((w.E + 3) / 4), dim3(256), 0, s, w, tab, span, tiles);
+      if (err) return err;
+    }
     if (span.tile_mask != nullptr) return 0;  // the scatter works the slots out
   }
-  hipLaunchKernelGGL((route_slots<DT, PV>), dim3(tiles), dim3(block), lds, s, w, tab, span,
-                     tiles > 1 ? 1u : 0u);
-  return (int)hipGetLastError();
+  const uint32_t scanned = tiles > 1 ? 1 : 0;
+  return launch_kernel(route_slots<DT, PV>, dim3(tiles), dim3(block), lds, s, w, tab, span, scanned);
 }
 
 template <class DT>

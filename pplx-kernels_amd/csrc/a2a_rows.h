@@ -228,10 +228,10 @@ inline bool row_has_register_variant(const WorldDev &w) {
 }  // namespace
 }  // namespace pplx_amd
 
-// Picks the register variant for the row size and launches KERNEL<NV, EXACT, DT>.
+// Picks the register variant for the row size, launches KERNEL<NV, EXACT, DT> and returns what launch_kernel says.
 // Rows beyond 8 KiB exist only for dispatch_scatter (PPLX_LAUNCH_LARGE_ROW_VARIANT).
 #define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                               \
-  hipLaunchKernelGGL((KERNEL<NV, EXACT, DT>), grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS)
+  return launch_kernel(KERNEL<NV, EXACT, DT>, grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS)
 
 #define PPLX_DISPATCH_ROW_VARIANTS(KERNEL)                                                       \
   do {                                                                                           \

@@ -147,8 +147,7 @@ int launch_split_stage_tokens_t(const WorldHost &w, const SplitDev &sp, const DT
   const uint32_t lds = 0;
   const uint32_t tokens = w.G * w.M;
   if (!row_has_register_variant(w)) {
-    hipLaunchKernelGGL(split_stage_tokens_long<DT>, dim3(tokens), dim3(256), 0, s, w, tab, sp);
-    return (int)hipGetLastError();
+    return launch_kernel(split_stage_tokens_long<DT>, dim3(tokens), dim3(256), 0, s, w, tab, sp);
   }
   const uint64_t row_bytes = (uint64_t)tokens * sp.token_stride;
   const uint32_t write_through = row_bytes <= kWriteThroughMaxBytes ? 1u : 0u;
@@ -158,7 +157,6 @@ int launch_split_stage_tokens_t(const WorldHost &w, const SplitDev &sp, const DT
   PPLX_DISPATCH_ROW_VARIANTS(split_stage_tokens);
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
 #undef PPLX_ROW_KERNEL_ARGS
-  return (int)hipGetLastError();
 }
 
 template <class CT>
@@ -166,9 +164,9 @@ int launch_split_deliver_t(const WorldHost &w, const SplitDev &sp, const CT &tab
   const uint32_t nvec = w.H / 8;
   const uint32_t segments = (nvec + 8 * kWave - 1) / (8 * kWave);
   const uint64_t waves = (uint64_t)w.R * w.M * segments;
-  hipLaunchKernelGGL(split_deliver<CT>, dim3((uint32_t)((waves + 3) / 4)), dim3(256), 0, s, w, tab, sp, segments,
-                     make_fast_div(segments));
-  return (int)hipGetLastError();
+  const FastDiv by_segments = make_fast_div(segments);
+  return launch_kernel(split_deliver<CT>, dim3((uint32_t)((waves + 3) / 4)), dim3(256), 0, s, w, tab, sp, segments,
+                       by_segments);
 }
 
 }  // namespace

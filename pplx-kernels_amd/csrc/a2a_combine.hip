@@ -461,9 +461,9 @@ CombineForm combine_form(const WorldHost &w, int in_dtype) { return combine_form
 
 int launch_combine(const WorldHost &w, const CombineRank *inline_rows, int in_dtype, int out_dtype,
                    void *stream) {
-  if (inline_rows)
-    return launch_combine_t(w, make_inline(w, inline_rows), in_dtype, out_dtype, (hipStream_t)stream);
-  return launch_combine_t(w, HbmCombine{w.crank}, in_dtype, out_dtype, (hipStream_t)stream);
+  return with_table<InlineCombine>(w, inline_rows, HbmCombine{w.crank}, [&](const auto &tab) {
+    return launch_combine_t(w, tab, in_dtype, out_dtype, (hipStream_t)stream);
+  });
 }
 
 }  // namespace pplx_amd

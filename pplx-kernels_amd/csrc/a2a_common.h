@@ -5,6 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <iterator>
 #include <type_traits>
 
 #include "a2a_device.h"
@@ -35,16 +36,16 @@ typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-struct InlineDispatch {  // the table itself is the kernel argument
-  DispatchRank rows[kInlineRanks];
+template <uint32_t N> struct InlineDispatch {  // the table itself is the kernel argument
+  DispatchRank rows[N];
   __device__ __forceinline__ const DispatchRank &at(uint32_t i) const { return rows[i]; }
 };
 struct HbmDispatch {
   const DispatchRank *rows;
   __device__ __forceinline__ const DispatchRank &at(uint32_t i) const { return rows[i]; }
 };
-struct InlineCombine {
-  CombineRank rows[kInlineRanks];
+template <uint32_t N> struct InlineCombine {
+  CombineRank rows[N];
   __device__ __forceinline__ const CombineRank &at(uint32_t i) const { return rows[i]; }
 };
 struct HbmCombine {
@@ -268,16 +269,17 @@ __device__ __forceinline__ uint32_t combine_rank_tokens(const WorldDev &w, const
   return n < w.M ? n : w.M;
 }
 
-inline InlineDispatch make_inline(const WorldDev &w, const DispatchRank *rows) {
-  InlineDispatch t{};
-  for (uint32_t i = 0; i < w.R && i < kInlineRanks; ++i) t.rows[i] = rows[i];
-  return t;
-}
-
-inline InlineCombine make_inline(const WorldDev &w, const CombineRank *rows) {
-  InlineCombine t{};
-  for (uint32_t i = 0; i < w.R && i < kInlineRanks; ++i) t.rows[i] = rows[i];
-  return t;
+// Calls `launch` with the world's rank table: among the arguments, in the shorter of the two forms that hold it, or
+// where `rows` is NULL in HBM.
+template <template <uint32_t> class Inline, class Row, class Hbm, class Launch>
+int with_table(const WorldDev &w, const Row *rows, const Hbm &in_hbm, Launch &&launch) {
+  auto with = [&](auto table) {
+    for (uint32_t i = 0; i < w.R && i < std::size(table.rows); ++i) table.rows[i] = rows[i];
+    return launch(table);
+  };
+  if (!rows) return launch(in_hbm);
+  if (w.R <= kShortInlineRanks) return with(Inline<kShortInlineRanks>{});
+  return with(Inline<kInlineRanks>{});
 }
 
 }  // namespace

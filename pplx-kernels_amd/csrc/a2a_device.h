@@ -209,6 +209,11 @@ inline StageLayout stage_layout(uint32_t row_bytes, uint32_t scales, uint64_t to
 // tables in the arguments / in HBM, dispatch and combine of one buffer set: 1 rank, 32 tokens of 2 KiB 3.77 / 3.50 and
 // 3.27 / 2.87; 64 x 1 DSv3 tokens 5.53 / 5.26 and 4.01 / 3.58; 8 x 128 12.69 / 12.51 and 22.12 / 21.90.
 constexpr uint32_t kInlineRanks = 64;
+// A table of up to this many ranks goes in an argument of that size (1152 bytes for dispatch, 640 for combine) and not in
+// one for kInlineRanks: what a launch costs the host grows with its arguments (2.27 us at 1240 bytes, 2.49 at 9304), which
+// are filled and copied besides.  Steps, us, 64 ranks' room / this: 8 x 4 tokens, per-rank calls 18.2 / 17.2; 4 ranks in
+// groups of two, 20 tokens, one call 9.2 / 8.5; 8 x 128, split 37.6 / 35.1.  Eight is what a node holds.
+constexpr uint32_t kShortInlineRanks = 8;
 constexpr uint32_t kBindBatch = 64;
 // A one-launch dispatch whose rows (all picks of all tokens) stay within this many bytes and go through registers
 // stores them write-through into the 256 MB last-level cache instead of streaming them past it.  That pays where

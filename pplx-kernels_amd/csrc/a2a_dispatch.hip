@@ -326,7 +326,7 @@ __device__ __forceinline__ void count_earlier_picks(const WorldDev &w, const Tab
 // numbers of picks in one kernel / apart, medians of two runs of 360 launches: 512-byte rows, 8 x 128 tokens, top-8 6.28 6.36 /
 // 6.12 6.24, 8 x 512, top-4 7.64 7.72 / 7.44 7.64; 1 KiB rows, 8 x 128, top-8 level at 6.20 - 6.32).
 template <int NV, bool EXACT, class DT, bool MANY>
-__global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, DT tab, FusedShape shape) {
+__device__ __forceinline__ void dispatch_in_one(const WorldDev &w, const DT &tab, const FusedShape &shape) {
   const uint32_t ksplit = shape.ksplit, kper = shape.kper, tokens_per_block = shape.tokens_per_block;
   const uint32_t pick_vector = shape.pick_vector, write_through = shape.write_through;
   constexpr uint32_t kFusedThreads = fused_threads(NV);
@@ -468,6 +468,20 @@ __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, 
       if (dispatch_group_overflows(w, rows, g)) atomicOr(w.faults, kFaultTooManyTokens);
     }
   }
+}
+
+template <int NV, bool EXACT, class DT, bool MANY>
+__global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, DT tab, FusedShape shape) {
+  dispatch_in_one<NV, EXACT, DT, MANY>(w, tab, shape);
+}
+// ... with a table of few ranks among the arguments
+template <int NV, bool EXACT, class DT, bool MANY>
+__global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused_few(WorldDev w, DT tab, FusedShape shape) {
+  dispatch_in_one<NV, EXACT, DT, MANY>(w, tab, shape);
+}
+template <int NV, bool EXACT, class DT, bool MANY> constexpr auto fused_kernel() {
+  if constexpr (std::is_same_v<DT, InlineDispatch<kShortInlineRanks>>) return dispatch_fused_few<NV, EXACT, DT, MANY>;
+  else return dispatch_fused<NV, EXACT, DT, MANY>;
 }
 
 // Rows longer than the register variants cover: stream each vector K times.
@@ -768,14 +782,14 @@ int launch_fused_t(const WorldHost &w, const DT &tab, uint32_t pick_vector, hipS
   const uint32_t write_through = row_bytes <= (staged ? kLdsWriteThroughMaxBytes : kWriteThroughMaxBytes) ? 1u : 0u;
   const FusedShape shape{ksplit, kper, tokens_per_block, pick_vector, write_through};
 #define PPLX_ROW_KERNEL_ARGS shape
-#define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                                                       \
-  do {                                                                                                                   \
-    if (w.K > 8) return launch_kernel(KERNEL<NV, EXACT, DT, true>, grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS);   \
-    return launch_kernel(KERNEL<NV, EXACT, DT, false>, grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS);               \
+#define PPLX_LAUNCH_ROW_VARIANT(KERNEL, NV, EXACT)                                                              \
+  do {                                                                                                          \
+    if (w.K > 8) return launch_kernel(KERNEL<NV, EXACT, DT, true>(), grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS); \
+    return launch_kernel(KERNEL<NV, EXACT, DT, false>(), grid, block, lds, s, w, tab, PPLX_ROW_KERNEL_ARGS);    \
   } while (0)
 #define PPLX_LAUNCH_LARGE_ROW_VARIANT(KERNEL) return (int)hipErrorInvalidValue
-  if (staged) PPLX_LAUNCH_ROW_VARIANT(dispatch_fused, 0, false);
-  else PPLX_DISPATCH_ROW_VARIANTS(dispatch_fused);
+  if (staged) PPLX_LAUNCH_ROW_VARIANT(fused_kernel, 0, false);
+  else PPLX_DISPATCH_ROW_VARIANTS(fused_kernel);
 #undef PPLX_LAUNCH_LARGE_ROW_VARIANT
 #undef PPLX_LAUNCH_ROW_VARIANT
 #undef PPLX_ROW_KERNEL_ARGS
@@ -909,8 +923,9 @@ int launch_bind_combine(CombineRank *table, const BindCombineBatch &b, void *str
 
 int launch_dispatch(const WorldHost &w, const DispatchRank *inline_rows, uint32_t pick_vector, void *stream) {
   if (pick_vector != 4 && pick_vector != 2) pick_vector = 1;
-  if (inline_rows) return launch_dispatch_t(w, make_inline(w, inline_rows), pick_vector, (hipStream_t)stream);
-  return launch_dispatch_t(w, HbmDispatch{w.drank}, pick_vector, (hipStream_t)stream);
+  return with_table<InlineDispatch>(w, inline_rows, HbmDispatch{w.drank}, [&](const auto &tab) {
+    return launch_dispatch_t(w, tab, pick_vector, (hipStream_t)stream);
+  });
 }
 
 }  // namespace pplx_amd

@@ -173,13 +173,15 @@ int launch_split_deliver_t(const WorldHost &w, const SplitDev &sp, const CT &tab
 
 int launch_split_stage_tokens(const WorldHost &w, const SplitDev &sp, const DispatchRank *inline_rows,
                               void *stream) {
-  if (inline_rows) return launch_split_stage_tokens_t(w, sp, make_inline(w, inline_rows), (hipStream_t)stream);
-  return launch_split_stage_tokens_t(w, sp, HbmDispatch{w.drank}, (hipStream_t)stream);
+  return with_table<InlineDispatch>(w, inline_rows, HbmDispatch{w.drank}, [&](const auto &tab) {
+    return launch_split_stage_tokens_t(w, sp, tab, (hipStream_t)stream);
+  });
 }
 
 int launch_split_deliver(const WorldHost &w, const SplitDev &sp, const CombineRank *inline_rows, void *stream) {
-  if (inline_rows) return launch_split_deliver_t(w, sp, make_inline(w, inline_rows), (hipStream_t)stream);
-  return launch_split_deliver_t(w, sp, HbmCombine{w.crank}, (hipStream_t)stream);
+  return with_table<InlineCombine>(w, inline_rows, HbmCombine{w.crank}, [&](const auto &tab) {
+    return launch_split_deliver_t(w, sp, tab, (hipStream_t)stream);
+  });
 }
 
 }  // namespace pplx_amd

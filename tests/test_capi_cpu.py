@@ -288,6 +288,13 @@ def test_one_launch_dispatch_of_short_rows_leaves_room_for_two_workgroups():
     assert all(v <= 64 for v in short.values()), short
 
 
+def test_one_launch_dispatch_with_a_short_table_leaves_the_same_room():
+    """The same for the kernels that take a table of few ranks among their arguments."""
+    name = re.compile(r"18dispatch_fused_fewILi([123])ELb1E.*Lb0EEE")
+    short = {k[".name"]: k[".vgpr_count"] for k in _gpu_kernels_of(ops._LIB_PATH) if name.search(k[".name"])}
+    assert len(short) == 3 and all(v <= 64 for v in short.values()), short
+
+
 def test_bench_refuses_more_than_one_gpu():
     """Every simulated rank shares one GPU's HBM: `bench.py --gpus N` with N above 1 (or under a
     launcher that sets WORLD_SIZE) exits with a message that says so, before it touches a GPU."""

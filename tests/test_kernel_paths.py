@@ -732,3 +732,43 @@ def test_binding_for_a_destroyed_world_fails_at_the_launch():
     for launch in (bound.dispatch, bound.combine):
         with pytest.raises(RuntimeError, match="the world has been destroyed"):
             launch()
+
+
+# ---------------------------------------------------------------------------
+# Rank tables among the arguments: up to eight ranks in a short one
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize("ranks,dp", [(1, 1), (7, 1), (8, 1), (8, 4), (9, 1), (10, 2), (63, 1), (64, 2)])
+@pytest.mark.parametrize("tokens,H,form", [(40, 1024, ONE_LAUNCH), (4160, 64, TABLES)])
+def test_tables_of_few_and_of_many_ranks(ranks, dp, tokens, H, form):
+    E = 2 * ranks if ranks > 1 else 8
+    M = tokens * dp // ranks + 1
+    spec = WorkloadSpec("tables", 17, ranks, E, min(3, E), H, M, torch.bfloat16, dp_size=dp, tokens="uniform")
+    assert ops.plan_of(ops.Config(M, E, spec.experts_per_token, ranks, dp, H, 2 * H, 0)).dispatch_form == form
+    step = DeviceStep(spec, generate(spec, seed=ranks))
+    world = make_world(spec, group_name="tables")
+    step.dispatch_world(world)
+    expected = check_dispatch_against_oracle(step)
+    step.expert_y_all.normal_(generator=torch.Generator(device="cuda").manual_seed(ranks))
+    step.combine_world(world)
+    check_combine_against_oracle(step, expected.slot_map)
+    for t in (step.expert_num_tokens_all, step.expert_x_all):
+        t.zero_()
+    for t in step.out_tokens:
+        t.fill_(float("nan"))
+    for do_send in (True, False):
+        for r, ata in enumerate(world.ranks):
+            ata.dispatch(
+                out_expert_num_tokens=step.expert_num_tokens[r], out_expert_x=step.expert_x[r], out_expert_x_scale=None,
+                dp_x=step.dp_x[r], dp_x_scale=None, indices=step.indices[r], bound_m=step.bound_m[r],
+                do_send=do_send, do_recv=not do_send,
+            )  # fmt: skip
+    check_dispatch_against_oracle(step, expected)
+    for do_send in (True, False):
+        for r, ata in enumerate(world.ranks):
+            ata.combine(
+                out_tokens=step.out_tokens[r], indices=step.indices[r], weights=step.weights[r],
+                expert_y=step.expert_y[r], bound_m=step.bound_m[r], do_send=do_send, do_recv=not do_send,
+            )  # fmt: skip
+    check_combine_against_oracle(step, expected.slot_map)
+    assert world.faults() == 0
+    world.destroy()

@@ -61,6 +61,61 @@ const char *status_name(int status) {
 // ---------------------------------------------------------------------------
 constexpr int kOps = 2, kModes = 3;  // (dispatch, combine) x (NONE, SEND, RECV)
 
+// The tensors of one recorded call.  Those of a call from Python are kept by their Python objects, whose counters are plain
+// words: a reference to the tensor itself is an atomic operation to take and another to let go, 80 ns for the seven of a
+// dispatch.  An object keeps its tensor, and the tensor's storage goes with either.
+class Kept {
+ public:
+  Kept() = default;
+  Kept(Kept &&) = default;
+  Kept &operator=(Kept &&) = default;
+  Kept(const Kept &) = delete;
+  Kept &operator=(const Kept &) = delete;
+  ~Kept() { clear(); }
+  bool empty() const { return tensors_.empty() && objects_.empty(); }
+  size_t size() const { return tensors_.size() + objects_.size(); }
+  bool has_objects() const { return !objects_.empty(); }
+  void add(const at::Tensor &t) { tensors_.push_back(t); }
+  void add(PyObject *o) {  // under the interpreter lock
+    objects_.push_back(o);
+    Py_INCREF(o);
+  }
+  void take(Kept &other) {
+    tensors_.insert(tensors_.end(), std::make_move_iterator(other.tensors_.begin()),
+                    std::make_move_iterator(other.tensors_.end()));
+    other.tensors_.clear();
+    objects_.insert(objects_.end(), other.objects_.begin(), other.objects_.end());
+    other.objects_.clear();
+  }
+  // (what lets objects go takes the interpreter lock, unless it has gone with the interpreter)
+  void clear() {
+    tensors_.clear();
+    if (objects_.empty()) return;
+    if (Py_IsInitialized()) {
+      const PyGILState_STATE held = PyGILState_Ensure();
+      clear_objects();
+      PyGILState_Release(held);
+    }
+    objects_.clear();
+  }
+  void clear_under_gil() {
+    tensors_.clear();
+    clear_objects();
+  }
+
+ private:
+  void clear_objects() {
+    // (a callback of a tensor may come back to the call that is being let go)
+    std::vector<PyObject *> gone;
+    gone.swap(objects_);
+    for (PyObject *o : gone) Py_DECREF(o);
+    gone.clear();
+    if (objects_.empty()) objects_.swap(gone);  // (with its memory)
+  }
+  std::vector<at::Tensor> tensors_;
+  std::vector<PyObject *> objects_;
+};
+
 struct World {
   std::string key;
   uint64_t id = 0;  // never given out again, unlike the address `ptr`
@@ -71,7 +126,7 @@ struct World {
   // A step's kernels are enqueued by the last rank to call, so the tensors of the ranks that
   // called earlier are kept alive until then: a temporary such as x.to(device) must not go
   // back to the caching allocator before it has been read.
-  std::array<std::vector<std::vector<at::Tensor>>, kOps * kModes> held;
+  std::array<std::vector<Kept>, kOps * kModes> held;
 
   World() = default;
   World(const World &) = delete;
@@ -189,9 +244,9 @@ fptr_t create_rank(const std::string &transport, const std::string &group_name, 
 // A launched step's tensors change places with the cleared vectors of the thread's step before, so that
 // neither side allocates again from step to step.
 struct Released {
-  typedef std::vector<std::vector<at::Tensor>> PerRank;
+  typedef std::vector<Kept> PerRank;
   PerRank step;
-  std::vector<at::Tensor> others;
+  Kept others;
   bool has_step = false;
 
   Released() = default;
@@ -199,7 +254,15 @@ struct Released {
   Released &operator=(const Released &) = delete;
   ~Released() {
     if (!has_step) return;
-    for (auto &tensors : step) tensors.clear();
+    bool objects = false;
+    for (const Kept &kept : step) objects = objects || kept.has_objects();
+    if (objects && Py_IsInitialized()) {
+      const PyGILState_STATE held = PyGILState_Ensure();  // (once for all ranks)
+      for (Kept &kept : step) kept.clear_under_gil();
+      PyGILState_Release(held);
+    } else {
+      for (Kept &kept : step) kept.clear();
+    }
     if (spare().empty()) spare().swap(step);  // (a callback of a tensor may have left its own)
   }
   void take_step(PerRank &held) {
@@ -208,10 +271,7 @@ struct Released {
     held.swap(step);
     has_step = true;
   }
-  void take(std::vector<at::Tensor> &kept) {
-    others.insert(others.end(), std::make_move_iterator(kept.begin()), std::make_move_iterator(kept.end()));
-    kept.clear();
-  }
+  void take(Kept &kept) { others.take(kept); }
 
  private:
   static PerRank &spare() {
@@ -323,11 +383,11 @@ void check_dispatch(const at::Tensor &outExpertNumTokens, const at::Tensor &outE
   check_tensor(indices, 2, "indices");
   TORCH_CHECK(indices.scalar_type() == at::kUInt32, "indices must be of type UInt32");
   check_bound_m(boundM);
-  TORCH_CHECK(indices.size(0) == dpX.size(0), "indices.size(0) must be equal to dpX.size(0)");
+  TORCH_CHECK(indices.sizes()[0] == dpX.sizes()[0], "indices.size(0) must be equal to dpX.size(0)");
 }
 
 void check_picks(const at::Tensor &indices, uint64_t experts_per_token) {
-  TORCH_CHECK(indices.size(1) == (int64_t)experts_per_token, "indices.size(1) must be equal to the experts per token");
+  TORCH_CHECK(indices.sizes()[1] == (int64_t)experts_per_token, "indices.size(1) must be equal to the experts per token");
 }
 
 // The views of csrc/bindings/all_to_all_ops.cpp:165-195
@@ -337,27 +397,27 @@ pplx_a2a_dispatch_args_t pack_dispatch(const at::Tensor &outExpertNumTokens, con
                                        const at::Tensor *boundM) {
   pplx_a2a_dispatch_args_t a{};
   a.out_expert_num_tokens = static_cast<int32_t *>(outExpertNumTokens.data_ptr());
-  a.out_expert_num_tokens_stride = outExpertNumTokens.stride(0);
+  a.out_expert_num_tokens_stride = outExpertNumTokens.strides()[0];
   const int64_t esz = (int64_t)outExpertX.element_size();
   a.out_expert_x = outExpertX.data_ptr();
-  a.out_expert_x_stride_row = outExpertX.stride(1) * esz;
-  a.out_expert_x_stride_expert = outExpertX.stride(0) * esz;
-  a.out_expert_x_rows = outExpertX.size(1);
+  a.out_expert_x_stride_row = outExpertX.strides()[1] * esz;
+  a.out_expert_x_stride_expert = outExpertX.strides()[0] * esz;
+  a.out_expert_x_rows = outExpertX.sizes()[1];
   if (outExpertXScale) {
     a.out_expert_x_scale = static_cast<float *>(outExpertXScale->data_ptr());
-    a.out_expert_x_scale_stride_elem = outExpertXScale->stride(2);
-    a.out_expert_x_scale_stride_row = outExpertXScale->stride(1);
-    a.out_expert_x_scale_stride_expert = outExpertXScale->stride(0);
+    a.out_expert_x_scale_stride_elem = outExpertXScale->strides()[2];
+    a.out_expert_x_scale_stride_row = outExpertXScale->strides()[1];
+    a.out_expert_x_scale_stride_expert = outExpertXScale->strides()[0];
   }
   a.dp_x = dpX.data_ptr();
-  a.dp_x_stride_row = dpX.stride(0) * (int64_t)dpX.element_size();
+  a.dp_x_stride_row = dpX.strides()[0] * (int64_t)dpX.element_size();
   if (dpXScale) {
     a.dp_x_scale = static_cast<const float *>(dpXScale->data_ptr());
-    a.dp_x_scale_stride_elem = dpXScale->stride(1);
-    a.dp_x_scale_stride_row = dpXScale->stride(0);
+    a.dp_x_scale_stride_elem = dpXScale->strides()[1];
+    a.dp_x_scale_stride_row = dpXScale->strides()[0];
   }
   a.indices = static_cast<const uint32_t *>(indices.data_ptr());
-  a.m = (uint32_t)indices.size(0);
+  a.m = (uint32_t)indices.sizes()[0];
   a.bound_m = boundM ? static_cast<const uint32_t *>(boundM->data_ptr()) : nullptr;
   return a;
 }
@@ -382,24 +442,25 @@ pplx_a2a_combine_args_t pack_combine(const at::Tensor &outTokens, const at::Tens
                                      const at::Tensor *boundM) {
   pplx_a2a_combine_args_t a{};
   a.out_tokens = outTokens.data_ptr();
-  a.out_tokens_stride_row = outTokens.stride(0);
+  a.out_tokens_stride_row = outTokens.strides()[0];
   a.out_dtype = dtype_code(outTokens.scalar_type());
   a.indices = static_cast<const uint32_t *>(indices.data_ptr());
   a.weights = static_cast<const float *>(weights.data_ptr());
-  a.weights_stride_row = weights.stride(0);
+  a.weights_stride_row = weights.strides()[0];
   a.expert_y = expertY.data_ptr();
-  a.expert_y_stride_row = expertY.stride(1);
-  a.expert_y_stride_expert = expertY.stride(0);
-  a.expert_y_rows = expertY.size(1);
+  a.expert_y_stride_row = expertY.strides()[1];
+  a.expert_y_stride_expert = expertY.strides()[0];
+  a.expert_y_rows = expertY.sizes()[1];
   a.in_dtype = dtype_code(expertY.scalar_type());
-  a.m = (uint32_t)indices.size(0);
+  a.m = (uint32_t)indices.sizes()[0];
   a.bound_m = boundM ? static_cast<const uint32_t *>(boundM->data_ptr()) : nullptr;
   return a;
 }
 
+constexpr const char *kUnknownHandle = "pplx_kernels: invalid state: the handle has been destroyed";
 RankRef find_rank(fptr_t ptr) {
   auto it = g_ranks.find(ptr);
-  TORCH_CHECK(it != g_ranks.end(), "pplx_kernels: invalid state: the handle has been destroyed");
+  TORCH_CHECK(it != g_ranks.end(), kUnknownHandle);
   return it->second;
 }
 
@@ -415,11 +476,17 @@ void clear_held(World &world, int op, Released &released) {
   }
 }
 
+// The tensors of a call, and where it came from Python their objects (None among them).
+struct CallTensors {
+  std::initializer_list<const at::Tensor *> tensors;
+  PyObject *const *objects = nullptr;
+};
+
 // After a call into the library: the tensors of a recorded call are kept, and everything kept
 // for the phase is let go once the library holds no recorded call of it any more (the phase
 // has been launched, or the library gave the step up).
-void settle_held(World &world, uint32_t rank, int op, int mode, bool recorded,
-                 std::initializer_list<const at::Tensor *> tensors, Released &released) {
+void settle_held(World &world, uint32_t rank, int op, int mode, bool recorded, const CallTensors &call,
+                 Released &released) {
   uint32_t pending = 0;
   (void)pplx_a2a_world_recorded_calls(world.ptr, op, mode, &pending);
   auto &per_rank = world.held[op * kModes + mode];
@@ -428,10 +495,13 @@ void settle_held(World &world, uint32_t rank, int op, int mode, bool recorded,
     return;
   }
   if (!recorded) return;
-  auto &kept = per_rank[rank];
+  Kept &kept = per_rank[rank];
   if (!kept.empty()) released.take(kept);
-  for (const at::Tensor *t : tensors) {
-    if (t) kept.push_back(*t);
+  size_t i = 0;
+  for (const at::Tensor *t : call.tensors) {
+    if (t && call.objects) kept.add(call.objects[i]);
+    else if (t) kept.add(*t);
+    ++i;
   }
 }
 
@@ -460,7 +530,8 @@ void *current_stream_of(const at::Tensor &t) {
 // csrc/bindings/all_to_all_ops.cpp:122-196.  Optional tensors arrive as pointers (NULL = None).
 void dispatch_core(fptr_t ptr, const at::Tensor &outExpertNumTokens, const at::Tensor &outExpertX,
                    const at::Tensor *outExpertXScale, const at::Tensor &dpX, const at::Tensor *dpXScale,
-                   const at::Tensor &indices, const at::Tensor *boundM, bool doSend, bool doRecv) {
+                   const at::Tensor &indices, const at::Tensor *boundM, bool doSend, bool doRecv,
+                   PyObject *const *objects = nullptr) {
   Released released;
   std::lock_guard<std::mutex> lock(g_mu);
   World *world = nullptr;
@@ -472,7 +543,8 @@ void dispatch_core(fptr_t ptr, const at::Tensor &outExpertNumTokens, const at::T
     auto found = g_ranks.find(ptr);
     if (found != g_ranks.end()) world = found->second.world;
     check_dispatch(outExpertNumTokens, outExpertX, outExpertXScale, dpX, dpXScale, indices, boundM);
-    const RankRef ref = find_rank(ptr);
+    TORCH_CHECK(world, kUnknownHandle);
+    const RankRef ref = found->second;
     check_picks(indices, world->cfg.experts_per_token);
     const int mode = split_mode_of(doSend, doRecv);
 
@@ -487,7 +559,7 @@ void dispatch_core(fptr_t ptr, const at::Tensor &outExpertNumTokens, const at::T
     // stream is the current one of the tensors' device (csrc/bindings/all_to_all_ops.cpp:163,194).
     const int st = pplx_a2a_dispatch((pplx_a2a_t *)ptr, &a, mode, current_stream_of(indices));
     settle_held(*world, ref.rank, 0, mode, st == PPLX_A2A_OK,
-                {&outExpertNumTokens, &outExpertX, outExpertXScale, &dpX, dpXScale, &indices, boundM}, released);
+                {{&outExpertNumTokens, &outExpertX, outExpertXScale, &dpX, dpXScale, &indices, boundM}, objects}, released);
     arguments_refused = st == PPLX_A2A_INVALID_ARGUMENT;
     A2A_CHECK(st);
   } catch (const c10::Error &err) {
@@ -499,7 +571,8 @@ void dispatch_core(fptr_t ptr, const at::Tensor &outExpertNumTokens, const at::T
 
 // csrc/bindings/all_to_all_ops.cpp:238-311
 void combine_core(fptr_t ptr, const at::Tensor &outTokens, const at::Tensor &indices, const at::Tensor &weights,
-                  const at::Tensor &expertY, const at::Tensor *boundM, bool doSend, bool doRecv) {
+                  const at::Tensor &expertY, const at::Tensor *boundM, bool doSend, bool doRecv,
+                  PyObject *const *objects = nullptr) {
   Released released;
   std::lock_guard<std::mutex> lock(g_mu);
   World *world = nullptr;
@@ -508,7 +581,8 @@ void combine_core(fptr_t ptr, const at::Tensor &outTokens, const at::Tensor &ind
     auto found = g_ranks.find(ptr);
     if (found != g_ranks.end()) world = found->second.world;
     check_combine(outTokens, indices, weights, expertY, boundM);
-    const RankRef ref = find_rank(ptr);
+    TORCH_CHECK(world, kUnknownHandle);
+    const RankRef ref = found->second;
     const int mode = split_mode_of(doSend, doRecv);
 
     const pplx_a2a_combine_args_t a = pack_combine(outTokens, indices, weights, expertY, boundM);
@@ -516,7 +590,7 @@ void combine_core(fptr_t ptr, const at::Tensor &outTokens, const at::Tensor &ind
     arguments_refused = false;
     if (mode != PPLX_A2A_SPLIT_NONE) reserve_split_locked(*world, (int)expertY.element_size());
     const int st = pplx_a2a_combine((pplx_a2a_t *)ptr, &a, mode, current_stream_of(indices));
-    settle_held(*world, ref.rank, 1, mode, st == PPLX_A2A_OK, {&outTokens, &indices, &weights, &expertY, boundM},
+    settle_held(*world, ref.rank, 1, mode, st == PPLX_A2A_OK, {{&outTokens, &indices, &weights, &expertY, boundM}, objects},
                 released);
     arguments_refused = st == PPLX_A2A_INVALID_ARGUMENT;
     A2A_CHECK(st);
@@ -613,7 +687,7 @@ PyObject *py_dispatch(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
                 tensor_arg(args[2], "out_expert_x"), optional_tensor_arg(args[3], "out_expert_x_scale"),
                 tensor_arg(args[4], "dp_x"), optional_tensor_arg(args[5], "dp_x_scale"),
                 tensor_arg(args[6], "indices"), optional_tensor_arg(args[7], "bound_m"),
-                PyObject_IsTrue(args[8]) == 1, PyObject_IsTrue(args[9]) == 1);
+                PyObject_IsTrue(args[8]) == 1, PyObject_IsTrue(args[9]) == 1, args + 1);
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }
@@ -625,7 +699,7 @@ PyObject *py_combine(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   combine_core(int_arg(args[0], "fptr"), tensor_arg(args[1], "out_tokens"), tensor_arg(args[2], "indices"),
                tensor_arg(args[3], "weights"), tensor_arg(args[4], "expert_y"),
                optional_tensor_arg(args[5], "bound_m"), PyObject_IsTrue(args[6]) == 1,
-               PyObject_IsTrue(args[7]) == 1);
+               PyObject_IsTrue(args[7]) == 1, args + 1);
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }

@@ -1153,6 +1153,53 @@ def test_a_kept_tensor_may_call_back_when_it_goes():
         a.destroy()
 
 
+@pytest.mark.parametrize("last", ["op", "method", "thread"])
+def test_temporaries_of_both_call_paths_outlive_their_callers(last):
+    """Ranks that call through the registered ops and ranks that call the methods, in one step, all with temporaries
+    that only the recorded calls keep; the step's last call comes by either path, or from another thread."""
+    import gc
+    import threading
+    import weakref
+
+    from pplx_kernels import ops
+
+    spec = _small_spec(name="bothpaths", in_dtype=FP8, hidden_dim=512)
+    step = DeviceStep(spec, generate(spec))
+    ranks = _make_ranks(spec, "bothpaths")
+    refs, gone = [], []
+
+    def call(r: int, through_op: bool) -> None:
+        kw = _dispatch_kw(step, r)
+        for name in ("dp_x", "dp_x_scale", "indices"):
+            kw[name] = kw[name].clone()
+            refs.append(weakref.ref(kw[name], lambda _: gone.append(r)))
+        if through_op:
+            torch.ops.pplx_kernels.all_to_all_intranode_dispatch(ranks[r]._ptr, *kw.values(), True, True)
+        else:
+            ranks[r].dispatch(**kw)
+
+    assert list(_dispatch_kw(step, 0)) == [
+        "out_expert_num_tokens", "out_expert_x", "out_expert_x_scale", "dp_x", "dp_x_scale", "indices", "bound_m"
+    ]  # fmt: skip
+    R = spec.world_size
+    for r in range(R - 1):
+        call(r, r % 2 == 0)
+    assert ops._C.held_tensors(ranks[0]._ptr) == 7 * (R - 1)
+    for _ in range(4):  # (memory that had been given back would be overwritten)
+        torch.full_like(step.dp_x[0].view(torch.uint8), 255)
+    if last == "thread":
+        t = threading.Thread(target=call, args=(R - 1, False))
+        t.start()
+        t.join()
+    else:
+        call(R - 1, last == "op")
+    gc.collect()
+    assert ops._C.held_tensors(ranks[0]._ptr) == 0 and len(gone) == 3 * R
+    check_dispatch_against_oracle(step)
+    for a in ranks:
+        a.destroy()
+
+
 def test_a_step_is_abandoned_when_a_rank_is_refused():
     """Rank 2's arguments fail their checks after ranks 0 and 1 have called: the half-assembled
     step is given up (nothing of it has reached the GPU), the tensors kept for it are let go,

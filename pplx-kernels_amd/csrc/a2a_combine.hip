@@ -28,6 +28,14 @@ template <> struct OutVectors<_Float16> {
   typedef f16x8 by8;
 };
 
+// Streaming or plain.  (By the compiler's own stores: it sees to what may follow a 16-byte store, which it does not know in
+// inline asm to be one, before the registers stored are written again.)
+template <RowStore POLICY, typename V> __device__ __forceinline__ void out_store(V v, PPLX_GLOBAL V *p) {
+  static_assert(POLICY == RowStore::kStream || POLICY == RowStore::kPlain, "out_store");
+  if constexpr (POLICY == RowStore::kStream) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
 template <typename T> struct Row8;
 template <> struct Row8<float> {
   struct Raw {
@@ -55,13 +63,13 @@ template <> struct Row8<float> {
   template <int N> static __device__ __forceinline__ void settle(Raw *raw) {
     SettleAll<2 * N>::of(reinterpret_cast<f32x4 *>(raw));
   }
-  template <typename U>
+  template <typename U, RowStore POLICY>
   static __device__ __forceinline__ void store(uint64_t row, Place p, uint32_t H, const f32x8 &acc) {
     typedef typename OutVectors<U>::by4 vec_t;
     PPLX_GLOBAL vec_t *out = global_ptr<vec_t>(row);
     const f32x4 a = __builtin_shufflevector(acc, acc, 0, 1, 2, 3), b = __builtin_shufflevector(acc, acc, 4, 5, 6, 7);
-    if (p.a < H / 4) __builtin_nontemporal_store(__builtin_convertvector(a, vec_t), out + p.a);
-    if (p.b < H / 4) __builtin_nontemporal_store(__builtin_convertvector(b, vec_t), out + p.b);
+    if (p.a < H / 4) out_store<POLICY>(__builtin_convertvector(a, vec_t), out + p.a);
+    if (p.b < H / 4) out_store<POLICY>(__builtin_convertvector(b, vec_t), out + p.b);
   }
 };
 // The 16-bit types.
@@ -77,10 +85,10 @@ template <typename V> struct Row8By16 {
     return __builtin_nontemporal_load(global_cptr<V>(row) + p);
   }
   template <int N> static __device__ __forceinline__ void settle(Raw *raw) { SettleAll<N>::of(raw); }
-  template <typename U>
+  template <typename U, RowStore POLICY>
   static __device__ __forceinline__ void store(uint64_t row, Place p, uint32_t H, const f32x8 &acc) {
     typedef typename OutVectors<U>::by8 vec_t;
-    if (p < H / 8) __builtin_nontemporal_store(__builtin_convertvector(acc, vec_t), global_ptr<vec_t>(row) + p);
+    if (p < H / 8) out_store<POLICY>(__builtin_convertvector(acc, vec_t), global_ptr<vec_t>(row) + p);
   }
 };
 template <> struct Row8<__bf16> : Row8By16<u32x4> {
@@ -164,7 +172,7 @@ __device__ __forceinline__ void reduce_picks(f32x8 (&acc)[VPL], uint32_t K, uint
 // 1024 tokens 267 and 275.  Copies of a token carry the same weights, so nothing is made of that case.
 template <typename T, typename U, class CT, int KB, int VPL, bool GROUPED>
 __global__ __launch_bounds__(kWavesPerBlock * kWave) void combine_gather(WorldDev w, CT tab, uint32_t segments,
-                                                                         FastDiv by_segments) {
+                                                                         FastDiv by_segments, uint32_t plain_stores) {
   const uint32_t lane = lane_id();
   const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave);
   const uint32_t token = fast_div(wave, by_segments);
@@ -215,8 +223,18 @@ __global__ __launch_bounds__(kWavesPerBlock * kWave) void combine_gather(WorldDe
   for (int v = 0; v < VPL; ++v) at[v] = Row::clamped(Row::place(segment * VPL + v, lane), w.H);
   f32x8 acc[VPL];
   auto store = [&](uint64_t out) {
+    if (plain_stores) {
+      // (fenced: stores of two branches that differ in their hint alone would be made one, without the hint)
+      asm volatile("" ::: "memory");
 #pragma unroll
-    for (int v = 0; v < VPL; ++v) Row::template store<U>(out, Row::place(segment * VPL + v, lane), w.H, acc[v]);
+      for (int v = 0; v < VPL; ++v)
+        Row::template store<U, RowStore::kPlain>(out, Row::place(segment * VPL + v, lane), w.H, acc[v]);
+      asm volatile("" ::: "memory");
+      return;
+    }
+#pragma unroll
+    for (int v = 0; v < VPL; ++v)
+      Row::template store<U, RowStore::kStream>(out, Row::place(segment * VPL + v, lane), w.H, acc[v]);
   };
   if constexpr (!GROUPED) {
     reduce_picks<T, KB, VPL>(acc, w.K, row, weight, 0, no_row == 0, at);
@@ -257,17 +275,34 @@ bool combine_per_group(const WorldHost &w, size_t elem_bytes) {
          (uint64_t)w.R * w.M * w.K * w.H * elem_bytes > kGroupGatherMinBytes;
 }
 
+// Combined rows whose length is no multiple of half a 128-byte line, the unit in which memory takes writes, begin anywhere:
+// stores that stream past the caches cut half lines there, and a small step's kernel ends waiting for those partial writes.
+// Plain stores meet in the caches first.  Dispatch + combine on three buffer sets, 8 ranks, top-2 of 32, us, streaming /
+// plain: 2968 wide, 8 x 16 tokens 7.3 / 7.0, 8 x 64 8.6 / 8.3, 8 x 128 (5.8 MiB) 11.3 / 10.8; 5384 wide, 8 x 64 (5.3 MiB) 10.9 / 10.4;
+// 2008 wide, top-4, 8 x 128 12.2 / 11.8; groups of two, top-3, 2968 wide, 8 x 100 9.9 / 9.6 (45 shapes of groups of two 0.97).
+// Beyond, the lines that stay behind cost what follows more than that: plain stores for 5384 wide, top-4, 8 x 200 34.5 / 37.8, 7176
+// wide, top-2, 8 x 256 35.2 / 40.8.  Rows of whole half lines are level in small steps.  (The same in dispatch, plain instead of
+// written-through stores, gives 2 % of the smallest steps and costs 6 % at 8 x 128 tokens; pieces that begin at half lines of the
+// output instead of the row's start gave nothing in large steps.)
+constexpr uint64_t kPlainStoresMaxBytes = 6ull << 20;
+bool plain_stores(const WorldHost &w) {
+  const uint64_t row = 2ull * w.H;
+  return row % 64 != 0 && (uint64_t)w.R * w.M * row <= kPlainStoresMaxBytes;
+}
+
 template <typename T, typename U, class CT, int KB, int VPL>
 int launch_combine_v(const WorldHost &w, const CT &tab, bool grouped, hipStream_t s) {
-  static_assert(sizeof(WorldDev) + sizeof(HbmCombine) + sizeof(uint32_t) + sizeof(FastDiv) <= kShortArguments,
+  static_assert(sizeof(WorldDev) + sizeof(HbmCombine) + 2 * sizeof(uint32_t) + sizeof(FastDiv) <= kShortArguments,
                 "arguments of combine_gather");
   const uint32_t nvec_segments = (w.H / 8 + kWave - 1) / kWave;
   const uint32_t segments = (nvec_segments + VPL - 1) / VPL;
   const uint64_t waves = (uint64_t)(grouped ? w.G : w.R) * w.M * segments;
   const dim3 grid((uint32_t)((waves + kWavesPerBlock - 1) / kWavesPerBlock)), block(kWavesPerBlock * kWave);
   const FastDiv by_segments = make_fast_div(segments);
-  if (grouped) return launch_kernel(combine_gather<T, U, CT, KB, VPL, true>, grid, block, 0, s, w, tab, segments, by_segments);
-  return launch_kernel(combine_gather<T, U, CT, KB, VPL, false>, grid, block, 0, s, w, tab, segments, by_segments);
+  const uint32_t plain = plain_stores(w) ? 1 : 0;
+  if (grouped)
+    return launch_kernel(combine_gather<T, U, CT, KB, VPL, true>, grid, block, 0, s, w, tab, segments, by_segments, plain);
+  return launch_kernel(combine_gather<T, U, CT, KB, VPL, false>, grid, block, 0, s, w, tab, segments, by_segments, plain);
 }
 
 // Whether 8 KiB pieces of a 16-bit row make workgroups that come out even, two to four of them to each of the 256 CUs,

@@ -772,3 +772,40 @@ def test_tables_of_few_and_of_many_ranks(ranks, dp, tokens, H, form):
     check_combine_against_oracle(step, expected.slot_map)
     assert world.faults() == 0
     world.destroy()
+
+
+# ---------------------------------------------------------------------------
+# Combined rows that cut half lines: plain stores up to 6 MiB of them
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize(
+    "M,H,K,dp,y_dtype",
+    [
+        (1, 8, 1, 1, torch.bfloat16),  # the smallest
+        (3, 40, 2, 1, torch.float16),
+        (9, 992, 6, 1, torch.bfloat16),  # whole half lines: streaming
+        (9, 1000, 6, 1, torch.bfloat16),
+        (70, 2008, 1, 1, torch.bfloat16),  # pieces of several KiB
+        (33, 520, 4, 1, torch.float32),
+        (33, 520, 5, 2, torch.float32),
+        (100, 2968, 3, 4, torch.float16),  # rows shared by a group's members, each stored by itself
+        (392, 1000, 2, 1, torch.bfloat16),  # 5.98 MiB
+        (394, 1000, 2, 1, torch.bfloat16),  # 6.01 MiB
+    ],
+)
+def test_combined_rows_that_cut_half_lines(M, H, K, dp, y_dtype):
+    spec = WorkloadSpec(
+        "cutrows", 23, 8, 16, K, H, M, torch.bfloat16, out_dtype=torch.bfloat16, expert_y_dtype=y_dtype, dp_size=dp,
+        tokens="uniform" if M > 1 else "full",
+    )  # fmt: skip
+    step = DeviceStep(spec, generate(spec, seed=M + H))
+    world = make_world(spec, group_name="cutrows")
+    for replay in range(2):
+        for t in step.out_tokens:
+            t.fill_(float("nan"))
+        step.dispatch_world(world)
+        expected = check_dispatch_against_oracle(step)
+        step.expert_y_all.normal_(generator=torch.Generator(device="cuda").manual_seed(replay))
+        step.combine_world(world)
+        check_combine_against_oracle(step, expected.slot_map)
+    assert world.faults() == 0
+    world.destroy()

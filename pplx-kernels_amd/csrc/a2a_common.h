@@ -87,7 +87,9 @@ __device__ __forceinline__ PPLX_GLOBAL V *as_global(V *p) {
 //                  fit there no longer waits for HBM to take them (dispatch of 8 x 128 DSv3
 //                  tokens: 18.9 instead of 22.6 us; from about 240 MB per step on it is the
 //                  slowest of the three).
-// The compiler offers no builtin for the scoped forms, hence the asm; they are plain vector stores.
+// The compiler offers no builtin for the scoped forms, hence the asm; they are plain vector stores.  A store of 16 bytes
+// wants two wait states before its data registers are written again; the compiler sees to that behind its own stores, not
+// behind asm, hence the s_nop (a kernel whose next instruction wrote them stored wrong values; dispatch measures the same).
 enum class RowStore { kStream, kStreamThrough, kKeep, kPlain };
 
 template <RowStore POLICY, typename V>
@@ -99,13 +101,13 @@ __device__ __forceinline__ void row_store(V v, PPLX_GLOBAL V *p) {
     __builtin_nontemporal_store(v, p);
   } else if constexpr (POLICY == RowStore::kStreamThrough) {
     if constexpr (sizeof(V) == 16) {
-      asm volatile("global_store_dwordx4 %0, %1, off sc1 nt" ::"v"(p), "v"(v) : "memory");
+      asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
     } else {
       asm volatile("global_store_dword %0, %1, off sc1 nt" ::"v"(p), "v"(v) : "memory");
     }
   } else {
     if constexpr (sizeof(V) == 16) {
-      asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
+      asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
     } else {
       asm volatile("global_store_dword %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
     }

@@ -88,7 +88,7 @@ struct alignas(16) CombineRank {
 static_assert(sizeof(CombineRank) == 80, "CombineRank layout");
 
 // Geometry + scratch of a world; passed to every kernel by value, and kept short: in some processes a launch with more
-// than kShortArguments bytes of arguments costs the host 3.4 to 4 us instead of 2.6 (9 KiB no more than 1 KiB).  Beside a
+// than kShortArguments bytes of arguments costs the host 2.75 us and more instead of 2.25 (9 KiB 3.15).  Beside a
 // table in HBM the one-launch dispatch, the scatters and the gather of combine stay within them; the routing kernels, whose
 // RouteSpan alone is 56 bytes, do not.
 constexpr size_t kShortArguments = 112;
@@ -202,7 +202,7 @@ inline StageLayout stage_layout(uint32_t row_bytes, uint32_t scales, uint64_t to
 }
 
 // A step's rank tables reach the kernels in one of two ways.  Worlds of up to kInlineRanks ranks pass them as
-// kernel arguments (9 KiB for dispatch, 5 KiB for combine; HIP on gfx950 takes kernel
+// kernel arguments (up to 9 KiB for dispatch and 5 KiB for combine; HIP on gfx950 takes kernel
 // arguments well beyond 4 KiB, eagerly and as graph nodes).  Larger worlds (drank / crank), and steps that were bound
 // beforehand (pplx_a2a_bound_create), go through tables in HBM, written by bind kernels that take up to kBindBatch rows as
 // arguments each.  Kernels read those faster than their arguments, which no cache holds from one launch to the next.  Us,

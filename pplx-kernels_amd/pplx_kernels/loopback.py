@@ -6,7 +6,7 @@ hand all ranks' tensors over at once; the library then makes one pass over them
 (``pplx_a2a_world_dispatch`` / ``pplx_a2a_world_combine``).  The kernels, the results and
 the argument checks are the same as for ``world_size`` per-rank calls.  The checks, the packing
 and the launch run in compiled code: packed in Python, a step of four ranks took 33 us of host
-time for 10 us of kernels (now 10 us a step), and a bound step 13 us (now 9.5).
+time for 10 us of kernels (now 8.5 us a step), and a bound step 13 us (now 9).
 
 ``capture()`` records whatever the body enqueues on the current stream into a hipGraph
 through the library's own capture entry points, so a step can be replayed without any
@@ -164,7 +164,7 @@ class LoopbackWorld:
         returns a :class:`BoundStep` that launches them as often as wanted, fastest on the stream
         that is current now: the rank tables are written to device memory there (by two small kernels,
         unless the stream is captured), and the step's kernels read them.  Binding takes 18 us of the
-        host for one rank, 60 for 8 and 390 for 64, 10 of them for the tables, which save 1 to 2 us a
+        host for one rank, 60 for 8 and 390 for 64, 10 of them for the tables, which save about 1 us a
         step: a step that is bound for fewer than some ten launches loses by them."""
         d_args = (ops.DispatchArgs * self.world_size)()
         c_args = (ops.CombineArgs * self.world_size)()

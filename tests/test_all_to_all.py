@@ -1200,6 +1200,110 @@ def test_temporaries_of_both_call_paths_outlive_their_callers(last):
         a.destroy()
 
 
+def _swap(t, other):
+    torch.utils.swap_tensors(t, other)
+
+
+def _set(t, other):
+    t.set_(other)
+
+
+def _set_data(t, other):
+    t.data = other
+
+
+@pytest.mark.parametrize("change", [_swap, _set, _set_data])
+@pytest.mark.parametrize("through_op", [False, True])
+@pytest.mark.parametrize("op", ["dispatch", "combine"])
+def test_memory_of_a_recorded_call_outlives_a_change_of_its_tensors(op, through_op, change):
+    """A recorded call names memory.  Its tensors get other memory before the step's last rank calls, and nothing of the
+    program's keeps what they had: the step works on it all the same.  (A tensor that a registered op recorded is
+    referred to twice and refuses to be swapped.)"""
+    spec = _small_spec(name="changed", in_dtype=FP8, hidden_dim=512)
+    step = DeviceStep(spec, generate(spec))
+    ranks = _make_ranks(spec, "changed")
+    kw_of = _dispatch_kw if op == "dispatch" else _combine_kw
+
+    def call(r: int, kw: dict) -> None:
+        if through_op:
+            getattr(torch.ops.pplx_kernels, f"all_to_all_intranode_{op}")(ranks[r]._ptr, *kw.values(), True, True)
+        else:
+            getattr(ranks[r], op)(**kw)
+
+    if op == "combine":
+        for r in range(spec.world_size):
+            ranks[r].dispatch(**_dispatch_kw(step, r))
+        expected = check_dispatch_against_oracle(step)
+        step.expert_y_all.normal_()
+    kept = []
+    for r in range(spec.world_size - 1):
+        kw = {name: t.view(t.shape) if name.startswith("out_") else t.clone() for name, t in kw_of(step, r).items()}
+        call(r, kw)
+        for t in kw.values():
+            before, other = t.data_ptr(), torch.full_like(t.view(torch.uint8), 255).view(t.dtype)
+            if through_op and change is _swap:
+                with pytest.raises(RuntimeError):
+                    change(t, other)
+                assert t.data_ptr() == before
+            else:
+                change(t, other)
+                assert t.data_ptr() != before
+            del other
+            kept += [t, torch.full_like(t.view(torch.uint8), 255)]  # (in the place of memory that had been given back)
+    call(spec.world_size - 1, kw_of(step, spec.world_size - 1))
+    if op == "dispatch":
+        check_dispatch_against_oracle(step)
+    else:
+        check_combine_against_oracle(step, expected.slot_map)
+    for a in ranks:
+        a.destroy()
+
+
+@pytest.mark.parametrize("last_through_op", [False, True])
+@pytest.mark.parametrize("scales", [False, True])
+@pytest.mark.parametrize("op", ["dispatch", "combine"])
+def test_every_temporary_input_outlives_its_caller(op, scales, last_through_op):
+    """All inputs of the ranks that call early are temporaries, with optional ones left out or not: none goes before the
+    step's last call, whatever takes the place of memory that was given back."""
+    import weakref
+
+    spec = _small_spec(name="temporaries", in_dtype=FP8 if scales else torch.bfloat16, hidden_dim=512)
+    step = DeviceStep(spec, generate(spec))
+    ranks = _make_ranks(spec, "temporaries")
+    R = spec.world_size
+    if op == "combine":
+        for r in range(R):
+            ranks[r].dispatch(**_dispatch_kw(step, r))
+        expected = check_dispatch_against_oracle(step)
+        step.expert_y_all.normal_()
+    refs, gone, fillers = [], [], []
+
+    def call(r: int, through_op: bool) -> list[int]:
+        kw = (_dispatch_kw if op == "dispatch" else _combine_kw)(step, r)
+        for name, t in kw.items():
+            if t is not None and not name.startswith("out_"):
+                kw[name] = t.clone()
+                refs.append(weakref.ref(kw[name], lambda _: gone.append(r)))
+        if through_op:
+            getattr(torch.ops.pplx_kernels, f"all_to_all_intranode_{op}")(ranks[r]._ptr, *kw.values(), True, True)
+        else:
+            getattr(ranks[r], op)(**kw)
+        return [t.numel() * t.element_size() for t in kw.values() if t is not None]
+
+    for r in range(R - 1):
+        for nbytes in call(r, r % 2 == 0):
+            fillers.append(torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda"))
+        assert not gone
+    call(R - 1, last_through_op)
+    assert len(gone) == len(refs) == R * (4 if op == "combine" or scales else 3)
+    if op == "dispatch":
+        check_dispatch_against_oracle(step)
+    else:
+        check_combine_against_oracle(step, expected.slot_map)
+    for a in ranks:
+        a.destroy()
+
+
 def test_a_step_is_abandoned_when_a_rank_is_refused():
     """Rank 2's arguments fail their checks after ranks 0 and 1 have called: the half-assembled
     step is given up (nothing of it has reached the GPU), the tensors kept for it are let go,

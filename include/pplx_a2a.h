@@ -251,6 +251,8 @@ typedef struct pplx_a2a_combine_plan {
   int32_t per_group;
 } pplx_a2a_combine_plan_t;
 int pplx_a2a_combine_plan(const pplx_a2a_config_t *cfg, int in_dtype, pplx_a2a_combine_plan_t *out);
+/* Whether combine stores the rows of a step plainly (1) or past the caches (0). */
+int pplx_a2a_combine_stores(const pplx_a2a_config_t *cfg, int32_t *plain);
 
 /* Parts of a step for pplx_a2a_world_abandon_step. */
 #define PPLX_A2A_ABANDON_DISPATCH 1u

@@ -1269,6 +1269,15 @@ int pplx_a2a_combine_plan(const pplx_a2a_config_t *cfg, int in_dtype, pplx_a2a_c
   return PPLX_A2A_OK;
 }
 
+int pplx_a2a_combine_stores(const pplx_a2a_config_t *cfg, int32_t *plain) {
+  if (!cfg || !plain) return fail(PPLX_A2A_INVALID_ARGUMENT, "cfg / plain is NULL");
+  if (int st = check_config(*cfg)) return st;
+  WorldHost d{};
+  fill_geometry(*cfg, d);
+  *plain = combine_stores_plainly(d);
+  return PPLX_A2A_OK;
+}
+
 int pplx_a2a_world_faults(pplx_a2a_world_t *w, void *stream, uint32_t *out_bits) {
   if (!w || !out_bits) return fail(PPLX_A2A_INVALID_ARGUMENT, "world / out_bits is NULL");
   DeviceScope scope(w->device);

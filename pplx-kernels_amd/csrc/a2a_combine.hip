@@ -281,11 +281,15 @@ bool combine_per_group(const WorldHost &w, size_t elem_bytes) {
 // plain: 2968 wide, 8 x 16 tokens 7.3 / 7.0, 8 x 64 8.6 / 8.3, 8 x 128 (5.8 MiB) 11.3 / 10.8; 5384 wide, 8 x 64 (5.3 MiB) 10.9 / 10.4;
 // 2008 wide, top-4, 8 x 128 12.2 / 11.8; groups of two, top-3, 2968 wide, 8 x 100 9.9 / 9.6 (45 shapes of groups of two 0.97).
 // Beyond, the lines that stay behind cost what follows more than that: plain stores for 5384 wide, top-4, 8 x 200 34.5 / 37.8, 7176
-// wide, top-2, 8 x 256 35.2 / 40.8.  Rows of whole half lines are level in small steps.  (The same in dispatch, plain instead of
+// wide, top-2, 8 x 256 35.2 / 40.8.  Both kinds of store over 488 to 7176 wide rows, top-1 to top-8, groups of one, two and four, plain
+// over streaming, mean (lowest to highest): 252 steps of 1 to 5.9 MiB 0.977 (0.943 to 1.019; top-8 0.98), 48 of 6.2 and 7 MiB 0.985 (to
+// 1.016), 60 of 8 MiB 0.999 (0.969 to 1.043), 24 of 10 MiB 1.002 (to 1.058), 60 of 12 MiB 1.007 (to 1.084), 48 of 16 and 24 MiB 1.013
+// (to 1.116): 6 MiB is where the worst of them begin to lose.  Rows are counted for every rank, present or not, as in all
+// rules here.  Rows of whole half lines are level in small steps.  (The same in dispatch, plain instead of
 // written-through stores, gives 2 % of the smallest steps and costs 6 % at 8 x 128 tokens; pieces that begin at half lines of the
 // output instead of the row's start gave nothing in large steps.)
 constexpr uint64_t kPlainStoresMaxBytes = 6ull << 20;
-bool plain_stores(const WorldHost &w) {
+bool plain_stores(const WorldDev &w) {
   const uint64_t row = 2ull * w.H;
   return row % 64 != 0 && (uint64_t)w.R * w.M * row <= kPlainStoresMaxBytes;
 }
@@ -493,6 +497,7 @@ int launch_combine_t(const WorldHost &w, const CT &tab, int in_dtype, int out_dt
 }  // namespace
 
 CombineForm combine_form(const WorldHost &w, int in_dtype) { return combine_form_of(w, in_dtype == 0 ? 4 : 2); }
+bool combine_stores_plainly(const WorldHost &w) { return plain_stores(w); }
 
 int launch_combine(const WorldHost &w, const CombineRank *inline_rows, int in_dtype, int out_dtype,
                    void *stream) {

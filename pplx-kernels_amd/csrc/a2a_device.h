@@ -293,6 +293,8 @@ struct CombineForm {
   bool per_group;
 };
 CombineForm combine_form(const WorldHost &w, int in_dtype);
+// Whether it stores the combined rows plainly, not past the caches.
+bool combine_stores_plainly(const WorldHost &w);
 // LDS bytes the routing kernels need for a given geometry.
 uint32_t route_lds_bytes(uint32_t num_experts, uint32_t tile_chunks);
 

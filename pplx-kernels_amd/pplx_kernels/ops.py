@@ -57,6 +57,7 @@ EXPORTED_SYMBOLS = (
     "pplx_a2a_plan",
     "pplx_a2a_plan_on",
     "pplx_a2a_combine_plan",
+    "pplx_a2a_combine_stores",
     "pplx_a2a_bound_bytes",
     "pplx_a2a_bound_create",
     "pplx_a2a_bound_launch",
@@ -199,6 +200,7 @@ def load_library() -> ctypes.CDLL:
             ctypes.POINTER(Config), i32, u32, ctypes.POINTER(Plan), ctypes.POINTER(i32),
         ]  # fmt: skip
         lib.pplx_a2a_combine_plan.argtypes = [ctypes.POINTER(Config), i32, ctypes.POINTER(CombinePlan)]
+        lib.pplx_a2a_combine_stores.argtypes = [ctypes.POINTER(Config), ctypes.POINTER(i32)]
         lib.pplx_a2a_world_of.argtypes = [vp]
         lib.pplx_a2a_world_of.restype = vp
         lib.pplx_a2a_world_recorded_calls.argtypes = [vp, i32, i32, ctypes.POINTER(u32)]
@@ -245,6 +247,13 @@ def combine_plan_of(config: Config, y_dtype: torch.dtype = torch.bfloat16) -> tu
         load_library().pplx_a2a_combine_plan(ctypes.byref(config), DTYPE_CODE[y_dtype], ctypes.byref(plan))
     )
     return plan.picks, plan.pieces, bool(plan.per_group)
+
+
+def combine_stores_plainly(config: Config) -> bool:
+    """Whether combine stores the rows of a step of this geometry plainly, not past the caches (no GPU needed)."""
+    plain = ctypes.c_int32()
+    check_status(load_library().pplx_a2a_combine_stores(ctypes.byref(config), ctypes.byref(plain)))
+    return bool(plain.value)
 
 
 def check_status(status: int) -> None:

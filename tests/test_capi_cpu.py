@@ -295,6 +295,39 @@ def test_one_launch_dispatch_with_a_short_table_leaves_the_same_room():
     assert len(short) == 3 and all(v <= 64 for v in short.values()), short
 
 
+def test_combine_kernels_hold_both_kinds_of_store(tmp_path):
+    """The gathers of combine store as they are told at the launch, past the caches or plainly.  The compiler makes one
+    store of two that differ in nothing else, unless something keeps them apart: each kernel has as many of either."""
+    import struct
+    import subprocess
+
+    objdump = "/opt/rocm/llvm/bin/llvm-objdump"
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
+    data = open(ops._LIB_PATH, "rb").read()
+    stores: dict[str, list[str]] = {}
+    pos = data.find(b"\x7fELF")
+    while pos >= 0:
+        if data[pos + 4] == 2 and struct.unpack_from("<H", data, pos + 18)[0] == 224:  # ELF64, EM_AMDGPU
+            (e_shoff,) = struct.unpack_from("<Q", data, pos + 0x28)
+            e_shentsize, e_shnum = struct.unpack_from("<HH", data, pos + 0x3A)
+            code = data[pos : pos + e_shoff + e_shentsize * e_shnum]
+            if b"combine_gather" in code:
+                path = tmp_path / f"{pos}.co"
+                path.write_bytes(code)
+                kernel = None
+                for line in subprocess.run([objdump, "-d", path], capture_output=True, text=True, check=True).stdout.splitlines():
+                    if line.endswith(">:"):
+                        kernel = line.split("<")[1][:-2]
+                    elif "global_store" in line and "combine_gather" in kernel:
+                        stores.setdefault(kernel, []).append(line.split("//")[0])
+        pos = data.find(b"\x7fELF", pos + 4)
+    assert len(stores) > 100
+    for kernel, lines in stores.items():
+        streaming = sum(line.rstrip().endswith(" nt") for line in lines)
+        assert streaming > 0 and 2 * streaming == len(lines), (kernel, lines)
+
+
 def test_bench_refuses_more_than_one_gpu():
     """Every simulated rank shares one GPU's HBM: `bench.py --gpus N` with N above 1 (or under a
     launcher that sets WORLD_SIZE) exits with a message that says so, before it touches a GPU."""

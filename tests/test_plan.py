@@ -243,6 +243,28 @@ def test_pieces_of_combine(tokens, topk, hidden, dtype, dp, picks, pieces):
 
 
 @pytest.mark.parametrize(
+    "M,H,K,dp,plain",
+    [
+        (1, 8, 1, 1, True),
+        (9, 992, 6, 1, False),  # whole half lines
+        (9, 984, 6, 1, True),
+        (9, 1000, 6, 1, True),
+        (393, 1000, 2, 1, True),  # 8 x 393 x 2000 bytes, 3456 below 6 MiB
+        (394, 1000, 2, 1, False),
+        (393, 1000, 2, 2, True),  # each rank of a group stores rows of its own
+        (394, 1000, 2, 2, False),
+        (393, 1000, 2, 4, True),
+        (394, 1000, 2, 4, False),
+        (4096, 96, 8, 1, False),  # 6 MiB of whole half lines
+        (16384, 24, 8, 1, True),  # 6 MiB of rows of 48 bytes
+        (16385, 24, 8, 1, False),
+    ],
+)
+def test_stores_of_combine(M, H, K, dp, plain):
+    assert ops.combine_stores_plainly(ops.Config(M, 32, K, 8, dp, H, 2 * H, 0)) == plain
+
+
+@pytest.mark.parametrize(
     "lds,tokens,row,topk,one_launch",
     [
         # 8 x 2 rows of 12 KiB and the tables beside them fit any device's LDS, sixteen rows of 10128 bytes only

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "a2a_device.h"
+#include "a2a_device_scope.h"
 #include "pplx_a2a.h"
 
 // Profiler ranges around the launch sequences, like the reference's nvtxRangePush("dispatch") /
@@ -79,34 +80,6 @@ class ProfilerRange {
   }
   ProfilerRange(const ProfilerRange &) = delete;
   ProfilerRange &operator=(const ProfilerRange &) = delete;
-};
-
-// Restores the caller's current device on scope exit.  A process that sees one device has no other: asking for the
-// current one would cost each launch 55 ns.
-class DeviceScope {
- public:
-  explicit DeviceScope(int device) {
-    static const bool single = [] {
-      int n = 0;
-      return hipGetDeviceCount(&n) == hipSuccess && n == 1;
-    }();
-    if (single && device == 0) {
-      ok_ = true;
-      return;
-    }
-    ok_ = hipGetDevice(&prev_) == hipSuccess;
-    if (ok_ && prev_ != device) ok_ = hipSetDevice(device) == hipSuccess;
-    switched_ = ok_ && prev_ != device;
-  }
-  ~DeviceScope() {
-    if (switched_) (void)hipSetDevice(prev_);
-  }
-  bool ok() const { return ok_; }
-
- private:
-  int prev_ = 0;
-  bool ok_ = false;
-  bool switched_ = false;
 };
 
 }  // namespace

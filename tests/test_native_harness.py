@@ -33,3 +33,12 @@ def test_division_helper_of_the_kernels_matches_integer_division():
     the hardware's division on millions of (numerator, divisor) pairs.  Needs no GPU."""
     proc = subprocess.run([BIN, "--host-only"], capture_output=True, text=True, timeout=120)
     assert proc.returncode == 0 and "pass [fast_div" in proc.stdout, proc.stdout[-2000:] + proc.stderr[-2000:]
+
+
+@pytest.mark.parametrize("devices", [-1, 0, 1, 2, 3])
+def test_device_scope(devices):
+    """The library selects a world's device around each call and restores the caller's; a process that sees one device
+    is not asked.  One device is all that the GPU tests see."""
+    exe = os.path.join(os.path.dirname(BIN), "test_device_scope")
+    proc = subprocess.run([exe, str(devices)], capture_output=True, text=True, timeout=60)
+    assert proc.returncode == 0 and "ALL PASSED" in proc.stdout, proc.stdout[-2000:] + proc.stderr[-2000:]

@@ -15,8 +15,9 @@ namespace {
 
 // Launches `kernel` on arguments of its parameters' own types (or types derived from them) and returns a hipError_t as
 // int.  By hipLaunchKernel, which takes the addresses of the arguments, and not by <<<>>>: that copies every argument into
-// its stub, a rank table of 9 KiB twice, and passes the launch's shape by a stack of the thread's.  Host time of a launch,
-// us, <<<>>> / this: 104 bytes of arguments 2.45 / 2.25, 176 bytes 2.97 / 2.76, 9 KiB 3.41 / 3.16.
+// its stub, a rank table of 9 KiB twice, and passes the launch's shape by a stack of the thread's.  Host time of a launch
+// (bench_launch), us, <<<>>> / this, which differs between processes: 104 bytes of arguments 2.29 / 2.13 or 2.68 / 2.56, 176 bytes
+// 2.31 / 2.17 or 3.53 / 3.40, 1240 bytes 2.38 / 2.24 or 4.09 / 3.95, 9304 bytes 2.95 / 2.70 or 4.01 / 3.87.
 template <typename P, typename A> const void *argument(const A &a) {
   static_assert(std::is_same_v<P, A> || std::is_base_of_v<P, A>, "an argument that would be converted");
   return static_cast<const P *>(&a);

@@ -88,7 +88,7 @@ struct alignas(16) CombineRank {
 static_assert(sizeof(CombineRank) == 80, "CombineRank layout");
 
 // Geometry + scratch of a world; passed to every kernel by value, and kept short: in some processes a launch with more
-// than kShortArguments bytes of arguments costs the host 2.75 us and more instead of 2.25 (9 KiB 3.15).  Beside a
+// than kShortArguments bytes of arguments costs the host 3.4 to 3.95 us instead of 2.55 (in the others 2.2, 9 KiB 2.7).  Beside a
 // table in HBM the one-launch dispatch, the scatters and the gather of combine stay within them; the routing kernels, whose
 // RouteSpan alone is 56 bytes, do not.
 constexpr size_t kShortArguments = 112;
@@ -210,9 +210,10 @@ inline StageLayout stage_layout(uint32_t row_bytes, uint32_t scales, uint64_t to
 // 3.27 / 2.87; 64 x 1 DSv3 tokens 5.53 / 5.26 and 4.01 / 3.58; 8 x 128 12.69 / 12.51 and 22.12 / 21.90.
 constexpr uint32_t kInlineRanks = 64;
 // A table of up to this many ranks goes in an argument of that size (1152 bytes for dispatch, 640 for combine) and not in
-// one for kInlineRanks: what a launch costs the host grows with its arguments (2.27 us at 1240 bytes, 2.49 at 9304), which
-// are filled and copied besides.  Steps, us, 64 ranks' room / this: 8 x 4 tokens, per-rank calls 18.2 / 17.2; 4 ranks in
-// groups of two, 20 tokens, one call 9.2 / 8.5; 8 x 128, split 37.6 / 35.1.  Eight is what a node holds.
+// one for kInlineRanks, which is filled and copied at each launch and costs more to launch in processes where that grows
+// with the arguments (2.24 us at 1240 bytes, 2.70 at 9304; in the others both take 3.9).  Steps, us, 64 ranks' room / this:
+// 8 x 4 tokens, per-rank calls 18.2 / 17.2; 4 ranks in groups of two, 20 tokens, one call 9.2 / 8.5; 8 x 128, split
+// 37.6 / 35.1.  Eight is what a node holds.  (A third kind of table makes the library 8.1 MB instead of 5.5.)
 constexpr uint32_t kShortInlineRanks = 8;
 constexpr uint32_t kBindBatch = 64;
 // A one-launch dispatch whose rows (all picks of all tokens) stay within this many bytes and go through registers

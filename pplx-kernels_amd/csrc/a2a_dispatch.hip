@@ -474,7 +474,8 @@ template <int NV, bool EXACT, class DT, bool MANY>
 __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused(WorldDev w, DT tab, FusedShape shape) {
   dispatch_in_one<NV, EXACT, DT, MANY>(w, tab, shape);
 }
-// ... with a table of few ranks among the arguments
+// ... with a table of few ranks among the arguments.  The same code, which the table's type alone would tell apart: the name of
+// its own is for what counts the built library's kernels by name (the registers of the short rows' forms).
 template <int NV, bool EXACT, class DT, bool MANY>
 __global__ __launch_bounds__(fused_threads(NV)) void dispatch_fused_few(WorldDev w, DT tab, FusedShape shape) {
   dispatch_in_one<NV, EXACT, DT, MANY>(w, tab, shape);

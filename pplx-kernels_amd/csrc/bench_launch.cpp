@@ -1,18 +1,24 @@
 // What a launch costs on the GPU at hand, whatever the kernel does: the floor under the latency
 // of the decode-sized steps, whose two kernels run for 4-6 us each.
 //
-// Empty kernels (one workgroup, and 256 workgroups of 1024 threads; with 64 bytes and with 9 KiB
-// of kernel arguments, the size of an inline rank table) are timed three ways, back to back on one
-// stream: eager launches, replays of a captured graph holding one such kernel, and replays of a
-// graph holding two.  Two figures per line: microseconds per launch (or replay) on the GPU's
-// side, from HIP events around the whole batch, and microseconds of host time per call.
+// Empty kernels of 256 workgroups of 1024 threads are launched as the library launches its own
+// (launch_kernel), with as many bytes of arguments as its kernels have: 104 beside a table in
+// device memory, 176 in the routing, 1240 with a rank table of up to eight ranks, 9304 with one of
+// 64.  They are timed three ways, back to back on one stream: eager launches, replays of a
+// captured graph holding one such kernel, and replays of a graph holding two.  Two figures per
+// line: microseconds per launch (or replay) on the GPU's side, from HIP events around the whole
+// batch, and microseconds of host time per call.  Then the host time of an eager launch again,
+// by launch_kernel and by <<<>>> in turn, the median of nine batches of each.
 //
 //   bench_launch [batch]       (default 2000 launches per figure)
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
+
+#include "a2a_common.h"
 
 #define HIP_OK(expr)                                                                       \
   do {                                                                                     \
@@ -23,11 +29,8 @@
     }                                                                                      \
   } while (0)
 
-struct SmallArgs {
-  unsigned long long v[8];
-};
-struct TableArgs {
-  unsigned long long v[1152];  // 9 KiB, an inline table of 64 ranks
+template <int BYTES> struct Arguments {  // (beside the pointer)
+  unsigned long long v[BYTES / 8 - 1];
 };
 
 template <class Args>
@@ -63,7 +66,9 @@ Figure time_batch(hipStream_t stream, int batch, Launch launch) {
 template <class Args>
 void run(const char *what, dim3 grid, dim3 block, hipStream_t stream, int batch, unsigned long long *sink) {
   Args args{};
-  auto eager = [&] { hipLaunchKernelGGL(empty_kernel<Args>, grid, block, 0, stream, args, sink); };
+  auto eager = [&] {
+    HIP_OK((hipError_t)pplx_amd::launch_kernel(empty_kernel<Args>, grid, block, 0, stream, args, sink));
+  };
   const Figure e = time_batch(stream, batch, eager);
   Figure g[2];
   for (int nodes = 1; nodes <= 2; ++nodes) {
@@ -83,6 +88,27 @@ void run(const char *what, dim3 grid, dim3 block, hipStream_t stream, int batch,
          e2.host_us, g[0].gpu_us, g[0].host_us, g[1].gpu_us, g[1].host_us);
 }
 
+// Host time of an eager launch, either way.
+template <class Args>
+void compare(hipStream_t stream, int batch, unsigned long long *sink) {
+  constexpr int kBatches = 9;
+  const dim3 grid(256), block(1024);
+  Args args{};
+  double ours[kBatches], theirs[kBatches];
+  for (int i = 0; i < kBatches; ++i) {
+    ours[i] = time_batch(stream, batch, [&] {
+                HIP_OK((hipError_t)pplx_amd::launch_kernel(empty_kernel<Args>, grid, block, 0, stream, args, sink));
+              }).host_us;
+    theirs[i] = time_batch(stream, batch, [&] {
+                  empty_kernel<Args><<<grid, block, 0, stream>>>(args, sink);
+                }).host_us;
+  }
+  std::sort(ours, ours + kBatches);
+  std::sort(theirs, theirs + kBatches);
+  printf("%6zu bytes   launch_kernel %6.2f   <<<>>> %6.2f\n", sizeof(Args) + sizeof(sink), ours[kBatches / 2],
+         theirs[kBatches / 2]);
+}
+
 int main(int argc, char **argv) {
   const int batch = argc > 1 ? atoi(argv[1]) : 2000;
   int n_dev = 0;
@@ -99,10 +125,15 @@ int main(int argc, char **argv) {
          batch);
   printf("%-44s %17s   %17s   %17s   %17s\n", "kernel", "1 eager launch", "2 eager launches", "graph of 1 node",
          "graph of 2 nodes");
-  run<SmallArgs>("1 workgroup x 64, 64 B of arguments", dim3(1), dim3(64), stream, batch, sink);
-  run<SmallArgs>("256 workgroups x 1024, 64 B of arguments", dim3(256), dim3(1024), stream, batch, sink);
-  run<TableArgs>("1 workgroup x 64, 9 KiB of arguments", dim3(1), dim3(64), stream, batch, sink);
-  run<TableArgs>("256 workgroups x 1024, 9 KiB of arguments", dim3(256), dim3(1024), stream, batch, sink);
+  run<Arguments<104>>("104 bytes of arguments", dim3(256), dim3(1024), stream, batch, sink);
+  run<Arguments<176>>("176 bytes of arguments", dim3(256), dim3(1024), stream, batch, sink);
+  run<Arguments<1240>>("1240 bytes of arguments", dim3(256), dim3(1024), stream, batch, sink);
+  run<Arguments<9304>>("9304 bytes of arguments", dim3(256), dim3(1024), stream, batch, sink);
+  printf("\nhost us per eager launch\n");
+  compare<Arguments<104>>(stream, batch, sink);
+  compare<Arguments<176>>(stream, batch, sink);
+  compare<Arguments<1240>>(stream, batch, sink);
+  compare<Arguments<9304>>(stream, batch, sink);
   HIP_OK(hipFree(sink));
   HIP_OK(hipStreamDestroy(stream));
   return 0;

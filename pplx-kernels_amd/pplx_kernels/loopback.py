@@ -6,7 +6,7 @@ hand all ranks' tensors over at once; the library then makes one pass over them
 (``pplx_a2a_world_dispatch`` / ``pplx_a2a_world_combine``).  The kernels, the results and
 the argument checks are the same as for ``world_size`` per-rank calls.  The checks, the packing
 and the launch run in compiled code: packed in Python, a step of four ranks took 33 us of host
-time for 10 us of kernels (now 8.5 us a step), and a bound step 13 us (now 9).
+time for 10 us of kernels (now 9 us a step), and a bound step 13 us (now 9).
 
 ``capture()`` records whatever the body enqueues on the current stream into a hipGraph
 through the library's own capture entry points, so a step can be replayed without any
